@@ -102,10 +102,13 @@ extern "C" int dsim_waveforms_create(dsim_sim *sim, uint32_t n_wave, uint32_t n_
         delete W;
         return rc;
     }
-    // padded trajectory columns stay zero; phases start at zero
-    hipError_t e = hipMemset(W->traj.p, 0, W->traj.n * 4);
-    if (e == hipSuccess) e = hipMemset(W->phase.p, 0, nw * 4);
-    if (e == hipSuccess) e = hipMemset(W->comp.p, 0, W->comp.n * 4);
+    // padded trajectory columns stay zero; phases start at zero.  Cleared on
+    // the handle's stream, before the walk it records: hipMemset returns before
+    // the device is done and does not order with that (non-blocking) stream.
+    hipStream_t st = dsim_host::sim_stream(sim);
+    hipError_t e = hipMemsetAsync(W->traj.p, 0, W->traj.n * 4, st);
+    if (e == hipSuccess) e = hipMemsetAsync(W->phase.p, 0, nw * 4, st);
+    if (e == hipSuccess) e = hipMemsetAsync(W->comp.p, 0, W->comp.n * 4, st);
     if (e != hipSuccess) {
         delete W;
         return fail(DSIM_ERR_HIP, "waveform init: %s", hipGetErrorString(e));
@@ -123,8 +126,8 @@ extern "C" int dsim_waveforms_set_buffer(dsim_waveforms *W, uint32_t buffer_step
     HIP_TRY(hipStreamSynchronize(dsim_host::sim_stream(W->sim)));
     W->traj.release();
     if (int rc = W->traj.alloc((size_t)3 * buffer_steps * W->n_pad)) return rc;
-    // padded trajectory columns stay zero
-    HIP_TRY(hipMemset(W->traj.p, 0, W->traj.n * 4));
+    // padded trajectory columns stay zero (cleared in the walk's stream order)
+    HIP_TRY(hipMemsetAsync(W->traj.p, 0, W->traj.n * 4, dsim_host::sim_stream(W->sim)));
     W->buffer = buffer_steps;
     return DSIM_OK;
 }

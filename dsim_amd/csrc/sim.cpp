@@ -182,11 +182,11 @@ static int sync_and_check(dsim_sim *s) {
     uint32_t fl[4] = {0, 0, 0, 0};
     HIP_TRY(hipMemcpy(fl, s->flags.p, 16, hipMemcpyDeviceToHost));
     if (fl[0] & 1u) {
-        HIP_TRY(hipMemset(s->flags.p, 0, 16));
+        HIP_TRY(hipMemsetAsync(s->flags.p, 0, 16, s->stream));
         return fail(DSIM_ERR_OVERFLOW, "a spin exceeded 4096 collisions in one step");
     }
     if (fl[0] & 4u) {
-        HIP_TRY(hipMemset(s->flags.p, 0, 16));
+        HIP_TRY(hipMemsetAsync(s->flags.p, 0, 16, s->stream));
         return fail(DSIM_ERR_STATE, "collision search numbered a grid entry out of range");
     }
     return DSIM_OK;
@@ -238,7 +238,8 @@ extern "C" int dsim_set_state_aos(dsim_sim *s, const float *pos, const dsim_spin
         HIP_TRY(hipMemcpy(s->ff(F_X), a.data(), n * 4, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(s->ff(F_Y), b.data(), n * 4, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(s->ff(F_Z), c.data(), n * 4, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemset(s->f(F_WRAP), 0, (size_t)n * 4));  // new positions: no crossings yet
+        // new positions: no crossings yet (in stream order with the next walk)
+        HIP_TRY(hipMemsetAsync(s->f(F_WRAP), 0, (size_t)n * 4, s->stream));
     }
     if (spins) {
         std::vector<float> m(n), ph(n);

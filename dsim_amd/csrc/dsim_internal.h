@@ -29,10 +29,21 @@ struct StepParams {
     const float4 *tri_mt;
     const uint32_t *cell_start;
     const uint32_t *cell_tri;
-    const float4 *cell_plane;  // plane (n, n.v0) of cell_tri[k], cell-major
-    const float4 *cell_mt;     // [3] per entry: v0 (w: triangle index), e1, e2
-    uint32_t n_entries;        // length of cell_tri and cell_plane
-    const float *cell_clear;   // per-cell distance lower bound, or null (no skipping)
+    // search lists of the walk: entry k of cell c, walk_start[c] <= k <
+    // walk_start[c + 1], is the triangles walk_ent[k] (.y kNone: one only) of
+    // one plane; walk_rec holds two records per entry (walk_cell_major) or per
+    // triangle: the plane (n, n.v0) and the lateral bound (see walk_test)
+    const uint32_t *walk_start;
+    const uint2 *walk_ent;
+    const float4 *walk_rec;
+    uint32_t walk_cell_major;
+    float walk_eps;
+    // per fine cell, a lower bound of the distance to any triangle in units of
+    // fine_q, or null (no skipping); fine_w is 0 on axes of one cell, which the
+    // distance leaves out, and 1 on the others
+    const uint8_t *fine;
+    uint32_t fine_dims[3];
+    float fine_inv[3], fine_w[3], fine_q;
     const uint8_t *fiber_myelin;
     uint32_t n_fibers;
     uint32_t dims[3];
@@ -58,10 +69,10 @@ struct StepParams {
     float *disp;      // [3][n] unwrapped displacement
     float *mom;       // [3][n] moment
     float *momc;      // [3][n] Kahan compensation
-    uint32_t *hits;   // membrane hits per spin since the last reorder, or null
+    uint32_t *searches;  // collision searches per spin since the last reorder, or null
     uint32_t *wrap;   // periodic voxel crossings per spin (three signed 10-bit counts), used
                       // for the phase of the unwrapped position when moments are off
-    uint32_t hit_window;  // steps those counts cover (0: no history)
+    uint32_t search_window;  // steps those counts cover (0: no history)
     float *traj;          // displacement after each step of the launch by spin id, in
                           // tiles of kTrajTile spins: k = 3 * step + axis of spin s at
                           // [s / kTrajTile][k / kTrajChunk][s % kTrajTile][k % kTrajChunk]
@@ -73,7 +84,7 @@ struct StepParams {
     uint64_t step0;
     const float4 *inject;  // [iters][n]
     uint32_t *trace;       // [iters][n][5]
-    uint32_t *flags;       // status word: bit 0 collision loop guard hit, bit 2 entry out of range
+    uint32_t *flags;       // status word: bit 0 collision loop guard hit
     unsigned long long *stats;  // [kWalkStats] work counters (counting build of the walk)
     uint32_t *queue;       // [8] slot counters of the persistent walk, or null (fixed blocks)
     uint32_t queue_run;    // slots per queue run (persistent walk; set at launch)
@@ -125,7 +136,6 @@ constexpr uint32_t kMaxJobs = 256;
 // Spins per workgroup of the physical-mode step kernels (k_walk and
 // k_walk_batch): one wave.
 constexpr uint32_t kWalkBlockSpins = 64;
-
 struct WalkJob {
     StepParams p;
     uint32_t iters;

@@ -14,15 +14,16 @@
 //                   per-cell counts
 //   radix sort      stable by cell: lists in ascending triangle order
 //   exclusive scan  of the counts -> cell_start
-//   k_cell_records  cell-major plane and triangle records
 //   k_ring_*        Chebyshev ring distance to the nearest occupied cell
 //   k_clearance     the clearance of each cell
+//   build_walk_tables  the walk's search lists and fine clearance (both builds)
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_reduce.hpp>
 #include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <vector>
@@ -280,22 +281,6 @@ __global__ __launch_bounds__(kBlock) void k_pairs(Geom g, uint32_t n_tri, const 
     }
 }
 
-// Per grid entry in cell order: the plane of its triangle, and v0 (with the
-// triangle index in .w), e1, e2 of its Moller-Trumbore record.
-__global__ __launch_bounds__(kBlock) void k_cell_records(uint32_t n_entries, const uint32_t *tri,
-                                                         const float4 *mt, float4 *plane,
-                                                         float4 *cm) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n_entries) return;
-    const uint32_t t = tri[k];
-    const float4 *r = mt + (size_t)t * 4;
-    plane[k] = r[0];
-    const float4 v0 = r[1];
-    cm[(size_t)k * 3 + 0] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(t));
-    cm[(size_t)k * 3 + 1] = r[2];
-    cm[(size_t)k * 3 + 2] = r[3];
-}
-
 __global__ __launch_bounds__(kBlock) void k_ring_init(uint32_t n_cells, const uint32_t *start,
                                                       uint32_t *ring) {
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
@@ -410,9 +395,369 @@ __global__ __launch_bounds__(kBlock) void k_clearance(Geom g, const uint32_t *ri
     out[c] = float_sqrt_floor(best2);
 }
 
+// Fine clearance: the walk completes a step from o to p without a search when
+// the clearances of the fine cells of o and p add up to more than the step's
+// length (the two balls cover the segment).  Each byte is the distance from
+// its fine cell to the nearest triangle of the grid, rounded down to a
+// multiple of q after taking off the margin for the walk's float arithmetic.
+//
+// The distance comes from the exact point-triangle distance of the cell's
+// centre, less the cell's half diagonal, over the triangles listed in the 3^k
+// grid cells around it (a triangle listed in none of them is no nearer than
+// the edge of that block), or from the grid's own clearance where that is
+// larger.  On an axis of one cell every distance is taken in the projection
+// along it: the bound then holds whatever the coordinate on that axis, and a
+// step's length leaves the axis out.
+struct FineGeom {
+    uint32_t sub[3];    // fine cells per grid cell and axis (1 on collapsed axes)
+    uint32_t dims[3];   // fine cells per axis
+    float cell[3];      // fine cell edge
+    float w[3];         // 0 on collapsed axes
+    float half_diag, q;
+};
+constexpr float kFineMargin = 1e-5f;  // covers FP32 rounding of positions, distances and lookups
+constexpr float kFineRange = 32.0f;   // q = grid cell / kFineRange: bytes reach 8 grid cells
+
+struct D3 {
+    double x, y, z;
+};
+__device__ __forceinline__ D3 operator-(D3 a, D3 b) { return D3{a.x - b.x, a.y - b.y, a.z - b.z}; }
+__device__ __forceinline__ double dotv(D3 a, D3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__device__ __forceinline__ D3 cross3(D3 a, D3 b) {
+    return D3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+}
+// Squared distance of r (point - a) from the segment a + t e.
+__device__ __forceinline__ double seg_dist2(D3 r, D3 e) {
+    const double ee = dotv(e, e);
+    const double t = ee > 0.0 ? fmin(fmax(dotv(r, e) / ee, 0.0), 1.0) : 0.0;
+    const D3 d = D3{r.x - t * e.x, r.y - t * e.y, r.z - t * e.z};
+    return dotv(d, d);
+}
+
+// Squared distance of point c from the triangle with record m, in the
+// projection w: the nearest of the three edges, or the plane's where the
+// point projects into the triangle or within the margin of it.  In double and
+// from the edges the walk tests (the normal of a long thin triangle is off by
+// more than the margin in FP32); a degenerate triangle is its edges.
+__device__ double tri_dist2(const float4 *__restrict__ m, D3 c, D3 w) {
+    const float4 v4 = m[1], a4 = m[2], b4 = m[3];
+    const D3 e1 = D3{a4.x * w.x, a4.y * w.y, a4.z * w.z};
+    const D3 e2 = D3{b4.x * w.x, b4.y * w.y, b4.z * w.z};
+    const D3 r = D3{(c.x - v4.x) * w.x, (c.y - v4.y) * w.y, (c.z - v4.z) * w.z};
+    const D3 e3 = e2 - e1, r1 = r - e1;
+    double d2 = fmin(fmin(seg_dist2(r, e1), seg_dist2(r, e2)), seg_dist2(r1, e3));
+    const D3 n = cross3(e1, e2);
+    const double nn = dotv(n, n);
+    if (nn > 0.0) {
+        const double k = -(double)kFineMargin * sqrt(nn);
+        if (dotv(n, cross3(e1, r)) >= k * sqrt(dotv(e1, e1)) &&
+            dotv(n, cross3(r, e2)) >= k * sqrt(dotv(e2, e2)) &&
+            dotv(n, cross3(e3, r1)) >= k * sqrt(dotv(e3, e3))) {
+            const double h = dotv(n, r);
+            d2 = fmin(d2, h * h / nn);
+        }
+    }
+    return d2;
+}
+
+__global__ __launch_bounds__(kBlock) void k_fine_clearance(Geom g, FineGeom f,
+                                                           const uint32_t *__restrict__ start,
+                                                           const uint32_t *__restrict__ tri,
+                                                           const float4 *__restrict__ mt,
+                                                           const float *__restrict__ coarse,
+                                                           uint8_t *__restrict__ out) {
+    const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (uint64_t)f.dims[0] * f.dims[1] * f.dims[2]) return;
+    const uint32_t fx = (uint32_t)(i % f.dims[0]), fy = (uint32_t)(i / f.dims[0] % f.dims[1]),
+                   fz = (uint32_t)(i / ((uint64_t)f.dims[0] * f.dims[1]));
+    const uint32_t fi[3] = {fx, fy, fz};
+    int32_t c[3], a0[3], a1[3];
+    float edge = 3.0e38f, ctr[3];
+    bool inner = true;
+    for (int k = 0; k < 3; ++k) {
+        c[k] = (int32_t)(fi[k] / f.sub[k]);
+        ctr[k] = g.lo[k] + ((float)fi[k] + 0.5f) * f.cell[k];
+        a0[k] = a1[k] = c[k];
+        if (f.w[k] == 0.0f) continue;
+        // the block of neighbours lies in the grid; its faces are one grid
+        // cell and the fine cell's offset away
+        inner &= c[k] > 0 && c[k] + 1 < (int32_t)g.dims[k];
+        a0[k] = c[k] - 1; a1[k] = c[k] + 1;
+        const uint32_t o = fi[k] % f.sub[k];
+        edge = fminf(edge, g.cell[k] + (float)min(o, f.sub[k] - 1 - o) * f.cell[k]);
+    }
+    double d = coarse[((uint64_t)c[2] * g.dims[1] + c[1]) * g.dims[0] + c[0]];
+    if (inner && d < edge) {
+        const double reach = (double)edge + f.half_diag;
+        double d2 = reach * reach;
+        const D3 p = D3{ctr[0], ctr[1], ctr[2]}, w = D3{f.w[0], f.w[1], f.w[2]};
+        for (int32_t z = a0[2]; z <= a1[2]; ++z)
+            for (int32_t y = a0[1]; y <= a1[1]; ++y) {
+                // the cells of a row are consecutive, and so are their entries
+                const uint64_t row = ((uint64_t)z * g.dims[1] + y) * g.dims[0];
+                const uint32_t k1 = start[row + a1[0] + 1];
+                for (uint32_t k = start[row + a0[0]]; k < k1; ++k)
+                    d2 = fmin(d2, tri_dist2(mt + (size_t)tri[k] * 4, p, w));
+            }
+        d = fmax(d, sqrt(d2) - f.half_diag);
+    }
+    out[i] = (uint8_t)fmin(fmax(floor((d - kFineMargin) / f.q), 0.0), 255.0);
+}
+
+// ---- search lists of the walk ---------------------------------------------- //
+// A wall facet is two triangles of one plane (equal records), so a search that lists them as one entry tests half the planes.  And
+// most planes a segment crosses it crosses beyond the facet (a wall's
+// neighbouring facets are nearly one plane): the lateral record bounds the
+// facet across its narrow direction, and rejects those before the triangle
+// test.
+
+constexpr uint32_t kNoTri = 0xFFFFFFFFu;
+
+// Sort key of triangle t: a hash of its plane and first vertex, whose equality
+// k_pair_triangles checks on the full records.
+__device__ __forceinline__ uint64_t mix64(uint64_t h, uint32_t v) {
+    h = (h ^ v) * 0x9E3779B97F4A7C15ull;
+    return h ^ (h >> 29);
+}
+__global__ __launch_bounds__(kBlock) void k_plane_keys(uint32_t n_tri, const float4 *mt,
+                                                       uint64_t *keys, uint32_t *vals) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= n_tri) return;
+    const float4 a = mt[(size_t)t * 4], v = mt[(size_t)t * 4 + 1];
+    const float f[7] = {a.x, a.y, a.z, a.w, v.x, v.y, v.z};
+    uint64_t h = 1;
+    for (int k = 0; k < 7; ++k) h = mix64(h, __float_as_uint(f[k] + 0.0f));  // -0 as +0
+    keys[t] = h;
+    vals[t] = t;
+}
+
+// Pairs the triangles of each run of equal keys two by two, in ascending
+// order (the sort is stable), where their planes are equal: every side test
+// then gives one result for both.
+__global__ __launch_bounds__(kBlock) void k_pair_triangles(uint32_t n_tri, const uint64_t *keys,
+                                                           const uint32_t *vals, const float4 *mt,
+                                                           uint32_t *partner) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n_tri || (i > 0 && keys[i] == keys[i - 1])) return;  // the run's first thread
+    uint32_t k = i;
+    while (k < n_tri && keys[k] == keys[i]) {
+        const uint32_t t = vals[k];
+        partner[t] = kNoTri;
+        if (k + 1 < n_tri && keys[k + 1] == keys[i]) {
+            const uint32_t u = vals[k + 1];
+            const float4 p = mt[(size_t)t * 4], q = mt[(size_t)u * 4];
+            if (p.x == q.x && p.y == q.y && p.z == q.z && p.w == q.w) {
+                partner[t] = u;
+                partner[u] = t;
+                k += 2;
+                continue;
+            }
+        }
+        ++k;
+    }
+}
+
+// Records of triangle t and its partner: the plane, and the lateral record
+// (d / W, m / W) with d the unit vector in the plane across the triangle's
+// longest edge and [m - W, m + W] the extent of both along d, widened by
+// kFineMargin; (0, 0, 0, 0), which bounds nothing, for a degenerate triangle.
+// eps: the largest distance of a vertex from its own record's plane.
+__global__ __launch_bounds__(kBlock) void k_walk_records(uint32_t n_tri, const float4 *mt,
+                                                         const uint32_t *partner, float4 *rec,
+                                                         uint32_t *eps) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= n_tri) return;
+    const float4 pl = mt[(size_t)t * 4];
+    double lo = 0, hi = 0, dev = 0;
+    D3 d = D3{0, 0, 0};
+    uint32_t u = t;
+    for (int q = 0; q < 2; ++q) {
+        const float4 v4 = mt[(size_t)u * 4 + 1], a4 = mt[(size_t)u * 4 + 2],
+                     b4 = mt[(size_t)u * 4 + 3];
+        const D3 v0 = D3{v4.x, v4.y, v4.z}, e1 = D3{a4.x, a4.y, a4.z}, e2 = D3{b4.x, b4.y, b4.z};
+        const D3 e3 = e2 - e1;
+        if (q == 0) {
+            const double l1 = dotv(e1, e1), l2 = dotv(e2, e2), l3 = dotv(e3, e3);
+            const D3 l = l1 >= l2 && l1 >= l3 ? e1 : l2 >= l3 ? e2 : e3;
+            d = cross3(cross3(e1, e2), l);
+            const double n = sqrt(dotv(d, d));
+            d = n > 0.0 ? D3{d.x / n, d.y / n, d.z / n} : D3{0, 0, 0};
+            lo = hi = dotv(d, v0);
+        }
+        const double c0 = dotv(d, v0), c1 = c0 + dotv(d, e1), c2 = c0 + dotv(d, e2);
+        lo = fmin(lo, fmin(c0, fmin(c1, c2)));
+        hi = fmax(hi, fmax(c0, fmax(c1, c2)));
+        const D3 n = D3{pl.x, pl.y, pl.z};
+        const double s0 = dotv(n, v0) - (double)pl.w;
+        dev = fmax(dev, fmax(fabs(s0), fmax(fabs(s0 + dotv(n, e1)), fabs(s0 + dotv(n, e2)))));
+        u = partner[t];
+        if (u == kNoTri) break;
+    }
+    const double W = 0.5 * (hi - lo) + kFineMargin, m = 0.5 * (hi + lo);
+    const bool ok = dotv(d, d) > 0.5 && W < 1e30;  // false for a degenerate or NaN triangle
+    rec[(size_t)t * 2] = pl;
+    rec[(size_t)t * 2 + 1] = ok ? make_float4((float)(d.x / W), (float)(d.y / W), (float)(d.z / W),
+                                              (float)(m / W))
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (ok && dev < 1.0) atomicMax(eps, __float_as_uint((float)dev));
+}
+
+// Entries of cell c: EMIT false counts them, true writes them at start[c]
+// (and their records, cell-major).  A triangle whose partner precedes it in
+// the cell's list is that one's entry.
+template <bool EMIT>
+__global__ __launch_bounds__(kBlock) void k_walk_lists(uint32_t n_cells, const uint32_t *cell_start,
+                                                       const uint32_t *cell_tri,
+                                                       const uint32_t *partner, uint32_t *start,
+                                                       uint2 *ent, const float4 *rec,
+                                                       float4 *cell_rec) {
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= n_cells) return;
+    const uint32_t k0 = cell_start[c], k1 = cell_start[c + 1];
+    uint32_t n = EMIT ? start[c] : 0u;
+    for (uint32_t k = k0; k < k1; ++k) {
+        const uint32_t t = cell_tri[k], u = partner[t];
+        bool with = false;
+        if (u != kNoTri) {  // lists are in ascending triangle order
+            uint32_t a = k0, b = k1;
+            while (a < b) {
+                const uint32_t m = (a + b) >> 1;
+                if (cell_tri[m] < u) a = m + 1; else b = m;
+            }
+            with = a < k1 && cell_tri[a] == u;
+        }
+        if (with && u < t) continue;
+        if (EMIT) {
+            ent[n] = make_uint2(t, with ? u : kNoTri);
+            if (cell_rec) {
+                cell_rec[(size_t)n * 2] = rec[(size_t)t * 2];
+                cell_rec[(size_t)n * 2 + 1] = rec[(size_t)t * 2 + 1];
+            }
+        }
+        ++n;
+    }
+    if (!EMIT) start[c] = n;
+}
+
 uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
 }  // namespace
+
+// Fine cells per grid cell and axis.  Planar grids take 4 (16 bytes a grid
+// cell), three-dimensional ones 2 (8 bytes), less where the table would pass
+// kFineMaxBytes.
+constexpr uint32_t kFineSub2D = 4, kFineSub3D = 2;
+constexpr uint64_t kFineMaxBytes = 1ull << 29;
+
+static int build_fine_clearance(dsim_substrate *S, hipStream_t st) {
+    int axes = 0;
+    for (int k = 0; k < 3; ++k) axes += S->dims[k] > 1;
+    if (axes == 0 || !S->d_clearance.p) return DSIM_OK;  // no table: every step searches
+    uint32_t sub = axes == 3 ? kFineSub3D : kFineSub2D;
+    uint64_t n = 0;
+    FineGeom f{};
+    for (;; sub /= 2) {
+        n = 1;
+        for (int k = 0; k < 3; ++k) {
+            f.sub[k] = S->dims[k] > 1 ? sub : 1;
+            f.dims[k] = S->dims[k] * f.sub[k];
+            n *= f.dims[k];
+        }
+        if (sub == 1 || n <= kFineMaxBytes) break;
+    }
+    Geom g{};
+    g.kind = S->kind;
+    float smallest = 3.0e38f, h2 = 0.0f;
+    for (int k = 0; k < 3; ++k) {
+        g.dims[k] = S->dims[k]; g.lo[k] = S->lo[k]; g.cell[k] = S->cell[k];
+        f.cell[k] = S->cell[k] / (float)f.sub[k];
+        f.w[k] = S->dims[k] > 1 ? 1.0f : 0.0f;
+        if (f.w[k] != 0.0f) {
+            smallest = std::min(smallest, S->cell[k]);
+            h2 += 0.25f * f.cell[k] * f.cell[k];
+        }
+        S->fine_dims[k] = f.dims[k];
+        S->fine_inv[k] = S->inv_cell[k] * (float)f.sub[k];
+        S->fine_w[k] = f.w[k];
+    }
+    f.half_diag = std::sqrt(h2) * 1.00001f;
+    f.q = S->fine_q = smallest / kFineRange;
+    if (int rc = S->d_fine.alloc(n)) return rc;
+    hipLaunchKernelGGL(k_fine_clearance, dim3(blocks_for(n)), dim3(kBlock), 0, st, g, f,
+                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_mt.p, S->d_clearance.p,
+                       S->d_fine.p);
+    HIP_TRY(hipGetLastError());
+    return DSIM_OK;
+}
+
+namespace {
+template <class T>
+struct TempBuf : DevBuf<T> {
+    ~TempBuf() { this->release(); }
+};
+}  // namespace
+
+static int build_search_lists(dsim_substrate *S, hipStream_t st) {
+    const uint32_t nT = S->n_tri, nC = S->n_cells;
+    const size_t nt1 = std::max<uint32_t>(nT, 1);
+    const bool cell_major = S->kind != DSIM_GRID_TRIBOX;
+    TempBuf<uint64_t> keys, keys2;
+    TempBuf<uint32_t> vals, vals2, partner, eps;
+    TempBuf<float4> rec;
+    TempBuf<uint8_t> temp;
+    int rc;
+    if ((rc = keys.alloc(nt1)) || (rc = keys2.alloc(nt1)) || (rc = vals.alloc(nt1)) ||
+        (rc = vals2.alloc(nt1)) || (rc = partner.alloc(nt1)) || (rc = eps.alloc(1)) ||
+        (rc = rec.alloc(nt1 * 2)) || (rc = S->walk_start.alloc((size_t)nC + 1)))
+        return rc;
+    HIP_TRY(hipMemsetAsync(eps.p, 0, 4, st));
+    size_t tb_sort = 0, tb_scan = 0;
+    if (nT)
+        HIP_TRY(rocprim::radix_sort_pairs(nullptr, tb_sort, keys.p, keys2.p, vals.p, vals2.p, nT, 0,
+                                          64, st));
+    HIP_TRY(rocprim::exclusive_scan(nullptr, tb_scan, S->walk_start.p, S->walk_start.p, 0u,
+                                    (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
+    if ((rc = temp.alloc(std::max({tb_sort, tb_scan, (size_t)1})))) return rc;
+    if (nT) {
+        hipLaunchKernelGGL(k_plane_keys, dim3(blocks_for(nT)), dim3(kBlock), 0, st, nT, S->tri_mt.p,
+                           keys.p, vals.p);
+        HIP_TRY(rocprim::radix_sort_pairs(temp.p, tb_sort, keys.p, keys2.p, vals.p, vals2.p, nT, 0,
+                                          64, st));
+        hipLaunchKernelGGL(k_pair_triangles, dim3(blocks_for(nT)), dim3(kBlock), 0, st, nT, keys2.p,
+                           vals2.p, S->tri_mt.p, partner.p);
+        hipLaunchKernelGGL(k_walk_records, dim3(blocks_for(nT)), dim3(kBlock), 0, st, nT, S->tri_mt.p,
+                           partner.p, rec.p, eps.p);
+    }
+    hipLaunchKernelGGL(k_walk_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, nC,
+                       S->d_cell_start.p, S->d_cell_tri.p, partner.p, S->walk_start.p,
+                       (uint2 *)nullptr, (const float4 *)nullptr, (float4 *)nullptr);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemsetAsync(S->walk_start.p + nC, 0, 4, st));
+    HIP_TRY(rocprim::exclusive_scan(temp.p, tb_scan, S->walk_start.p, S->walk_start.p, 0u,
+                                    (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
+    uint32_t n = 0;
+    float dev = 0.0f;
+    HIP_TRY(hipMemcpyAsync(&n, S->walk_start.p + nC, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&dev, eps.p, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    const size_t n1 = std::max<uint32_t>(n, 1);
+    if ((rc = S->walk_ent.alloc(n1)) || (cell_major && (rc = S->walk_rec.alloc(n1 * 2)))) return rc;
+    hipLaunchKernelGGL(k_walk_lists<true>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, nC,
+                       S->d_cell_start.p, S->d_cell_tri.p, partner.p, S->walk_start.p, S->walk_ent.p,
+                       rec.p, S->walk_rec.p);
+    HIP_TRY(hipGetLastError());
+    // side distances are off by the record's own error and by FP32 rounding at
+    // coordinates up to 2 (three fused operations of half an ulp, 4e-7)
+    S->walk_eps = 2.0f * dev + 1e-6f;
+    if (!cell_major) std::swap(S->walk_rec, static_cast<DevBuf<float4> &>(rec));
+    HIP_TRY(hipStreamSynchronize(st));  // the temporary arrays are freed on return
+    return DSIM_OK;
+}
+
+int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
+    if (int rc = build_search_lists(S, st)) return rc;
+    return build_fine_clearance(S, st);
+}
 
 extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_grid_params *grid,
                                             dsim_substrate **out) {
@@ -575,21 +920,6 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
     GRID_TRY(hipMemcpyAsync(&S->max_per_cell, maxc.p, 4, hipMemcpyDeviceToHost, st));
     S->n_entries = n_pairs;
 
-    // cell-major records (not for exact-membership grids: their long
-    // triangles are listed in many cells, so entries keep only the index)
-    const bool cell_major = grid->kind != DSIM_GRID_TRIBOX;
-    if (cell_major && ((rc = S->cell_plane.alloc(np1)) || (rc = S->cell_mt.alloc(np1 * 3))))
-        return bail(rc);
-    if (!cell_major) {
-    } else if (n_pairs) {
-        hipLaunchKernelGGL(k_cell_records, dim3(blocks_for(n_pairs)), dim3(kBlock), 0, st,
-                           n_pairs, S->d_cell_tri.p, S->tri_mt.p, S->cell_plane.p, S->cell_mt.p);
-        GRID_TRY(hipGetLastError());
-    } else {
-        GRID_TRY(hipMemsetAsync(S->cell_plane.p, 0, 16, st));
-        GRID_TRY(hipMemsetAsync(S->cell_mt.p, 0, 48, st));
-    }
-
     // clearance (AABB and exact-membership grids)
     if (grid->kind != DSIM_GRID_REFERENCE) {
         if ((rc = ring.alloc(S->n_cells)) || (rc = S->d_clearance.alloc(S->n_cells)))
@@ -617,6 +947,7 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
                            S->d_clearance.p);
         GRID_TRY(hipGetLastError());
     }
+    if ((rc = dsim_host::build_walk_tables(S, st))) return bail(rc);
     GRID_TRY(hipStreamSynchronize(st));
 #undef GRID_TRY
     cleanup();

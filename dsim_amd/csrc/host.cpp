@@ -551,27 +551,11 @@ extern "C" int dsim_substrate_create(const dsim_mesh *mesh, const dsim_grid_para
     }
     std::vector<uint32_t> ct = S->cell_tri;
     if (ct.empty()) ct.push_back(0);  // keep a valid pointer for empty grids
-    // Per grid entry, in cell order: the plane of its triangle (the
-    // prefilter of a cell's candidates reads contiguous memory), and the
-    // triangle's Moller-Trumbore vertices with its index in v0.w, so the test
-    // needs no second lookup through cell_tri.
-    // Exact-membership grids list long triangles in many cells: their
-    // entries keep only the index and the step reads the triangle's record.
-    const bool cell_major = grid->kind != DSIM_GRID_TRIBOX;
-    std::vector<float4> cp(cell_major ? ct.size() : 0), cm(cell_major ? ct.size() * 3 : 0);
-    for (size_t k = 0; k < cp.size(); ++k) {
-        if (S->cell_tri.empty()) break;
-        const float4 *r = &mt[(size_t)ct[k] * 4];
-        cp[k] = r[0];
-        cm[k * 3 + 0] = float4{r[1].x, r[1].y, r[1].z, bits_to_float(ct[k])};
-        cm[k * 3 + 1] = r[2];
-        cm[k * 3 + 2] = r[3];
-    }
-    if ((rc = upload(S->d_cell_tri, ct)) || (cell_major && (rc = upload(S->cell_plane, cp))) ||
-        (cell_major && (rc = upload(S->cell_mt, cm)))) {
+    if ((rc = upload(S->d_cell_tri, ct)) || (rc = dsim_host::build_walk_tables(S, nullptr))) {
         delete S;
         return rc;
     }
+    HIP_TRY(hipStreamSynchronize(nullptr));
     *out = S;
     return DSIM_OK;
 }
@@ -676,10 +660,10 @@ extern "C" int dsim_substrate_label_axis(const dsim_substrate *s, uint32_t *axis
 
 extern "C" int dsim_substrate_bytes(const dsim_substrate *s, uint64_t *bytes) {
     if (!s || !bytes) return fail(DSIM_ERR_ARG, "NULL argument");
-    *bytes = (uint64_t)s->tri_ref.n * 16 + s->tri_mt.n * 16 + s->tri_aabb.n * 16 + s->cell_plane.n * 16 +
-             s->cell_mt.n * 16 +
+    *bytes = (uint64_t)s->tri_ref.n * 16 + s->tri_mt.n * 16 + s->tri_aabb.n * 16 + s->walk_rec.n * 16 +
+             s->walk_ent.n * 8 + s->walk_start.n * 4 +
              s->d_cell_start.n * 4 + s->d_cell_tri.n * 4 + s->fiber_myelin.n + s->d_clearance.n * 4 +
-             s->d_helpers.n * 4;
+             s->d_helpers.n * 4 + s->d_fine.n;
     return DSIM_OK;
 }
 

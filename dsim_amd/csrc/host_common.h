@@ -81,6 +81,13 @@ int upload(DevBuf<T> &d, const std::vector<T> &h) {
 
 }  // namespace dsim_host
 
+struct dsim_substrate;
+namespace dsim_host {
+// Builds the walk's search lists and fine clearance from the device grid,
+// records and clearance (grid.hip).
+int build_walk_tables(dsim_substrate *S, hipStream_t st);
+}  // namespace dsim_host
+
 #define HIP_TRY(expr)                                                                        \
     do {                                                                                     \
         hipError_t e_ = (expr);                                                              \
@@ -98,9 +105,23 @@ struct dsim_substrate {
     uint32_t dims[3] = {0, 0, 0};
     float lo[3] = {0, 0, 0}, cell[3] = {0, 0, 0}, inv_cell[3] = {0, 0, 0};
     std::vector<float> clearance;  // per cell: lower bound of the distance to any triangle
-    dsim_host::DevBuf<float4> tri_ref, tri_mt, tri_aabb, cell_plane, cell_mt;
+    dsim_host::DevBuf<float4> tri_ref, tri_mt, tri_aabb;
     dsim_host::DevBuf<uint32_t> d_cell_start, d_cell_tri;
     dsim_host::DevBuf<float> d_clearance, d_helpers;
+    // Search lists of the physical-mode walk (build_walk_tables): per grid cell
+    // its triangles, two of one plane in one entry (the second kNone where there
+    // is none), and the entries' plane and lateral records, cell-major for
+    // reference and AABB grids and by triangle (walk_rec[2 t]) for
+    // exact-membership grids, whose long triangles are listed in many cells.
+    dsim_host::DevBuf<uint32_t> walk_start;
+    dsim_host::DevBuf<uint2> walk_ent;
+    dsim_host::DevBuf<float4> walk_rec;
+    float walk_eps = 0;  // bound of the error of a side distance (see walk_test, kernels.hip)
+    // Fine clearance of the walk: one byte per fine cell, a lower bound of the distance to any registered triangle
+    // in units of fine_q; axes with one grid cell are collapsed (fine_w 0).
+    dsim_host::DevBuf<uint8_t> d_fine;
+    uint32_t fine_dims[3] = {0, 0, 0};
+    float fine_inv[3] = {0, 0, 0}, fine_w[3] = {0, 0, 0}, fine_q = 0;
     dsim_host::DevBuf<uint8_t> fiber_myelin;
     int refs = 0;
     bool on_device = false;
@@ -109,8 +130,9 @@ struct dsim_substrate {
     bool device_built = false;
     uint32_t n_entries = 0;
     ~dsim_substrate() {
-        tri_ref.release(); tri_mt.release(); tri_aabb.release(); cell_plane.release(); cell_mt.release();
-        d_clearance.release(); d_helpers.release();
+        tri_ref.release(); tri_mt.release(); tri_aabb.release();
+        walk_start.release(); walk_ent.release(); walk_rec.release();
+        d_clearance.release(); d_helpers.release(); d_fine.release();
         d_cell_start.release(); d_cell_tri.release(); fiber_myelin.release();
     }
 };

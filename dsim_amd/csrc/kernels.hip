@@ -45,6 +45,10 @@ __device__ __forceinline__ void mwc_randn(uint32_t &s0, uint32_t &s1, float &n1,
 // Philox4x32-10 (Salmon et al., SC'11).  The 32x32->64 products compile to
 // one v_mad_u64_u32 each.
 __device__ __forceinline__ uint4 philox(uint4 c, uint32_t k0, uint32_t k1) {
+    // the round keys are wave-uniform: formed here with scalar additions, not
+    // hoisted out of a caller's step loop, where eighteen of them would crowd
+    // out its other scalars (each spilled one costs a vector instruction)
+    asm volatile("" : "+s"(k0), "+s"(k1));
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         const uint64_t p0 = (uint64_t)0xD2511F53u * c.x;
@@ -293,32 +297,31 @@ __device__ __forceinline__ bool better(const Hit &c, const Hit &b) {
     return (c.d < b.d) || (c.d == b.d && c.idx < b.idx);
 }
 
-// Where the walk reads a grid entry's records: kRecsCellMajor from the
-// cell-major copies (AABB and reference grids), kRecsIndirect from the
-// triangle's own record through cell_tri (exact-membership grids keep no
-// copy), kRecsEither deciding per launch parameter (a uniform branch; the
+// Where the walk reads a search entry's records: kRecsCellMajor by entry (AABB
+// and reference grids), kRecsIndirect by its triangle (exact-membership
+// grids), kRecsEither deciding per launch parameter (a uniform branch; the
 // batched kernel, whose jobs may use either kind of grid).
-// Moller-Trumbore vertices of grid entry k and its triangle index.
+//
+// Does the segment o-p cross the plane of entry k (first triangle tri) where
+// its facet may be?  The
+// plane's sides decide as crosses_plane does.  The lateral record (e, m) gives
+// each end's coordinate w across the facet's narrow direction, scaled so that
+// the facet lies within [-1, 1]; at the crossing it is
+// (w0 s1 - w1 s0) / (s1 - s0).  The bound allows for the error of the side
+// distances (walk_eps), which moves the crossing along the segment, so a
+// segment rejected here is one the triangle test rejects.
 template <int RECS>
-__device__ __forceinline__ uint32_t entry_mt(const StepParams &P, uint32_t k, float4 &v0,
-                                             float4 &e1, float4 &e2) {
-    if (RECS == kRecsCellMajor || (RECS == kRecsEither && P.cell_mt)) {
-        v0 = P.cell_mt[(size_t)k * 3 + 0];
-        e1 = P.cell_mt[(size_t)k * 3 + 1];
-        e2 = P.cell_mt[(size_t)k * 3 + 2];
-        return __float_as_uint(v0.w);
-    }
-    const uint32_t t = P.cell_tri[k];
-    v0 = P.tri_mt[(size_t)t * 4 + 1];
-    e1 = P.tri_mt[(size_t)t * 4 + 2];
-    e2 = P.tri_mt[(size_t)t * 4 + 3];
-    return t;
-}
-// Plane (n, n.v0) of grid entry k's triangle.
-template <int RECS>
-__device__ __forceinline__ float4 entry_plane(const StepParams &P, uint32_t k) {
-    if (RECS == kRecsCellMajor || (RECS == kRecsEither && P.cell_plane)) return P.cell_plane[k];
-    return P.tri_mt[(size_t)P.cell_tri[k] * 4];
+__device__ __forceinline__ bool walk_test(const StepParams &P, uint32_t k, uint32_t tri,
+                                          const float4 o, const float4 p) {
+    const size_t r = RECS == kRecsIndirect || (RECS == kRecsEither && !P.walk_cell_major) ? tri : k;
+    const float4 pl = P.walk_rec[2 * r], e = P.walk_rec[2 * r + 1];
+    const float s0 = fmaf(pl.x, o.x, fmaf(pl.y, o.y, fmaf(pl.z, o.z, -pl.w)));
+    const float s1 = fmaf(pl.x, p.x, fmaf(pl.y, p.y, fmaf(pl.z, p.z, -pl.w)));
+    const float w0 = fmaf(e.x, o.x, fmaf(e.y, o.y, fmaf(e.z, o.z, -e.w)));
+    const float w1 = fmaf(e.x, p.x, fmaf(e.y, p.y, fmaf(e.z, p.z, -e.w)));
+    const float far = fabsf(fmaf(w0, s1, -(w1 * s0)));
+    const float lim = fmaf(P.walk_eps, fabsf(w0) + fabsf(w1) + 1.0f, fabsf(s1 - s0));
+    return ((s0 > 0.0f) != (s1 > 0.0f)) & !(far > lim);
 }
 
 // cubeCollDetect, spinKernelCpu.cpp:311-337, over one CSR cell.
@@ -328,30 +331,19 @@ __device__ __forceinline__ void cell_test(const StepParams &P, uint32_t cell, ui
                                           float pz, Hit &best) {
     uint32_t k0 = P.cell_start[cell], k1 = P.cell_start[cell + 1];
     for (uint32_t k = k0; k < k1; ++k) {
-        if (MODE == 0) {
-            uint32_t t = P.cell_tri[k];
-            if (t == excluded) continue;
-            Hit c;
-            test_ref(P.tri_ref, t, ox, oy, oz, px, py, pz, c);
-            if (better<MODE>(c, best)) best = c;
-        } else {
-            // the cell-major plane record rejects most candidates without
-            // touching the triangle record
-            if (!crosses_plane(entry_plane<kRecsEither>(P, k), ox, oy, oz, px, py, pz)) continue;
-            uint32_t t = P.cell_tri[k];
-            if (t == excluded) continue;
-            Hit c;
-            test_mt_crossing(P.tri_mt, t, ox, oy, oz, px, py, pz, c);
-            if (better<MODE>(c, best)) best = c;
-        }
+        uint32_t t = P.cell_tri[k];
+        if (t == excluded) continue;
+        Hit c;
+        test_ref(P.tri_ref, t, ox, oy, oz, px, py, pz, c);
+        if (better<MODE>(c, best)) best = c;
     }
 }
 
-// reflectPos, spinKernelCpu.cpp:406-422.
+// reflectPos, spinKernelCpu.cpp:406-422 (MODE 1: wall holds the normal).
 template <int MODE>
 __device__ __forceinline__ void reflect(const StepParams &P, float sx, float sy, float sz,
-                                        float tx, float ty, float tz, const Hit &h, float &rx,
-                                        float &ry, float &rz) {
+                                        float tx, float ty, float tz, const Hit &h,
+                                        const float4 wall, float &rx, float &ry, float &rz) {
     if ((P.reflection_type == 0) | (h.type > 1)) {
         rx = sx; ry = sy; rz = sz;
         return;
@@ -364,13 +356,12 @@ __device__ __forceinline__ void reflect(const StepParams &P, float sx, float sy,
         ry = -2 * nx * ny * qx + (1 - 2 * ny * ny) * qy - 2 * ny * nz * qz + h.py;
         rz = -2 * nx * nz * qx - 2 * ny * nz * qy + (1 - 2 * nz * nz) * qz + h.pz;
     } else {
-        const float4 pl = P.tri_mt[h.idx * 4];
         float qx = tx - h.px, qy = ty - h.py, qz = tz - h.pz;
-        float dn = fmaf(pl.x, qx, fmaf(pl.y, qy, pl.z * qz));
+        float dn = fmaf(wall.x, qx, fmaf(wall.y, qy, wall.z * qz));
         float k = -2.0f * dn;
-        rx = fmaf(k, pl.x, qx) + h.px;
-        ry = fmaf(k, pl.y, qy) + h.py;
-        rz = fmaf(k, pl.z, qz) + h.pz;
+        rx = fmaf(k, wall.x, qx) + h.px;
+        ry = fmaf(k, wall.y, qy) + h.py;
+        rz = fmaf(k, wall.z, qz) + h.pz;
     }
 }
 
@@ -464,7 +455,7 @@ __device__ __forceinline__ void collide(const StepParams &P, float ox, float oy,
         ncoll += 1;
         float thr = umax - (umax - umin) * P.perm;
         if (u <= thr) {
-            reflect<MODE>(P, ox, oy, oz, px, py, pz, best, ex, ey, ez);
+            reflect<MODE>(P, ox, oy, oz, px, py, pz, best, float4(), ex, ey, ez);
             umax = thr;
         } else {
             umin = thr;
@@ -478,27 +469,25 @@ __device__ __forceinline__ void collide(const StepParams &P, float ox, float oy,
     px = ex; py = ey; pz = ez;
 }
 
-// Clearance shortcut.  The clearance of a cell bounds from below the distance
-// from any point of the cell to any triangle registered in the grid, so a
-// spin inside the cell can walk a path shorter than that without a search
-// finding a hit.  Two allowances keep the float arithmetic on the safe side:
-// kClearMargin for a position that rounds into the cell from just outside it,
-// and kStepSlack per step for the rounding of the new position (half an ulp
-// per coordinate at |x| < 2, 1.1e-7 as a vector) and of the step length.
-constexpr float kClearMargin = 1e-5f;
+// Clearance shortcut.  The clearance at a point bounds from below its distance
+// to any triangle registered in the grid, so a step whose length is less than
+// the sum of its end points' clearances crosses none: the two balls cover it.
+// The table's bytes carry the margin for FP32 positions (grid.hip); kStepSlack
+// covers the rounding of the new position (half an ulp per coordinate at
+// |x| < 2, 1.1e-7 as a vector) and of the step's length.
 constexpr float kStepSlack = 4e-7f;
 
-// Clearance budget of a spin at (x, y, z): the cell's clearance less the
-// margin, or -1 (no shortcut) outside the grid, where lookups clamp to an
-// edge cell that does not contain the position.
+// Clearance at (x, y, z), or a value that no sum brings above a step's length
+// outside the grid.
 __device__ __forceinline__ float clearance_at(const StepParams &P, float x, float y, float z) {
-    const float qx = floorf((x - P.lo[0]) * P.inv_cell[0]);
-    const float qy = floorf((y - P.lo[1]) * P.inv_cell[1]);
-    const float qz = floorf((z - P.lo[2]) * P.inv_cell[2]);
-    if (!(qx >= 0.0f && qx < (float)P.dims[0] && qy >= 0.0f && qy < (float)P.dims[1] &&
-          qz >= 0.0f && qz < (float)P.dims[2]))
-        return -1.0f;
-    return P.cell_clear[cell_hash(P, (uint32_t)qx, (uint32_t)qy, (uint32_t)qz)] - kClearMargin;
+    const int qx = (int)floorf((x - P.lo[0]) * P.fine_inv[0]);
+    const int qy = (int)floorf((y - P.lo[1]) * P.fine_inv[1]);
+    const int qz = (int)floorf((z - P.lo[2]) * P.fine_inv[2]);
+    if ((uint32_t)qx >= P.fine_dims[0] || (uint32_t)qy >= P.fine_dims[1] ||
+        (uint32_t)qz >= P.fine_dims[2])
+        return -1e30f;
+    return P.fine_q *
+           (float)P.fine[((uint32_t)qz * P.fine_dims[1] + (uint32_t)qy) * P.fine_dims[0] + (uint32_t)qx];
 }
 
 // ------------------------------------------------------------------------ //
@@ -597,39 +586,47 @@ __global__ __launch_bounds__(64) void k_step(StepParams P, uint32_t iters) {
 // ------------------------------------------------------------------------ //
 // Physical-mode walk, laid out for 64-wide wavefronts.
 //
-// Each lane runs a small state machine: it either starts its next step (draw
-// normals, propose the end point, take the clearance shortcut if it applies)
-// or has a segment of the current step pending a collision search.  Every
-// trip round the wave loop does one search round for all pending lanes
-// together, so a lane whose step ended without a hit starts its next step
-// while another lane is still reflecting.
+// Each lane walks one spin.  The wave's loop advances the lanes that are free
+// (end the last step, draw the next one; a step whose end points' clearances
+// cover it needs no search) and then searches the segments of the others
+// together.  A lane whose step ended without a hit starts its next one while
+// another lane is still reflecting.
 //
 // The search is compacted over the wave in two passes.  Each pending lane
-// lists the CSR ranges of the cells its segment's bounding box covers, and a
-// wave prefix sum numbers the (lane, grid entry) pairs.  The plane pass tests
-// 64 pairs per trip, whatever lane they belong to, against the entry's plane
-// record and queues the pairs whose plane the segment crosses; the triangle
-// pass runs Moller-Trumbore on the queue, 64 pairs per trip.  The nearest hit
-// per lane is an LDS atomic minimum over (t bits, triangle index): for t > 0
-// the float bits order like the values, so this is the same (t, then index)
-// order as a scan of the lane's cells in any order; the pair holding the
-// minimum then writes its hit point for the lane.
+// lists the entries of the rows of cells that its segment's bounding box covers
+// (the cells of a row are consecutive, and so are their entries), and a wave
+// prefix sum numbers the (lane, entry) pairs.  The plane pass tests 128 pairs
+// per trip, whatever lane they belong to, against the entry's plane and facet
+// bound, and queues the triangles of those the segment may cross; the triangle
+// pass runs Moller-Trumbore on the queue, 64 per trip.
+// The nearest hit per lane is an LDS atomic minimum over (t bits, triangle
+// index): for t > 0 the float bits order like the values, so this is the same
+// (t, then index) order as a scan of the lane's cells in any order; the pair
+// holding the minimum then writes the hit for the lane.
+//
+// Bound: VALU issue (about 73 % of the slots at four waves a SIMD; the inner
+// turn takes some 230 instructions, a search round 350 and more).  1e6 spins,
+// 2000 axons, 12,000 steps: 380 ms, against 544 ms with a per-cell clearance
+// budget (67 % of the steps searched, here 24 %, and 12 % again after a hit)
+// and one list entry a triangle (5.0 plane and 1.9 triangle tests a step, here
+// 1.8 and 0.9).
 // ------------------------------------------------------------------------ //
-constexpr uint32_t kWaveSegs = 256;   // cell ranges listed per wave and search round
+constexpr uint32_t kWaveRows = 128;   // cell rows listed per wave and search round
 constexpr uint32_t kPass = 128;       // pairs per pass: two per lane, loads in flight together
-// plane crossings awaiting the triangle test; the scratch of 16 waves (four
-// per SIMD) then takes 155.6 KB of a CU's 160 KB LDS
+// Triangles awaiting their test (a pass queues 256 at most); the scratch of 16
+// waves (four per SIMD) then takes 155.6 KB of a CU's 160 KB LDS.
 constexpr uint32_t kWaveQueue = 384;
 
 struct WaveScratch {
-    uint2 seg[kWaveSegs];  // (first entry - lane-local pair number, lane-local end)
+    uint2 row[kWaveRows];  // (first entry - lane-local pair number, lane-local end)
     float4 o[64];          // segment start; .w = excluded triangle
-    float4 p[64];          // segment end
+    float4 p[64];          // segment end; .w = squared length
     float4 hit[64];        // nearest hit point; .w = hit type
-    uint2 meta[64];        // (first pair number, first slot in seg)
+    float4 wall[64];       // normal and info of its triangle
+    uint2 meta[64];        // (first pair number, first row)
     unsigned long long best[64];
     uint32_t map[kPass];   // lane + 1 at the pass position where its pairs start
-    uint2 queue[kWaveQueue];  // (grid entry, lane)
+    uint2 queue[kWaveQueue];  // (triangle, lane)
 };
 
 // Orders this wave's LDS accesses: a wave's LDS instructions complete in
@@ -683,181 +680,197 @@ struct WalkCounters {
 };
 __device__ __forceinline__ uint32_t popc(unsigned long long m) { return (uint32_t)__popcll(m); }
 
-// FP32 triangle test of queue entry q (cell-major record) for its lane; the
-// lane's minimum key in best[] is lowered to it on a hit.  Returns true for a
-// near-grazing entry, which wave_graze_pass decides.
-template <int RECS>
-__device__ __forceinline__ bool queue_test(const StepParams &P, WaveScratch &L, uint32_t q,
-                                           uint32_t qlen, Hit &h, uint32_t &owner,
-                                           unsigned long long &key) {
-    h.type = 0;
-    owner = 0;
-    key = ~0ull;
-    if (q >= qlen) return false;
-    const uint2 e = L.queue[q];
-    owner = e.y;
-    float4 v0, e1, e2;
-    const uint32_t t = entry_mt<RECS>(P, e.x, v0, e1, e2);
-    const float4 so = L.o[owner], sp = L.p[owner];
-    if (t == __float_as_uint(so.w)) return false;
-    if (mt_fp32(v0, e1, e2, t, so.x, so.y, so.z, sp.x, sp.y, sp.z, sp.w, h)) return true;
-    if (h.type) {
-        key = hit_key(h.d, t);
-        atomicMin(&L.best[owner], key);
+// The lane holding a segment's minimum so far records its hit.
+__device__ __forceinline__ void record_hit(WaveScratch &L, const Hit &h, uint32_t seg,
+                                           unsigned long long key, const float4 pl, float info) {
+    if (h.type && L.best[seg] == key) {
+        L.hit[seg] = make_float4(h.px, h.py, h.pz, __uint_as_float(h.type));
+        L.wall[seg] = make_float4(pl.x, pl.y, pl.z, info);
     }
-    return false;
 }
 
 // FP64 re-test of the near-grazing queue entries in [0, qlen) (found again
 // by the FP32 test), one entry per lane per trip, with the nearest-hit
 // bookkeeping of the FP32 pass.  Wave-uniform qlen.
-template <int RECS, bool STATS>
+template <bool STATS>
 __device__ __forceinline__ void wave_graze_pass(const StepParams &P, WaveScratch &L,
                                                 uint32_t lane, uint32_t qlen, WalkCounters &C) {
     for (uint32_t qb = 0; qb < qlen; qb += 64) {
         wave_lds_sync();
         Hit h;
         h.type = 0;
-        uint32_t owner = 0;
+        uint32_t seg = 0;
         unsigned long long key = ~0ull;
+        float4 pl = make_float4(0.f, 0.f, 0.f, 0.f), v0 = pl;
         const uint32_t q = qb + lane;
         bool graze = false;
         if (q < qlen) {
             const uint2 e = L.queue[q];
-            float4 v0, e1, e2;
-            const uint32_t t = entry_mt<RECS>(P, e.x, v0, e1, e2);
+            const uint32_t t = e.x;
+            const float4 *m = P.tri_mt + (size_t)t * 4;
+            v0 = m[1];
+            const float4 e1 = m[2], e2 = m[3];
             const float4 so = L.o[e.y], sp = L.p[e.y];
             graze = t != __float_as_uint(so.w) &&
                     mt_fp32(v0, e1, e2, t, so.x, so.y, so.z, sp.x, sp.y, sp.z, sp.w, h);
             if (graze) {
                 mt_fp64(v0, e1, e2, t, so.x, so.y, so.z, sp.x, sp.y, sp.z, h);
                 if (h.type) {
-                    owner = e.y;
+                    seg = e.y;
+                    pl = m[0];
                     key = hit_key(h.d, t);
-                    atomicMin(&L.best[owner], key);
+                    atomicMin(&L.best[seg], key);
                 }
+            } else {
+                h.type = 0;  // decided by the FP32 pass
             }
         }
         if (STATS) C.v[kStatGraze] += popc(__ballot(graze));
         wave_lds_sync();
-        if (h.type && L.best[owner] == key)
-            L.hit[owner] = make_float4(h.px, h.py, h.pz, __uint_as_float(h.type));
+        record_hit(L, h, seg, key, pl, v0.w);
     }
 }
 
-// Triangle pass over queue[0, qlen): nearest hit per lane into best[] and its
-// point into hit[].  Wave-uniform qlen.
-template <int RECS, bool STATS>
+// Triangle pass over queue[0, qlen): each segment's nearest hit into best[],
+// hit[] and wall[].  Wave-uniform qlen.
+template <bool STATS>
 __device__ __forceinline__ void wave_triangle_pass(const StepParams &P, WaveScratch &L,
                                                    uint32_t lane, uint32_t qlen,
                                                    WalkCounters &C) {
     if (STATS) {
         C.v[kStatTriangle] += qlen;
-        C.v[kStatTriPasses] += (qlen + kPass - 1) / kPass;
+        C.v[kStatTriPasses] += (qlen + 63) / 64;
     }
     bool graze = false;
-    for (uint32_t qb = 0; qb < qlen; qb += kPass) {
+    for (uint32_t qb = 0; qb < qlen; qb += 64) {
         wave_lds_sync();
-        Hit ha, hb;
-        uint32_t oa, ob;
-        unsigned long long ka, kb;
-        graze |= queue_test<RECS>(P, L, qb + lane, qlen, ha, oa, ka);
-        graze |= queue_test<RECS>(P, L, qb + 64 + lane, qlen, hb, ob, kb);
+        Hit h;
+        h.type = 0;
+        uint32_t seg = 0;
+        unsigned long long key = ~0ull;
+        float4 pl = make_float4(0.f, 0.f, 0.f, 0.f), v0 = pl;
+        if (qb + lane < qlen) {
+            const uint2 e = L.queue[qb + lane];
+            const uint32_t t = e.x;
+            seg = e.y;
+            const float4 *m = P.tri_mt + (size_t)t * 4;
+            pl = m[0];
+            v0 = m[1];
+            const float4 e1 = m[2], e2 = m[3];
+            const float4 so = L.o[seg], sp = L.p[seg];
+            if (t != __float_as_uint(so.w)) {
+                graze |= mt_fp32(v0, e1, e2, t, so.x, so.y, so.z, sp.x, sp.y, sp.z, sp.w, h);
+                if (h.type) {
+                    key = hit_key(h.d, t);
+                    atomicMin(&L.best[seg], key);
+                }
+            }
+        }
         wave_lds_sync();
-        // the pair holding the lane's minimum so far records its hit point; a
-        // later pass that lowers the minimum overwrites it
-        if (ha.type && L.best[oa] == ka)
-            L.hit[oa] = make_float4(ha.px, ha.py, ha.pz, __uint_as_float(ha.type));
-        if (hb.type && L.best[ob] == kb)
-            L.hit[ob] = make_float4(hb.px, hb.py, hb.pz, __uint_as_float(hb.type));
+        // a later trip that lowers the minimum overwrites the record
+        record_hit(L, h, seg, key, pl, v0.w);
     }
-    if (__builtin_expect(__ballot(graze) != 0, 0)) wave_graze_pass<RECS, STATS>(P, L, lane, qlen, C);
+    if (__builtin_expect(__ballot(graze) != 0, 0)) wave_graze_pass<STATS>(P, L, lane, qlen, C);
     wave_lds_sync();
 }
 
-// Plane test of pair j for its owner lane: sets k (grid entry) and whether
-// the owner's segment crosses the entry's plane.
+// Queues the triangles of the lanes with c set.
+__device__ __forceinline__ void queue_push(WaveScratch &L, bool c, uint2 tri, uint32_t seg,
+                                           uint32_t &qlen) {
+    const unsigned long long b = __ballot(c);
+    if (b == 0ull) return;
+    if (c) L.queue[qlen + lane_rank(b)] = make_uint2(tri.x, seg);
+    qlen += popc(b);
+    const bool two = c && tri.y != kNone;
+    const unsigned long long b2 = __ballot(two);
+    if (two) L.queue[qlen + lane_rank(b2)] = make_uint2(tri.y, seg);
+    qlen += popc(b2);
+}
+
+// Test of pair j for its owner lane: whether the owner's segment may cross the
+// entry's facet, and the entry's triangles.
 template <int RECS>
 __device__ __forceinline__ bool pair_crosses(const StepParams &P, const WaveScratch &L,
                                              uint32_t j, uint32_t total, uint32_t owner,
-                                             uint32_t &k) {
-    k = 0;
+                                             uint2 &tri) {
     if (j >= total) return false;
     const uint2 m = L.meta[owner];
     const uint32_t r = j - m.x;
     uint32_t s = m.y;
-    uint2 e = L.seg[s];
-    while (r >= e.y && s + 1 < kWaveSegs) e = L.seg[++s];
-    k = e.x + r;
-    if (k >= P.n_entries) {  // cannot happen when the numbering is right
-        atomicOr(P.flags, 4u);
-        k = 0;
-    }
-    const float4 so = L.o[owner], sp = L.p[owner];
-    return crosses_plane(entry_plane<RECS>(P, k), so.x, so.y, so.z, sp.x, sp.y, sp.z);
+    uint2 e = L.row[s];
+    while (r >= e.y && s + 1 < kWaveRows) e = L.row[++s];
+    const uint32_t k = e.x + r;
+    tri = P.walk_ent[k];
+    return walk_test<RECS>(P, k, tri.x, L.o[owner], L.p[owner]);
 }
+
+// A hit point of FP32 arithmetic may lie this far outside the cells that list
+// its triangle, and a clipped segment's ends this far from their exact place.
+constexpr float kBoxPad = 1e-5f;
 
 // One search round, called by all 64 lanes of the wave together.  For each
 // lane with `search` set, either finds the nearest hit of the segment o-p
-// (excluding `excluded`): returns true with key = hit_key(t, triangle) (or ~0
-// when there is none) and the hit point and type in `hit`; or returns false
-// when the wave's cell list is full in this search round, or when the lane's
-// cell box is longer than the list and cells remain (the lane searches again).
-// A box of more than kWaveSegs cells is searched kWaveSegs cells per round, in
-// x-fastest order from cell `slice` (0 for a new segment; advanced here), its
-// nearest hit carried in best[]/hit[] from round to round.
+// (excluding `excluded`; all of them lie between t0 and t1 of it) and returns
+// true with best[lane] = hit_key(t, triangle), ~0 when there is none, hit[lane]
+// and wall[lane]; or returns false when the wave's row list is full in this
+// round, or when the lane's box has more rows than the list and some remain
+// (the lane searches again).  A box of more than kWaveRows rows is searched
+// kWaveRows rows per round, along y first, from row `slice` (0 for a new
+// segment; advanced here), its nearest hit carried from round to round.
 template <int RECS, bool STATS>
 __device__ __forceinline__ bool wave_search(const StepParams &P, WaveScratch &L, uint32_t lane,
                                             bool search, float ox, float oy, float oz, float px,
-                                            float py, float pz, uint32_t excluded,
-                                            uint32_t &slice, unsigned long long &key,
-                                            float4 &hit, WalkCounters &C) {
-    uint32_t x0 = 0, x1 = 0, y0 = 0, y1 = 0, z0 = 0, z1 = 0, ncell = 0;
+                                            float py, float pz, float t0, float t1,
+                                            uint32_t excluded, uint32_t &slice, WalkCounters &C) {
+    uint32_t x0 = 0, y0 = 0, z0 = 0, x1 = 0, y1 = 0, z1 = 0, rows = 0;
     if (search) {
-        uint32_t sx, sy, sz, tx, ty, tz;
-        cell_of<1>(P, ox, oy, oz, sx, sy, sz);
-        cell_of<1>(P, px, py, pz, tx, ty, tz);
-        x0 = min(sx, tx); x1 = max(sx, tx);
-        y0 = min(sy, ty); y1 = max(sy, ty);
-        z0 = min(sz, tz); z1 = max(sz, tz);
-        ncell = (x1 - x0 + 1) * (y1 - y0 + 1) * (z1 - z0 + 1);
+        const float dx = px - ox, dy = py - oy, dz = pz - oz;
+        const float ax = fmaf(t0, dx, ox), ay = fmaf(t0, dy, oy), az = fmaf(t0, dz, oz);
+        const float bx = fmaf(t1, dx, ox), by = fmaf(t1, dy, oy), bz = fmaf(t1, dz, oz);
+        cell_of<1>(P, fminf(ax, bx) - kBoxPad, fminf(ay, by) - kBoxPad, fminf(az, bz) - kBoxPad, x0,
+                   y0, z0);
+        cell_of<1>(P, fmaxf(ax, bx) + kBoxPad, fmaxf(ay, by) + kBoxPad, fmaxf(az, bz) + kBoxPad, x1,
+                   y1, z1);
+        rows = (y1 - y0 + 1) * (z1 - z0 + 1);
+        L.o[lane] = make_float4(ox, oy, oz, __uint_as_float(excluded));
+        L.p[lane] = make_float4(px, py, pz, fmaf(dx, dx, fmaf(dy, dy, dz * dz)));
     }
-    // a lane lists at most kWaveSegs cells of its box per round; one that does
+    // a lane lists at most kWaveRows rows of its box per round; one that does
     // not fit behind the lanes before it waits for the next round (the first
     // lane always fits)
-    const uint32_t nreq = search ? min(ncell - slice, kWaveSegs) : 0u;
+    const uint32_t nreq = search ? min(rows - slice, kWaveRows) : 0u;
     const uint32_t send = wave_incl_sum(nreq);
     const uint32_t soff = send - nreq;
-    const bool coop = nreq > 0 && send <= kWaveSegs;
+    const bool coop = nreq > 0 && send <= kWaveRows;
     uint32_t cnt = 0;
     if (coop) {
-        uint32_t cx = x0, cy = y0, cz = z0;
+        const uint32_t ny = y1 - y0 + 1, width = x1 - x0 + 1;
+        uint32_t y = 0, cell = cell_hash(P, x0, y0, z0);
         if (slice) {  // a later slice of a long box
-            const uint32_t nx = x1 - x0 + 1, ny = y1 - y0 + 1;
-            cx += slice % nx;
-            cy += (slice / nx) % ny;
-            cz += slice / (nx * ny);
+            y = slice % ny;
+            cell += y * P.dims[0] + (slice / ny) * P.dims[1] * P.dims[0];
         }
-        for (uint32_t s = 0; s < nreq; s += 4) {
-            uint32_t k0[4], k1[4];
+        for (uint32_t s = 0; s < nreq; s += 2) {
+            uint32_t k0[2], k1[2];
 #pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
+            for (uint32_t q = 0; q < 2; ++q) {
                 k0[q] = k1[q] = 0;
                 if (s + q < nreq) {
-                    const uint32_t c = cell_hash(P, cx, cy, cz);
-                    k0[q] = P.cell_start[c];
-                    k1[q] = P.cell_start[c + 1];
-                    if (++cx > x1) { cx = x0; if (++cy > y1) { cy = y0; ++cz; } }
+                    k0[q] = P.walk_start[cell];
+                    k1[q] = P.walk_start[cell + width];
+                    cell += P.dims[0];
+                    if (++y == ny) { y = 0; cell += (P.dims[1] - ny) * P.dims[0]; }
                 }
             }
 #pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
+            for (uint32_t q = 0; q < 2; ++q) {
                 if (s + q < nreq) {
-                    L.seg[soff + s + q] = make_uint2(k0[q] - cnt, cnt + (k1[q] - k0[q]));
+                    L.row[soff + s + q] = make_uint2(k0[q] - cnt, cnt + (k1[q] - k0[q]));
                     cnt += k1[q] - k0[q];
                 }
             }
         }
+        if (slice == 0) L.best[lane] = ~0ull;  // later slices keep the minimum so far
     }
     const uint32_t cend = wave_incl_sum(cnt);
     const uint32_t off = cend - cnt;
@@ -865,16 +878,12 @@ __device__ __forceinline__ bool wave_search(const StepParams &P, WaveScratch &L,
     if (STATS) {
         C.v[kStatSearchLanes] += popc(__ballot(coop));
         C.v[kStatDeferred] += popc(__ballot(nreq > 0 && !coop));
-        C.v[kStatCells] += __builtin_amdgcn_readlane(wave_incl_sum(coop ? nreq : 0u), 63);
+        C.v[kStatCells] += __builtin_amdgcn_readlane(
+            wave_incl_sum(coop ? nreq * (x1 - x0 + 1) : 0u), 63);
         C.v[kStatPlane] += total;
         C.v[kStatPasses] += (total + kPass - 1) / kPass;
     }
-    if (coop) {
-        L.o[lane] = make_float4(ox, oy, oz, __uint_as_float(excluded));
-        L.p[lane] = make_float4(px, py, pz, seg_len2(ox, oy, oz, px, py, pz));
-        L.meta[lane] = make_uint2(off, soff);
-        if (slice == 0) L.best[lane] = ~0ull;  // later slices keep the minimum so far
-    }
+    if (coop) L.meta[lane] = make_uint2(off, soff);
     uint32_t qlen = 0;  // wave-uniform
     for (uint32_t base = 0; base < total; base += kPass) {
         L.map[lane] = 0;
@@ -885,30 +894,25 @@ __device__ __forceinline__ bool wave_search(const StepParams &P, WaveScratch &L,
         // owner of pass position q: the last lane whose pairs start at or
         // before it (position 0 always holds the lane covering `base`)
         const uint32_t own_a = wave_incl_max(L.map[lane]);
-        const uint32_t own_b = max(wave_incl_max(L.map[lane + 64]),
-                                   __builtin_amdgcn_readlane(own_a, 63));
-        uint32_t ka, kb;
-        const bool ca = pair_crosses<RECS>(P, L, base + lane, total, own_a - 1, ka);
-        const bool cb = pair_crosses<RECS>(P, L, base + 64 + lane, total, own_b - 1, kb);
-        const unsigned long long ba = __ballot(ca), bb = __ballot(cb);
-        if (ca) L.queue[qlen + lane_rank(ba)] = make_uint2(ka, own_a - 1);
-        qlen += (uint32_t)__popcll(ba);
-        if (cb) L.queue[qlen + lane_rank(bb)] = make_uint2(kb, own_b - 1);
-        qlen += (uint32_t)__popcll(bb);
-        if (qlen > kWaveQueue - kPass) {
-            wave_triangle_pass<RECS, STATS>(P, L, lane, qlen, C);
+        uint2 ta, tb;
+        bool cb = false;
+        uint32_t own_b = 1;
+        if (base + 64 < total) {
+            own_b = max(wave_incl_max(L.map[lane + 64]), __builtin_amdgcn_readlane(own_a, 63));
+            cb = pair_crosses<RECS>(P, L, base + 64 + lane, total, own_b - 1, tb);
+        }
+        const bool ca = pair_crosses<RECS>(P, L, base + lane, total, own_a - 1, ta);
+        queue_push(L, ca, ta, own_a - 1, qlen);
+        queue_push(L, cb, tb, own_b - 1, qlen);
+        if (qlen > kWaveQueue - 2 * kPass) {  // a pass queues two triangles a pair at most
+            wave_triangle_pass<STATS>(P, L, lane, qlen, C);
             qlen = 0;
         }
     }
-    if (qlen) wave_triangle_pass<RECS, STATS>(P, L, lane, qlen, C);
+    if (qlen) wave_triangle_pass<STATS>(P, L, lane, qlen, C);
     wave_lds_sync();
-    key = ~0ull;
-    const bool done = coop && slice + nreq >= ncell;
+    const bool done = coop && slice + nreq >= rows;
     if (coop && !done) slice += nreq;
-    if (done) {
-        key = L.best[lane];
-        if (key != ~0ull) hit = L.hit[lane];
-    }
     return done;
 }
 
@@ -980,10 +984,13 @@ constexpr uint32_t kQueueMinSteps = 768;
 // TRAJBUF (trajectory runs): each lane keeps its last four steps'
 // displacements in registers and stores them as three 16-byte chunks every
 // fourth step (launches and buffers are multiples of four steps).
+//
+// A wave walks `per_wave` spins (64, or fewer where there are not enough to
+// fill the device), lanes beyond that none.
 template <int BOUND, int RNG, int INSTR, bool MOMENT, int RECS, bool QUEUE = false,
           bool TRAJBUF = false>
 __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, uint32_t iters,
-                                          WaveScratch &L) {
+                                          uint32_t per_wave, WaveScratch &L) {
     constexpr bool PERIODIC = BOUND != kBoundClamp;
     constexpr bool TRACE = INSTR == kInstrTrace, STATS = INSTR == kInstrStats;
     WalkCounters C;
@@ -994,11 +1001,19 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
     uint32_t sid = 0, comp = 0, fiber = kFiberNone, s0 = 0, s1 = 0;
     float x = 0.f, y = 0.f, z = 0.f, mag = 0.f, ph = 0.f;
     float dx = 0.f, dy = 0.f, dz = 0.f, mx = 0.f, my = 0.f, mz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
-    float safe = -1.0f;
+    float clear = -1e30f;  // clearance at (x, y, z)
     float tb[TRAJBUF ? 12 : 1];  // TRAJBUF: displacements of the last four steps
     // voxel crossings (periodic phase): the unwrapped position is x + kx * period
     int kx = 0, ky = 0, kz = 0;
-    uint32_t nhit = 0, hit_total = 0;
+    uint32_t nsearch = 0, hit_total = 0;
+    // step length and decay of the spin's compartment
+    float sd = 0.f, dc = 0.f;
+    auto enter = [&] {
+        sd = comp == 0 ? P.std_dev[0] : comp == 1 ? P.std_dev[1]
+           : comp == 2 ? P.std_dev[2] : P.std_dev[3];
+        dc = comp == 0 ? P.decay[0] : comp == 1 ? P.decay[1]
+           : comp == 2 ? P.decay[2] : P.decay[3];
+    };
     auto load = [&](uint32_t i) {
         sid = P.spin_id ? P.spin_id[i] : i;
         x = P.x[i]; y = P.y[i]; z = P.z[i];
@@ -1007,14 +1022,15 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
         if (PERIODIC && !MOMENT) unpack_wrap(P.wrap[i], kx, ky, kz);
         const uint32_t lab = P.label[i];
         comp = lab & 0xFFu; fiber = (lab >> 8) & 0xFFFFu;
+        enter();
         if (RNG == kRngMwc) { s0 = P.seed[2 * i]; s1 = P.seed[2 * i + 1]; }
         if (MOMENT) {
             dx = P.disp[i]; dy = P.disp[P.n + i]; dz = P.disp[2 * P.n + i];
             mx = P.mom[i]; my = P.mom[P.n + i]; mz = P.mom[2 * P.n + i];
             cx = P.momc[i]; cy = P.momc[P.n + i]; cz = P.momc[2 * P.n + i];
         }
-        if (P.cell_clear) safe = clearance_at(P, x, y, z);
-        nhit = 0;
+        if (P.fine) clear = clearance_at(P, x, y, z);
+        nsearch = 0;
     };
     auto store = [&](uint32_t i) {
         P.x[i] = x; P.y[i] = y; P.z[i] = z;
@@ -1028,8 +1044,7 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
             P.mom[i] = mx; P.mom[P.n + i] = my; P.mom[2 * P.n + i] = mz;
             P.momc[i] = cx; P.momc[P.n + i] = cy; P.momc[2 * P.n + i] = cz;
         }
-        if (P.hits) P.hits[i] += nhit;
-        if (STATS) hit_total += nhit;
+        if (P.searches) P.searches[i] += nsearch;
     };
     // The persistent walk (QUEUE): lanes take slots from their XCD's queue,
     // the finishing lanes of a trip together (one atomic per wave).
@@ -1043,193 +1058,222 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
         return want ? queue_slot(q, base + lane_rank(m), P.n, P.queue_run) : P.n;
     };
     // lanes past the last spin stay in the loop (done) for the wave operations
-    uint32_t i = QUEUE ? take(true) : block * blockDim.x + threadIdx.x;
+    uint32_t i = QUEUE ? take(true) : lane < per_wave ? block * per_wave + lane : P.n;
     bool live = i < P.n;
+    if (STATS) C.v[kStatWaves] = __ballot(live) != 0ull;
     if (live) load(i);
     uint32_t it = live ? 0u : iters;
     // the pending segment of the current step and its permeation interval
-    bool pending = false, refresh = false;
+    bool pending = false, complete = false;
     float ox = 0.f, oy = 0.f, oz = 0.f, px = 0.f, py = 0.f, pz = 0.f;
     float u = 0.f, umax = 1.f, umin = 0.f;
+    float t0 = 0.f, t1 = 1.f;  // part of the pending segment that may hold a hit
     uint32_t excluded = kNone, first = kNone, last = kNone, ncoll = 0;
-    uint32_t slice = 0;  // cells of the segment's box searched so far
-    while (__ballot(it < iters) != 0ull) {
-        bool complete = false;
+    uint32_t slice = 0;  // rows of the segment's box searched so far
+    for (;;) {
+        // Advance: lanes end their completed step and start the next one; in
+        // the persistent walk twice before a search, whose fixed part then
+        // serves more segments (fixed blocks end with their slowest lane, which
+        // would wait).  1e6 spins, 2000 axons: 383 ms an acquisition with two
+        // turns, 397 with one, 387 with three, 405 with eight; 1e4 spins: 45.7
+        // ms with one, 51.7 with eight.
+        constexpr uint32_t kTurns = QUEUE ? 2 : 1;
+        for (uint32_t adv = 0;;) {
+            if (complete) {
+                complete = false;
+                // `clear` is the proposed end point's: the step may have ended
+                // elsewhere (a hit, a clamp, a wrap)
+                bool moved = ncoll != 0;
+                if (!PERIODIC) {
+                    const float wx = px, wy = py, wz = pz;
+                    if (px > P.clamp_hi) px = P.clamp_hi; else if (px < P.clamp_lo) px = P.clamp_lo;
+                    if (py > P.clamp_hi) py = P.clamp_hi; else if (py < P.clamp_lo) py = P.clamp_lo;
+                    if (pz > P.clamp_hi) pz = P.clamp_hi; else if (pz < P.clamp_lo) pz = P.clamp_lo;
+                    moved |= (px != wx) | (py != wy) | (pz != wz);
+                }
+                if (MOMENT) {
+                    dx += px - x; dy += py - y; dz += pz - z;
+                }
+                if (PERIODIC) {
+                    if (BOUND == kBoundCube) {
+                        // few steps leave the voxel: one test for all axes
+                        if (!(fmaxf(fmaxf(fabsf(px), fabsf(py)), fabsf(pz)) < 1.0f)) {
+                            moved = true;
+                            wrap_axis(px, -1.0f, 1.0f, 2.0f, kx);
+                            wrap_axis(py, -1.0f, 1.0f, 2.0f, ky);
+                            wrap_axis(pz, -1.0f, 1.0f, 2.0f, kz);
+                        }
+                    } else {
+                        const float wx = px, wy = py, wz = pz;
+                        wrap_axis(px, P.wrap_lo[0], P.wrap_hi[0], P.wrap_len[0], kx);
+                        wrap_axis(py, P.wrap_lo[1], P.wrap_hi[1], P.wrap_len[1], ky);
+                        wrap_axis(pz, P.wrap_lo[2], P.wrap_hi[2], P.wrap_len[2], kz);
+                        moved |= (px != wx) | (py != wy) | (pz != wz);
+                    }
+                }
+                if (P.fine && moved) clear = clearance_at(P, px, py, pz);
+                x = px; y = py; z = pz;
+                mag = fmaf(-mag, dc, mag);
+                // spinKernelCpu.cpp:490 with the post-step position; in a periodic
+                // voxel that is the unwrapped position (x + k * period, exactly x
+                // for a spin that has not crossed a face)
+                if (!MOMENT && !PERIODIC) ph += (P.gx * x + P.gy * y + P.gz * z) * P.pc;
+                if (!MOMENT && PERIODIC) {
+                    const float lx = BOUND == kBoundCube ? 2.0f : P.wrap_len[0];
+                    const float ly = BOUND == kBoundCube ? 2.0f : P.wrap_len[1];
+                    const float lz = BOUND == kBoundCube ? 2.0f : P.wrap_len[2];
+                    const float ux = x + (float)kx * lx;
+                    const float uy = y + (float)ky * ly;
+                    const float uz = z + (float)kz * lz;
+                    ph += (P.gx * ux + P.gy * uy + P.gz * uz) * P.pc;
+                }
+                if (MOMENT && P.weight != 0.0f) {
+                    float yv, tv;
+                    yv = fmaf(P.weight, dx, -cx); tv = mx + yv; cx = (tv - mx) - yv; mx = tv;
+                    yv = fmaf(P.weight, dy, -cy); tv = my + yv; cy = (tv - my) - yv; my = tv;
+                    yv = fmaf(P.weight, dz, -cz); tv = mz + yv; cz = (tv - mz) - yv; mz = tv;
+                }
+                if (TRAJBUF) {
+                    // unwrapped displacement after this step, k = 3 * it + axis,
+                    // shifted into the four-step window; stored when it is full
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) tb[q] = tb[q + 3];
+                    tb[9] = dx; tb[10] = dy; tb[11] = dz;
+                    if ((it & 3u) == 3u) {
+                        float4 *tr = reinterpret_cast<float4 *>(
+                            P.traj + (size_t)(sid / kTrajTile) * P.traj_stride +
+                            (size_t)(3 * (it - 3) / kTrajChunk) * (kTrajTile * kTrajChunk)) +
+                            sid % kTrajTile;
+                        tr[0] = make_float4(tb[0], tb[1], tb[2], tb[3]);
+                        tr[kTrajTile] = make_float4(tb[4], tb[5], tb[6], tb[7]);
+                        tr[2 * kTrajTile] = make_float4(tb[8], tb[9], tb[10], tb[11]);
+                    }
+                } else if (MOMENT && P.traj) {
+                    // unwrapped displacement after this step, k = 3 * it + axis
+                    // of the spin's tile
+                    float *tr = P.traj + (size_t)(sid / kTrajTile) * P.traj_stride +
+                                (sid % kTrajTile) * kTrajChunk;
+#pragma unroll
+                    for (uint32_t a = 0; a < 3; ++a) {
+                        const uint32_t k = 3 * it + a;
+                        tr[(size_t)(k / kTrajChunk) * (kTrajTile * kTrajChunk) + k % kTrajChunk] =
+                            a == 0 ? dx : a == 1 ? dy : dz;
+                    }
+                }
+                if (TRACE) {
+                    uint32_t qx, qy, qz;
+                    cell_of<1>(P, x, y, z, qx, qy, qz);
+                    uint32_t *tr = P.trace + ((size_t)it * P.n + sid) * 5;
+                    tr[0] = first; tr[1] = last; tr[2] = ncoll;
+                    tr[3] = cell_hash(P, qx, qy, qz);
+                    tr[4] = comp | (fiber << 8);
+                }
+                ++it;
+            }
+            if (QUEUE) {
+                // a lane whose spin has walked its steps stores it and takes the
+                // next slot of its queue
+                const bool fin = live && it == iters;
+                if (__ballot(fin) != 0ull) {
+                    if (fin) store(i);
+                    if (STATS) C.v[kStatSteps] += popc(__ballot(fin)) * iters;
+                    const uint32_t ni = take(fin);
+                    if (fin) {
+                        i = ni;
+                        live = i < P.n;
+                        if (live) {
+                            load(i);
+                            it = 0;
+                        }
+                    }
+                }
+            }
+            const bool go = it < iters && !pending;
+            const unsigned long long mg = __ballot(go);
+            if (mg == 0ull || (adv >= kTurns && __ballot(pending) != 0ull)) break;
+            ++adv;
+            if (go) {
+                float n0, n1, n2;
+                if (RNG == kRngInject) {
+                    const float4 r = P.inject[(size_t)it * P.n + sid];
+                    n0 = r.x; n1 = r.y; n2 = r.z; u = r.w;
+                } else if (RNG == kRngMwc) {
+                    mwc_randn(s0, s1, n0, n1, n2, u);
+                } else {
+                    philox_draw(P.key0, P.key1, sid, P.step0 + it, n0, n1, n2, u);
+                }
+                ox = x; oy = y; oz = z;
+                px = fmaf(n0, sd, x); py = fmaf(n1, sd, y); pz = fmaf(n2, sd, z);
+                first = last = excluded = kNone;
+                ncoll = 0;
+                umax = 1.0f; umin = 0.0f;
+                pending = true;
+                t0 = 0.0f; t1 = 1.0f;
+                if (P.fine) {
+                    const float clear_p = clearance_at(P, px, py, pz);
+                    const float w0 = n0 * P.fine_w[0], w1 = n1 * P.fine_w[1], w2 = n2 * P.fine_w[2];
+                    const float len =
+                        sd * __builtin_amdgcn_sqrtf(fmaf(w0, w0, fmaf(w1, w1, w2 * w2))) + kStepSlack;
+                    if (len < clear + clear_p) {
+                        pending = false;
+                        complete = true;
+                        if (STATS) ++shortcuts;
+                    } else {
+                        // the balls around the ends hold no triangle: search what
+                        // lies between
+                        const float r = __builtin_amdgcn_rcpf(len);
+                        t0 = fmaxf(clear * r, 0.0f);
+                        t1 = 1.0f - fmaxf(clear_p * r, 0.0f);
+                    }
+                    clear = clear_p;  // unless the step ends elsewhere
+                }
+            }
+        }
+        // Search the pending segments together.
+        const unsigned long long mp = __ballot(pending);
+        if (mp == 0ull) break;  // every lane has walked its steps
         if (STATS) {
             C.v[kStatTrips] += 1;
             C.v[kStatLiveLaneTrips] += popc(__ballot(it < iters));
         }
-        if (it < iters && !pending) {
-            float n0, n1, n2;
-            if (RNG == kRngInject) {
-                const float4 q = P.inject[(size_t)it * P.n + sid];
-                n0 = q.x; n1 = q.y; n2 = q.z; u = q.w;
-            } else if (RNG == kRngMwc) {
-                mwc_randn(s0, s1, n0, n1, n2, u);
-            } else {
-                philox_draw(P.key0, P.key1, sid, P.step0 + it, n0, n1, n2, u);
-            }
-            const float sd = comp == 0 ? P.std_dev[0] : comp == 1 ? P.std_dev[1]
-                           : comp == 2 ? P.std_dev[2] : P.std_dev[3];
-            ox = x; oy = y; oz = z;
-            px = fmaf(n0, sd, x); py = fmaf(n1, sd, y); pz = fmaf(n2, sd, z);
-            first = last = excluded = kNone;
-            ncoll = 0;
-            umax = 1.0f; umin = 0.0f;
-            pending = true;
-            refresh = true;
+        if (pending) nsearch += 1;
+        const bool done = wave_search<RECS, STATS>(P, L, lane, pending, ox, oy, oz, px, py, pz, t0, t1,
+                                                   excluded, slice, C);
+        if (pending && done) {
+            const unsigned long long key = L.best[lane];
             slice = 0;
-            if (P.cell_clear) {
-                // no triangle lies within `safe` of the path walked since the
-                // last check, so a shorter step cannot hit one
-                const float len =
-                    sd * __builtin_amdgcn_sqrtf(fmaf(n0, n0, fmaf(n1, n1, n2 * n2))) + kStepSlack;
-                if (len < safe) {
-                    safe -= len;
-                    pending = false;
-                    refresh = false;
-                    complete = true;
-                    if (STATS) ++shortcuts;
-                }
-            }
-        }
-        unsigned long long key;
-        float4 hp;
-        const bool searched =
-            wave_search<RECS, STATS>(P, L, lane, pending, ox, oy, oz, px, py, pz, excluded, slice,
-                                     key, hp, C);
-        if (pending && searched) {
             if (key == ~0ull) {
                 pending = false;
                 complete = true;
             } else {
-                const uint32_t idx = (uint32_t)key;
+                const float4 hp = L.hit[lane], so = L.o[lane], wall = L.wall[lane];
                 Hit h;
                 h.px = hp.x; h.py = hp.y; h.pz = hp.z;
                 h.type = __float_as_uint(hp.w);
-                h.idx = idx;
-                if (ncoll == 0) first = idx;
-                last = idx;
+                h.idx = (uint32_t)key;
+                if (ncoll == 0) first = h.idx;
+                last = h.idx;
                 ncoll += 1;
-                nhit += 1;
+                if (STATS) hit_total += 1;
                 const float thr = umax - (umax - umin) * P.perm;
                 float ex = px, ey = py, ez = pz;
                 if (u <= thr) {
-                    reflect<1>(P, ox, oy, oz, px, py, pz, h, ex, ey, ez);
+                    reflect<1>(P, so.x, so.y, so.z, px, py, pz, h, wall, ex, ey, ez);
                     umax = thr;
                 } else {
                     umin = thr;
-                    transit<1>(P, tri_info_of(P, idx, 1), comp, fiber);
+                    transit<1>(P, __float_as_uint(wall.w), comp, fiber);
+                    enter();
                 }
+                // the rest of the step starts on the triangle
                 ox = h.px; oy = h.py; oz = h.pz;
                 px = ex; py = ey; pz = ez;
-                excluded = idx;
-                slice = 0;
+                t0 = 0.0f; t1 = 1.0f;
+                excluded = h.idx;
                 if (ncoll == 4096) {
                     atomicOr(P.flags, 1u);
                     pending = false;
                     complete = true;
-                }
-            }
-        }
-        if (complete) {
-            if (!PERIODIC) {
-                if (px > P.clamp_hi) px = P.clamp_hi; else if (px < P.clamp_lo) px = P.clamp_lo;
-                if (py > P.clamp_hi) py = P.clamp_hi; else if (py < P.clamp_lo) py = P.clamp_lo;
-                if (pz > P.clamp_hi) pz = P.clamp_hi; else if (pz < P.clamp_lo) pz = P.clamp_lo;
-            }
-            if (MOMENT) {
-                dx += px - x; dy += py - y; dz += pz - z;
-            }
-            if (PERIODIC) {
-                const float wx = px, wy = py, wz = pz;
-                if (BOUND == kBoundCube) {
-                    wrap_axis(px, -1.0f, 1.0f, 2.0f, kx);
-                    wrap_axis(py, -1.0f, 1.0f, 2.0f, ky);
-                    wrap_axis(pz, -1.0f, 1.0f, 2.0f, kz);
-                } else {
-                    wrap_axis(px, P.wrap_lo[0], P.wrap_hi[0], P.wrap_len[0], kx);
-                    wrap_axis(py, P.wrap_lo[1], P.wrap_hi[1], P.wrap_len[1], ky);
-                    wrap_axis(pz, P.wrap_lo[2], P.wrap_hi[2], P.wrap_len[2], kz);
-                }
-                refresh |= (px != wx) | (py != wy) | (pz != wz);
-            }
-            x = px; y = py; z = pz;
-            if (P.cell_clear && refresh) safe = clearance_at(P, x, y, z);
-            const float dc = comp == 0 ? P.decay[0] : comp == 1 ? P.decay[1]
-                           : comp == 2 ? P.decay[2] : P.decay[3];
-            mag = fmaf(-mag, dc, mag);
-            // spinKernelCpu.cpp:490 with the post-step position; in a periodic
-            // voxel that is the unwrapped position (x + k * period, exactly x
-            // for a spin that has not crossed a face)
-            if (!MOMENT && !PERIODIC) ph += (P.gx * x + P.gy * y + P.gz * z) * P.pc;
-            if (!MOMENT && PERIODIC) {
-                const float lx = BOUND == kBoundCube ? 2.0f : P.wrap_len[0];
-                const float ly = BOUND == kBoundCube ? 2.0f : P.wrap_len[1];
-                const float lz = BOUND == kBoundCube ? 2.0f : P.wrap_len[2];
-                const float ux = x + (float)kx * lx;
-                const float uy = y + (float)ky * ly;
-                const float uz = z + (float)kz * lz;
-                ph += (P.gx * ux + P.gy * uy + P.gz * uz) * P.pc;
-            }
-            if (MOMENT && P.weight != 0.0f) {
-                float yv, tv;
-                yv = fmaf(P.weight, dx, -cx); tv = mx + yv; cx = (tv - mx) - yv; mx = tv;
-                yv = fmaf(P.weight, dy, -cy); tv = my + yv; cy = (tv - my) - yv; my = tv;
-                yv = fmaf(P.weight, dz, -cz); tv = mz + yv; cz = (tv - mz) - yv; mz = tv;
-            }
-            if (TRAJBUF) {
-                // unwrapped displacement after this step, k = 3 * it + axis,
-                // shifted into the four-step window; stored when it is full
-#pragma unroll
-                for (int q = 0; q < 9; ++q) tb[q] = tb[q + 3];
-                tb[9] = dx; tb[10] = dy; tb[11] = dz;
-                if ((it & 3u) == 3u) {
-                    float4 *tr = reinterpret_cast<float4 *>(
-                        P.traj + (size_t)(sid / kTrajTile) * P.traj_stride +
-                        (size_t)(3 * (it - 3) / kTrajChunk) * (kTrajTile * kTrajChunk)) +
-                        sid % kTrajTile;
-                    tr[0] = make_float4(tb[0], tb[1], tb[2], tb[3]);
-                    tr[kTrajTile] = make_float4(tb[4], tb[5], tb[6], tb[7]);
-                    tr[2 * kTrajTile] = make_float4(tb[8], tb[9], tb[10], tb[11]);
-                }
-            } else if (MOMENT && P.traj) {
-                // unwrapped displacement after this step, k = 3 * it + axis
-                // of the spin's tile
-                float *tr = P.traj + (size_t)(sid / kTrajTile) * P.traj_stride +
-                            (sid % kTrajTile) * kTrajChunk;
-#pragma unroll
-                for (uint32_t a = 0; a < 3; ++a) {
-                    const uint32_t k = 3 * it + a;
-                    tr[(size_t)(k / kTrajChunk) * (kTrajTile * kTrajChunk) + k % kTrajChunk] =
-                        a == 0 ? dx : a == 1 ? dy : dz;
-                }
-            }
-            if (TRACE) {
-                uint32_t qx, qy, qz;
-                cell_of<1>(P, x, y, z, qx, qy, qz);
-                uint32_t *tr = P.trace + ((size_t)it * P.n + sid) * 5;
-                tr[0] = first; tr[1] = last; tr[2] = ncoll;
-                tr[3] = cell_hash(P, qx, qy, qz);
-                tr[4] = comp | (fiber << 8);
-            }
-            ++it;
-        }
-        if (QUEUE) {
-            // a lane whose spin has walked its steps stores it and takes the
-            // next slot of its queue
-            const bool fin = live && it == iters;
-            if (__ballot(fin) != 0ull) {
-                if (fin) store(i);
-                if (STATS) C.v[kStatSteps] += popc(__ballot(fin)) * iters;
-                const uint32_t ni = take(fin);
-                if (fin) {
-                    i = ni;
-                    live = i < P.n;
-                    if (live) {
-                        load(i);
-                        it = 0;
-                    }
                 }
             }
         }
@@ -1239,43 +1283,42 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
         if (!QUEUE) C.v[kStatSteps] = popc(__ballot(live)) * iters;
         C.v[kStatHits] = __builtin_amdgcn_readlane(wave_incl_sum(hit_total), 63);
         C.v[kStatShortcut] = __builtin_amdgcn_readlane(wave_incl_sum(shortcuts), 63);
-        C.v[kStatWaves] = 1;
         if (lane == 0)
             for (uint32_t k = 0; k < kWalkStats; ++k)
                 if (C.v[k]) atomicAdd(P.stats + k, (unsigned long long)C.v[k]);
     }
 }
 
-template <int BOUND, int RNG, int INSTR, bool MOMENT, int RECS>
 // One wave per workgroup: every wave runs until its own slowest lane is done,
-// and a finished wave frees its slot for the next block at once (with four
-// waves per workgroup the slot waited for the slowest of the four).
-__global__ __launch_bounds__(kWalkBlockSpins) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(
-    StepParams P, uint32_t iters) {
-    __shared__ WaveScratch scratch[1];
-    walk_body<BOUND, RNG, INSTR, MOMENT, RECS>(P, xcd_block(kWalkXcdRun), iters, scratch[0]);
+// and a finished wave frees its slot for the next block at once.  per_wave
+// spins a wave (see launch_one).
+template <int BOUND, int RNG, int INSTR, bool MOMENT, int RECS>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(
+    StepParams P, uint32_t iters, uint32_t per_wave) {
+    __shared__ WaveScratch scratch;
+    walk_body<BOUND, RNG, INSTR, MOMENT, RECS>(P, xcd_block(kWalkXcdRun), iters, per_wave, scratch);
 }
 
 // The walk of trajectory runs (moment mode, Philox): k_walk with the
 // trajectory stores gathered four steps at a time (walk_body's TRAJBUF).
 template <int BOUND, int RECS>
-__global__ __launch_bounds__(kWalkBlockSpins) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_traj(
-    StepParams P, uint32_t iters) {
-    __shared__ WaveScratch scratch[1];
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_traj(
+    StepParams P, uint32_t iters, uint32_t per_wave) {
+    __shared__ WaveScratch scratch;
     walk_body<BOUND, kRngPhilox, kInstrNone, true, RECS, false, true>(P, xcd_block(kWalkXcdRun),
-                                                                      iters, scratch[0]);
+                                                                      iters, per_wave, scratch);
 }
 
 // Persistent walk: one one-wave workgroup per resident slot (block b on XCD
-// b mod 8); each lane walks a spin's steps, stores it and takes the next slot
-// from its XCD's queue, so no lane idles while its wave waits for the slowest
-// spin of a fixed block.  Spins are independent (Philox counters keyed by the
+// b mod 8); each lane walks a spin's steps, stores it and takes the next slot from
+// its XCD's queue, so no lane idles while its wave waits for the slowest spin
+// of a fixed block.  Spins are independent (Philox counters keyed by the
 // spin id), so the results equal k_walk's.
 template <int BOUND, int INSTR, bool MOMENT, int RECS>
-__global__ __launch_bounds__(kWalkBlockSpins) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_queue(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_queue(
     StepParams P, uint32_t iters) {
-    __shared__ WaveScratch scratch[1];
-    walk_body<BOUND, kRngPhilox, INSTR, MOMENT, RECS, true>(P, blockIdx.x, iters, scratch[0]);
+    __shared__ WaveScratch scratch;
+    walk_body<BOUND, kRngPhilox, INSTR, MOMENT, RECS, true>(P, blockIdx.x, iters, 64u, scratch);
 }
 
 // Batched walk for the server: the blocks of one launch are shared out over
@@ -1286,16 +1329,16 @@ __global__ __launch_bounds__(kWalkBlockSpins) __attribute__((amdgpu_waves_per_eu
 // table's total exit at once, so one launch shape (and one captured graph)
 // serves any mix of jobs.
 template <int BOUND, int RECS>
-__global__ __launch_bounds__(kWalkBlockSpins) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_batch(const WalkTable *__restrict__ T) {
-    __shared__ WaveScratch scratch[1];
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_batch(const WalkTable *__restrict__ T) {
+    __shared__ WaveScratch scratch;
     const uint32_t b = xcd_block(kBatchXcdRun);
     if (b >= T->total_blocks) return;
     uint32_t j = 0;
     for (uint32_t st = kMaxJobs / 2; st; st >>= 1)
         if (j + st < T->n_jobs && T->block_start[j + st] <= b) j += st;
     const WalkJob &J = T->job[j];
-    walk_body<BOUND, kRngPhilox, kInstrNone, true, RECS>(J.p, b - T->block_start[j], J.iters,
-                                                    scratch[0]);
+    walk_body<BOUND, kRngPhilox, kInstrNone, true, RECS>(J.p, b - T->block_start[j], J.iters, 64u,
+                                                         scratch);
 }
 
 hipError_t launch_walk_batch(const WalkTable *table, uint32_t grid_blocks, bool periodic,
@@ -1315,8 +1358,8 @@ hipError_t launch_walk_batch(const WalkTable *table, uint32_t grid_blocks, bool 
     return hipGetLastError();
 }
 
-// Resident one-wave workgroups of the walk on this device (four per SIMD).
-static uint32_t resident_walk_blocks() {
+// Resident waves of the walk on this device (four per SIMD).
+static uint32_t resident_walk_waves() {
     static uint32_t cached = 0;
     if (!cached) {
         int dev = 0, cus = 0;
@@ -1329,56 +1372,70 @@ static uint32_t resident_walk_blocks() {
     return cached;
 }
 
-template <int MODE, int BOUND, int RNG, int INSTR, bool MOMENT>
-static void launch_one(const StepParams &p, uint32_t iters, hipStream_t s) {
-    if constexpr (MODE == 1 && RNG == kRngPhilox && INSTR != kInstrTrace) {
-        // the persistent walk once every resident slot has two spins or more
-        // and a launch walks at least kQueueMinSteps steps; not while a
-        // trajectory is recorded (its lanes, at different steps of different
-        // spins, would scatter every trajectory store over 64 rows).  Lanes
-        // take a queue slot per spin walked, so short launches turn the eight
-        // queue counters into a stream of atomics: 4e6 spins in 128-step
-        // launches walked 2.3x slower than fixed blocks, at 512 steps 3 %
-        // slower, at 768 3 % faster.
-        const uint32_t slots = resident_walk_blocks();
-        if (p.queue && !p.traj && p.n >= 2 * slots * kWalkBlockSpins && iters >= kQueueMinSteps) {
-            if (hipMemsetAsync(p.queue, 0, kXcds * sizeof(uint32_t), s) != hipSuccess) return;
-            StepParams pq = p;
-            pq.queue_run = queue_run(p.n);
-            if (p.cell_mt)
-                hipLaunchKernelGGL((k_walk_queue<BOUND, INSTR, MOMENT, kRecsCellMajor>), dim3(slots),
-                                   dim3(kWalkBlockSpins), 0, s, pq, iters);
-            else
-                hipLaunchKernelGGL((k_walk_queue<BOUND, INSTR, MOMENT, kRecsIndirect>), dim3(slots),
-                                   dim3(kWalkBlockSpins), 0, s, pq, iters);
-            return;
-        }
-    }
-    if constexpr (MODE == 1 && MOMENT && RNG == kRngPhilox && INSTR == kInstrNone) {
+template <int BOUND, int RNG, int INSTR, bool MOMENT>
+static void launch_blocks(const StepParams &p, uint32_t iters, uint32_t per_wave, hipStream_t s) {
+    const dim3 g((p.n + per_wave - 1) / per_wave), b(64);
+    if constexpr (MOMENT && RNG == kRngPhilox && INSTR == kInstrNone) {
         // four-step windows need whole windows per launch
         if (p.traj && iters % 4 == 0) {
-            if (p.cell_mt)
-                hipLaunchKernelGGL((k_walk_traj<BOUND, kRecsCellMajor>),
-                                   dim3((p.n + kWalkBlockSpins - 1) / kWalkBlockSpins),
-                                   dim3(kWalkBlockSpins), 0, s, p, iters);
+            if (p.walk_cell_major)
+                hipLaunchKernelGGL((k_walk_traj<BOUND, kRecsCellMajor>), g, b, 0, s, p, iters,
+                                   per_wave);
             else
-                hipLaunchKernelGGL((k_walk_traj<BOUND, kRecsIndirect>),
-                                   dim3((p.n + kWalkBlockSpins - 1) / kWalkBlockSpins),
-                                   dim3(kWalkBlockSpins), 0, s, p, iters);
+                hipLaunchKernelGGL((k_walk_traj<BOUND, kRecsIndirect>), g, b, 0, s, p, iters,
+                                   per_wave);
             return;
         }
     }
+    if (p.walk_cell_major)
+        hipLaunchKernelGGL((k_walk<BOUND, RNG, INSTR, MOMENT, kRecsCellMajor>), g, b, 0, s, p,
+                           iters, per_wave);
+    else
+        hipLaunchKernelGGL((k_walk<BOUND, RNG, INSTR, MOMENT, kRecsIndirect>), g, b, 0, s, p,
+                           iters, per_wave);
+}
+
+template <int MODE, int BOUND, int RNG, int INSTR, bool MOMENT>
+static void launch_one(const StepParams &p, uint32_t iters, hipStream_t s) {
     if constexpr (MODE == 0) {
         hipLaunchKernelGGL((k_step<0, BOUND != kBoundClamp, RNG, INSTR == kInstrTrace, MOMENT>),
                            dim3((p.n + 63) / 64), dim3(64), 0, s, p, iters);
-    } else if (p.cell_mt) {
-        hipLaunchKernelGGL((k_walk<BOUND, RNG, INSTR, MOMENT, kRecsCellMajor>),
-                           dim3((p.n + kWalkBlockSpins - 1) / kWalkBlockSpins),
-                           dim3(kWalkBlockSpins), 0, s, p, iters);
+        return;
     } else {
-        hipLaunchKernelGGL((k_walk<BOUND, RNG, INSTR, MOMENT, kRecsIndirect>),
-                           dim3((p.n + kWalkBlockSpins - 1) / kWalkBlockSpins),
-                           dim3(kWalkBlockSpins), 0, s, p, iters);
+        const uint32_t waves = resident_walk_waves();
+        if constexpr (RNG == kRngPhilox && INSTR != kInstrTrace) {
+            // the persistent walk once every resident lane has two spins or more
+            // and a launch walks at least kQueueMinSteps steps; not while a
+            // trajectory is recorded (its lanes, at different steps of different
+            // spins, would scatter every trajectory store over 64 rows).  Lanes
+            // take a queue slot per spin walked, so short launches turn the eight
+            // queue counters into a stream of atomics: 4e6 spins in 128-step
+            // launches walked 2.3x slower than fixed blocks, at 512 steps 3 %
+            // slower, at 768 3 % faster.
+            if (p.queue && !p.traj && p.n >= 2 * waves * 64u && iters >= kQueueMinSteps) {
+                if (hipMemsetAsync(p.queue, 0, kXcds * sizeof(uint32_t), s) != hipSuccess) return;
+                StepParams pq = p;
+                pq.queue_run = queue_run(p.n);
+                const dim3 g(waves), b(64);
+                if (p.walk_cell_major)
+                    hipLaunchKernelGGL((k_walk_queue<BOUND, INSTR, MOMENT, kRecsCellMajor>), g, b, 0,
+                                       s, pq, iters);
+                else
+                    hipLaunchKernelGGL((k_walk_queue<BOUND, INSTR, MOMENT, kRecsIndirect>), g, b, 0,
+                                       s, pq, iters);
+                return;
+            }
+        }
+        // Too few spins to fill every resident wave: fewer a wave (4 at least),
+        // as long as the waves are all resident at once.  A wave's turn costs
+        // about the same whatever its spins, and it ends with its slowest one.
+        // 1e4 spins: 55.8 ms at 64 spins a wave, 48.4 at 16, 45.6 at 8, 43.8 at
+        // 4; 1e5 spins: 29.9 ms at 64, 21.9 at 32 (3126 waves), 24.8 at 16 (6251,
+        // more than reside).  (The counting build keeps 64: its waves are counted.)
+        uint32_t pw = 64;
+        if constexpr (INSTR == kInstrNone)
+            while (pw > 4 && (p.n + pw / 2 - 1) / (pw / 2) <= waves) pw /= 2;
+        launch_blocks<BOUND, RNG, INSTR, MOMENT>(p, iters, pw, s);
     }
 }
 
@@ -2364,6 +2421,7 @@ hipError_t launch_moment_reset(uint32_t n, const float *x, const float *y, const
 }
 
 // ------------------------------------------------------------------------ //
+// ------------------------------------------------------------------------ //
 // Spatial reordering of spins (Morton order of their grid cells), so that the
 // lanes of a wavefront walk the same cells and triangle records.
 // ------------------------------------------------------------------------ //
@@ -2376,21 +2434,25 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {  // 10 bits -> every t
     return v;
 }
 
-// Sort key of a spin: its membrane-hit rate since the last reorder in 16
-// bands, highest first, then the Morton index of its cell.  Spins that hit at
-// like rates share a wavefront, so no lane holds the wave back for long; the
-// busiest workgroups are dispatched first; and within a band the Morton order
-// keeps neighbouring blocks on neighbouring triangles.  Resets the hit counts.
+// Sort key of a spin: the rate of its collision searches since the last
+// reorder in 16 bands, highest first, then the Morton index of its cell.
+// Spins that search at like rates share a wavefront: its search rounds are
+// then full where they are frequent and rare where they are not, and no lane
+// holds the wave back for long.  The busiest workgroups are dispatched first,
+// and within a band the Morton order keeps neighbouring blocks on neighbouring
+// triangles.  Resets the counts.
 __global__ __launch_bounds__(256) void k_sort_key(StepParams P, uint32_t *keys, uint32_t *vals) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= P.n) return;
     uint32_t cx, cy, cz;
     cell_of<1>(P, P.x[i], P.y[i], P.z[i], cx, cy, cz);
     uint32_t band = 0;
-    if (P.hits) {
-        if (P.hit_window)
-            band = (uint32_t)min<uint64_t>(15, (uint64_t)P.hits[i] * 16u / P.hit_window);
-        P.hits[i] = 0;
+    if (P.searches) {
+        // no history yet: the extra-axonal space, between the walls, first
+        band = P.search_window
+                   ? (uint32_t)min<uint64_t>(15, (uint64_t)P.searches[i] * 16u / P.search_window)
+                   : (P.label[i] & 0xFFu) == 0 ? 8u : 0u;
+        P.searches[i] = 0;
     }
     const uint32_t morton = spread3(cx) | (spread3(cy) << 1) | (spread3(cz) << 2);
     keys[i] = ((15u - band) << 28) | (morton >> 2);

@@ -215,7 +215,7 @@ int run_round(dsim_server *S, uint32_t *n_active, uint32_t *n_queued) {
         uint32_t total = 0;
         for (Req *r : S->active) {
             if (!r->ready || r->read_out || r->r.boundary != (uint32_t)(kind >> 1) ||
-                r->lobe_left == 0 || (r->sub->cell_mt.p == nullptr) != ((kind & 1) != 0) ||
+                r->lobe_left == 0 || (r->sub->kind == DSIM_GRID_TRIBOX) != ((kind & 1) != 0) ||
                 walk_blocks(r->r.n_spins) > cap)
                 continue;
             jobs.push_back(r);

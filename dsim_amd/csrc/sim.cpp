@@ -25,7 +25,7 @@ namespace {
 enum Field {
     F_X, F_Y, F_Z, F_MAG, F_PHASE, F_LABEL, F_ID,
     F_DISP, F_MOM = F_DISP + 3, F_MOMC = F_MOM + 3, F_X0 = F_MOMC + 3,
-    F_HITS = F_X0 + 3,  // membrane hits since the last reorder (orders the next one)
+    F_SEARCHES = F_X0 + 3,  // collision searches since the last reorder (orders the next one)
     F_WRAP,             // periodic voxel crossings (phase of the unwrapped position)
     F_COUNT
 };
@@ -185,10 +185,6 @@ static int sync_and_check(dsim_sim *s) {
         HIP_TRY(hipMemsetAsync(s->flags.p, 0, 16, s->stream));
         return fail(DSIM_ERR_OVERFLOW, "a spin exceeded 4096 collisions in one step");
     }
-    if (fl[0] & 4u) {
-        HIP_TRY(hipMemsetAsync(s->flags.p, 0, 16, s->stream));
-        return fail(DSIM_ERR_STATE, "collision search numbered a grid entry out of range");
-    }
     return DSIM_OK;
 }
 
@@ -324,14 +320,18 @@ static dsim::StepParams step_params(dsim_sim *s) {
     P.tri_mt = b->tri_mt.p;
     P.cell_start = b->d_cell_start.p;
     P.cell_tri = b->d_cell_tri.p;
-    P.cell_plane = b->cell_plane.p;
-    P.cell_mt = b->cell_mt.p;
-    P.n_entries = (uint32_t)b->d_cell_tri.n;
-    P.cell_clear = s->prm.mode == DSIM_MODE_PHYSICAL ? b->d_clearance.p : nullptr;
+    P.walk_start = b->walk_start.p;
+    P.walk_ent = b->walk_ent.p;
+    P.walk_rec = b->walk_rec.p;
+    P.walk_cell_major = b->kind != DSIM_GRID_TRIBOX;
+    P.walk_eps = b->walk_eps;
+    P.fine = s->prm.mode == DSIM_MODE_PHYSICAL ? b->d_fine.p : nullptr;
+    P.fine_q = b->fine_q;
     P.fiber_myelin = b->fiber_myelin.p;
     P.n_fibers = b->n_fibers;
     for (int k = 0; k < 3; ++k) {
         P.dims[k] = b->dims[k]; P.lo[k] = b->lo[k]; P.cell[k] = b->cell[k]; P.inv_cell[k] = b->inv_cell[k];
+        P.fine_dims[k] = b->fine_dims[k]; P.fine_inv[k] = b->fine_inv[k]; P.fine_w[k] = b->fine_w[k];
     }
     for (int c = 0; c < 4; ++c) {
         P.std_dev[c] = s->prm.std_dev[c];
@@ -355,7 +355,7 @@ static dsim::StepParams step_params(dsim_sim *s) {
     P.spin_id = s->f(F_ID);
     P.seed = s->seed.p;
     P.disp = s->ff(F_DISP); P.mom = s->ff(F_MOM); P.momc = s->ff(F_MOMC);
-    P.hits = s->sorting() ? s->f(F_HITS) : nullptr;
+    P.searches = s->sorting() ? s->f(F_SEARCHES) : nullptr;
     P.wrap = s->f(F_WRAP);
     P.key0 = (uint32_t)s->prm.seed;
     P.key1 = (uint32_t)(s->prm.seed >> 32);
@@ -364,12 +364,12 @@ static dsim::StepParams step_params(dsim_sim *s) {
     return P;
 }
 
-// Reorders the spins by their recent membrane-hit rate, then by the Morton
+// Reorders the spins by their recent rate of searches, then by the Morton
 // index of their cell (the key is built on the device).
 static int spatial_sort(dsim_sim *s) {
     dsim::StepParams P = step_params(s);
-    // hit counts cover the steps since the last reorder (none before the first)
-    P.hit_window = s->steps_since_sort < (1ull << 31) ? (uint32_t)s->steps_since_sort : 0u;
+    // the counts cover the steps since the last reorder (none before the first)
+    P.search_window = s->steps_since_sort < (1ull << 31) ? (uint32_t)s->steps_since_sort : 0u;
     const uint32_t *perm = nullptr;
     hipError_t e = dsim::launch_sort_perm(P, s->keys_a.p, s->keys_b.p, s->vals_a.p, s->vals_b.p,
                                           s->sort_tmp.p, s->sort_tmp.n, s->stream, &perm);

@@ -106,8 +106,8 @@ typedef struct {
     uint64_t seed;            /* Philox key */
     float spin_radius;        /* clamp margin (spinSystem.cpp:61: 0.005) */
     uint32_t sort_interval;   /* physical mode with Philox: reorder spins in device memory
-                               * every this many steps (0 = never), by recent membrane-hit
-                               * rate, then cell.  Results do not depend on it. */
+                               * every this many steps (0 = never), by recent rate of collision
+                               * searches, then cell.  Results do not depend on it. */
     uint32_t steps_per_launch; /* steps fused per kernel launch (0 = 1024; with reordering at
                                   most sort_interval) */
     float voxel_lo[3];        /* periodic voxel [voxel_lo, voxel_hi) per axis, normalised;     */
@@ -296,9 +296,10 @@ enum {
     DSIM_STAT_TRIPS = 1,         /* trips round a wave's loop (one search round each) */
     DSIM_STAT_SEARCH_LANES = 2,  /* lanes searching, summed over trips */
     DSIM_STAT_CELLS = 3,         /* grid cells listed by searching lanes */
-    DSIM_STAT_PLANE_TESTS = 4,   /* (segment, grid entry) plane tests */
+    DSIM_STAT_PLANE_TESTS = 4,   /* (segment, search entry) plane tests; an entry is a cell's
+                                  * triangle, or two of one plane */
     DSIM_STAT_PLANE_PASSES = 5,  /* wave passes of the plane test */
-    DSIM_STAT_TRI_TESTS = 6,     /* Moller-Trumbore tests (plane crossings) */
+    DSIM_STAT_TRI_TESTS = 6,     /* Moller-Trumbore tests (facets the segment may cross) */
     DSIM_STAT_TRI_PASSES = 7,    /* wave passes of the triangle test */
     DSIM_STAT_FP64_TESTS = 8,    /* near-grazing FP64 re-tests */
     DSIM_STAT_HITS = 9,          /* membrane hits */

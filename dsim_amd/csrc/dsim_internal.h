@@ -29,6 +29,12 @@ struct StepParams {
     const float4 *tri_mt;
     const uint32_t *cell_start;
     const uint32_t *cell_tri;
+    // reference mode on a reference grid, or null: per list entry of cell_tri two
+    // records, the triangle's normal and (first vertex, triangle), and per cell
+    // 27 bits: bit (dx + 1) + 3 (dy + 1) + 9 (dz + 1) is set if any cell of the box
+    // from the cell to its neighbour (dx, dy, dz) lists a triangle
+    const float4 *ref_rec;
+    const uint32_t *ref_mask;
     // search lists of the walk: entry k of cell c, walk_start[c] <= k <
     // walk_start[c + 1], is the triangles walk_ent[k] (.y kNone: one only) of
     // one plane; walk_rec holds two records per entry (walk_cell_major) or per

@@ -602,6 +602,43 @@ __global__ __launch_bounds__(kBlock) void k_walk_records(uint32_t n_tri, const f
     if (ok && dev < 1.0) atomicMax(eps, __float_as_uint((float)dev));
 }
 
+// Reference mode: per list entry the triangle's normal and its first vertex
+// with the triangle's index.
+__global__ __launch_bounds__(kBlock) void k_ref_records(uint32_t n, const uint32_t *tri,
+                                                        const float4 *ref, float4 *rec) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t t = tri[k];
+    const float4 a = ref[(size_t)t * 4], d = ref[(size_t)t * 4 + 3];
+    rec[(size_t)k * 2] = make_float4(a.x, a.y, a.z, 0.f);
+    rec[(size_t)k * 2 + 1] = make_float4(d.x, d.y, d.z, __uint_as_float(t));
+}
+
+// StepParams::ref_mask of each cell; boxes reach no further than the grid.
+__global__ __launch_bounds__(kBlock) void k_ref_masks(uint32_t dx, uint32_t dy, uint32_t dz,
+                                                      const uint32_t *start, uint32_t *mask) {
+    const uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (c >= (uint64_t)dx * dy * dz) return;
+    const int x = (int)(c % dx), y = (int)(c / dx % dy), z = (int)(c / ((uint64_t)dx * dy));
+    uint32_t listed = 0, m = 0;  // same bit order
+    for (int k = 0; k < 27; ++k) {
+        const int qx = x + k % 3 - 1, qy = y + k / 3 % 3 - 1, qz = z + k / 9 - 1;
+        if (qx < 0 || qy < 0 || qz < 0 || qx >= (int)dx || qy >= (int)dy || qz >= (int)dz) continue;
+        const uint64_t q = ((uint64_t)qz * dy + qy) * dx + qx;
+        if (start[q + 1] > start[q]) listed |= 1u << k;
+    }
+    for (int k = 0; k < 27; ++k) {
+        const int ex = k % 3 - 1, ey = k / 3 % 3 - 1, ez = k / 9 - 1;
+        bool any = false;
+        for (int b = 0; b < 8; ++b) {
+            const int bx = b & 1 ? ex : 0, by = b & 2 ? ey : 0, bz = b & 4 ? ez : 0;
+            any |= (listed >> ((bx + 1) + 3 * (by + 1) + 9 * (bz + 1))) & 1u;
+        }
+        if (any) m |= 1u << k;
+    }
+    mask[c] = m;
+}
+
 // Entries of cell c: EMIT false counts them, true writes them at start[c]
 // (and their records, cell-major).  A triangle whose partner precedes it in
 // the cell's list is that one's entry.
@@ -754,7 +791,28 @@ static int build_search_lists(dsim_substrate *S, hipStream_t st) {
     return DSIM_OK;
 }
 
+// Masks of grids up to this many cells (256 MB); larger ones list every box.
+constexpr uint32_t kRefMaskCells = 1u << 26;
+
+static int build_ref_tables(dsim_substrate *S, hipStream_t st) {
+    const uint32_t n = (uint32_t)S->d_cell_tri.n;  // one unused entry where the grid lists none
+    if (int rc = S->ref_rec.alloc((size_t)n * 2)) return rc;
+    if (S->n_tri) {
+        hipLaunchKernelGGL(k_ref_records, dim3(blocks_for(n)), dim3(kBlock), 0, st, n,
+                           S->d_cell_tri.p, S->tri_ref.p, S->ref_rec.p);
+        HIP_TRY(hipGetLastError());
+    }
+    if (S->n_cells > kRefMaskCells) return DSIM_OK;
+    if (int rc = S->ref_mask.alloc(S->n_cells)) return rc;
+    hipLaunchKernelGGL(k_ref_masks, dim3(blocks_for(S->n_cells)), dim3(kBlock), 0, st, S->dims[0],
+                       S->dims[1], S->dims[2], S->d_cell_start.p, S->ref_mask.p);
+    HIP_TRY(hipGetLastError());
+    return DSIM_OK;
+}
+
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
+    if (S->kind == DSIM_GRID_REFERENCE)
+        if (int rc = build_ref_tables(S, st)) return rc;
     if (int rc = build_search_lists(S, st)) return rc;
     return build_fine_clearance(S, st);
 }

@@ -108,6 +108,10 @@ struct dsim_substrate {
     dsim_host::DevBuf<float4> tri_ref, tri_mt, tri_aabb;
     dsim_host::DevBuf<uint32_t> d_cell_start, d_cell_tri;
     dsim_host::DevBuf<float> d_clearance, d_helpers;
+    // Reference grids: entry records and neighbour masks of the reference mode
+    // (StepParams::ref_rec, ref_mask).
+    dsim_host::DevBuf<float4> ref_rec;
+    dsim_host::DevBuf<uint32_t> ref_mask;
     // Search lists of the physical-mode walk (build_walk_tables): per grid cell
     // its triangles, two of one plane in one entry (the second kNone where there
     // is none), and the entries' plane and lateral records, cell-major for
@@ -132,6 +136,7 @@ struct dsim_substrate {
     ~dsim_substrate() {
         tri_ref.release(); tri_mt.release(); tri_aabb.release();
         walk_start.release(); walk_ent.release(); walk_rec.release();
+        ref_rec.release(); ref_mask.release();
         d_clearance.release(); d_helpers.release(); d_fine.release();
         d_cell_start.release(); d_cell_tri.release(); fiber_myelin.release();
     }

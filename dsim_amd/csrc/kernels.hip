@@ -128,16 +128,30 @@ struct Hit {
 };
 
 // triCollDetect, spinKernelCpu.cpp:354-395 (softsurfer test, reference order).
+// r = num / den in (0,1) needs num and den of one sign with |num| <= |den|; the
+// division (and the rest of the record) is only needed then.
+__device__ __forceinline__ bool ref_plane(const float4 a, const float4 d, float ox, float oy,
+                                          float oz, float px, float py, float pz, float &num,
+                                          float &den) {
+    num = a.x * (d.x - ox) + a.y * (d.y - oy) + a.z * (d.z - oz);
+    den = a.x * (px - ox) + a.y * (py - oy) + a.z * (pz - oz);
+    return (num > 0.0f && den >= num) || (num < 0.0f && den <= num);
+}
+__device__ __forceinline__ bool ref_plane(const float4 a, const float4 d, float ox, float oy,
+                                          float oz, float px, float py, float pz) {
+    float num, den;
+    return ref_plane(a, d, ox, oy, oz, px, py, pz, num, den);
+}
+// The whole test of triangle t; wall takes its normal and info.
 __device__ __forceinline__ void test_ref(const float4 *__restrict__ R, uint32_t t, float ox,
-                                         float oy, float oz, float px, float py, float pz, Hit &h) {
+                                         float oy, float oz, float px, float py, float pz, Hit &h,
+                                         float4 &wall) {
     h.type = 0;
     const float4 a = R[t * 4 + 0];
     const float4 d = R[t * 4 + 3];
-    float num = a.x * (d.x - ox) + a.y * (d.y - oy) + a.z * (d.z - oz);
-    float den = a.x * (px - ox) + a.y * (py - oy) + a.z * (pz - oz);
-    // r in (0,1) needs num and den of one sign with |num| <= |den|; the
-    // division (and the rest of the record) is only needed then.
-    if (!((num > 0.0f && den >= num) || (num < 0.0f && den <= num))) return;
+    wall = make_float4(a.x, a.y, a.z, d.w);
+    float num, den;
+    if (!ref_plane(a, d, ox, oy, oz, px, py, pz, num, den)) return;
     float r = num / den;
     if (!((0 < r) & (r < 1))) return;
     const float4 b = R[t * 4 + 1];
@@ -289,14 +303,6 @@ __device__ __forceinline__ void test_mt(const float4 *__restrict__ M, uint32_t t
     test_mt_crossing(M, t, ox, oy, oz, px, py, pz, h);
 }
 
-template <int MODE>
-__device__ __forceinline__ bool better(const Hit &c, const Hit &b) {
-    if (c.type == 0) return false;
-    if (MODE == 0) return c.d < b.d;
-    if (b.type == 0) return true;
-    return (c.d < b.d) || (c.d == b.d && c.idx < b.idx);
-}
-
 // Where the walk reads a search entry's records: kRecsCellMajor by entry (AABB
 // and reference grids), kRecsIndirect by its triangle (exact-membership
 // grids), kRecsEither deciding per launch parameter (a uniform branch; the
@@ -324,22 +330,7 @@ __device__ __forceinline__ bool walk_test(const StepParams &P, uint32_t k, uint3
     return ((s0 > 0.0f) != (s1 > 0.0f)) & !(far > lim);
 }
 
-// cubeCollDetect, spinKernelCpu.cpp:311-337, over one CSR cell.
-template <int MODE>
-__device__ __forceinline__ void cell_test(const StepParams &P, uint32_t cell, uint32_t excluded,
-                                          float ox, float oy, float oz, float px, float py,
-                                          float pz, Hit &best) {
-    uint32_t k0 = P.cell_start[cell], k1 = P.cell_start[cell + 1];
-    for (uint32_t k = k0; k < k1; ++k) {
-        uint32_t t = P.cell_tri[k];
-        if (t == excluded) continue;
-        Hit c;
-        test_ref(P.tri_ref, t, ox, oy, oz, px, py, pz, c);
-        if (better<MODE>(c, best)) best = c;
-    }
-}
-
-// reflectPos, spinKernelCpu.cpp:406-422 (MODE 1: wall holds the normal).
+// reflectPos, spinKernelCpu.cpp:406-422; wall holds the triangle's normal.
 template <int MODE>
 __device__ __forceinline__ void reflect(const StepParams &P, float sx, float sy, float sz,
                                         float tx, float ty, float tz, const Hit &h,
@@ -349,8 +340,7 @@ __device__ __forceinline__ void reflect(const StepParams &P, float sx, float sy,
         return;
     }
     if (MODE == 0) {
-        const float4 a = P.tri_ref[h.idx * 4];
-        float nx = a.x, ny = a.y, nz = a.z;
+        float nx = wall.x, ny = wall.y, nz = wall.z;
         float qx = tx - h.px, qy = ty - h.py, qz = tz - h.pz;
         rx = (1 - 2 * nx * nx) * qx - 2 * nx * ny * qy - 2 * nx * nz * qz + h.px;
         ry = -2 * nx * ny * qx + (1 - 2 * ny * ny) * qy - 2 * ny * nz * qz + h.py;
@@ -398,77 +388,6 @@ __device__ __forceinline__ void transit(const StepParams &P, uint32_t info, uint
     }
 }
 
-__device__ __forceinline__ uint32_t tri_info_of(const StepParams &P, uint32_t t, int mode) {
-    return mode == 0 ? __float_as_uint(P.tri_ref[t * 4 + 3].w)
-                     : __float_as_uint(P.tri_mt[t * 4 + 1].w);
-}
-
-// collDetectRectGrid, spinKernelCpu.cpp:198-301.  MODE 0 stops at the first
-// cell (x-major walk) holding a hit; MODE 1 visits the whole cell range and
-// keeps the nearest hit (t, then triangle index).
-template <int MODE>
-__device__ __forceinline__ void collide(const StepParams &P, float ox, float oy, float oz,
-                                        float &px, float &py, float &pz, float u, uint32_t &comp,
-                                        uint32_t &fiber, uint32_t &first, uint32_t &last,
-                                        uint32_t &ncoll) {
-    float ex = px, ey = py, ez = pz;
-    uint32_t excluded = kNone;
-    float umax = 1.0f, umin = 0.0f;
-    for (int guard = 0; guard < 4096; ++guard) {
-        uint32_t sx, sy, sz, tx, ty, tz;
-        cell_of<MODE>(P, ox, oy, oz, sx, sy, sz);
-        cell_of<MODE>(P, px, py, pz, tx, ty, tz);
-        uint32_t ix = (uint32_t)((tx > sx) - (tx < sx));
-        uint32_t iy = (uint32_t)((ty > sy) - (ty < sy));
-        uint32_t iz = (uint32_t)((tz > sz) - (tz < sz));
-        Hit best;
-        best.type = 0;
-        best.idx = kNone;
-        best.d = (MODE == 0) ? 400000000.0f : 2.0f;
-        best.px = best.py = best.pz = 0.0f;
-        uint32_t cx = sx;
-        do {
-            uint32_t cy = sy;
-            do {
-                uint32_t cz = sz;
-                do {
-                    uint32_t cell = cell_hash(P, cx, cy, cz);
-                    if (MODE == 0) {
-                        Hit c;
-                        c.type = 0;
-                        c.idx = kNone;
-                        c.d = 400000000.0f;
-                        cell_test<0>(P, cell, excluded, ox, oy, oz, px, py, pz, c);
-                        best = c;
-                    } else {
-                        cell_test<1>(P, cell, excluded, ox, oy, oz, px, py, pz, best);
-                    }
-                    cz += iz;
-                } while (cz != tz + iz && (MODE == 1 || best.type == 0));
-                cy += iy;
-            } while (cy != ty + iy && (MODE == 1 || best.type == 0));
-            cx += ix;
-        } while (cx != tx + ix && (MODE == 1 || best.type == 0));
-        if (best.type == 0) break;
-        if (ncoll == 0) first = best.idx;
-        last = best.idx;
-        ncoll += 1;
-        float thr = umax - (umax - umin) * P.perm;
-        if (u <= thr) {
-            reflect<MODE>(P, ox, oy, oz, px, py, pz, best, float4(), ex, ey, ez);
-            umax = thr;
-        } else {
-            umin = thr;
-            transit<MODE>(P, tri_info_of(P, best.idx, MODE), comp, fiber);
-        }
-        ox = best.px; oy = best.py; oz = best.pz;
-        px = ex; py = ey; pz = ez;
-        excluded = best.idx;
-        if (guard == 4095) atomicOr(P.flags, 1u);
-    }
-    px = ex; py = ey; pz = ez;
-}
-
 // Clearance shortcut.  The clearance at a point bounds from below its distance
 // to any triangle registered in the grid, so a step whose length is less than
 // the sum of its end points' clearances crosses none: the two balls cover it.
@@ -488,99 +407,6 @@ __device__ __forceinline__ float clearance_at(const StepParams &P, float x, floa
         return -1e30f;
     return P.fine_q *
            (float)P.fine[((uint32_t)qz * P.fine_dims[1] + (uint32_t)qy) * P.fine_dims[0] + (uint32_t)qx];
-}
-
-// ------------------------------------------------------------------------ //
-// Reference-mode step kernel: cpuIntegrate (spinKernelCpu.cpp:430-499) for
-// `iters` steps per launch with the spin's state held in registers.
-// ------------------------------------------------------------------------ //
-template <int MODE, bool PERIODIC, int RNG, bool TRACE, bool MOMENT>
-__global__ __launch_bounds__(64) void k_step(StepParams P, uint32_t iters) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.n) return;
-    // the spin's identity keys its random stream, injected normals and trace
-    const uint32_t sid = P.spin_id ? P.spin_id[i] : i;
-    float x = P.x[i], y = P.y[i], z = P.z[i];
-    float mag = P.mag[i];
-    float ph = MOMENT ? 0.0f : P.phase[i];
-    uint32_t lab = P.label[i];
-    uint32_t comp = lab & 0xFFu, fiber = (lab >> 8) & 0xFFFFu;
-    uint32_t s0 = 0, s1 = 0;
-    if (RNG == kRngMwc) { s0 = P.seed[2 * i]; s1 = P.seed[2 * i + 1]; }
-    float dx = 0.f, dy = 0.f, dz = 0.f, mx = 0.f, my = 0.f, mz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
-    if (MOMENT) {
-        dx = P.disp[i]; dy = P.disp[P.n + i]; dz = P.disp[2 * P.n + i];
-        mx = P.mom[i]; my = P.mom[P.n + i]; mz = P.mom[2 * P.n + i];
-        cx = P.momc[i]; cy = P.momc[P.n + i]; cz = P.momc[2 * P.n + i];
-    }
-    for (uint32_t it = 0; it < iters; ++it) {
-        const uint64_t gstep = P.step0 + it;
-        float n0, n1, n2, u = 0.0f;
-        if (RNG == kRngInject) {
-            float4 q = P.inject[(size_t)it * P.n + sid];
-            n0 = q.x; n1 = q.y; n2 = q.z; u = q.w;
-        } else if (RNG == kRngMwc) {
-            mwc_randn(s0, s1, n0, n1, n2, u);
-        } else {
-            philox_draw(P.key0, P.key1, sid, gstep, n0, n1, n2, u);
-        }
-        const float sd = comp == 0 ? P.std_dev[0] : comp == 1 ? P.std_dev[1]
-                       : comp == 2 ? P.std_dev[2] : P.std_dev[3];
-        const float ox = x, oy = y, oz = z;
-        float px, py, pz;
-        if (MODE == 0) {
-            px = x + n0 * sd; py = y + n1 * sd; pz = z + n2 * sd;
-        } else {
-            px = fmaf(n0, sd, x); py = fmaf(n1, sd, y); pz = fmaf(n2, sd, z);
-        }
-        uint32_t first = kNone, last = kNone, ncoll = 0;
-        collide<MODE>(P, ox, oy, oz, px, py, pz, u, comp, fiber, first, last, ncoll);
-        if (!PERIODIC) {
-            // spinKernelCpu.cpp:469-474
-            if (px > P.clamp_hi) px = P.clamp_hi; else if (px < P.clamp_lo) px = P.clamp_lo;
-            if (py > P.clamp_hi) py = P.clamp_hi; else if (py < P.clamp_lo) py = P.clamp_lo;
-            if (pz > P.clamp_hi) pz = P.clamp_hi; else if (pz < P.clamp_lo) pz = P.clamp_lo;
-        }
-        if (MOMENT) {
-            dx += px - ox; dy += py - oy; dz += pz - oz;
-        }
-        if (PERIODIC) {
-            if (px >= 1.0f) px -= 2.0f; else if (px < -1.0f) px += 2.0f;
-            if (py >= 1.0f) py -= 2.0f; else if (py < -1.0f) py += 2.0f;
-            if (pz >= 1.0f) pz -= 2.0f; else if (pz < -1.0f) pz += 2.0f;
-        }
-        x = px; y = py; z = pz;
-        const float t2 = comp == 0 ? P.t2[0] : comp == 1 ? P.t2[1] : comp == 2 ? P.t2[2] : P.t2[3];
-        const float dc = comp == 0 ? P.decay[0] : comp == 1 ? P.decay[1]
-                       : comp == 2 ? P.decay[2] : P.decay[3];
-        if (MODE == 0) mag += -mag / t2 * P.dt;          // spinKernelCpu.cpp:486
-        else mag = fmaf(-mag, dc, mag);
-        if (!MOMENT) ph += (P.gx * x + P.gy * y + P.gz * z) * P.pc;  // spinKernelCpu.cpp:490
-        if (MOMENT && P.weight != 0.0f) {
-            float yv, tv;
-            yv = fmaf(P.weight, dx, -cx); tv = mx + yv; cx = (tv - mx) - yv; mx = tv;
-            yv = fmaf(P.weight, dy, -cy); tv = my + yv; cy = (tv - my) - yv; my = tv;
-            yv = fmaf(P.weight, dz, -cz); tv = mz + yv; cz = (tv - mz) - yv; mz = tv;
-        }
-        if (TRACE) {
-            uint32_t qx, qy, qz;
-            cell_of<MODE>(P, x, y, z, qx, qy, qz);
-            uint32_t *tr = P.trace + ((size_t)it * P.n + sid) * 5;
-            tr[0] = first; tr[1] = last; tr[2] = ncoll;
-            tr[3] = cell_hash(P, qx, qy, qz);
-            tr[4] = comp | (fiber << 8);
-        }
-    }
-    P.x[i] = x; P.y[i] = y; P.z[i] = z;
-    P.mag[i] = mag;
-    if (!MOMENT) P.phase[i] = ph;
-    P.label[i] = comp | (fiber << 8);
-    if (RNG == kRngMwc) { P.seed[2 * i] = s0; P.seed[2 * i + 1] = s1; }
-    if (MOMENT) {
-        P.disp[i] = dx; P.disp[P.n + i] = dy; P.disp[2 * P.n + i] = dz;
-        P.mom[i] = mx; P.mom[P.n + i] = my; P.mom[2 * P.n + i] = mz;
-        P.momc[i] = cx; P.momc[P.n + i] = cy; P.momc[2 * P.n + i] = cz;
-    }
 }
 
 // ------------------------------------------------------------------------ //
@@ -1321,6 +1147,392 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     walk_body<BOUND, kRngPhilox, INSTR, MOMENT, RECS, true>(P, blockIdx.x, iters, 64u, scratch);
 }
 
+// ------------------------------------------------------------------------ //
+// Reference-mode steps: cpuIntegrate (spinKernelCpu.cpp:430-499), `iters` steps
+// per launch with the spins' state in registers, laid out as the walk above:
+// a lane a spin, every lane that is free starts its next step, the segments of
+// the others are searched together.
+//
+// collDetectRectGrid (spinKernelCpu.cpp:198-301) visits the cells from the
+// start cell towards the end cell, x outermost, and stops at the first that
+// holds a hit, taking its nearest (the first of equals).  Here all cells of
+// the box are listed in that order, their (lane, entry) pairs numbered over
+// the wave and tested 128 at a time against the entry's plane; the pairs that
+// cross it go through the rest of triCollDetect from a queue.  The lane's
+// minimum over (cell's place in the order, squared distance) is what the
+// visit in order finds, and among equals the lowest triangle is the first (the
+// lists ascend).  A step to a neighbouring cell at most asks one mask word of
+// its start cell whether any cell of the box lists anything.
+//
+// Bound: a wave's instruction stream and the latency of its dependent loads.
+// With a lane searching its own cells one entry after another (two dependent
+// loads an entry, a wave as slow as its slowest lane) ten steps took 0.24 ms
+// for 1e3 spins and 500 steps 52 ms for 1e6.
+// ------------------------------------------------------------------------ //
+constexpr uint32_t kRefCells = 128;  // cells listed per wave and search round
+constexpr uint32_t kRefQueue = 256;  // pairs awaiting the triangle test (a pass queues 128)
+
+struct RefScratch {
+    uint2 cell[kRefCells];  // (first entry - lane-local pair number, lane-local end)
+    float4 o[64];           // segment start; .w = excluded triangle
+    float4 p[64];           // segment end
+    float4 hit[64];         // nearest hit point; .w = hit type
+    float4 wall[64];        // normal and info of its triangle
+    uint2 meta[64];         // (first pair number, first cell)
+    unsigned long long best[64];  // (cell's place, squared distance)
+    uint32_t tri[64];             // lowest triangle of those at `best`
+    uint32_t map[kPass];    // lane + 1 at the pass position where its pairs start
+    uint2 queue[kRefQueue];  // (triangle, lane | cell's place << 6)
+};
+
+// floor((v - lo) / cell), clamped, as calcCubePos rounds it: the quotient by
+// multiplication decides unless it is too near a whole number.
+__device__ __forceinline__ uint32_t ref_cell(float v, float lo, float cell, float inv, uint32_t n) {
+    const float d = v - lo;
+    float q = d * inv;
+    if (!(fabsf(q - rintf(q)) > 1e-6f * fmaxf(fabsf(q), 1.0f))) q = d / cell;
+    return clamp_cell(floorf(q), n);
+}
+
+// Triangle pass over queue[0, qlen) (wave-uniform): triCollDetect's decision
+// for each pair, the lanes' minima into best[], tri[], hit[] and wall[].
+__device__ __forceinline__ void ref_triangle_pass(const StepParams &P, RefScratch &L, uint32_t lane,
+                                                  uint32_t qlen) {
+    for (uint32_t qb = 0; qb < qlen; qb += 64) {
+        wave_lds_sync();
+        Hit h;
+        h.type = 0;
+        uint32_t own = 0;
+        unsigned long long key = ~0ull, was = ~0ull;
+        float4 wall = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (qb + lane < qlen) {
+            const uint2 e = L.queue[qb + lane];
+            own = e.y & 63u;
+            const float4 so = L.o[own], sp = L.p[own];
+            was = L.best[own];
+            test_ref(P.tri_ref, e.x, so.x, so.y, so.z, sp.x, sp.y, sp.z, h, wall);
+            // the reference's search starts from this distance
+            if (h.type && h.d < 400000000.0f)
+                key = ((unsigned long long)(e.y >> 6) << 32) | __float_as_uint(h.d);
+            else
+                h.type = 0;
+        }
+        wave_lds_sync();
+        if (h.type) atomicMin(&L.best[own], key);
+        wave_lds_sync();
+        const bool at = h.type && L.best[own] == key;
+        if (at && was != key) L.tri[own] = kNone;  // a new minimum: no triangle yet
+        wave_lds_sync();
+        if (at) atomicMin(&L.tri[own], h.idx);
+        wave_lds_sync();
+        if (at && L.tri[own] == h.idx) {
+            L.hit[own] = make_float4(h.px, h.py, h.pz, __uint_as_float(h.type));
+            L.wall[own] = wall;
+        }
+    }
+    wave_lds_sync();
+}
+
+// Plane test of pair j for its owner lane (the first conditions of
+// triCollDetect): whether the rest of the test is needed, and the pair's queue
+// entry.
+template <bool MAJOR>
+__device__ __forceinline__ bool ref_pair(const StepParams &P, const RefScratch &L, uint32_t j,
+                                         uint32_t total, uint32_t owner, uint2 &entry) {
+    if (j >= total) return false;
+    const uint2 m = L.meta[owner];
+    const uint32_t r = j - m.x;
+    uint32_t s = m.y;
+    uint2 e = L.cell[s];
+    while (r >= e.y && s + 1 < kRefCells) e = L.cell[++s];
+    const uint32_t k = e.x + r;
+    float4 a, d;
+    uint32_t t;
+    if (MAJOR) {
+        a = P.ref_rec[(size_t)k * 2];
+        d = P.ref_rec[(size_t)k * 2 + 1];
+        t = __float_as_uint(d.w);
+    } else {
+        t = P.cell_tri[k];
+        a = P.tri_ref[(size_t)t * 4];
+        d = P.tri_ref[(size_t)t * 4 + 3];
+    }
+    const float4 so = L.o[owner], sp = L.p[owner];
+    entry = make_uint2(t, owner | ((s - m.y) << 6));
+    return t != __float_as_uint(so.w) &&
+           ref_plane(a, d, so.x, so.y, so.z, sp.x, sp.y, sp.z);
+}
+
+// One search round, called by all 64 lanes together: for each lane with
+// `search` set the hit of the segment o-p that the visit of its box's cells in
+// order finds first, best[lane] ~0 when there is none.  Returns false when the
+// wave's cell list is full (the lane searches again), or when no hit is found
+// yet and cells remain: a box is searched kRefCells cells per round, from cell
+// `slice` of the order (0 for a new segment; advanced here).  (sx, sy, sz) and
+// (tx, ty, tz): the cells of o and p.
+template <bool MAJOR>
+__device__ __forceinline__ bool ref_search(const StepParams &P, RefScratch &L, uint32_t lane,
+                                           bool search, float ox, float oy, float oz, float px,
+                                           float py, float pz, uint32_t sx, uint32_t sy, uint32_t sz,
+                                           uint32_t tx, uint32_t ty, uint32_t tz,
+                                           uint32_t excluded, uint32_t &slice) {
+    const int ix = (int)(tx > sx) - (int)(tx < sx), iy = (int)(ty > sy) - (int)(ty < sy),
+              iz = (int)(tz > sz) - (int)(tz < sz);
+    const uint32_t ny = (uint32_t)abs((int)(ty - sy)) + 1, nz = (uint32_t)abs((int)(tz - sz)) + 1;
+    const uint32_t cells = ((uint32_t)abs((int)(tx - sx)) + 1) * ny * nz;
+    const uint32_t nreq = search ? min(cells - slice, kRefCells) : 0u;
+    const uint32_t send = wave_incl_sum(nreq);
+    const uint32_t soff = send - nreq;
+    const bool coop = nreq > 0 && send <= kRefCells;
+    uint32_t cnt = 0;
+    if (coop) {
+        L.o[lane] = make_float4(ox, oy, oz, __uint_as_float(excluded));
+        L.p[lane] = make_float4(px, py, pz, 0.f);
+        L.best[lane] = ~0ull;
+        uint32_t x = 0, y = 0, z = 0;
+        if (slice) {  // a later slice of a long box
+            z = slice % nz;
+            y = slice / nz % ny;
+            x = slice / (nz * ny);
+        }
+        for (uint32_t q0 = 0; q0 < nreq; q0 += 4) {
+            uint32_t k0[4], k1[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                k0[q] = k1[q] = 0;
+                if (q0 + q < nreq) {
+                    const uint32_t c = cell_hash(P, sx + (uint32_t)(ix * (int)x),
+                                                 sy + (uint32_t)(iy * (int)y),
+                                                 sz + (uint32_t)(iz * (int)z));
+                    k0[q] = P.cell_start[c];
+                    k1[q] = P.cell_start[c + 1];
+                    if (++z == nz) { z = 0; if (++y == ny) { y = 0; ++x; } }
+                }
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                if (q0 + q < nreq) {
+                    L.cell[soff + q0 + q] = make_uint2(k0[q] - cnt, cnt + (k1[q] - k0[q]));
+                    cnt += k1[q] - k0[q];
+                }
+            }
+        }
+    }
+    const uint32_t cend = wave_incl_sum(cnt);
+    const uint32_t off = cend - cnt;
+    const uint32_t total = __builtin_amdgcn_readlane(cend, 63);
+    if (coop) L.meta[lane] = make_uint2(off, soff);
+    uint32_t qlen = 0;  // wave-uniform
+    for (uint32_t base = 0; base < total; base += kPass) {
+        L.map[lane] = 0;
+        L.map[lane + 64] = 0;
+        wave_lds_sync();
+        if (cnt && off < base + kPass && off + cnt > base) L.map[off > base ? off - base : 0] = lane + 1;
+        wave_lds_sync();
+        const uint32_t own_a = wave_incl_max(L.map[lane]);
+        uint2 ea, eb;
+        bool cb = false;
+        if (base + 64 < total) {
+            const uint32_t own_b = max(wave_incl_max(L.map[lane + 64]),
+                                       __builtin_amdgcn_readlane(own_a, 63));
+            cb = ref_pair<MAJOR>(P, L, base + 64 + lane, total, own_b - 1, eb);
+        }
+        const bool ca = ref_pair<MAJOR>(P, L, base + lane, total, own_a - 1, ea);
+        const unsigned long long ba = __ballot(ca), bb = __ballot(cb);
+        if (ca) L.queue[qlen + lane_rank(ba)] = ea;
+        qlen += popc(ba);
+        if (cb) L.queue[qlen + lane_rank(bb)] = eb;
+        qlen += popc(bb);
+        if (qlen > kRefQueue - kPass) {
+            ref_triangle_pass(P, L, lane, qlen);
+            qlen = 0;
+        }
+    }
+    if (qlen) ref_triangle_pass(P, L, lane, qlen);
+    wave_lds_sync();
+    if (!coop) return false;
+    if (L.best[lane] != ~0ull || slice + nreq >= cells) return true;
+    slice += nreq;
+    return false;
+}
+
+template <int RNG, bool TRACE, bool MOMENT, bool MAJOR>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_ref_walk(
+    StepParams P, uint32_t iters, uint32_t per_wave) {
+    __shared__ RefScratch L;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t i = blockIdx.x * per_wave + lane;
+    const bool live = lane < per_wave && i < P.n;
+    // the spin's identity keys its random stream, injected normals and trace
+    uint32_t sid = 0, comp = 0, fiber = kFiberNone, s0 = 0, s1 = 0;
+    float x = 0.f, y = 0.f, z = 0.f, mag = 0.f, ph = 0.f;
+    float dx = 0.f, dy = 0.f, dz = 0.f, mx = 0.f, my = 0.f, mz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
+    uint32_t sx = 0, sy = 0, sz = 0;  // cell of the segment's start
+    uint32_t tx = 0, ty = 0, tz = 0;  // and of its end
+    auto cell_at = [&](float vx, float vy, float vz, uint32_t &qx, uint32_t &qy, uint32_t &qz) {
+        qx = ref_cell(vx, P.lo[0], P.cell[0], P.inv_cell[0], P.dims[0]);
+        qy = ref_cell(vy, P.lo[1], P.cell[1], P.inv_cell[1], P.dims[1]);
+        qz = ref_cell(vz, P.lo[2], P.cell[2], P.inv_cell[2], P.dims[2]);
+    };
+    if (live) {
+        sid = P.spin_id ? P.spin_id[i] : i;
+        x = P.x[i]; y = P.y[i]; z = P.z[i];
+        mag = P.mag[i];
+        if (!MOMENT) ph = P.phase[i];
+        const uint32_t lab = P.label[i];
+        comp = lab & 0xFFu; fiber = (lab >> 8) & 0xFFFFu;
+        if (RNG == kRngMwc) { s0 = P.seed[2 * i]; s1 = P.seed[2 * i + 1]; }
+        if (MOMENT) {
+            dx = P.disp[i]; dy = P.disp[P.n + i]; dz = P.disp[2 * P.n + i];
+            mx = P.mom[i]; my = P.mom[P.n + i]; mz = P.mom[2 * P.n + i];
+            cx = P.momc[i]; cy = P.momc[P.n + i]; cz = P.momc[2 * P.n + i];
+        }
+        cell_at(x, y, z, sx, sy, sz);
+    }
+    uint32_t it = live ? 0u : iters;
+    bool pending = false, complete = false;
+    float ox = 0.f, oy = 0.f, oz = 0.f, px = 0.f, py = 0.f, pz = 0.f;
+    float u = 0.f, umax = 1.f, umin = 0.f;
+    uint32_t excluded = kNone, first = kNone, last = kNone, ncoll = 0, slice = 0;
+    // state after collision number `sat` of the step (a power of two from 16 on)
+    float sox = 0.f, soy = 0.f, soz = 0.f, spx = 0.f, spy = 0.f, spz = 0.f, sumax = 0.f, sumin = 0.f;
+    uint32_t sex = 0, slab = 0, sat = 0;
+    for (;;) {
+        if (complete) {
+            complete = false;
+            const float ux = px, uy = py, uz = pz;
+            // spinKernelCpu.cpp:469-474
+            if (px > P.clamp_hi) px = P.clamp_hi; else if (px < P.clamp_lo) px = P.clamp_lo;
+            if (py > P.clamp_hi) py = P.clamp_hi; else if (py < P.clamp_lo) py = P.clamp_lo;
+            if (pz > P.clamp_hi) pz = P.clamp_hi; else if (pz < P.clamp_lo) pz = P.clamp_lo;
+            if (MOMENT) {
+                dx += px - x; dy += py - y; dz += pz - z;
+            }
+            x = px; y = py; z = pz;
+            // the next step starts in the cell this one ended in
+            sx = tx; sy = ty; sz = tz;
+            if ((px != ux) | (py != uy) | (pz != uz)) cell_at(x, y, z, sx, sy, sz);
+            const float t2 = comp == 0 ? P.t2[0] : comp == 1 ? P.t2[1] : comp == 2 ? P.t2[2] : P.t2[3];
+            mag += -mag / t2 * P.dt;                                     // spinKernelCpu.cpp:486
+            if (!MOMENT) ph += (P.gx * x + P.gy * y + P.gz * z) * P.pc;  // spinKernelCpu.cpp:490
+            if (MOMENT && P.weight != 0.0f) {
+                float yv, tv;
+                yv = fmaf(P.weight, dx, -cx); tv = mx + yv; cx = (tv - mx) - yv; mx = tv;
+                yv = fmaf(P.weight, dy, -cy); tv = my + yv; cy = (tv - my) - yv; my = tv;
+                yv = fmaf(P.weight, dz, -cz); tv = mz + yv; cz = (tv - mz) - yv; mz = tv;
+            }
+            if (TRACE) {
+                uint32_t *tr = P.trace + ((size_t)it * P.n + sid) * 5;
+                tr[0] = first; tr[1] = last; tr[2] = ncoll;
+                tr[3] = cell_hash(P, sx, sy, sz);
+                tr[4] = comp | (fiber << 8);
+            }
+            ++it;
+        }
+        if (it < iters && !pending) {
+            float n0, n1, n2;
+            if (RNG == kRngInject) {
+                const float4 r = P.inject[(size_t)it * P.n + sid];
+                n0 = r.x; n1 = r.y; n2 = r.z; u = r.w;
+            } else if (RNG == kRngMwc) {
+                mwc_randn(s0, s1, n0, n1, n2, u);
+            } else {
+                philox_draw(P.key0, P.key1, sid, P.step0 + it, n0, n1, n2, u);
+            }
+            const float sd = comp == 0 ? P.std_dev[0] : comp == 1 ? P.std_dev[1]
+                           : comp == 2 ? P.std_dev[2] : P.std_dev[3];
+            ox = x; oy = y; oz = z;
+            px = x + n0 * sd; py = y + n1 * sd; pz = z + n2 * sd;
+            first = last = excluded = kNone;
+            ncoll = 0;
+            umax = 1.0f; umin = 0.0f;
+            slice = 0;
+            cell_at(px, py, pz, tx, ty, tz);
+            pending = true;
+            if (P.ref_mask) {
+                const uint32_t ex = tx - sx + 1u, ey = ty - sy + 1u, ez = tz - sz + 1u;
+                if (ex < 3u && ey < 3u && ez < 3u) {
+                    const uint32_t m = P.ref_mask[cell_hash(P, sx, sy, sz)];
+                    if (!((m >> (ex + 3u * ey + 9u * ez)) & 1u)) {
+                        pending = false;
+                        complete = true;
+                    }
+                }
+            }
+        }
+        if (__ballot(pending) == 0ull) {
+            if (__ballot(complete) == 0ull) break;  // every lane has walked its steps
+            continue;
+        }
+        const bool done = ref_search<MAJOR>(P, L, lane, pending, ox, oy, oz, px, py, pz, sx, sy, sz, tx,
+                                            ty, tz, excluded, slice);
+        if (pending && done) {
+            slice = 0;
+            if (L.best[lane] == ~0ull) {
+                pending = false;
+                complete = true;
+            } else {
+                const float4 hp = L.hit[lane], wall = L.wall[lane];
+                Hit h;
+                h.px = hp.x; h.py = hp.y; h.pz = hp.z;
+                h.type = __float_as_uint(hp.w);
+                h.idx = L.tri[lane];
+                if (ncoll == 0) first = h.idx;
+                last = h.idx;
+                ncoll += 1;
+                const float thr = umax - (umax - umin) * P.perm;
+                float ex = px, ey = py, ez = pz;
+                if (u <= thr) {
+                    reflect<0>(P, ox, oy, oz, px, py, pz, h, wall, ex, ey, ez);
+                    umax = thr;
+                } else {
+                    umin = thr;
+                    transit<0>(P, __float_as_uint(wall.w), comp, fiber);
+                }
+                ox = h.px; oy = h.py; oz = h.pz;
+                px = ex; py = ey; pz = ez;
+                excluded = h.idx;
+                cell_at(ox, oy, oz, sx, sy, sz);
+                cell_at(px, py, pz, tx, ty, tz);
+                // A step whose loop does not end (a facet's two triangles hit in
+                // turn) repeats its state exactly: whole periods are left out.
+                // Searched for one by one, a wave took milliseconds for it.
+                if (ncoll >= 16) {
+                    const bool same = ncoll > 16 && sox == ox && soy == oy && soz == oz &&
+                                      spx == px && spy == py && spz == pz && sex == excluded &&
+                                      sumax == umax && sumin == umin && slab == (comp | (fiber << 8));
+                    if (same) {
+                        const uint32_t period = ncoll - sat;
+                        ncoll += (4096 - ncoll) / period * period;
+                    } else if ((ncoll & (ncoll - 1)) == 0) {
+                        sox = ox; soy = oy; soz = oz;
+                        spx = px; spy = py; spz = pz;
+                        sex = excluded; sumax = umax; sumin = umin;
+                        slab = comp | (fiber << 8);
+                        sat = ncoll;
+                    }
+                }
+                if (ncoll == 4096) {
+                    atomicOr(P.flags, 1u);
+                    pending = false;
+                    complete = true;
+                }
+            }
+        }
+    }
+    if (!live) return;
+    P.x[i] = x; P.y[i] = y; P.z[i] = z;
+    P.mag[i] = mag;
+    if (!MOMENT) P.phase[i] = ph;
+    P.label[i] = comp | (fiber << 8);
+    if (RNG == kRngMwc) { P.seed[2 * i] = s0; P.seed[2 * i + 1] = s1; }
+    if (MOMENT) {
+        P.disp[i] = dx; P.disp[P.n + i] = dy; P.disp[2 * P.n + i] = dz;
+        P.mom[i] = mx; P.mom[P.n + i] = my; P.mom[2 * P.n + i] = mz;
+        P.momc[i] = cx; P.momc[P.n + i] = cy; P.momc[2 * P.n + i] = cz;
+    }
+}
+
 // Batched walk for the server: the blocks of one launch are shared out over
 // the jobs of a table in device memory (job j owns blocks [block_start[j],
 // block_start[j+1])).  Each job is a whole simulation (its own substrate,
@@ -1397,12 +1609,25 @@ static void launch_blocks(const StepParams &p, uint32_t iters, uint32_t per_wave
 
 template <int MODE, int BOUND, int RNG, int INSTR, bool MOMENT>
 static void launch_one(const StepParams &p, uint32_t iters, hipStream_t s) {
+    const uint32_t waves = resident_walk_waves();
+    // Too few spins to fill every resident wave: fewer a wave (4 at least), as
+    // long as the waves are all resident at once.  A wave's turn costs about the
+    // same whatever its spins, and it ends with its slowest one.  Physical mode,
+    // 1e4 spins: 55.8 ms at 64 spins a wave, 48.4 at 16, 45.6 at 8, 43.8 at 4; 1e5
+    // spins: 29.9 ms at 64, 21.9 at 32 (3126 waves), 24.8 at 16 (6251, more than
+    // reside).  (The counting build keeps 64: its waves are counted.)
+    uint32_t pw = 64;
+    if constexpr (INSTR == kInstrNone)
+        while (pw > 4 && (p.n + pw / 2 - 1) / (pw / 2) <= waves) pw /= 2;
     if constexpr (MODE == 0) {
-        hipLaunchKernelGGL((k_step<0, BOUND != kBoundClamp, RNG, INSTR == kInstrTrace, MOMENT>),
-                           dim3((p.n + 63) / 64), dim3(64), 0, s, p, iters);
-        return;
+        const dim3 g((p.n + pw - 1) / pw), b(64);
+        if (p.ref_rec)
+            hipLaunchKernelGGL((k_ref_walk<RNG, INSTR == kInstrTrace, MOMENT, true>), g, b, 0, s, p,
+                               iters, pw);
+        else
+            hipLaunchKernelGGL((k_ref_walk<RNG, INSTR == kInstrTrace, MOMENT, false>), g, b, 0, s, p,
+                               iters, pw);
     } else {
-        const uint32_t waves = resident_walk_waves();
         if constexpr (RNG == kRngPhilox && INSTR != kInstrTrace) {
             // the persistent walk once every resident lane has two spins or more
             // and a launch walks at least kQueueMinSteps steps; not while a
@@ -1426,15 +1651,6 @@ static void launch_one(const StepParams &p, uint32_t iters, hipStream_t s) {
                 return;
             }
         }
-        // Too few spins to fill every resident wave: fewer a wave (4 at least),
-        // as long as the waves are all resident at once.  A wave's turn costs
-        // about the same whatever its spins, and it ends with its slowest one.
-        // 1e4 spins: 55.8 ms at 64 spins a wave, 48.4 at 16, 45.6 at 8, 43.8 at
-        // 4; 1e5 spins: 29.9 ms at 64, 21.9 at 32 (3126 waves), 24.8 at 16 (6251,
-        // more than reside).  (The counting build keeps 64: its waves are counted.)
-        uint32_t pw = 64;
-        if constexpr (INSTR == kInstrNone)
-            while (pw > 4 && (p.n + pw / 2 - 1) / (pw / 2) <= waves) pw /= 2;
         launch_blocks<BOUND, RNG, INSTR, MOMENT>(p, iters, pw, s);
     }
 }
@@ -2007,10 +2223,11 @@ __device__ __forceinline__ void ray_add(const LabelParams &P, uint32_t t, float4
         lo.z > rmaxz)
         return;
     Hit h;
+    float4 wall;
     if (P.use_mt)
         test_mt(P.tri_mt, t, sx, sy, sz, ex, ey, ez, h);
     else
-        test_ref(P.tri_ref, t, sx, sy, sz, ex, ey, ez, h);
+        test_ref(P.tri_ref, t, sx, sy, sz, ex, ey, ez, h, wall);
     if (h.type == 0) return;
     const uint32_t info = __float_as_uint(lo.w);
     const uint32_t f = info & 0xFFFFu, m = info >> 16;

@@ -320,6 +320,8 @@ static dsim::StepParams step_params(dsim_sim *s) {
     P.tri_mt = b->tri_mt.p;
     P.cell_start = b->d_cell_start.p;
     P.cell_tri = b->d_cell_tri.p;
+    P.ref_rec = b->ref_rec.p;
+    P.ref_mask = b->ref_mask.p;
     P.walk_start = b->walk_start.p;
     P.walk_ent = b->walk_ent.p;
     P.walk_rec = b->walk_rec.p;

@@ -676,6 +676,116 @@ __global__ __launch_bounds__(kBlock) void k_walk_lists(uint32_t n_cells, const u
     if (!EMIT) start[c] = n;
 }
 
+// The labeller's rows: the grid's cells along axis A, rows by the two other
+// axes (B, then C), and what decides whether a triangle is listed in them.
+struct RowGeom {
+    uint32_t dims[3];
+    float lo[3], cell[3];
+    int A, B, C;
+    float face;  // the grid's far face on A
+    bool exact;
+};
+
+// Does the triangle stand at the ends of rows rather than where their cells
+// list it?  AABB grids: its box starts past the grid's face on the ray's side
+// (no row lists it in a cell the ray can reach).  Exact-membership grids: its
+// box reaches past that face (the ray may cross it beyond the grid, where no
+// row cell lists it).
+__device__ __forceinline__ bool past_grid(const RowGeom &g, const float4 *box, uint32_t t) {
+    const float4 v = box[2 * (size_t)t + (g.exact ? 1 : 0)];
+    return (g.A == 0 ? v.x : g.A == 1 ? v.y : v.z) > g.face;
+}
+
+// A row entry's extents on the axes across (LabelParams::row_box).
+__device__ __forceinline__ float4 row_extent(const RowGeom &g, const float4 *box, uint32_t t) {
+    const float4 lo = box[2 * (size_t)t], hi = box[2 * (size_t)t + 1];
+    return make_float4(g.B == 0 ? lo.x : lo.y, g.B == 0 ? hi.x : hi.y, g.C == 1 ? lo.y : lo.z,
+                       g.C == 1 ? hi.y : hi.z);
+}
+
+// The triangles past the grid, after their count.
+__global__ __launch_bounds__(kBlock) void k_row_outside(RowGeom g, uint32_t n_tri,
+                                                        const float4 *box, uint32_t *outside) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t < n_tri && past_grid(g, box, t)) outside[1 + atomicAdd(&outside[0], 1u)] = t;
+}
+
+// Their entries: in every row whose cells' boxes, computed as label_cell does,
+// meet the triangle's on the axes across.  One block per triangle in turn.
+// EMIT false counts a row's; true fills the places before the row's end, and
+// counts them back to zero.
+template <bool EMIT>
+__global__ __launch_bounds__(kBlock) void k_row_ends(RowGeom g, const uint32_t *outside,
+                                                     const float4 *box, uint32_t *count,
+                                                     const uint32_t *start, uint32_t *tri,
+                                                     float4 *rec) {
+    const uint32_t n = outside[0], nb = g.dims[g.B], nc = g.dims[g.C];
+    for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
+        const uint32_t t = outside[1 + j];
+        const float4 e = row_extent(g, box, t);
+        // cell ranges to either side, then the boxes themselves
+        const float b0 = (e.x - g.lo[g.B]) / g.cell[g.B], b1 = (e.y - g.lo[g.B]) / g.cell[g.B];
+        const float c0 = (e.z - g.lo[g.C]) / g.cell[g.C], c1 = (e.w - g.lo[g.C]) / g.cell[g.C];
+        auto slack = [](float v) { return 1.0f + 1e-6f * fabsf(v); };
+        const int bl = (int)fminf(fmaxf(b0 - slack(b0), 0.0f), (float)(nb - 1));
+        const int bh = (int)fminf(fmaxf(b1 + slack(b1), 0.0f), (float)(nb - 1));
+        const int cl = (int)fminf(fmaxf(c0 - slack(c0), 0.0f), (float)(nc - 1));
+        const int ch = (int)fminf(fmaxf(c1 + slack(c1), 0.0f), (float)(nc - 1));
+        const uint32_t wide = (uint32_t)max(bh - bl + 1, 0);
+        const uint64_t all = (uint64_t)wide * (uint32_t)max(ch - cl + 1, 0);
+        for (uint64_t k = threadIdx.x; k < all; k += kBlock) {
+            const uint32_t b = bl + (uint32_t)(k % wide), c = cl + (uint32_t)(k / wide);
+            if (e.y < g.lo[g.B] + (float)b * g.cell[g.B] ||
+                e.x > g.lo[g.B] + (float)(b + 1) * g.cell[g.B] ||
+                e.w < g.lo[g.C] + (float)c * g.cell[g.C] ||
+                e.z > g.lo[g.C] + (float)(c + 1) * g.cell[g.C])
+                continue;
+            const uint32_t r = c * nb + b;
+            if (EMIT) {
+                const uint32_t at = start[(r + 1) * g.dims[g.A]] - atomicSub(&count[r], 1u);
+                tri[at] = t;
+                rec[at] = e;
+            } else {
+                atomicAdd(&count[r], 1u);
+            }
+        }
+    }
+}
+
+// Row entries of the cell at place r of the row order: the listed triangles
+// that the next cell of the row does not list, and for the row's last cell the
+// places of the entries of k_row_ends after them (ends counts a row's).  EMIT
+// false counts them, true writes those listed at start[r].
+template <bool EMIT>
+__global__ __launch_bounds__(kBlock) void k_row_lists(RowGeom g, uint32_t n_cells,
+                                                      const uint32_t *cell_start,
+                                                      const uint32_t *cell_tri, const float4 *box,
+                                                      const uint32_t *ends, uint32_t *start,
+                                                      uint32_t *tri, float4 *rec) {
+    const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
+    if (r >= n_cells) return;
+    uint32_t at[3];
+    at[g.A] = r % g.dims[g.A];
+    at[g.B] = r / g.dims[g.A] % g.dims[g.B];
+    at[g.C] = r / g.dims[g.A] / g.dims[g.B];
+    const uint32_t c = (at[2] * g.dims[1] + at[1]) * g.dims[0] + at[0];
+    const bool last = at[g.A] + 1 == g.dims[g.A];
+    const uint32_t next = c + (g.A == 0 ? 1u : g.A == 1 ? g.dims[0] : g.dims[0] * g.dims[1]);
+    uint32_t a = last ? 0u : cell_start[next], b = last ? 0u : cell_start[next + 1];
+    uint32_t n = EMIT ? start[r] : 0u;
+    for (uint32_t k = cell_start[c]; k < cell_start[c + 1]; ++k) {
+        const uint32_t t = cell_tri[k];
+        while (a < b && cell_tri[a] < t) ++a;  // both lists ascend
+        if ((a < b && cell_tri[a] == t) || past_grid(g, box, t)) continue;
+        if (EMIT) {
+            tri[n] = t;
+            rec[n] = row_extent(g, box, t);
+        }
+        ++n;
+    }
+    if (!EMIT) start[r] = n + (last ? ends[r / g.dims[g.A]] : 0u);
+}
+
 uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
 
 }  // namespace
@@ -810,7 +920,61 @@ static int build_ref_tables(dsim_substrate *S, hipStream_t st) {
     return DSIM_OK;
 }
 
+// Row lists of the labeller (LabelParams::row_start).
+static int build_row_lists(dsim_substrate *S, hipStream_t st) {
+    const uint32_t nT = S->n_tri, nC = S->n_cells;
+    RowGeom g{};
+    g.A = (int)S->label_axis;
+    g.B = g.A == 0 ? 1 : 0;
+    g.C = g.A == 2 ? 1 : 2;
+    g.exact = S->kind == DSIM_GRID_TRIBOX;
+    g.face = S->lo[g.A] + (float)S->dims[g.A] * S->cell[g.A];
+    for (int k = 0; k < 3; ++k) { g.dims[k] = S->dims[k]; g.lo[k] = S->lo[k]; g.cell[k] = S->cell[k]; }
+    const uint32_t n_rows = g.dims[g.B] * g.dims[g.C], n_blocks = std::min(nT, 1024u);
+    TempBuf<uint8_t> temp;
+    TempBuf<uint32_t> outside;  // and after it the rows' counts of their entries
+    int rc;
+    size_t tb = 0;
+    HIP_TRY(rocprim::exclusive_scan(nullptr, tb, S->row_start.p, S->row_start.p, 0u,
+                                    (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
+    if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = S->row_start.alloc((size_t)nC + 1)) ||
+        (rc = outside.alloc((size_t)nT + 1 + n_rows)))
+        return rc;
+    uint32_t *ends = outside.p + nT + 1;
+    HIP_TRY(hipMemsetAsync(outside.p, 0, outside.n * 4, st));
+    if (nT) {
+        hipLaunchKernelGGL(k_row_outside, dim3(blocks_for(nT)), dim3(kBlock), 0, st, g, nT,
+                           S->tri_aabb.p, outside.p);
+        hipLaunchKernelGGL(k_row_ends<false>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
+                           S->tri_aabb.p, ends, (const uint32_t *)nullptr, (uint32_t *)nullptr,
+                           (float4 *)nullptr);
+    }
+    hipLaunchKernelGGL(k_row_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
+                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, S->row_start.p,
+                       (uint32_t *)nullptr, (float4 *)nullptr);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemsetAsync(S->row_start.p + nC, 0, 4, st));
+    HIP_TRY(rocprim::exclusive_scan(temp.p, tb, S->row_start.p, S->row_start.p, 0u,
+                                    (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
+    uint32_t n = 0;
+    HIP_TRY(hipMemcpyAsync(&n, S->row_start.p + nC, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    const size_t n1 = std::max<uint32_t>(n, 1);  // a lane past its row's end reads entry 0
+    if ((rc = S->row_tri.alloc(n1)) || (rc = S->row_box.alloc(n1))) return rc;
+    hipLaunchKernelGGL(k_row_lists<true>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
+                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, S->row_start.p,
+                       S->row_tri.p, S->row_box.p);
+    if (nT)
+        hipLaunchKernelGGL(k_row_ends<true>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
+                           S->tri_aabb.p, ends, S->row_start.p, S->row_tri.p, S->row_box.p);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(st));
+    return DSIM_OK;
+}
+
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
+    if (S->kind != DSIM_GRID_REFERENCE)
+        if (int rc = build_row_lists(S, st)) return rc;
     if (S->kind == DSIM_GRID_REFERENCE)
         if (int rc = build_ref_tables(S, st)) return rc;
     if (int rc = build_search_lists(S, st)) return rc;

@@ -112,6 +112,9 @@ struct dsim_substrate {
     // (StepParams::ref_rec, ref_mask).
     dsim_host::DevBuf<float4> ref_rec;
     dsim_host::DevBuf<uint32_t> ref_mask;
+    // The labeller's rows (LabelParams::row_start); not for the reference grid.
+    dsim_host::DevBuf<uint32_t> row_start, row_tri;
+    dsim_host::DevBuf<float4> row_box;
     // Search lists of the physical-mode walk (build_walk_tables): per grid cell
     // its triangles, two of one plane in one entry (the second kNone where there
     // is none), and the entries' plane and lateral records, cell-major for
@@ -137,6 +140,7 @@ struct dsim_substrate {
         tri_ref.release(); tri_mt.release(); tri_aabb.release();
         walk_start.release(); walk_ent.release(); walk_rec.release();
         ref_rec.release(); ref_mask.release();
+        row_start.release(); row_tri.release(); row_box.release();
         d_clearance.release(); d_helpers.release(); d_fine.release();
         d_cell_start.release(); d_cell_tri.release(); fiber_myelin.release();
     }

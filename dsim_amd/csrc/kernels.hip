@@ -2181,15 +2181,15 @@ __device__ __forceinline__ uint32_t fiber_hash(uint32_t f) { return f * 0x9E3779
 // substrate's ray axis (the physical mode) or along the spin's dominant axis
 // (findSpinsInFibers), then for re-casts moved by a Philox jitter of up to
 // 0.05 per axis.
-__device__ __forceinline__ void label_ray(const LabelParams &P, uint32_t i, uint32_t tries,
-                                          float sx, float sy, float sz, float &ex, float &ey,
-                                          float &ez) {
+__device__ __forceinline__ void label_ray(const LabelParams &P, uint32_t axis, uint32_t i,
+                                          uint32_t tries, float sx, float sy, float sz, float &ex,
+                                          float &ey, float &ez) {
     ex = sx; ey = sy; ez = sz;
-    if (P.ray_axis == 1) {
+    if (axis == 1) {
         ex = (float)(1.1 * (double)P.xmax);
-    } else if (P.ray_axis == 2) {
+    } else if (axis == 2) {
         ey = (float)(1.1 * (double)P.ymax);
-    } else if (P.ray_axis == 3) {
+    } else if (axis == 3) {
         ez = (float)(1.1 * (double)P.zmax);
     } else if ((fabsf(sx) > fabsf(sy)) & (fabsf(sx) > fabsf(sz))) {
         ex = (float)(((sx >= 0) - (sx < 0)) * 1.1 * (double)P.xmax);
@@ -2212,29 +2212,38 @@ struct RaySums {
     uint32_t xf[3], xh[3], amb[3];
 };
 
-// Adds triangle t (box lo/hi, fibre and membrane in lo.w) if its box overlaps
-// the ray's box and the ray crosses it.
-__device__ __forceinline__ void ray_add(const LabelParams &P, uint32_t t, float4 lo, float4 hi,
-                                        float sx, float sy, float sz, float ex, float ey,
-                                        float ez, RaySums &R) {
+// The type of the ray's crossing of triangle t (0: none; 2, 3: through an edge
+// or vertex) where their boxes overlap, and of a triangle of membrane type 0-2.
+__device__ __forceinline__ uint32_t ray_hit(const LabelParams &P, bool use_mt, uint32_t t,
+                                            float4 lo, float4 hi, float sx, float sy, float sz,
+                                            float ex, float ey, float ez) {
     const float rminx = fminf(sx, ex), rminy = fminf(sy, ey), rminz = fminf(sz, ez);
     const float rmaxx = fmaxf(sx, ex), rmaxy = fmaxf(sy, ey), rmaxz = fmaxf(sz, ez);
     if (rminx > hi.x || lo.x > rmaxx || rminy > hi.y || lo.y > rmaxy || rminz > hi.z ||
-        lo.z > rmaxz)
-        return;
+        lo.z > rmaxz || __float_as_uint(lo.w) >> 16 > 2u)
+        return 0u;
     Hit h;
     float4 wall;
-    if (P.use_mt)
+    if (use_mt)
         test_mt(P.tri_mt, t, sx, sy, sz, ex, ey, ez, h);
     else
         test_ref(P.tri_ref, t, sx, sy, sz, ex, ey, ez, h, wall);
-    if (h.type == 0) return;
-    const uint32_t info = __float_as_uint(lo.w);
-    const uint32_t f = info & 0xFFFFu, m = info >> 16;
-    if (m > 2) return;
-    R.xf[m] ^= f + 1u;
-    R.xh[m] ^= fiber_hash(f);
-    if (h.type >= 2) R.amb[m] += 1;
+    return (uint32_t)h.type;
+}
+
+// Adds triangle t (box lo/hi, fibre and membrane in lo.w) if the ray crosses it.
+__device__ __forceinline__ void ray_add(const LabelParams &P, uint32_t t, float4 lo, float4 hi,
+                                        float sx, float sy, float sz, float ex, float ey,
+                                        float ez, RaySums &R) {
+    const uint32_t type = ray_hit(P, P.use_mt, t, lo, hi, sx, sy, sz, ex, ey, ez);
+    if (type == 0) return;
+    const uint32_t info = __float_as_uint(lo.w), f = info & 0xFFFFu;
+    for (uint32_t m = 0; m < 3; ++m) {  // no index into R: it stays in registers
+        const bool on = info >> 16 == m;
+        R.xf[m] ^= on ? f + 1u : 0u;
+        R.xh[m] ^= on ? fiber_hash(f) : 0u;
+        R.amb[m] += on && type >= 2u ? 1u : 0u;
+    }
 }
 
 // The label a ray's sums give: the first membrane type (axon, myelin, glia)
@@ -2246,7 +2255,9 @@ __device__ __forceinline__ bool ray_label(const RaySums &R, uint32_t &comp, uint
     fib = kFiberNone;
     uint32_t nedge = 0;
     bool found = false, multi = false;
-    for (uint32_t m = 0; m < 3 && !found; ++m) {
+#pragma unroll
+    for (uint32_t m = 0; m < 3; ++m) {
+        if (found) continue;
         nedge += R.amb[m];
         if (R.xf[m] != 0u) {
             const uint32_t f = R.xf[m] - 1u;
@@ -2274,7 +2285,7 @@ __global__ __launch_bounds__(256) void k_label(LabelParams P) {
     uint32_t out_comp = 0, out_fiber = kFiberNone;
     while (__syncthreads_or(!done)) {
         float ex, ey, ez;
-        label_ray(P, i, tries, sx, sy, sz, ex, ey, ez);
+        label_ray(P, P.ray_axis, i, tries, sx, sy, sz, ex, ey, ez);
         RaySums R = {};
         for (uint32_t t0 = 0; t0 < P.n_tri; t0 += 256) {
             __syncthreads();
@@ -2301,7 +2312,7 @@ __global__ __launch_bounds__(256) void k_label(LabelParams P) {
     }
     if (live) {
         P.label[i] = out_comp | (out_fiber << 8);
-        P.tries[i] = tries;
+        if (tries > P.max_tries) atomicAdd(P.n_ambiguous, 1u);
     }
 }
 
@@ -2309,24 +2320,6 @@ hipError_t launch_label(const LabelParams &p, hipStream_t s) {
     if (p.n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_label, dim3((p.n + 255) / 256), dim3(256), 0, s, p);
     return hipGetLastError();
-}
-
-// Is the triangle (box lo, hi) taken by the outside list rather than by the
-// row walk?  AABB grids: its box starts past the grid's face on the ray's
-// side (no grid row lists it in a cell the ray can reach).  Exact-membership
-// grids: its box reaches past that face (the ray may cross it beyond the grid,
-// where no row cell lists it).
-__device__ __forceinline__ bool past_grid(const LabelParams &P, float4 lo, float4 hi) {
-    const int a = (int)P.ray_axis - 1;
-    if (P.exact_grid) return (a == 0 ? hi.x : a == 1 ? hi.y : hi.z) > P.hi[a];
-    return (a == 0 ? lo.x : a == 1 ? lo.y : lo.z) > P.hi[a];
-}
-
-__global__ __launch_bounds__(256) void k_label_outside(LabelParams P) {
-    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= P.n_tri) return;
-    if (past_grid(P, P.tri_aabb[2 * t], P.tri_aabb[2 * t + 1]))
-        P.outside[atomicAdd(P.n_outside, 1u)] = t;
 }
 
 // Cell of coordinate v on axis a whose membership box, lo + c cell to
@@ -2338,96 +2331,166 @@ __device__ __forceinline__ uint32_t label_cell(const LabelParams &P, float v, in
     return c;
 }
 
-// Is triangle t listed in cell c (lists are in ascending triangle order)?
-__device__ __forceinline__ bool listed(const LabelParams &P, uint32_t c, uint32_t t) {
-    uint32_t a = P.cell_start[c], b = P.cell_start[c + 1];
-    while (a < b) {
-        const uint32_t m = (a + b) >> 1;
-        const uint32_t v = P.cell_tri[m];
-        if (v == t) return true;
-        if (v < t) a = m + 1; else b = m;
-    }
-    return false;
+// The first ray of each spin along the substrate's ray axis A (k_label's
+// try 0).  Candidates are the entries of the ray's grid row from the spin's
+// cell on (row_start, built with the substrate: an entry stands at the last
+// cell of each run of the row's cells that list its triangle, and at the
+// row's end those that the grid may not list where the ray meets them), so
+// each triangle is considered once.  For an AABB grid these are k_label's
+// candidates: those are the triangles whose boxes hold a point of the ray; for
+// one that does not start past the grid, the point of the ray at
+// max(box lo_A, s_A) lies in the grid box, so the cell of the row holding it
+// meets the triangle's box and lists it (the grid lists a triangle in every
+// cell whose closed membership box meets its bounding box, and the cells'
+// boxes tile the grid box).  An exact-membership grid lists a triangle that
+// lies inside the grid box on the ray's side in the cell of the row that holds
+// a crossing, and in a contiguous run of the row's cells (a convex triangle
+// meets a convex row of boxes in an interval), so every crossing is counted
+// once.  The others stand at the end of every row whose cells' boxes meet
+// theirs across the ray.
+//
+// What bounds it: the lines its gathers touch in the vector cache, and their
+// latency.
+// kRowLanes lanes of a spin read neighbouring entries (16 bytes each, the
+// extent across the ray, which turns most entries away) and the survivors of
+// the wave's spins are queued in LDS and tested 64 at a time, so the crossing
+// test runs with full lanes.  The sums of a spin do not depend on the order,
+// so the result equals k_label's first try.  Spins with an ambiguous ray,
+// outside the grid box, or beyond the ray's end are queued for the re-cast
+// kernels.  10^6 spins among 280,000 triangles (285 row entries and 70
+// overlapping boxes a spin): 1.09 ms; walking the cells' lists with a search
+// for each triangle in the cell before, and a list of all triangles past the
+// grid's face for every spin, 42.7 ms.
+// Spins by row group for k_label_row (76 us for the ranks of 10^6 spins, bound
+// by the counts' atomics; 10 us for the rest): the group of each spin's row and its
+// rank there (the spins of a group in any order; labels do not depend on it),
+// the groups' first places, and the order.
+template <int A>
+__global__ __launch_bounds__(256) void k_label_group_rank(LabelParams P, uint32_t *count,
+                                                          uint2 *place) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= P.n) return;
+    constexpr int B = A == 0 ? 1 : 0, C = A == 2 ? 1 : 2;  // the axes across
+    const float b = (B == 0 ? P.x : P.y)[i], c = (C == 1 ? P.y : P.z)[i];
+    const uint32_t r = label_cell(P, c, C) * P.dims[B] + label_cell(P, b, B);
+    const uint32_t group = (uint32_t)((uint64_t)r * kLabelGroups / (P.dims[B] * P.dims[C]));
+    place[i] = make_uint2(group, atomicAdd(&count[group], 1u));
 }
 
-// Lanes that share one spin's row walk (consecutive lanes of a wave).
-constexpr uint32_t kRowLanes = 8;
+__global__ __launch_bounds__(1024) void k_label_group_start(uint32_t *count) {
+    __shared__ uint32_t wave[16];
+    constexpr uint32_t per = kLabelGroups / 1024;
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    uint32_t v[per], sum = 0;
+    for (uint32_t k = 0; k < per; ++k) { v[k] = count[t * per + k]; sum += v[k]; }
+    const uint32_t inc = wave_incl_sum(sum);
+    if (lane == 63u) wave[w] = inc;
+    __syncthreads();
+    uint32_t base = inc - sum;
+    for (uint32_t k = 0; k < w; ++k) base += wave[k];
+    for (uint32_t k = 0; k < per; ++k) { count[t * per + k] = base; base += v[k]; }
+}
 
-// The first ray of each spin along the substrate's ray axis A (k_label's
-// try 0): candidates are the triangles listed in the cells of the ray's grid
-// row from the spin's cell on, each considered once (in the first of those
-// cells that lists it), plus the triangles whose boxes start past the grid's
-// face on the ray's side.  For an AABB grid these are k_label's candidates:
-// those are the triangles whose boxes hold a point of the ray; for one that
-// does not start past the grid, the point of the ray at max(box lo_A, s_A)
-// lies in the grid box, so the cell of the row holding it meets the
-// triangle's box and lists it (the grid lists a triangle in every cell whose
-// closed membership box meets its bounding box, and the cells' boxes tile the
-// grid box).  An exact-membership grid lists a triangle that lies inside the
-// grid box on the ray's side in the cell of the row that holds a crossing,
-// and in a contiguous run of the row's cells (a convex triangle meets a
-// convex row of boxes in an interval), so every crossing is counted once; a
-// triangle reaching past that face is taken by the outside list.  The kRowLanes lanes of a spin take every
-// kRowLanes-th cell and outside triangle and combine their sums; the sums do
-// not depend on the order, so the result equals k_label's first try.  Spins
-// with an ambiguous ray, outside the grid box, or beyond the ray's end are
-// queued for the re-cast kernels.
+__global__ __launch_bounds__(256) void k_label_order(uint32_t n, const uint32_t *start,
+                                                     const uint2 *place, uint32_t *order) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) order[start[place[i].x] + place[i].y] = i;
+}
+
+constexpr uint32_t kRowLanes = 8, kRowSpins = 64 / kRowLanes, kRowQueue = 192;
+static_assert(kRowQueue >= 3 * 64, "a round adds up to 128 entries to fewer than 64");
+
+template <int A>
 __global__ __launch_bounds__(256) void k_label_row(LabelParams P) {
-    const uint32_t gid = blockIdx.x * 256 + threadIdx.x;
-    const uint32_t i = gid / kRowLanes, g = gid % kRowLanes;
-    const bool live = i < P.n;  // every lane stays for the shuffles below
-    const int A = (int)P.ray_axis - 1;
-    float s3[3] = {0.f, 0.f, 0.f};
+    __shared__ float ray[4][kRowSpins][6];
+    __shared__ uint32_t sums[4][kRowSpins][9];
+    __shared__ uint2 queue[4][kRowQueue];
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t slot = lane / kRowLanes, g = lane % kRowLanes;
+    // each die (blocks go round them in turn) takes a run of the spin order
+    const uint32_t block = P.order ? blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds
+                                   : blockIdx.x;
+    const uint32_t at = (block * 4 + w) * kRowSpins + slot;
+    const bool live = at < P.n;  // every lane stays for the wave's queue
+    const uint32_t i = live && P.order ? P.order[at] : at;
+    constexpr int B = A == 0 ? 1 : 0, C = A == 2 ? 1 : 2;  // the axes across
+    float s3[3] = {0.f, 0.f, 0.f}, e3[3];
     if (live) { s3[0] = P.x[i]; s3[1] = P.y[i]; s3[2] = P.z[i]; }
-    const float sx = s3[0], sy = s3[1], sz = s3[2];
-    float ex, ey, ez;
-    label_ray(P, i, 0u, sx, sy, sz, ex, ey, ez);
-    const float eA = A == 0 ? ex : A == 1 ? ey : ez;
+    label_ray(P, A + 1u, i, 0u, s3[0], s3[1], s3[2], e3[0], e3[1], e3[2]);
+    if (g == 0)
+        for (int k = 0; k < 3; ++k) {
+            ray[w][slot][k] = s3[k];
+            ray[w][slot][3 + k] = e3[k];
+        }
+    for (uint32_t k = g; k < 9; k += kRowLanes) sums[w][slot][k] = 0;
     // the row walk covers rays that start in the grid box and run towards +A
-    const bool row = live && sx >= P.lo[0] && sx <= P.hi[0] && sy >= P.lo[1] &&
-                     sy <= P.hi[1] && sz >= P.lo[2] && sz <= P.hi[2] && s3[A] <= eA;
-    RaySums R = {};
+    const bool row = live && s3[0] >= P.lo[0] && s3[0] <= P.hi[0] && s3[1] >= P.lo[1] &&
+                     s3[1] <= P.hi[1] && s3[2] >= P.lo[2] && s3[2] <= P.hi[2] && s3[A] <= e3[A];
+    uint32_t k = 0, end = 0;
     if (row) {
-        uint32_t c3[3] = {label_cell(P, sx, 0), label_cell(P, sy, 1), label_cell(P, sz, 2)};
-        const uint32_t stride[3] = {1u, P.dims[0], P.dims[0] * P.dims[1]};
-        const uint32_t cA0 = c3[A];
-        c3[A] = 0;
-        const uint32_t rowc = (c3[2] * P.dims[1] + c3[1]) * P.dims[0] + c3[0];
-        const uint32_t sA = stride[A];
-        for (uint32_t cA = cA0 + g; cA < P.dims[A]; cA += kRowLanes) {
-            const uint32_t c = rowc + cA * sA;
-            for (uint32_t k = P.cell_start[c]; k < P.cell_start[c + 1]; ++k) {
-                const uint32_t t = P.cell_tri[k];
-                const float4 lo = P.tri_aabb[2 * t], hi = P.tri_aabb[2 * t + 1];
-                if (past_grid(P, lo, hi)) continue;              // in the outside list
-                if (cA > cA0 && listed(P, c - sA, t)) continue;  // considered one cell back
-                ray_add(P, t, lo, hi, sx, sy, sz, ex, ey, ez, R);
+        const uint32_t r = (label_cell(P, s3[C], C) * P.dims[B] + label_cell(P, s3[B], B)) *
+                           P.dims[A];
+        k = P.row_start[r + label_cell(P, s3[A], A)] + g;
+        end = P.row_start[r + P.dims[A]];
+    }
+    uint32_t queued = 0;
+    auto push = [&](bool on, uint32_t t) {
+        const uint64_t m = __ballot(on);
+        if (on) queue[w][queued + lane_rank(m)] = make_uint2(slot, t);
+        queued += (uint32_t)__popcll(m);
+    };
+    auto test = [&](uint32_t first, uint32_t count) {
+        wave_lds_sync();
+        if (lane < count) {
+            const uint2 q = queue[w][first + lane];
+            const float *v = ray[w][q.x];
+            const float4 lo = P.tri_aabb[2 * (size_t)q.y], hi = P.tri_aabb[2 * (size_t)q.y + 1];
+            const uint32_t type = ray_hit(P, true, q.y, lo, hi, v[0], v[1], v[2], v[3], v[4],
+                                          v[5]);
+            if (type) {
+                const uint32_t info = __float_as_uint(lo.w), f = info & 0xFFFFu;
+                uint32_t *sum = &sums[w][q.x][info >> 16];
+                atomicXor(&sum[0], f + 1u);
+                atomicXor(&sum[3], fiber_hash(f));
+                if (type >= 2u) atomicAdd(&sum[6], 1u);
             }
         }
-        const uint32_t no = *P.n_outside;
-        for (uint32_t j = g; j < no; j += kRowLanes) {
-            const uint32_t t = P.outside[j];
-            ray_add(P, t, P.tri_aabb[2 * t], P.tri_aabb[2 * t + 1], sx, sy, sz, ex, ey, ez, R);
+        wave_lds_sync();
+    };
+    // two entries a lane and round: both loads are in flight together
+    while (__ballot(k < end)) {
+        const bool in0 = k < end, in1 = k + kRowLanes < end;
+        const uint32_t k0 = in0 ? k : 0u, k1 = in1 ? k + kRowLanes : k0;
+        const float4 b0 = P.row_box[k0], b1 = P.row_box[k1];
+        const float vb = s3[B], vc = s3[C];
+        const bool on0 = in0 && !(vb > b0.y || b0.x > vb || vc > b0.w || b0.z > vc);
+        const bool on1 = in1 && !(vb > b1.y || b1.x > vb || vc > b1.w || b1.z > vc);
+        push(on0, on0 ? P.row_tri[k0] : 0u);
+        push(on1, on1 ? P.row_tri[k1] : 0u);
+        while (queued >= 64u) {
+            queued -= 64u;
+            test(queued, 64u);
         }
+        k += 2 * kRowLanes;
     }
-    for (uint32_t off = 1; off < kRowLanes; off <<= 1)
-        for (uint32_t m = 0; m < 3; ++m) {
-            R.xf[m] ^= __shfl_xor(R.xf[m], off, 64);
-            R.xh[m] ^= __shfl_xor(R.xh[m], off, 64);
-            R.amb[m] += __shfl_xor(R.amb[m], off, 64);
-        }
+    test(0u, queued);
     if (!live || g != 0) return;
     if (!row) {
         P.retry[atomicAdd(P.n_retry, 1u)] = make_uint2(i, 0u);
         return;
     }
+    RaySums R;
+    for (uint32_t m = 0; m < 3; ++m) {
+        R.xf[m] = sums[w][slot][m];
+        R.xh[m] = sums[w][slot][3 + m];
+        R.amb[m] = sums[w][slot][6 + m];
+    }
     uint32_t comp, fib;
     if (ray_label(R, comp, fib)) {
         P.label[i] = comp | (fib << 8);
-        P.tries[i] = 0;
     } else if (P.max_tries == 0) {  // no re-cast allowed: keep the first result
         P.label[i] = comp | (fib << 8);
-        P.tries[i] = 1;
+        atomicAdd(P.n_ambiguous, 1u);
     } else {
         P.retry[atomicAdd(P.n_retry, 1u)] = make_uint2(i, 1u);  // re-cast with a jitter
     }
@@ -2458,7 +2521,7 @@ __global__ __launch_bounds__(256) void k_label_group(LabelParams P) {
         uint32_t out_comp = 0, out_fiber = kFiberNone;
         while (__syncthreads_or(!done)) {
             float ex, ey, ez;
-            label_ray(P, i, tries, sx, sy, sz, ex, ey, ez);
+            label_ray(P, P.ray_axis, i, tries, sx, sy, sz, ex, ey, ez);
             RaySums R = {};
             for (uint32_t t0 = 0; t0 < P.n_tri; t0 += 256) {
                 __syncthreads();
@@ -2490,15 +2553,20 @@ __global__ __launch_bounds__(256) void k_label_group(LabelParams P) {
         }
         if (live && g == 0) {
             P.label[i] = out_comp | (out_fiber << 8);
-            P.tries[i] = tries;
+            if (tries > P.max_tries) atomicAdd(P.n_ambiguous, 1u);
         }
     }
 }
 
-// Queued spins when the queue is short: one block per spin, its 256 threads
-// sharing out the triangles, so a spin's re-casts take microseconds.
-__global__ __launch_bounds__(256) void k_label_spin(LabelParams P) {
-    __shared__ uint32_t part[4][9];
+// Queued spins when the queue is short: one block per spin, its threads
+// sharing out the triangles, kSpinLoads boxes of a thread in flight together:
+// with few blocks the latency of the loads is what a spin's re-casts take.  A
+// spin among 280,000 triangles (9 MB of boxes): 183 us; of 256 threads with one
+// box in flight 374 us.
+constexpr uint32_t kSpinThreads = 1024, kSpinLoads = 4;
+
+__global__ __launch_bounds__(kSpinThreads) void k_label_spin(LabelParams P) {
+    __shared__ uint32_t part[kSpinThreads / 64][9];
     const uint32_t count = *P.n_retry;
     if (count > kRetryPerBlockMax) return;  // k_label_group takes a long queue
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
@@ -2510,11 +2578,20 @@ __global__ __launch_bounds__(256) void k_label_spin(LabelParams P) {
         uint32_t out_comp = 0, out_fiber = kFiberNone;
         for (;;) {
             float ex, ey, ez;
-            label_ray(P, i, tries, sx, sy, sz, ex, ey, ez);
+            label_ray(P, P.ray_axis, i, tries, sx, sy, sz, ex, ey, ez);
             RaySums R = {};
-            for (uint32_t t = threadIdx.x; t < P.n_tri; t += 256)
-                ray_add(P, t, P.tri_aabb[2 * t], P.tri_aabb[2 * t + 1], sx, sy, sz, ex, ey, ez,
-                        R);
+            for (uint32_t t0 = threadIdx.x; t0 < P.n_tri; t0 += kSpinThreads * kSpinLoads) {
+                float4 lo[kSpinLoads], hi[kSpinLoads];
+                for (uint32_t k = 0; k < kSpinLoads; ++k) {
+                    const uint32_t t = min(t0 + k * kSpinThreads, P.n_tri - 1);
+                    lo[k] = P.tri_aabb[2 * (size_t)t];
+                    hi[k] = P.tri_aabb[2 * (size_t)t + 1];
+                }
+                for (uint32_t k = 0; k < kSpinLoads; ++k) {
+                    const uint32_t t = t0 + k * kSpinThreads;
+                    if (t < P.n_tri) ray_add(P, t, lo[k], hi[k], sx, sy, sz, ex, ey, ez, R);
+                }
+            }
             for (uint32_t off = 1; off < 64; off <<= 1)
                 for (uint32_t m = 0; m < 3; ++m) {
                     R.xf[m] ^= __shfl_xor(R.xf[m], off, 64);
@@ -2529,7 +2606,7 @@ __global__ __launch_bounds__(256) void k_label_spin(LabelParams P) {
                 }
             __syncthreads();
             RaySums T = {};
-            for (uint32_t v = 0; v < 4; ++v)
+            for (uint32_t v = 0; v < kSpinThreads / 64; ++v)
                 for (uint32_t m = 0; m < 3; ++m) {
                     T.xf[m] ^= part[v][m];
                     T.xh[m] ^= part[v][3 + m];
@@ -2543,19 +2620,35 @@ __global__ __launch_bounds__(256) void k_label_spin(LabelParams P) {
         }
         if (threadIdx.x == 0) {
             P.label[i] = out_comp | (out_fiber << 8);
-            P.tries[i] = tries;
+            if (tries > P.max_tries) atomicAdd(P.n_ambiguous, 1u);
         }
     }
 }
 
+// The row walk along axis A, and before it the spins' order.
+template <int A>
+static void launch_rows(const LabelParams &p, hipStream_t s) {
+    constexpr uint32_t per_block = 4 * kRowSpins;
+    uint32_t blocks = (p.n + per_block - 1) / per_block;
+    if (p.order) {
+        const dim3 spins((p.n + 255) / 256);
+        hipLaunchKernelGGL(k_label_group_rank<A>, spins, dim3(256), 0, s, p, p.group, p.retry);
+        hipLaunchKernelGGL(k_label_group_start, dim3(1), dim3(1024), 0, s, p.group);
+        hipLaunchKernelGGL(k_label_order, spins, dim3(256), 0, s, p.n, p.group, p.retry, p.order);
+        blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+    }
+    hipLaunchKernelGGL(k_label_row<A>, dim3(blocks), dim3(256), 0, s, p);
+}
+
 hipError_t launch_label_row(const LabelParams &p, hipStream_t s) {
     if (p.n == 0) return hipSuccess;
-    if (p.n_tri)
-        hipLaunchKernelGGL(k_label_outside, dim3((p.n_tri + 255) / 256), dim3(256), 0, s, p);
-    const uint64_t lanes = (uint64_t)p.n * kRowLanes;
-    hipLaunchKernelGGL(k_label_row, dim3((uint32_t)((lanes + 255) / 256)), dim3(256), 0, s, p);
+    switch (p.ray_axis) {
+        case 1: launch_rows<0>(p, s); break;
+        case 2: launch_rows<1>(p, s); break;
+        default: launch_rows<2>(p, s); break;
+    }
     // the re-casts: the kernel that does not fit the queue's length exits at once
-    hipLaunchKernelGGL(k_label_spin, dim3(kRetryPerBlockMax), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(k_label_spin, dim3(kRetryPerBlockMax), dim3(kSpinThreads), 0, s, p);
     const uint32_t groups = (p.n + kGroupSpins - 1) / kGroupSpins;
     hipLaunchKernelGGL(k_label_group, dim3(groups < 4096u ? groups : 4096u), dim3(256), 0, s, p);
     return hipGetLastError();

@@ -48,7 +48,10 @@ struct dsim_sim {
     uint64_t step = 0;
     hipStream_t stream = nullptr;
     DevBuf<uint32_t> state, alt;  // F_COUNT * n words each (alt only when sorting)
-    DevBuf<uint32_t> seed, flags, tries;
+    DevBuf<uint32_t> seed, flags;
+    // labelling: counters (groups, ambiguous, queued), then per spin the retry
+    // queue's entry and the place in the row order; made on the first call
+    DevBuf<uint32_t> label_work;
     DevBuf<double> partial, out;
     DevBuf<float> grads;
     DevBuf<float4> inject;
@@ -73,7 +76,7 @@ struct dsim_sim {
     }
     ~dsim_sim() {
         for (auto &e : ev) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
-        for (auto *b : {&state, &alt, &seed, &flags, &tries, &trace, &keys_a, &keys_b, &vals_a,
+        for (auto *b : {&state, &alt, &seed, &flags, &label_work, &trace, &keys_a, &keys_b, &vals_a,
                         &vals_b})
             b->release();
         partial.release(); out.release(); grads.release(); inject.release(); sort_tmp.release();
@@ -130,7 +133,6 @@ extern "C" int dsim_sim_create(dsim_substrate *sub, const dsim_params *p, uint32
     int rc;
     if ((rc = S->state.alloc(m * F_COUNT)) || (rc = S->flags.alloc(4)) || (rc = S->queue.alloc(8)) ||
         (rc = S->partial.alloc((size_t)dsim::kSignalBlocks * 15)) || (rc = S->out.alloc(15)) ||
-        (rc = S->tries.alloc(m)) ||
         (p->rng == DSIM_RNG_MWC && (rc = S->seed.alloc(2 * m)))) {
         delete S;
         return rc;
@@ -641,7 +643,6 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     L.n = s->n;
     L.x = s->ff(F_X); L.y = s->ff(F_Y); L.z = s->ff(F_Z);
     L.label = s->f(F_LABEL);
-    L.tries = s->tries.p;
     L.xmax = xmax; L.ymax = ymax; L.zmax = zmax;
     L.max_tries = max_tries;
     // the physical mode casts along the substrate's ray axis (+x unless the
@@ -654,23 +655,24 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     const dsim_substrate *sub = s->sub;
     const bool rows = L.ray_axis && sub->kind != DSIM_GRID_REFERENCE && sub->n_cells > 0 &&
                       s->n > 0;
-    dsim_host::DevBuf<uint32_t> work;  // retry queue, counters, outside list
-    hipError_t e;
+    constexpr size_t counters = dsim::kLabelGroups + 2;  // even: the uint2 queue follows
+    const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
+    if (!s->label_work.p)
+        if (int rc = s->label_work.alloc(words)) return rc;
+    uint32_t *w = s->label_work.p;
+    L.group = w;
+    L.n_ambiguous = w + counters - 2;
+    L.n_retry = w + counters - 1;
+    hipError_t e = hipMemsetAsync(w, 0, counters * 4, s->stream);
+    if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
     if (rows) {
-        const size_t q = 2 * (size_t)s->n;  // the queue's uint2 entries sit at the aligned start
-        if (int rc = work.alloc(q + 2 + (size_t)sub->n_tri)) return rc;
-        L.retry = reinterpret_cast<uint2 *>(work.p);
-        L.n_outside = work.p + q;
-        L.n_retry = work.p + q + 1;
-        L.outside = work.p + q + 2;
-        e = hipMemsetAsync(L.n_outside, 0, 8, s->stream);
-        if (e != hipSuccess) {
-            work.release();
-            return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
-        }
-        L.cell_start = sub->d_cell_start.p;
-        L.cell_tri = sub->d_cell_tri.p;
-        L.exact_grid = sub->kind == DSIM_GRID_TRIBOX ? 1u : 0u;
+        L.retry = reinterpret_cast<uint2 *>(w + counters);
+        const uint64_t row_bytes = (uint64_t)sub->row_tri.n * 20 + (uint64_t)sub->n_tri * 96;
+        L.order = s->n >= dsim::kLabelOrderMin && row_bytes > dsim::kXcdL2Bytes
+                      ? w + counters + 2 * (size_t)s->n : nullptr;
+        L.row_start = sub->row_start.p;
+        L.row_tri = sub->row_tri.p;
+        L.row_box = sub->row_box.p;
         for (int k = 0; k < 3; ++k) {
             L.dims[k] = sub->dims[k];
             L.lo[k] = sub->lo[k];
@@ -682,20 +684,10 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     } else {
         e = dsim::launch_label(L, s->stream);
     }
-    if (e != hipSuccess) {
-        work.release();
-        return fail(DSIM_ERR_HIP, "label launch: %s", hipGetErrorString(e));
-    }
+    if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label launch: %s", hipGetErrorString(e));
     e = hipStreamSynchronize(s->stream);
-    work.release();
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
-    if (n_ambiguous) {
-        std::vector<uint32_t> t(s->n);
-        if (s->n) HIP_TRY(hipMemcpy(t.data(), s->tries.p, (size_t)s->n * 4, hipMemcpyDeviceToHost));
-        uint32_t a = 0;
-        for (uint32_t v : t) a += v > max_tries;
-        *n_ambiguous = a;
-    }
+    if (n_ambiguous) HIP_TRY(hipMemcpy(n_ambiguous, L.n_ambiguous, 4, hipMemcpyDeviceToHost));
     s->moment_ready = false;
     return DSIM_OK;
 }

@@ -218,7 +218,17 @@ constexpr uint32_t kPhaseSliceK = 32;  // k per LDS stage
 hipError_t launch_phase_gemm(const float *traj, uint32_t n, uint32_t n_pad, uint32_t k_len,
                              uint32_t k_fold, const uint16_t *g_hi, const uint16_t *g_lo,
                              uint32_t k_total, uint32_t k0, uint32_t n_wave, float *phase,
-                             uint32_t *comp, hipStream_t s);
+                             uint32_t *comp, bool from_zero, hipStream_t s);
+// The waveforms' operands: pc * grads [n_steps][n_wave][3] as bf16 hi + lo rows
+// [n_wpad][3 n_steps] (rows past n_wave zero) and their FP64 sums over the steps.
+hipError_t launch_phase_operands(const float *g, uint32_t n_steps, uint32_t n_wave,
+                                 uint32_t n_wpad, float pc, uint16_t *hi, uint16_t *lo,
+                                 double *gsum, hipStream_t s);
+// Rows s0 (even) to s0 + m of phase and of the unpacked compensation, [m][n_wave]
+// (either output may be null).
+hipError_t launch_phase_rows(uint32_t s0, uint32_t m, const float *phase, const uint32_t *comp,
+                             uint32_t n_wave, uint32_t n_wpad, float *p_out, float *c_out,
+                             hipStream_t s);
 // Signal of every waveform: per block of state slots and waveform the FP64
 // sums of m cos(phase), m sin(phase) and counts for the total and
 // compartments 0-3, phase = phase[id[s]][w] + gsum[w] . x0[s] (in FP64; mag,

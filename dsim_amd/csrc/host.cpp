@@ -11,6 +11,7 @@
 #include <cstring>
 #include <string>
 #include <thread>
+#include <mutex>
 #include <vector>
 
 #include <hip/hip_runtime_api.h>
@@ -351,6 +352,104 @@ uint32_t dsim_host::label_axis_of(const dsim_mesh *mesh) {
     return score[2] < score[1] ? 2 : 1;
 }
 
+namespace {
+
+struct PoolBlock {
+    void *p;
+    size_t bytes;
+    int device;
+};
+std::mutex pool_mu;
+std::vector<PoolBlock> pool;  // oldest first
+size_t pool_bytes = 0;
+uint64_t pool_users = 0;
+
+// The oldest block out of the pool (under pool_mu).
+PoolBlock pool_oldest() {
+    const PoolBlock b = pool.front();
+    pool.erase(pool.begin());
+    pool_bytes -= b.bytes;
+    return b;
+}
+
+// Gives every idle block back; false if there was none.
+bool pool_trim() {
+    std::vector<PoolBlock> idle;
+    {
+        std::lock_guard<std::mutex> l(pool_mu);
+        idle.swap(pool);
+        pool_bytes = 0;
+    }
+    for (const PoolBlock &b : idle) (void)hipFree(b.p);
+    return !idle.empty();
+}
+
+}  // namespace
+
+void *dsim_host::dev_alloc(size_t bytes, hipError_t *e) {
+    void *p = nullptr;
+    *e = hipMalloc(&p, bytes);
+    if (*e != hipSuccess && pool_trim()) {
+        (void)hipGetLastError();
+        *e = hipMalloc(&p, bytes);
+    }
+    return *e == hipSuccess ? p : nullptr;
+}
+
+void *dsim_host::pool_take(size_t bytes, size_t *got, hipError_t *e) {
+    *got = bytes;
+    *e = hipSuccess;
+    int device = 0;
+    if (hipGetDevice(&device) == hipSuccess) {
+        std::lock_guard<std::mutex> l(pool_mu);
+        size_t best = pool.size();
+        for (size_t k = 0; k < pool.size(); ++k)
+            if (pool[k].device == device && pool[k].bytes >= bytes &&
+                pool[k].bytes / 4 * 3 <= bytes && (best == pool.size() || pool[k].bytes < pool[best].bytes))
+                best = k;
+        if (best < pool.size()) {
+            const PoolBlock b = pool[best];
+            pool.erase(pool.begin() + best);
+            pool_bytes -= b.bytes;
+            *got = b.bytes;
+            return b.p;
+        }
+    }
+    return dev_alloc(bytes, e);
+}
+
+void dsim_host::pool_give(void *p, size_t bytes) {
+    int device = 0;
+    size_t total = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceTotalMem(&total, device) != hipSuccess)
+        total = 0;
+    const size_t limit = total / kPoolShare;
+    std::vector<PoolBlock> out;
+    if (bytes > limit) {
+        out.push_back({p, bytes, device});
+    } else {
+        std::lock_guard<std::mutex> l(pool_mu);
+        pool.push_back({p, bytes, device});
+        pool_bytes += bytes;
+        while (pool_bytes > limit || pool.size() > kPoolBlocks || (!pool_users && !pool.empty()))
+            out.push_back(pool_oldest());
+    }
+    for (const PoolBlock &b : out) (void)hipFree(b.p);
+}
+
+void dsim_host::pool_ref() {
+    std::lock_guard<std::mutex> l(pool_mu);
+    ++pool_users;
+}
+
+void dsim_host::pool_unref() {
+    {
+        std::lock_guard<std::mutex> l(pool_mu);
+        if (--pool_users) return;
+    }
+    pool_trim();
+}
+
 extern "C" const char *dsim_last_error(void) { return dsim_host::g_err.c_str(); }
 extern "C" int dsim_abi_version(void) { return DSIM_ABI_VERSION; }
 
@@ -620,9 +719,9 @@ extern "C" int dsim_alloc_array(void **dev_ptr, size_t bytes) {
     if (!dev_ptr) return fail(DSIM_ERR_ARG, "NULL pointer");
     *dev_ptr = nullptr;
     if (bytes == 0) return DSIM_OK;
-    hipError_t e = hipMalloc(dev_ptr, bytes);
-    if (e != hipSuccess) {
-        *dev_ptr = nullptr;
+    hipError_t e = hipSuccess;
+    *dev_ptr = dsim_host::dev_alloc(bytes, &e);
+    if (!*dev_ptr) {
         return fail(DSIM_ERR_NOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     }
     return DSIM_OK;

@@ -1742,10 +1742,100 @@ __device__ __forceinline__ void bf16_split2(float a, float b, uint32_t &hi, uint
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
 }
 
+// Nearest even in integers (any bit pattern).
+__device__ __forceinline__ uint16_t bf16_rne(float x) {
+    const uint32_t u = __float_as_uint(x);
+    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+}
+
 // Raw buffer descriptor over a wave-uniform base (gfx9 word 3; no stride, byte
 // offsets below 2^31).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void *base) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7fffffff, 0x00020000);
+}
+
+// The waveforms' operands of the phase GEMM: pc * G as bf16 hi + lo, k-major
+// rows [n_wpad][3 n_steps] of the gradients [n_steps][n_wave][3], waveforms past
+// n_wave zero.  A block turns a tile of 32 steps and 16 waveforms through LDS,
+// so both sides move whole lines: 1024 waveforms of 2048 steps (50 MB moved)
+// 16 us, and 54 us for the sums, a serial chain of FP64 additions; on the host
+// 36 ms.
+constexpr uint32_t kOperandSteps = 32, kOperandWaves = 16;
+__global__ __launch_bounds__(256) void k_phase_operands(const float *__restrict__ g, uint32_t n_steps,
+                                                        uint32_t n_wave, float pc,
+                                                        uint16_t *__restrict__ hi,
+                                                        uint16_t *__restrict__ lo) {
+    constexpr uint32_t row = 3 * kOperandWaves, cols = 3 * kOperandSteps;
+    __shared__ float tile[kOperandSteps][row + 1];
+    const uint32_t t0 = blockIdx.x * kOperandSteps, w0 = blockIdx.y * kOperandWaves;
+    for (uint32_t k = threadIdx.x; k < kOperandSteps * row; k += 256) {
+        const uint32_t t = k / row, j = k % row;
+        const bool in = t0 + t < n_steps && w0 + j / 3 < n_wave;
+        tile[t][j] = in ? pc * g[((size_t)(t0 + t) * n_wave + w0) * 3 + j] : 0.0f;
+    }
+    __syncthreads();
+    const size_t K = (size_t)3 * n_steps;
+    for (uint32_t k = threadIdx.x; k < kOperandWaves * cols; k += 256) {
+        const uint32_t w = k / cols, j = k % cols;  // column j: step j / 3, axis j % 3
+        if (t0 + j / 3 >= n_steps) continue;
+        const float v = tile[j / 3][3 * w + j % 3];
+        const uint16_t h = bf16_rne(v);
+        const size_t at = (size_t)(w0 + w) * K + (size_t)3 * t0 + j;
+        hi[at] = h;
+        lo[at] = bf16_rne(v - __uint_as_float((uint32_t)h << 16));
+    }
+}
+
+// gsum[w][a] = sum_t of pc * G in FP64, in the order of the steps.
+__global__ __launch_bounds__(64) void k_phase_gsum(const float *__restrict__ g, uint32_t n_steps,
+                                                   uint32_t n_wave, uint32_t n_wpad, float pc,
+                                                   double *__restrict__ gsum) {
+    const uint32_t j = blockIdx.x * 64u + threadIdx.x;  // waveform * 3 + axis
+    if (j >= n_wpad * 3u) return;
+    double sum = 0.0;
+    if (j < n_wave * 3u) {
+#pragma unroll 16
+        for (uint32_t t = 0; t < n_steps; ++t) sum += (double)(pc * g[(size_t)t * n_wave * 3 + j]);
+    }
+    gsum[j] = sum;
+}
+
+hipError_t launch_phase_operands(const float *g, uint32_t n_steps, uint32_t n_wave,
+                                 uint32_t n_wpad, float pc, uint16_t *hi, uint16_t *lo,
+                                 double *gsum, hipStream_t s) {
+    const dim3 grid((n_steps + kOperandSteps - 1) / kOperandSteps, n_wpad / kOperandWaves);
+    hipLaunchKernelGGL(k_phase_operands, grid, dim3(256), 0, s, g, n_steps, n_wave, pc, hi, lo);
+    hipLaunchKernelGGL(k_phase_gsum, dim3((n_wpad * 3 + 63) / 64), dim3(64), 0, s, g, n_steps, n_wave,
+                       n_wpad, pc, gsum);
+    return hipGetLastError();
+}
+
+// Rows s0 (even) to s0 + m of the pairs without the padded waveforms.
+__global__ __launch_bounds__(256) void k_phase_rows(uint32_t s0, uint32_t m,
+                                                    const float *__restrict__ phase,
+                                                    const uint32_t *__restrict__ comp,
+                                                    uint32_t n_wave, uint32_t n_wpad,
+                                                    float *__restrict__ p_out,
+                                                    float *__restrict__ c_out) {
+    const uint64_t all = (uint64_t)m * n_wave;
+    for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < all;
+         k += (uint64_t)gridDim.x * 256) {
+        const uint32_t r = (uint32_t)(k / n_wave), w = (uint32_t)(k % n_wave);
+        if (p_out) p_out[k] = phase[(size_t)(s0 + r) * n_wpad + w];
+        if (c_out) {
+            const uint32_t word = comp[(size_t)((s0 + r) / 2) * n_wpad + w];
+            c_out[k] = __uint_as_float(((s0 + r) & 1u) ? word & 0xffff0000u : word << 16);
+        }
+    }
+}
+
+hipError_t launch_phase_rows(uint32_t s0, uint32_t m, const float *phase, const uint32_t *comp,
+                             uint32_t n_wave, uint32_t n_wpad, float *p_out, float *c_out,
+                             hipStream_t s) {
+    const uint64_t blocks = ((uint64_t)m * n_wave + 255) / 256;
+    hipLaunchKernelGGL(k_phase_rows, dim3((uint32_t)(blocks < 16384 ? blocks : 16384)), dim3(256), 0,
+                       s, s0, m, phase, comp, n_wave, n_wpad, p_out, c_out);
+    return hipGetLastError();
 }
 
 // Register stage of one K slice of the phase GEMM (see k_phase_gemm) for
@@ -1829,7 +1919,8 @@ template <int TJ>
 __global__ __launch_bounds__(kPhaseThreads) void k_phase_gemm(
     const float *__restrict__ traj, uint32_t n_pad, uint32_t k_len, uint32_t k_fold,
     const uint16_t *__restrict__ g_hi, const uint16_t *__restrict__ g_lo, uint32_t k_total,
-    uint32_t k0, uint32_t n_wave, float *__restrict__ phase, uint32_t *__restrict__ comp) {
+    uint32_t k0, uint32_t n_wave, float *__restrict__ phase, uint32_t *__restrict__ comp,
+    bool from_zero) {
     constexpr uint32_t kTileN = 128u * TJ;
     constexpr uint32_t kAHalves = kPhaseTileM * kLdsPitch, kBHalves = kTileN * kLdsPitch;
     constexpr uint32_t kStage = 2 * kAHalves + 2 * kBHalves;
@@ -1878,21 +1969,34 @@ __global__ __launch_bounds__(kPhaseThreads) void k_phase_gemm(
     for (int r = 0; r < 4; ++r) lp[r] = ((4u * (lane >> 5) + r) * n_wave + (lane & 31u)) * 4u;
 #pragma unroll
     for (int r = 0; r < 2; ++r) lc[r] = ((2u * (lane >> 5) + r) * n_wave + (lane & 31u)) * 4u;
+    // The first product starts from zero: the pairs need no clearing, and 6 bytes
+    // a pair are neither written before nor read here.
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const uint32_t sp = (32u * i + 8u * (q / 4)) * n_wave * 4u;
-            const uint32_t sc = (16u * i + 4u * (q / 4)) * n_wave * 4u;
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                ps[i][j][q] = __uint_as_float(
-                    __builtin_amdgcn_raw_buffer_load_b32(rp, lp[q % 4] + 128u * j, sp, 0));
-                if (q % 2 == 0)
-                    pk[i][j][q / 2] =
-                        __builtin_amdgcn_raw_buffer_load_b32(rc, lc[(q % 4) / 2] + 128u * j, sc, 0);
+            for (int q = 0; q < 16; ++q) {
+                ps[i][j][q] = 0.0f;
+                pk[i][j][q / 2] = 0u;
             }
-        }
+    if (!from_zero) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const uint32_t sp = (32u * i + 8u * (q / 4)) * n_wave * 4u;
+                const uint32_t sc = (16u * i + 4u * (q / 4)) * n_wave * 4u;
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) {
+                    ps[i][j][q] = __uint_as_float(
+                        __builtin_amdgcn_raw_buffer_load_b32(rp, lp[q % 4] + 128u * j, sp, 0));
+                    if (q % 2 == 0)
+                        pk[i][j][q / 2] = __builtin_amdgcn_raw_buffer_load_b32(
+                            rc, lc[(q % 4) / 2] + 128u * j, sc, 0);
+                }
+            }
+    }
     __syncthreads();
     f32x16 acc[2][TJ];
 #pragma unroll
@@ -1992,7 +2096,7 @@ __global__ __launch_bounds__(kPhaseThreads) void k_phase_gemm(
 hipError_t launch_phase_gemm(const float *traj, uint32_t n, uint32_t n_pad, uint32_t k_len,
                              uint32_t k_fold, const uint16_t *g_hi, const uint16_t *g_lo,
                              uint32_t k_total, uint32_t k0, uint32_t n_wave, float *phase,
-                             uint32_t *comp, hipStream_t s) {
+                             uint32_t *comp, bool from_zero, hipStream_t s) {
     if (n == 0 || k_len == 0) return hipSuccess;
     if (k_fold == 0 || k_fold % kPhaseSliceK || k_len % kPhaseSliceK || n_wave % kPhaseTileN ||
         n_pad % kPhaseTileM)
@@ -2007,10 +2111,10 @@ hipError_t launch_phase_gemm(const float *traj, uint32_t n, uint32_t n_pad, uint
     const uint32_t grid = m_groups * 8u * (n_wave / tile_n);
     if (wide)
         hipLaunchKernelGGL(k_phase_gemm<2>, dim3(grid), dim3(kPhaseThreads), 0, s, traj, n_pad,
-                           k_len, k_fold, g_hi, g_lo, k_total, k0, n_wave, phase, comp);
+                           k_len, k_fold, g_hi, g_lo, k_total, k0, n_wave, phase, comp, from_zero);
     else
         hipLaunchKernelGGL(k_phase_gemm<1>, dim3(grid), dim3(kPhaseThreads), 0, s, traj, n_pad,
-                           k_len, k_fold, g_hi, g_lo, k_total, k0, n_wave, phase, comp);
+                           k_len, k_fold, g_hi, g_lo, k_total, k0, n_wave, phase, comp, from_zero);
     return hipGetLastError();
 }
 
@@ -2050,6 +2154,9 @@ __global__ __launch_bounds__(256) void k_phase_final(const double *partial, uint
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;  // waveform*15 + quantity
     if (i >= n_wave * 15u) return;
     double acc = 0.0;
+    // in the blocks' order, several loads in flight (512 blocks, 1024 waveforms:
+    // 25 us, one at a time 172 us)
+#pragma unroll 16
     for (uint32_t b = 0; b < n_blocks; ++b) acc += partial[(size_t)b * n_wave * 15 + i];
     out[i] = acc;
 }

@@ -4,7 +4,6 @@
 // readout (k_phase_partial).
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 #include <vector>
 
 #include <hip/hip_runtime_api.h>
@@ -15,27 +14,30 @@
 #include "host_common.h"
 #include "sim_internal.h"
 
-using dsim_host::DevBuf;
+using dsim_host::PoolBuf;
 using dsim_host::fail;
-using dsim_host::upload;
 
 struct dsim_waveforms {
     dsim_sim *sim = nullptr;
     uint32_t n = 0, n_pad = 0, n_wave = 0, n_steps = 0, chunk = 0, done = 0;
     uint32_t n_wpad = 0;          // waveforms padded with zero ones to a multiple of kPhaseTileN
     uint32_t buffer = 0;          // steps walked per trajectory buffer (a multiple of chunk)
-    DevBuf<uint16_t> g_hi, g_lo;  // [n_wpad][3*n_steps] bf16 bits, pc folded in
-    DevBuf<double> gsum;          // [n_wpad][3]: sum_t pc * G_w(t)
-    DevBuf<float> traj;           // n_pad / kTrajTile tiles of [3*len][kTrajTile] (len <= buffer)
-    DevBuf<float> phase;          // [n_pad][n_wpad] (rows past n: padding)
-    DevBuf<uint32_t> comp;        // [n_pad / 2][n_wpad]: Kahan compensation of spins 2m, 2m + 1
-                                  // as bf16 in the low and high half
-    DevBuf<double> partial, out;
+    // One allocation: gsum [n_wpad][3], sum_t pc * G_w(t); the readout's partial
+    // sums and out [n_wpad][15]; the bf16 halves g_hi, g_lo [n_wpad][3*n_steps]
+    // of the gradients, pc folded in.
+    PoolBuf<double> work;
+    double *gsum = nullptr, *partial = nullptr, *out = nullptr;
+    uint16_t *g_hi = nullptr, *g_lo = nullptr;
+    PoolBuf<float> traj;          // n_pad / kTrajTile tiles of [3*len][kTrajTile] (len <= buffer)
+    // phase [n_pad][n_wpad] (rows past n: padding), and after it comp
+    // [n_pad / 2][n_wpad]: Kahan compensation of spins 2m, 2m + 1 as bf16 in the
+    // low and high half.  Written by the first product, which starts from zero.
+    PoolBuf<float> phase;
+    uint32_t *comp = nullptr;
+    bool empty = true;            // no product yet: the pairs are zero and not in memory
     double walk_ms = 0.0, gemm_ms = 0.0;
     ~dsim_waveforms() {
-        g_hi.release(); g_lo.release(); gsum.release(); traj.release(); phase.release();
-        comp.release();
-        partial.release(); out.release();
+        work.release(); traj.release(); phase.release();
     }
 };
 
@@ -43,18 +45,14 @@ namespace {
 
 constexpr uint32_t kPhaseBlocks = 512;  // spin blocks of the readout
 
-uint16_t bf16_rne(float x) {
-    uint32_t u;
-    std::memcpy(&u, &x, 4);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+constexpr uint64_t kStagingBytes = 64ull << 20;  // of get_phase's row blocks, at most
 
-float bf16_val(uint16_t h) {
-    uint32_t u = (uint32_t)h << 16;
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
+// The pairs before any product, for a readout: zero.
+int clear_pairs(dsim_waveforms *W, hipStream_t st) {
+    if (!W->empty) return DSIM_OK;
+    HIP_TRY(hipMemsetAsync(W->phase.p, 0, W->phase.n * 4, st));
+    W->empty = false;
+    return DSIM_OK;
 }
 
 }  // namespace
@@ -80,35 +78,35 @@ extern "C" int dsim_waveforms_create(dsim_sim *sim, uint32_t n_wave, uint32_t n_
     W->n_steps = n_steps;
     W->chunk = chunk;
     W->buffer = chunk;
-    const size_t K = (size_t)3 * n_steps;
-    std::vector<uint16_t> hi(nwp * K, 0), lo(nwp * K, 0);
-    std::vector<double> gs((size_t)nwp * 3, 0.0);
-    for (uint32_t t = 0; t < n_steps; ++t)
-        for (uint32_t w = 0; w < n_wave; ++w)
-            for (uint32_t a = 0; a < 3; ++a) {
-                const float v = pc * grads[((size_t)t * n_wave + w) * 3 + a];
-                const uint16_t h = bf16_rne(v);
-                hi[w * K + 3 * t + a] = h;
-                lo[w * K + 3 * t + a] = bf16_rne(v - bf16_val(h));
-                gs[(size_t)w * 3 + a] += (double)v;
-            }
-    int rc;
+    const size_t K = (size_t)3 * n_steps, ng = (size_t)nwp * K;
     const size_t nw = (size_t)std::max<uint32_t>(W->n_pad, 1) * nwp;
-    if ((rc = upload(W->g_hi, hi)) || (rc = upload(W->g_lo, lo)) || (rc = upload(W->gsum, gs)) ||
-        (rc = W->traj.alloc((size_t)3 * chunk * W->n_pad)) || (rc = W->phase.alloc(nw)) ||
-        (rc = W->comp.alloc((size_t)std::max<uint32_t>(W->n_pad / 2, 1) * nwp)) ||
-        (rc = W->partial.alloc((size_t)kPhaseBlocks * nwp * 15)) ||
-        (rc = W->out.alloc((size_t)nwp * 15))) {
+    const size_t n_sum = (size_t)nwp * 3, n_part = (size_t)kPhaseBlocks * nwp * 15;
+    const size_t n_out = (size_t)nwp * 15;
+    PoolBuf<float> g;  // the gradients as given
+    int rc;
+    if ((rc = g.alloc((size_t)n_steps * n_wave * 3)) ||
+        (rc = W->work.alloc(n_sum + n_part + n_out + (2 * ng * 2 + 7) / 8)) ||
+        (rc = W->traj.alloc((size_t)3 * chunk * W->n_pad)) ||
+        (rc = W->phase.alloc(nw + (size_t)std::max<uint32_t>(W->n_pad / 2, 1) * nwp))) {
+        g.release();
         delete W;
         return rc;
     }
-    // padded trajectory columns stay zero; phases start at zero.  Cleared on
-    // the handle's stream, before the walk it records: hipMemset returns before
-    // the device is done and does not order with that (non-blocking) stream.
+    W->gsum = W->work.p;
+    W->partial = W->gsum + n_sum;
+    W->out = W->partial + n_part;
+    W->g_hi = reinterpret_cast<uint16_t *>(W->out + n_out);
+    W->g_lo = W->g_hi + ng;
+    W->comp = reinterpret_cast<uint32_t *>(W->phase.p + nw);
+    // The trajectory needs no clearing: padded spins reach only padded rows of
+    // the pairs, which nothing reads.
     hipStream_t st = dsim_host::sim_stream(sim);
-    hipError_t e = hipMemsetAsync(W->traj.p, 0, W->traj.n * 4, st);
-    if (e == hipSuccess) e = hipMemsetAsync(W->phase.p, 0, nw * 4, st);
-    if (e == hipSuccess) e = hipMemsetAsync(W->comp.p, 0, W->comp.n * 4, st);
+    hipError_t e = hipMemcpyAsync(g.p, grads, g.n * 4, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+        e = dsim::launch_phase_operands(g.p, n_steps, n_wave, nwp, pc, W->g_hi, W->g_lo, W->gsum, st);
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+    g.release();
     if (e != hipSuccess) {
         delete W;
         return fail(DSIM_ERR_HIP, "waveform init: %s", hipGetErrorString(e));
@@ -126,15 +124,13 @@ extern "C" int dsim_waveforms_set_buffer(dsim_waveforms *W, uint32_t buffer_step
     HIP_TRY(hipStreamSynchronize(dsim_host::sim_stream(W->sim)));
     W->traj.release();
     if (int rc = W->traj.alloc((size_t)3 * buffer_steps * W->n_pad)) return rc;
-    // padded trajectory columns stay zero (cleared in the walk's stream order)
-    HIP_TRY(hipMemsetAsync(W->traj.p, 0, W->traj.n * 4, dsim_host::sim_stream(W->sim)));
     W->buffer = buffer_steps;
     return DSIM_OK;
 }
 
 extern "C" int dsim_waveforms_destroy(dsim_waveforms *W) {
     if (!W) return DSIM_OK;
-    (void)hipStreamSynchronize(dsim_host::sim_stream(W->sim));
+    (void)hipStreamSynchronize(dsim_host::sim_stream(W->sim));  // the blocks go back to the pool
     delete W;
     return DSIM_OK;
 }
@@ -154,9 +150,9 @@ extern "C" int dsim_waveforms_run(dsim_waveforms *W, uint32_t steps, float *traj
         if ((rc = dsim_host::sim_walk_traj(W->sim, len, W->traj.p))) break;
         HIP_TRY(hipEventRecord(ev[1], st));
         hipError_t e = dsim::launch_phase_gemm(W->traj.p, W->n, W->n_pad, 3 * len, 3 * W->chunk,
-                                               W->g_hi.p, W->g_lo.p, 3 * W->n_steps,
-                                               3 * W->done, W->n_wpad, W->phase.p, W->comp.p,
-                                               st);
+                                               W->g_hi, W->g_lo, 3 * W->n_steps, 3 * W->done,
+                                               W->n_wpad, W->phase.p, W->comp, W->empty, st);
+        if (e == hipSuccess) W->empty = false;
         if (e != hipSuccess) {
             rc = fail(DSIM_ERR_HIP, "phase GEMM: %s", hipGetErrorString(e));
             break;
@@ -198,11 +194,12 @@ extern "C" int dsim_waveforms_signal(dsim_waveforms *W, double *out) {
     dsim_host::sim_readout_fields(W->sim, &mag, &label, &x0, &id);
     hipStream_t st = dsim_host::sim_stream(W->sim);
     const uint32_t nb = std::max<uint32_t>(1, std::min<uint32_t>(kPhaseBlocks, W->n));
-    hipError_t e = dsim::launch_phase_signal(W->n, W->phase.p, W->n_wpad, W->gsum.p, mag, label, x0,
-                                             id, W->partial.p, nb, W->out.p, st);
+    if (int rc = clear_pairs(W, st)) return rc;
+    hipError_t e = dsim::launch_phase_signal(W->n, W->phase.p, W->n_wpad, W->gsum, mag, label, x0, id,
+                                             W->partial, nb, W->out, st);
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "phase readout: %s", hipGetErrorString(e));
     std::vector<double> v((size_t)W->n_wpad * 15);
-    HIP_TRY(hipMemcpyAsync(v.data(), W->out.p, v.size() * 8, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(v.data(), W->out, v.size() * 8, hipMemcpyDeviceToHost, st));
     if (int rc = dsim_sync(W->sim)) return rc;
     for (uint32_t w = 0; w < W->n_wave; ++w) {
         const double *q = &v[(size_t)w * 15];
@@ -216,21 +213,33 @@ extern "C" int dsim_waveforms_signal(dsim_waveforms *W, double *out) {
 extern "C" int dsim_waveforms_get_phase(dsim_waveforms *W, float *phase, float *comp) {
     if (!W) return fail(DSIM_ERR_ARG, "NULL waveforms");
     if (int rc = dsim_sync(W->sim)) return rc;
-    const size_t m = (size_t)W->n * W->n_wave;
-    const uint32_t nwp = W->n_wpad;  // row stride of the device arrays
-    if (phase && m)
-        HIP_TRY(hipMemcpy2D(phase, (size_t)W->n_wave * 4, W->phase.p, (size_t)nwp * 4,
-                            (size_t)W->n_wave * 4, W->n, hipMemcpyDeviceToHost));
-    if (comp && m) {
-        std::vector<uint32_t> v((size_t)(W->n + 1) / 2 * nwp);
-        HIP_TRY(hipMemcpy(v.data(), W->comp.p, v.size() * 4, hipMemcpyDeviceToHost));
-        for (uint32_t s = 0; s < W->n; ++s)
-            for (uint32_t w = 0; w < W->n_wave; ++w) {
-                const uint32_t word = v[(size_t)(s / 2) * nwp + w];
-                const uint32_t bits = (s & 1u) ? (word & 0xffff0000u) : (word << 16);
-                std::memcpy(&comp[(size_t)s * W->n_wave + w], &bits, 4);
-            }
+    if (!W->n || (!phase && !comp)) return DSIM_OK;
+    hipStream_t st = dsim_host::sim_stream(W->sim);
+    if (int rc = clear_pairs(W, st)) return rc;
+    // blocks of whole spin pairs, without the padded waveforms, through a
+    // staging buffer: a copy of rows at a stride takes the runtime about 5 us
+    // a row
+    const uint64_t row = (uint64_t)W->n_wave * 4;
+    const uint32_t rows = (uint32_t)std::min<uint64_t>((W->n + 1u) & ~1u,
+                                                       std::max<uint64_t>(kStagingBytes / row & ~1ull, 2));
+    PoolBuf<float> stage;
+    if (int rc = stage.alloc((size_t)rows * W->n_wave * 2)) return rc;
+    float *c_stage = stage.p + (size_t)rows * W->n_wave;
+    hipError_t e = hipSuccess;
+    for (uint32_t s0 = 0; s0 < W->n && e == hipSuccess; s0 += rows) {
+        const uint32_t m = std::min(rows, W->n - s0);
+        const size_t bytes = (size_t)m * row, at = (size_t)s0 * W->n_wave;
+        e = dsim::launch_phase_rows(s0, m, W->phase.p, W->comp, W->n_wave, W->n_wpad,
+                                    phase ? stage.p : nullptr, comp ? c_stage : nullptr, st);
+        if (e == hipSuccess && phase)
+            e = hipMemcpyAsync(phase + at, stage.p, bytes, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess && comp)
+            e = hipMemcpyAsync(comp + at, c_stage, bytes, hipMemcpyDeviceToHost, st);
     }
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+    stage.release();
+    if (e != hipSuccess) return fail(DSIM_ERR_HIP, "phase copy: %s", hipGetErrorString(e));
     return DSIM_OK;
 }
 

@@ -90,6 +90,8 @@ struct dsim_server {
     Batch batch[4];  // [boundary * 2 + (grid entries read through cell_tri)]
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
+    dsim_server() { dsim_host::pool_ref(); }  // the requests' handles reuse their blocks
+    ~dsim_server() { dsim_host::pool_unref(); }
     double clock() const {
         return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     }
@@ -172,7 +174,9 @@ int ensure_batch(dsim_server *S, int kind) {
     Batch &B = S->batch[kind];
     if (B.exec) return DSIM_OK;
     HIP_TRY(hipHostMalloc((void **)&B.host, sizeof(dsim::WalkTable), hipHostMallocDefault));
-    HIP_TRY(hipMalloc((void **)&B.dev, sizeof(dsim::WalkTable)));
+    hipError_t ea = hipSuccess;
+    B.dev = static_cast<dsim::WalkTable *>(dsim_host::dev_alloc(sizeof(dsim::WalkTable), &ea));
+    if (!B.dev) return fail(DSIM_ERR_NOMEM, "hipMalloc: %s", hipGetErrorString(ea));
     // the launch shape never changes: blocks past the table's total exit at
     // once, so one captured launch serves every round
     HIP_TRY(hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal));

@@ -16,6 +16,7 @@
 #include "sim_internal.h"
 
 using dsim_host::DevBuf;
+using dsim_host::PoolBuf;
 using dsim_host::fail;
 
 namespace {
@@ -47,20 +48,17 @@ struct dsim_sim {
     uint32_t n = 0;
     uint64_t step = 0;
     hipStream_t stream = nullptr;
-    DevBuf<uint32_t> state, alt;  // F_COUNT * n words each (alt only when sorting)
-    DevBuf<uint32_t> seed, flags;
-    // labelling: counters (groups, ambiguous, queued), then per spin the retry
-    // queue's entry and the place in the row order; made on the first call
-    DevBuf<uint32_t> label_work;
-    DevBuf<double> partial, out;
-    DevBuf<float> grads;
-    DevBuf<float4> inject;
-    DevBuf<uint32_t> trace;
-    DevBuf<unsigned long long> stats;  // walk work counters while counting is on
-    DevBuf<uint32_t> queue;            // slot counters of the persistent walk
+    PoolBuf<uint32_t> state, alt;  // F_COUNT * n words each (alt only when sorting)
+    PoolBuf<uint32_t> seed, flags;
+    PoolBuf<double> partial, out;
+    PoolBuf<float> grads;
+    PoolBuf<float4> inject;
+    PoolBuf<uint32_t> trace;
+    PoolBuf<unsigned long long> stats;  // walk work counters while counting is on
+    PoolBuf<uint32_t> queue;            // slot counters of the persistent walk
     bool counting = false;
-    DevBuf<uint32_t> keys_a, keys_b, vals_a, vals_b;
-    DevBuf<uint8_t> sort_tmp;
+    PoolBuf<uint32_t> keys_a, keys_b, vals_a, vals_b;
+    PoolBuf<uint8_t> sort_tmp;
     uint64_t steps_since_sort = ~0ull;
     bool permuted = false;
     bool moment_ready = false;
@@ -74,15 +72,20 @@ struct dsim_sim {
     bool sorting() const {
         return prm.sort_interval > 0 && prm.mode == DSIM_MODE_PHYSICAL && prm.rng == DSIM_RNG_PHILOX;
     }
+    dsim_sim() { dsim_host::pool_ref(); }
     ~dsim_sim() {
+        // the blocks go back to the pool, which does not wait as hipFree does; no
+        // other stream holds work on them (the server waits for its rounds)
+        if (stream) (void)hipStreamSynchronize(stream);
         for (auto &e : ev) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
-        for (auto *b : {&state, &alt, &seed, &flags, &label_work, &trace, &keys_a, &keys_b, &vals_a,
+        for (auto *b : {&state, &alt, &seed, &flags, &trace, &keys_a, &keys_b, &vals_a,
                         &vals_b})
             b->release();
         partial.release(); out.release(); grads.release(); inject.release(); sort_tmp.release();
         stats.release(); queue.release();
         if (stream) (void)hipStreamDestroy(stream);
         if (sub) sub->refs--;
+        dsim_host::pool_unref();
     }
 };
 
@@ -417,6 +420,7 @@ static int run_steps(dsim_sim *s, dsim::StepParams P, uint32_t iters, int rng, b
         if ((uint64_t)iters * n * 16 > (1ull << 32))
             return fail(DSIM_ERR_ARG, "injected sequence too large (%u x %u)", iters, n);
         if (s->inject.n < (size_t)iters * n) {
+            HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
             s->inject.release();
             if (int rc = s->inject.alloc((size_t)iters * n)) return rc;
         }
@@ -427,6 +431,7 @@ static int run_steps(dsim_sim *s, dsim::StepParams P, uint32_t iters, int rng, b
         if ((uint64_t)iters * n * 20 > (1ull << 32))
             return fail(DSIM_ERR_ARG, "trace too large (%u x %u)", iters, n);
         if (s->trace.n < (size_t)iters * n * 5) {
+            HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
             s->trace.release();
             if (int rc = s->trace.alloc((size_t)iters * n * 5)) return rc;
         }
@@ -556,10 +561,12 @@ extern "C" int dsim_signal_moment(dsim_sim *s, uint32_t ndir, const float *g, fl
     if (!g || !out) return fail(DSIM_ERR_ARG, "NULL argument");
     const uint32_t nb = 256;
     if (s->grads.n < (size_t)ndir * 3) {
+        HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
         s->grads.release();
         if (int rc = s->grads.alloc((size_t)ndir * 3)) return rc;
     }
     if (s->partial.n < (size_t)ndir * nb * 15) {
+        HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
         s->partial.release();
         if (int rc = s->partial.alloc(
                 (size_t)std::max<size_t>(ndir * (size_t)nb, dsim::kSignalBlocks) * 15))
@@ -657,14 +664,15 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
                       s->n > 0;
     constexpr size_t counters = dsim::kLabelGroups + 2;  // even: the uint2 queue follows
     const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
-    if (!s->label_work.p)
-        if (int rc = s->label_work.alloc(words)) return rc;
-    uint32_t *w = s->label_work.p;
+    // counters (groups, ambiguous, queued), then per spin the retry queue's
+    // entry and the place in the row order
+    PoolBuf<uint32_t> work;
+    if (int rc = work.alloc(words)) return rc;
+    uint32_t *w = work.p;
     L.group = w;
     L.n_ambiguous = w + counters - 2;
     L.n_retry = w + counters - 1;
     hipError_t e = hipMemsetAsync(w, 0, counters * 4, s->stream);
-    if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
     if (rows) {
         L.retry = reinterpret_cast<uint2 *>(w + counters);
         const uint64_t row_bytes = (uint64_t)sub->row_tri.n * 20 + (uint64_t)sub->n_tri * 96;
@@ -680,14 +688,18 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
             L.inv_cell[k] = sub->inv_cell[k];
             L.hi[k] = sub->lo[k] + (float)sub->dims[k] * sub->cell[k];
         }
-        e = dsim::launch_label_row(L, s->stream);
+        if (e == hipSuccess) e = dsim::launch_label_row(L, s->stream);
     } else {
-        e = dsim::launch_label(L, s->stream);
+        if (e == hipSuccess) e = dsim::launch_label(L, s->stream);
     }
-    if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label launch: %s", hipGetErrorString(e));
-    e = hipStreamSynchronize(s->stream);
+    uint32_t ambiguous = 0;
+    if (e == hipSuccess && n_ambiguous)
+        e = hipMemcpyAsync(&ambiguous, L.n_ambiguous, 4, hipMemcpyDeviceToHost, s->stream);
+    const hipError_t es = hipStreamSynchronize(s->stream);
+    work.release();
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
-    if (n_ambiguous) HIP_TRY(hipMemcpy(n_ambiguous, L.n_ambiguous, 4, hipMemcpyDeviceToHost));
+    if (n_ambiguous) *n_ambiguous = ambiguous;
     s->moment_ready = false;
     return DSIM_OK;
 }

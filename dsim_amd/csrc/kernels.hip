@@ -2118,6 +2118,20 @@ hipError_t launch_phase_gemm(const float *traj, uint32_t n, uint32_t n_pad, uint
     return hipGetLastError();
 }
 
+// sin and cos of x, sincos' own, behind a wave-uniform branch: its reduction of
+// arguments past 2^30, two thirds of its instructions, is otherwise done for
+// every argument and selected away.
+__device__ __forceinline__ void wave_sincos(double x, double *s, double *c) {
+    const bool small = fabs(x) < 1073741824.0;
+    if (__ballot(!small)) {
+        asm volatile("" : "+v"(x));  // keeps the compiler from doing it before the branch
+        sincos(x, s, c);
+    } else {
+        __builtin_assume(small);
+        sincos(x, s, c);
+    }
+}
+
 // Readout of the waveform phases: one thread per waveform, one block row per
 // range of spins; FP64 phase (x0 term added in FP64), cos/sin and sums.
 __global__ __launch_bounds__(256) void k_phase_partial(uint32_t n, const float *__restrict__ phase,
@@ -2139,7 +2153,7 @@ __global__ __launch_bounds__(256) void k_phase_partial(uint32_t n, const float *
         const double ph = (double)phase[(size_t)id[s] * n_wave + w] + gx * (double)x0[s] +
                           gy * (double)x0[n + s] + gz * (double)x0[2 * n + s];
         double sn, cs;
-        sincos(ph, &sn, &cs);
+        wave_sincos(ph, &sn, &cs);
         const double m = (double)mag[s];
         const uint32_t c = (label[s] & 0xFFu) + 1u;
         v[0] += m * cs; v[5] += m * sn; v[10] += 1.0;
@@ -2178,37 +2192,112 @@ hipError_t launch_phase_signal(uint32_t n, const float *phase, uint32_t n_wave,
 // Signal readout: getMrSignal(double[]) (spinSystem.cpp:1452-1500), FP64.
 // Per-block partials then one fixed-order final pass (deterministic).
 // ------------------------------------------------------------------------ //
-__device__ __forceinline__ void block_reduce15(double (&v)[15], double *out) {
-    __shared__ double sh[15][256];
-    const int t = threadIdx.x;
-    for (int k = 0; k < 15; ++k) sh[k][t] = v[k];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (t < s)
-            for (int k = 0; k < 15; ++k) sh[k][t] += sh[k][t + s];
-        __syncthreads();
+// The lanes 4 H apart hand each other H of their 2 H sums and add.
+template <int H>
+__device__ __forceinline__ void hand_over(double (&w)[16], uint32_t &which) {
+    const bool up = threadIdx.x & (4 * H);
+    which += up ? H : 0;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+        const double keep = up ? w[j + H] : w[j], give = up ? w[j] : w[j + H];
+        w[j] = keep + __shfl_xor(give, 4 * H, 64);
     }
-    if (t < 15) out[t] = sh[t][0];
+}
+
+// Sums over a block of 256 by halving, in the order of a tree over the threads
+// (t and t + 128, then t + 64, then the lanes of the first wave): the two upper
+// levels through LDS, the rest by lane exchanges.  At each exchange a lane
+// keeps half of its sums and hands over the other half, so the 15 sums take 17
+// exchanges instead of 90.  Calls may follow one another.
+__device__ __forceinline__ void block_reduce15(double (&v)[15], double *out) {
+    __shared__ double sh[15][128];
+    const uint32_t t = threadIdx.x;
+    __syncthreads();  // the array's last readers are done
+    if (t >= 128)
+        for (int k = 0; k < 15; ++k) sh[k][t - 128] = v[k];
+    __syncthreads();
+    if (t < 128)
+        for (int k = 0; k < 15; ++k) v[k] += sh[k][t];
+    if (t >= 64 && t < 128)  // read back above by this thread alone
+        for (int k = 0; k < 15; ++k) sh[k][t] = v[k];
+    __syncthreads();
+    if (t >= 64) return;
+    double w[16];
+#pragma unroll
+    for (int k = 0; k < 15; ++k) w[k] = v[k] + sh[k][t + 64];
+    w[15] = 0.0;
+    uint32_t which = 0;  // the sum that w[0] ends as
+    hand_over<8>(w, which);
+    hand_over<4>(w, which);
+    hand_over<2>(w, which);
+    hand_over<1>(w, which);
+    w[0] += __shfl_xor(w[0], 2, 64);
+    w[0] += __shfl_xor(w[0], 1, 64);
+    if ((t & 3u) == 0u && which < 15u) out[which] = w[0];
+}
+
+// One thread's sums for a readout line: m cos(phase), m sin(phase) over all its
+// spins and by compartment (k = compartment + 1).  The counts, which all lines
+// share, are kept beside them as integers.
+struct LineSums {
+    double c[5], s[5];
+};
+// Adds a spin of magnitude m and compartment k - 1 at the lines' phases.  The
+// lanes of each compartment add under their own mask: a selected 0.0 for the
+// others would take three times the instructions.
+template <uint32_t L>
+__device__ __forceinline__ void line_add(LineSums (&v)[L], double m, const float (&ph)[L],
+                                         uint32_t k) {
+    double c[L], s[L];
+#pragma unroll
+    for (uint32_t l = 0; l < L; ++l) {
+        wave_sincos((double)ph[l], &s[l], &c[l]);
+        c[l] *= m;
+        s[l] *= m;
+        v[l].c[0] += c[l];
+        v[l].s[0] += s[l];
+    }
+#pragma unroll
+    for (uint32_t q = 1; q < 5; ++q) {
+        uint32_t kq = k;
+        asm("" : "+v"(kq));  // else the four become one add at an index k, in scratch
+        if (q == kq)
+#pragma unroll
+            for (uint32_t l = 0; l < L; ++l) {
+                v[l].c[q] += c[l];
+                v[l].s[q] += s[l];
+            }
+    }
+}
+__device__ __forceinline__ void line_reduce(const LineSums &v, const uint32_t count[5],
+                                            double *partial) {
+    double r[15];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        r[k] = v.c[k];
+        r[5 + k] = v.s[k];
+        r[10 + k] = (double)count[k];
+    }
+    block_reduce15(r, partial);
+}
+__device__ __forceinline__ void count_add(uint32_t count[5], uint32_t k) {
+    count[0]++;
+#pragma unroll
+    for (uint32_t q = 1; q < 5; ++q) count[q] += q == k ? 1u : 0u;
 }
 
 __global__ __launch_bounds__(256) void k_signal_partial(uint32_t n, const float *mag,
                                                         const float *phase, const uint32_t *label,
                                                         double *partial) {
-    double v[15];
-    for (int k = 0; k < 15; ++k) v[k] = 0.0;
+    LineSums v[1] = {};
+    uint32_t count[5] = {};
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        double m = (double)mag[i];
-        double c = cos((double)phase[i]) * m, s = sin((double)phase[i]) * m;
-        uint32_t k = (label[i] & 0xFFu) + 1u;
-        v[0] += c; v[5] += s; v[10] += 1.0;
-        for (uint32_t q = 1; q < 5; ++q) {
-            bool on = (q == k);
-            v[q] += on ? c : 0.0;
-            v[5 + q] += on ? s : 0.0;
-            v[10 + q] += on ? 1.0 : 0.0;
-        }
+        const uint32_t k = (label[i] & 0xFFu) + 1u;
+        const float ph[1] = {phase[i]};
+        count_add(count, k);
+        line_add<1>(v, (double)mag[i], ph, k);
     }
-    block_reduce15(v, partial + (size_t)blockIdx.x * 15);
+    line_reduce(v[0], count, partial + (size_t)blockIdx.x * 15);
 }
 
 __global__ __launch_bounds__(256) void k_partial_final(const double *partial, uint32_t n_blocks,
@@ -2231,15 +2320,31 @@ hipError_t launch_signal(uint32_t n, const float *mag, const float *phase, const
 }
 
 // Per-direction readout from gradient moments: phase_j = pc * g_j.(M + W x0).
-__global__ __launch_bounds__(256) void k_moment_partial(uint32_t n, const float *mag,
-                                                        const float *mom, const float *x0,
-                                                        float wsum, const uint32_t *label,
-                                                        const float *grads, float pc,
-                                                        double *partial) {
-    const uint32_t j = blockIdx.y;
-    const float gx = grads[3 * j], gy = grads[3 * j + 1], gz = grads[3 * j + 2];
-    double v[15];
-    for (int k = 0; k < 15; ++k) v[k] = 0.0;
+// Bound by the FP64 sine and cosine of every (spin, line) pair, and with few
+// pairs by the latency of the block sums; a block takes L lines of its spins,
+// which share the loads, the moment's x0 term and the counts.  10^6 spins, 65
+// lines: 205 us (250 with one line a block; 355 with sine and cosine apart, all
+// of a block's sums halved through LDS and zeros selected for the other
+// compartments); 60,000 spins, 13 lines: 14.6 us with one line, 19.2 with two
+// (26.1); 300,001 spins, 30 lines: 46.7 and 41.7 (65.5).
+constexpr uint32_t kReadoutLines = 2;
+constexpr uint64_t kReadoutPairs = 4u << 20;
+template <uint32_t L>
+__global__ __launch_bounds__(256) void k_moment_partial(uint32_t n, const float *__restrict__ mag,
+                                                        const float *__restrict__ mom,
+                                                        const float *__restrict__ x0, float wsum,
+                                                        const uint32_t *__restrict__ label,
+                                                        uint32_t first,
+                                                        const float *__restrict__ grads, float pc,
+                                                        double *__restrict__ partial) {
+    const uint32_t j0 = first + blockIdx.y * L;
+    float g[L][3];
+#pragma unroll
+    for (uint32_t l = 0; l < L; ++l)
+#pragma unroll
+        for (uint32_t a = 0; a < 3; ++a) g[l][a] = grads[3 * (j0 + l) + a];
+    LineSums v[L] = {};
+    uint32_t count[5] = {};
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         float mx = mom[i], my = mom[n + i], mz = mom[2 * n + i];
         if (x0 && wsum != 0.0f) {
@@ -2247,27 +2352,33 @@ __global__ __launch_bounds__(256) void k_moment_partial(uint32_t n, const float 
             my = fmaf(wsum, x0[n + i], my);
             mz = fmaf(wsum, x0[2 * n + i], mz);
         }
-        float ph = fmaf(gx, mx, fmaf(gy, my, gz * mz)) * pc;
-        double m = (double)mag[i];
-        double c = cos((double)ph) * m, s = sin((double)ph) * m;
-        uint32_t k = (label[i] & 0xFFu) + 1u;
-        v[0] += c; v[5] += s; v[10] += 1.0;
-        for (uint32_t q = 1; q < 5; ++q) {
-            bool on = (q == k);
-            v[q] += on ? c : 0.0;
-            v[5 + q] += on ? s : 0.0;
-            v[10 + q] += on ? 1.0 : 0.0;
-        }
+        const double m = (double)mag[i];
+        const uint32_t k = (label[i] & 0xFFu) + 1u;
+        count_add(count, k);
+        float ph[L];
+#pragma unroll
+        for (uint32_t l = 0; l < L; ++l)
+            ph[l] = fmaf(g[l][0], mx, fmaf(g[l][1], my, g[l][2] * mz)) * pc;
+        line_add<L>(v, m, ph, k);
     }
-    block_reduce15(v, partial + ((size_t)j * gridDim.x + blockIdx.x) * 15);
+#pragma unroll
+    for (uint32_t l = 0; l < L; ++l)
+        line_reduce(v[l], count, partial + ((size_t)(j0 + l) * gridDim.x + blockIdx.x) * 15);
 }
 
 hipError_t launch_moment_signal(uint32_t n, const float *mag, const float *mom, const float *x0,
                                 float wsum, const uint32_t *label, uint32_t ndir,
                                 const float *grads, float pc, double *partial, uint32_t n_blocks,
                                 double *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_moment_partial, dim3(n_blocks, ndir), dim3(256), 0, s, n, mag, mom, x0,
-                       wsum, label, grads, pc, partial);
+    // lines in twos where there is work enough to fill the device with them
+    const uint32_t groups = (uint64_t)n * ndir >= kReadoutPairs ? ndir / kReadoutLines : 0u;
+    const uint32_t done = groups * kReadoutLines;
+    if (groups)
+        hipLaunchKernelGGL(k_moment_partial<kReadoutLines>, dim3(n_blocks, groups), dim3(256), 0, s, n,
+                           mag, mom, x0, wsum, label, 0u, grads, pc, partial);
+    if (done < ndir)
+        hipLaunchKernelGGL(k_moment_partial<1>, dim3(n_blocks, ndir - done), dim3(256), 0, s, n, mag,
+                           mom, x0, wsum, label, done, grads, pc, partial);
     hipLaunchKernelGGL(k_partial_final, dim3(ndir), dim3(256), 0, s, partial, n_blocks, out);
     return hipGetLastError();
 }

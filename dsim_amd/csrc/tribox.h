@@ -84,16 +84,21 @@ __host__ __device__ inline bool tribox_separated(const TriBoxAxes &T, double eps
 }
 
 // The square of the largest separation over the axes (0 when none
-// separates): a lower bound of the squared distance between the two.
-__host__ __device__ inline double tribox_gap2(const TriBoxAxes &T) {
+// separates): a lower bound of the squared distance between the two.  Once it
+// reaches `enough` the rest of the axes is left out: for a caller that keeps
+// the smallest such square, any value from its own on is as good.  The
+// triangle's plane, which separates most, comes first.
+__host__ __device__ inline double tribox_gap2(const TriBoxAxes &T, double enough = 1e300) {
     double best = 0.0;
-    for (int q = 0; q < 13; ++q) {
+    for (int i = 0; i < 13; ++i) {
+        const int q = i == 0 ? 3 : i <= 3 ? i - 1 : i;
         double ax[3], aa;
         tribox_axis(T, q, ax);
         const double g = tribox_sep(T, ax, aa);
         if (g > 0.0 && aa > 0.0) {
             const double d2 = g * g / aa;
             if (d2 > best) best = d2;
+            if (best >= enough) break;
         }
     }
     return best;

@@ -176,6 +176,12 @@ hipError_t launch_moment_signal(uint32_t n, const float *mag, const float *mom, 
                                 float wsum, const uint32_t *label, uint32_t ndir,
                                 const float *grads, float pc, double *partial, uint32_t n_blocks,
                                 double *out, hipStream_t s);
+// Error flags, positions and spin data (either may be null) in spin order; id
+// null where slots are spins.
+hipError_t launch_pack_state(uint32_t n, const uint32_t *x, const uint32_t *y, const uint32_t *z,
+                             const uint32_t *mag, const uint32_t *phase, const uint32_t *label,
+                             const uint32_t *id, const uint32_t *flags, uint32_t *out_flags,
+                             uint32_t *pos, uint32_t *spins, hipStream_t s);
 hipError_t launch_label(const LabelParams &p, hipStream_t s);
 // Grid-row labelling of the first +x ray, then the tiled pass over the spins
 // it leaves (ambiguous rays, spins outside the grid).  The buffers of the

@@ -15,7 +15,6 @@
 #include "host_common.h"
 #include "sim_internal.h"
 
-using dsim_host::DevBuf;
 using dsim_host::PoolBuf;
 using dsim_host::fail;
 
@@ -39,6 +38,8 @@ const size_t kMaxEventPairs = 64;
 const uint32_t kDefaultStepsPerLaunch = 1024;
 // Longest launch of a walk that records trajectories (sim_walk_traj).
 const uint32_t kTrajLaunchSteps = 128;
+// State read-backs of at most this many words go through one copy.
+constexpr size_t kPackWords = 1u << 18;
 
 }  // namespace
 
@@ -49,8 +50,9 @@ struct dsim_sim {
     uint64_t step = 0;
     hipStream_t stream = nullptr;
     PoolBuf<uint32_t> state, alt;  // F_COUNT * n words each (alt only when sorting)
-    PoolBuf<uint32_t> seed, flags;
-    PoolBuf<double> partial, out;
+    PoolBuf<uint32_t> seed;
+    PoolBuf<double> partial;
+    PoolBuf<double> out;  // the signal's 15 sums, and after them the error flags (four words)
     PoolBuf<float> grads;
     PoolBuf<float4> inject;
     PoolBuf<uint32_t> trace;
@@ -67,6 +69,7 @@ struct dsim_sim {
     double ms_done = 0.0;
     uint64_t launches = 0, sorts = 0;
 
+    uint32_t *flags() { return reinterpret_cast<uint32_t *>(out.p + 15); }
     uint32_t *f(int k) { return state.p + (size_t)k * n; }
     float *ff(int k) { return reinterpret_cast<float *>(f(k)); }
     bool sorting() const {
@@ -78,7 +81,7 @@ struct dsim_sim {
         // other stream holds work on them (the server waits for its rounds)
         if (stream) (void)hipStreamSynchronize(stream);
         for (auto &e : ev) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
-        for (auto *b : {&state, &alt, &seed, &flags, &trace, &keys_a, &keys_b, &vals_a,
+        for (auto *b : {&state, &alt, &seed, &trace, &keys_a, &keys_b, &vals_a,
                         &vals_b})
             b->release();
         partial.release(); out.release(); grads.release(); inject.release(); sort_tmp.release();
@@ -134,8 +137,8 @@ extern "C" int dsim_sim_create(dsim_substrate *sub, const dsim_params *p, uint32
     }
     const size_t m = std::max<uint32_t>(n, 1);
     int rc;
-    if ((rc = S->state.alloc(m * F_COUNT)) || (rc = S->flags.alloc(4)) || (rc = S->queue.alloc(8)) ||
-        (rc = S->partial.alloc((size_t)dsim::kSignalBlocks * 15)) || (rc = S->out.alloc(15)) ||
+    if ((rc = S->state.alloc(m * F_COUNT)) || (rc = S->queue.alloc(8)) ||
+        (rc = S->partial.alloc((size_t)dsim::kSignalBlocks * 15)) || (rc = S->out.alloc(17)) ||
         (p->rng == DSIM_RNG_MWC && (rc = S->seed.alloc(2 * m)))) {
         delete S;
         return rc;
@@ -155,7 +158,7 @@ extern "C" int dsim_sim_create(dsim_substrate *sub, const dsim_params *p, uint32
         }
     }
     e = hipMemsetAsync(S->state.p, 0, m * F_COUNT * 4, S->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(S->flags.p, 0, 16, S->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(S->flags(), 0, 16, S->stream);
     // MWC seeds: a draw keyed by the Philox key, so a fresh handle walks a
     // random stream (an all-zero MWC state repeats one draw forever); callers
     // with the reference's seeds replace them with dsim_set_state_aos
@@ -182,15 +185,20 @@ extern "C" int dsim_sim_destroy(dsim_sim *s) {
     return DSIM_OK;
 }
 
-static int sync_and_check(dsim_sim *s) {
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    uint32_t fl[4] = {0, 0, 0, 0};
-    HIP_TRY(hipMemcpy(fl, s->flags.p, 16, hipMemcpyDeviceToHost));
+// Reports and clears the error flags fl, as read from the device.
+static int check_flags(dsim_sim *s, const uint32_t fl[4]) {
     if (fl[0] & 1u) {
-        HIP_TRY(hipMemsetAsync(s->flags.p, 0, 16, s->stream));
+        HIP_TRY(hipMemsetAsync(s->flags(), 0, 16, s->stream));
         return fail(DSIM_ERR_OVERFLOW, "a spin exceeded 4096 collisions in one step");
     }
     return DSIM_OK;
+}
+
+static int sync_and_check(dsim_sim *s) {
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    uint32_t fl[4] = {0, 0, 0, 0};
+    HIP_TRY(hipMemcpy(fl, s->flags(), 16, hipMemcpyDeviceToHost));
+    return check_flags(s, fl);
 }
 
 // Copies field k to the host in spin order (undoing the spatial reorder).
@@ -268,37 +276,47 @@ extern "C" int dsim_set_state_aos(dsim_sim *s, const float *pos, const dsim_spin
 extern "C" int dsim_get_state_aos(dsim_sim *s, float *pos, dsim_spin_data *spins,
                                   uint32_t *seeds) {
     if (int rc = check_sim(s)) return rc;
-    if (int rc = sync_and_check(s)) return rc;
     const uint32_t n = s->n;
-    if (n == 0) return DSIM_OK;
-    std::vector<uint32_t> id;
-    if (int rc = spin_ids(s, id)) return rc;
-    if (pos) {
-        std::vector<float> a(n), b(n), c(n);
-        int rc;
-        if ((rc = download_field(s, F_X, id, (uint32_t *)a.data())) ||
-            (rc = download_field(s, F_Y, id, (uint32_t *)b.data())) ||
-            (rc = download_field(s, F_Z, id, (uint32_t *)c.data())))
-            return rc;
-        for (uint32_t i = 0; i < n; ++i) { pos[3 * i] = a[i]; pos[3 * i + 1] = b[i]; pos[3 * i + 2] = c[i]; }
-    }
-    if (spins) {
-        std::vector<float> m(n), ph(n);
-        std::vector<uint32_t> lab(n);
-        int rc;
-        if ((rc = download_field(s, F_MAG, id, (uint32_t *)m.data())) ||
-            (rc = download_field(s, F_PHASE, id, (uint32_t *)ph.data())) ||
-            (rc = download_field(s, F_LABEL, id, lab.data())))
-            return rc;
-        for (uint32_t i = 0; i < n; ++i) {
-            memset(&spins[i], 0, sizeof(dsim_spin_data));
-            spins[i].signalMagnitude = m[i];
-            spins[i].signalPhase = ph[i];
-            spins[i].compartmentType = (uint8_t)(lab[i] & 0xFFu);
-            spins[i].insideFiber = (uint16_t)(lab[i] >> 8);
+    if (n == 0 || (!pos && !spins)) {
+        if (int rc = sync_and_check(s)) return rc;
+    } else {
+        // error flags, positions and spin data in spin order, made on the device
+        static_assert(sizeof(dsim_spin_data) == 12, "three words a spin");
+        const size_t part = (size_t)n * 3;  // words
+        const size_t words = 4 + (pos ? part : 0) + (spins ? part : 0);
+        PoolBuf<uint32_t> pack;
+        if (int rc = pack.alloc(words)) return rc;
+        uint32_t *d_pos = pos ? pack.p + 4 : nullptr;
+        uint32_t *d_spins = spins ? pack.p + 4 + (pos ? part : 0) : nullptr;
+        hipError_t e = dsim::launch_pack_state(n, s->f(F_X), s->f(F_Y), s->f(F_Z), s->f(F_MAG),
+                                               s->f(F_PHASE), s->f(F_LABEL),
+                                               s->permuted ? s->f(F_ID) : nullptr, s->flags(),
+                                               pack.p, d_pos, d_spins, s->stream);
+        // few spins in one copy; many straight into the caller's arrays, once
+        // the flags are known to be clear
+        const bool whole = words <= kPackWords;
+        std::vector<uint32_t> h(whole ? words : 4);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(h.data(), pack.p, h.size() * 4, hipMemcpyDeviceToHost, s->stream);
+        hipError_t es = hipStreamSynchronize(s->stream);
+        int rc = DSIM_OK;
+        if (e == hipSuccess) e = es;
+        if (e == hipSuccess) rc = check_flags(s, h.data());
+        if (e == hipSuccess && rc == DSIM_OK && whole) {
+            if (pos) memcpy(pos, h.data() + 4, part * 4);
+            if (spins) memcpy(spins, h.data() + words - part, part * 4);
+        } else if (e == hipSuccess && rc == DSIM_OK) {
+            if (pos) e = hipMemcpyAsync(pos, d_pos, part * 4, hipMemcpyDeviceToHost, s->stream);
+            if (e == hipSuccess && spins)
+                e = hipMemcpyAsync(spins, d_spins, part * 4, hipMemcpyDeviceToHost, s->stream);
+            es = hipStreamSynchronize(s->stream);
+            if (e == hipSuccess) e = es;
         }
+        pack.release();
+        if (rc) return rc;
+        if (e != hipSuccess) return fail(DSIM_ERR_HIP, "state copy: %s", hipGetErrorString(e));
     }
-    if (seeds) {
+    if (seeds && n) {
         if (!s->seed.p) return fail(DSIM_ERR_STATE, "rng is not MWC");
         HIP_TRY(hipMemcpy(seeds, s->seed.p, (size_t)n * 8, hipMemcpyDeviceToHost));
     }
@@ -366,7 +384,7 @@ static dsim::StepParams step_params(dsim_sim *s) {
     P.wrap = s->f(F_WRAP);
     P.key0 = (uint32_t)s->prm.seed;
     P.key1 = (uint32_t)(s->prm.seed >> 32);
-    P.flags = s->flags.p;
+    P.flags = s->flags();
     P.queue = s->prm.fixed_blocks ? nullptr : s->queue.p;
     return P;
 }
@@ -519,9 +537,12 @@ extern "C" int dsim_signal(dsim_sim *s, double out[5]) {
     hipError_t e = dsim::launch_signal(s->n, s->ff(F_MAG), s->ff(F_PHASE), s->f(F_LABEL),
                                        s->partial.p, dsim::kSignalBlocks, s->out.p, s->stream);
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "signal launch: %s", hipGetErrorString(e));
-    double v[15];
+    double v[17];  // the sums and the error flags
     HIP_TRY(hipMemcpyAsync(v, s->out.p, sizeof v, hipMemcpyDeviceToHost, s->stream));
-    if (int rc = sync_and_check(s)) return rc;
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    uint32_t fl[4];
+    memcpy(fl, v + 15, sizeof fl);
+    if (int rc = check_flags(s, fl)) return rc;
     for (int k = 0; k < 5; ++k)
         out[k] = v[10 + k] == 0.0 ? 0.0 : std::sqrt(v[k] * v[k] + v[5 + k] * v[5 + k]) / v[10 + k];
     return DSIM_OK;
@@ -572,13 +593,15 @@ extern "C" int dsim_signal_moment(dsim_sim *s, uint32_t ndir, const float *g, fl
                 (size_t)std::max<size_t>(ndir * (size_t)nb, dsim::kSignalBlocks) * 15))
             return rc;
     }
-    DevBuf<double> o;
+    PoolBuf<double> o;
     if (int rc = o.alloc((size_t)ndir * 15)) return rc;
-    HIP_TRY(hipMemcpyAsync(s->grads.p, g, (size_t)ndir * 12, hipMemcpyHostToDevice, s->stream));
-    hipError_t e = dsim::launch_moment_signal(s->n, s->ff(F_MAG), s->ff(F_MOM), s->ff(F_X0),
-                                              s->wsum, s->f(F_LABEL), ndir, s->grads.p, pc,
-                                              s->partial.p, nb, o.p, s->stream);
+    hipError_t e = hipMemcpyAsync(s->grads.p, g, (size_t)ndir * 12, hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess)
+        e = dsim::launch_moment_signal(s->n, s->ff(F_MAG), s->ff(F_MOM), s->ff(F_X0), s->wsum,
+                                       s->f(F_LABEL), ndir, s->grads.p, pc, s->partial.p, nb, o.p,
+                                       s->stream);
     if (e != hipSuccess) {
+        (void)hipStreamSynchronize(s->stream);
         o.release();
         return fail(DSIM_ERR_HIP, "moment signal: %s", hipGetErrorString(e));
     }

@@ -328,7 +328,7 @@ def served_bench(cs, envs, n_requests, round_steps=256, loads=(0.4,), overload_r
 def reference_mode_bench(n, steps, cpu_seconds, threads, cpu=True):
     """The reference-semantics path a drop-in user runs (spinKernelCpu.cpp
     arithmetic: softsurfer triangle test, first-cell walk over the 50^3 grid,
-    clamp box, MWC seeds; k_step on the device) on the small configuration's
+    clamp box, MWC seeds; k_ref_walk on the device) on the small configuration's
     mesh: device rate over `steps` steps of `n` spins, and the oracle's rate in
     the same mode on a sample of the same spins on the host cores."""
     import oracle as O

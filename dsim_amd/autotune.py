@@ -66,7 +66,7 @@ def tune(cfg, axons, n, *, cells_um=(0.15, 0.2, 0.25), sorts=SORTS,
     interval, then the largest cell (fewer reorders, smaller grid) is chosen,
     so that repeated runs settle on the same configuration.  Each candidate
     launches launch_steps(sort) steps at a time, its warm-up runs past the
-    first reorder keyed by measured hit rates, and it is timed over at least
+    first reorder keyed by measured search rates, and it is timed over at least
     `steps` and two of its reorder intervals (whole launches and their
     reorders)."""
     results = []
@@ -77,7 +77,7 @@ def tune(cfg, axons, n, *, cells_um=(0.15, 0.2, 0.25), sorts=SORTS,
             sub, sim = make_sim(env, n, sort_interval=srt, steps_per_launch=launch_steps(srt))
             sim.init_uniform(1.0)
             sim.label(env["xmax"], env["xmax"], env["xmax"])
-            # warm up past the first reorder keyed by measured hit rates
+            # warm up past the first reorder keyed by measured search rates
             timed = max(steps, 2 * srt)
             sec = time_steps(sim, timed, warm=max(warm, srt + 64))
             rate = n * timed / sec

@@ -254,7 +254,7 @@ struct Fields {
     uint32_t count;
 };
 hipError_t sort_temp_bytes(uint32_t n, size_t *bytes);
-// Sort keys of the spins (hit band, then cell Morton index) and the slot
+// Sort keys of the spins (band of search rate, then cell Morton index) and the slot
 // permutation that orders them, stably; *perm points at the permutation (one
 // of the two value buffers).
 hipError_t launch_sort_perm(const StepParams &p, uint32_t *keys_a, uint32_t *keys_b,

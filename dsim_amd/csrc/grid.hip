@@ -807,9 +807,10 @@ uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); 
 }  // namespace
 
 // Fine cells per grid cell and axis.  Planar grids take 4 (16 bytes a grid
-// cell), three-dimensional ones 2 (8 bytes), less where the table would pass
-// kFineMaxBytes.
-constexpr uint32_t kFineSub2D = 4, kFineSub3D = 2;
+// cell), less where the table would pass kFineMaxBytes; three-dimensional ones
+// take 1: with 2 (8 bytes) crossing bundles walk no faster (50,000 spins 22.8 ms
+// and 22.9, 24 served requests 71.9 and 72.3) and the table takes 20 ms to build.
+constexpr uint32_t kFineSub2D = 4, kFineSub3D = 1;
 constexpr uint64_t kFineMaxBytes = 1ull << 29;
 
 static int build_fine_clearance(dsim_substrate *S, hipStream_t st) {
@@ -936,8 +937,8 @@ static int build_ref_tables(dsim_substrate *S, hipStream_t st) {
     return DSIM_OK;
 }
 
-// Row lists of the labeller (LabelParams::row_start).
-static int build_row_lists(dsim_substrate *S, hipStream_t st) {
+int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t most,
+                               hipStream_t st) {
     const uint32_t nT = S->n_tri, nC = S->n_cells;
     RowGeom g{};
     g.A = (int)S->label_axis;
@@ -951,9 +952,9 @@ static int build_row_lists(dsim_substrate *S, hipStream_t st) {
     TempBuf<uint32_t> outside;  // and after it the rows' counts of their entries
     int rc;
     size_t tb = 0;
-    HIP_TRY(rocprim::exclusive_scan(nullptr, tb, S->row_start.p, S->row_start.p, 0u,
+    HIP_TRY(rocprim::exclusive_scan(nullptr, tb, R.start.p, R.start.p, 0u,
                                     (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
-    if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = S->row_start.alloc((size_t)nC + 1)) ||
+    if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = R.start.alloc((size_t)nC + 1)) ||
         (rc = outside.alloc((size_t)nT + 1 + n_rows)))
         return rc;
     uint32_t *ends = outside.p + nT + 1;
@@ -966,23 +967,27 @@ static int build_row_lists(dsim_substrate *S, hipStream_t st) {
                            (float4 *)nullptr);
     }
     hipLaunchKernelGGL(k_row_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
-                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, S->row_start.p,
+                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, R.start.p,
                        (uint32_t *)nullptr, (float4 *)nullptr);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemsetAsync(S->row_start.p + nC, 0, 4, st));
-    HIP_TRY(rocprim::exclusive_scan(temp.p, tb, S->row_start.p, S->row_start.p, 0u,
+    HIP_TRY(hipMemsetAsync(R.start.p + nC, 0, 4, st));
+    HIP_TRY(rocprim::exclusive_scan(temp.p, tb, R.start.p, R.start.p, 0u,
                                     (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
     uint32_t n = 0;
-    HIP_TRY(hipMemcpyAsync(&n, S->row_start.p + nC, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&n, R.start.p + nC, 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     const size_t n1 = std::max<uint32_t>(n, 1);  // a lane past its row's end reads entry 0
-    if ((rc = S->row_tri.alloc(n1)) || (rc = S->row_box.alloc(n1))) return rc;
+    if (((uint64_t)nC + 1) * 4 + (uint64_t)n1 * 20 > most) {
+        R.start.release();
+        return DSIM_OK;
+    }
+    if ((rc = R.tri.alloc(n1)) || (rc = R.box.alloc(n1))) return rc;
     hipLaunchKernelGGL(k_row_lists<true>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
-                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, S->row_start.p,
-                       S->row_tri.p, S->row_box.p);
+                       S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, R.start.p,
+                       R.tri.p, R.box.p);
     if (nT)
         hipLaunchKernelGGL(k_row_ends<true>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
-                           S->tri_aabb.p, ends, S->row_start.p, S->row_tri.p, S->row_box.p);
+                           S->tri_aabb.p, ends, R.start.p, R.tri.p, R.box.p);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     return DSIM_OK;
@@ -990,7 +995,7 @@ static int build_row_lists(dsim_substrate *S, hipStream_t st) {
 
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
     if (S->kind != DSIM_GRID_REFERENCE)
-        if (int rc = build_row_lists(S, st)) return rc;
+        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, st)) return rc;
     if (S->kind == DSIM_GRID_REFERENCE)
         if (int rc = build_ref_tables(S, st)) return rc;
     if (int rc = build_search_lists(S, st)) return rc;

@@ -761,7 +761,7 @@ extern "C" int dsim_substrate_bytes(const dsim_substrate *s, uint64_t *bytes) {
     if (!s || !bytes) return fail(DSIM_ERR_ARG, "NULL argument");
     *bytes = (uint64_t)s->tri_ref.n * 16 + s->tri_mt.n * 16 + s->tri_aabb.n * 16 + s->walk_rec.n * 16 +
              s->walk_ent.n * 8 + s->walk_start.n * 4 + s->ref_rec.n * 16 + s->ref_mask.n * 4 +
-             (s->row_start.n + s->row_tri.n) * 4 + s->row_box.n * 16 +
+             s->rows.bytes() +
              s->d_cell_start.n * 4 + s->d_cell_tri.n * 4 + s->fiber_myelin.n + s->d_clearance.n * 4 +
              s->d_helpers.n * 4 + s->d_fine.n;
     return DSIM_OK;

@@ -689,8 +689,19 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
     // counters (groups, ambiguous, queued), then per spin the retry queue's
     // entry and the place in the row order
+    dsim_host::RowLists own;  // of this call, where the substrate keeps none
+    if (rows && !sub->rows.start.p)
+        if (int rc = dsim_host::build_row_lists(sub, own, ~0ull, s->stream)) {
+            (void)hipStreamSynchronize(s->stream);
+            own.release();
+            return rc;
+        }
+    const dsim_host::RowLists &lists = own.start.p ? own : sub->rows;
     PoolBuf<uint32_t> work;
-    if (int rc = work.alloc(words)) return rc;
+    if (int rc = work.alloc(words)) {
+        own.release();
+        return rc;
+    }
     uint32_t *w = work.p;
     L.group = w;
     L.n_ambiguous = w + counters - 2;
@@ -698,12 +709,12 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     hipError_t e = hipMemsetAsync(w, 0, counters * 4, s->stream);
     if (rows) {
         L.retry = reinterpret_cast<uint2 *>(w + counters);
-        const uint64_t row_bytes = (uint64_t)sub->row_tri.n * 20 + (uint64_t)sub->n_tri * 96;
+        const uint64_t row_bytes = (uint64_t)lists.tri.n * 20 + (uint64_t)sub->n_tri * 96;
         L.order = s->n >= dsim::kLabelOrderMin && row_bytes > dsim::kXcdL2Bytes
                       ? w + counters + 2 * (size_t)s->n : nullptr;
-        L.row_start = sub->row_start.p;
-        L.row_tri = sub->row_tri.p;
-        L.row_box = sub->row_box.p;
+        L.row_start = lists.start.p;
+        L.row_tri = lists.tri.p;
+        L.row_box = lists.box.p;
         for (int k = 0; k < 3; ++k) {
             L.dims[k] = sub->dims[k];
             L.lo[k] = sub->lo[k];
@@ -720,6 +731,7 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
         e = hipMemcpyAsync(&ambiguous, L.n_ambiguous, 4, hipMemcpyDeviceToHost, s->stream);
     const hipError_t es = hipStreamSynchronize(s->stream);
     work.release();
+    own.release();
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
     if (n_ambiguous) *n_ambiguous = ambiguous;

@@ -43,6 +43,7 @@ def _mesh(axis, seed):
     (2, "tribox", (10, 10, 10), 33),
     (0, "aabb", (4, 512, 512), 32768),     # ordered by row: rows past the L2's size
     (2, "aabb", (300, 300, 4), 40001),
+    (0, "aabb", (4, 1100, 1100), 20001),   # lists too large to keep, made by the call
 ])
 def test_rows_match_the_pass_over_all_triangles(axis, grid, dims, n):
     print(f"case label rows axis {axis} {grid} {dims} spins {n}", flush=True)

@@ -808,8 +808,9 @@ uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); 
 
 // Fine cells per grid cell and axis.  Planar grids take 4 (16 bytes a grid
 // cell), less where the table would pass kFineMaxBytes; three-dimensional ones
-// take 1: with 2 (8 bytes) crossing bundles walk no faster (50,000 spins 22.8 ms
-// and 22.9, 24 served requests 71.9 and 72.3) and the table takes 20 ms to build.
+// take 1: with 2 (8 bytes) 50,000 spins among crossing bundles walk no faster
+// (22.8 ms and 22.9), the device full of larger substrates by 5% (1.34e10
+// spin-steps/s against 1.27e10), for 7 bytes a cell and twice the build time.
 constexpr uint32_t kFineSub2D = 4, kFineSub3D = 1;
 constexpr uint64_t kFineMaxBytes = 1ull << 29;
 

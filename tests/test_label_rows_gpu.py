@@ -22,8 +22,8 @@ def _need_gpu():
         pytest.fail("no HIP device visible: GPU tests need an MI355X")
 
 
-def _mesh(axis, seed):
-    V, T, I = _soup(160, seed)
+def _mesh(axis, seed, tris=160):
+    V, T, I = _soup(tris, seed)
     V = V.copy()
     if axis:  # the walls (along z) along x
         V = V[:, [2, 1, 0]]
@@ -43,17 +43,17 @@ def _mesh(axis, seed):
     (2, "tribox", (10, 10, 10), 33),
     (0, "aabb", (4, 512, 512), 32768),     # ordered by row: rows past the L2's size
     (2, "aabb", (300, 300, 4), 40001),
-    (0, "aabb", (4, 1100, 1100), 20001),   # lists too large to keep, made by the call
+    (0, "tribox", (58, 760, 764), 20001),  # lists too large to keep, made by the call
 ])
 def test_rows_match_the_pass_over_all_triangles(axis, grid, dims, n):
     print(f"case label rows axis {axis} {grid} {dims} spins {n}", flush=True)
-    V, T, I = _mesh(axis, 5)
+    V, T, I = _mesh(axis, 5, 12 if dims[1] > 700 else 160)
     pos = np.random.default_rng(n).uniform(-0.95, 0.95, (n, 3)).astype(np.float32)
     pos[:, axis] *= 0.6
     lo, hi = np.array([-1.0, -0.9, -0.8]), np.array([0.7, 0.8, 0.9])
     hi[axis] = 0.25  # triangles beyond it
     sub = D.Substrate(V, T, I, device=True, grid=grid, dims=dims, lo=tuple(lo),
-                      cell=tuple((hi - lo) / dims), eps=1e-5)
+                      cell=tuple((hi - lo) / dims), eps=1e-5, clearance_rings=1)
     assert sub.label_axis() == axis
     out = []
     for s in (D.Substrate(V, T, I, device=True, n_cubes=10), sub):
@@ -71,4 +71,4 @@ def test_rows_match_the_pass_over_all_triangles(axis, grid, dims, n):
         assert a[0] == b[0]
         np.testing.assert_array_equal(a[1], b[1])
         np.testing.assert_array_equal(a[2], b[2])
-    assert n < 100 or (out[0][0][1] > 0).sum() > n // 10
+    assert n < 100 or (out[0][0][1] > 0).sum() > n // 20

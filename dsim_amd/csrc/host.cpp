@@ -361,14 +361,14 @@ struct PoolBlock {
 };
 std::mutex pool_mu;
 std::vector<PoolBlock> pool;  // oldest first
-size_t pool_bytes = 0;
 uint64_t pool_users = 0;
 
-// The oldest block out of the pool (under pool_mu).
-PoolBlock pool_oldest() {
-    const PoolBlock b = pool.front();
-    pool.erase(pool.begin());
-    pool_bytes -= b.bytes;
+// The oldest block of the device (any for -1) out of the pool (under pool_mu).
+PoolBlock pool_oldest(int device) {
+    auto it = pool.begin();
+    while (device >= 0 && it->device != device) ++it;
+    const PoolBlock b = *it;
+    pool.erase(it);
     return b;
 }
 
@@ -378,7 +378,6 @@ bool pool_trim() {
     {
         std::lock_guard<std::mutex> l(pool_mu);
         idle.swap(pool);
-        pool_bytes = 0;
     }
     for (const PoolBlock &b : idle) (void)hipFree(b.p);
     return !idle.empty();
@@ -396,21 +395,23 @@ void *dsim_host::dev_alloc(size_t bytes, hipError_t *e) {
     return *e == hipSuccess ? p : nullptr;
 }
 
-void *dsim_host::pool_take(size_t bytes, size_t *got, hipError_t *e) {
+void *dsim_host::pool_take(size_t bytes, size_t *got, int *device, hipError_t *e) {
     *got = bytes;
     *e = hipSuccess;
-    int device = 0;
-    if (hipGetDevice(&device) == hipSuccess) {
+    if (hipGetDevice(device) != hipSuccess) {
+        *device = -1;  // not for the pool
+        return dev_alloc(bytes, e);
+    }
+    {
         std::lock_guard<std::mutex> l(pool_mu);
         size_t best = pool.size();
         for (size_t k = 0; k < pool.size(); ++k)
-            if (pool[k].device == device && pool[k].bytes >= bytes &&
+            if (pool[k].device == *device && pool[k].bytes >= bytes &&
                 pool[k].bytes / 4 * 3 <= bytes && (best == pool.size() || pool[k].bytes < pool[best].bytes))
                 best = k;
         if (best < pool.size()) {
             const PoolBlock b = pool[best];
             pool.erase(pool.begin() + best);
-            pool_bytes -= b.bytes;
             *got = b.bytes;
             return b.p;
         }
@@ -418,11 +419,9 @@ void *dsim_host::pool_take(size_t bytes, size_t *got, hipError_t *e) {
     return dev_alloc(bytes, e);
 }
 
-void dsim_host::pool_give(void *p, size_t bytes) {
-    int device = 0;
+void dsim_host::pool_give(void *p, size_t bytes, int device) {
     size_t total = 0;
-    if (hipGetDevice(&device) != hipSuccess || hipDeviceTotalMem(&total, device) != hipSuccess)
-        total = 0;
+    if (device < 0 || hipDeviceTotalMem(&total, device) != hipSuccess) total = 0;
     const size_t limit = total / kPoolShare;
     std::vector<PoolBlock> out;
     if (bytes > limit) {
@@ -430,9 +429,14 @@ void dsim_host::pool_give(void *p, size_t bytes) {
     } else {
         std::lock_guard<std::mutex> l(pool_mu);
         pool.push_back({p, bytes, device});
-        pool_bytes += bytes;
-        while (pool_bytes > limit || pool.size() > kPoolBlocks || (!pool_users && !pool.empty()))
-            out.push_back(pool_oldest());
+        size_t held = 0;  // idle on this device
+        for (const PoolBlock &b : pool) held += b.device == device ? b.bytes : 0;
+        while (held > limit) {
+            out.push_back(pool_oldest(device));
+            held -= out.back().bytes;
+        }
+        while (pool.size() > kPoolBlocks || (!pool_users && !pool.empty()))
+            out.push_back(pool_oldest(-1));
     }
     for (const PoolBlock &b : out) (void)hipFree(b.p);
 }

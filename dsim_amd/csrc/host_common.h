@@ -51,8 +51,9 @@ void *dev_alloc(size_t bytes, hipError_t *e);
 
 // Idle blocks of simulation and waveform handles, kept for the next handle
 // while any simulation or server is alive (pool_ref, pool_unref), up to
-// 1/kPoolShare of the device's memory, the oldest given back first, and all
-// given back when an allocation here would fail.  Handles come and go with
+// 1/kPoolShare of each device's memory, the oldest given back first, and all
+// given back when an allocation here would fail.  A block stays with the device
+// that was current when it was allocated, whichever is when it is given back.  Handles come and go with
 // every request or run of waveforms, and gigabytes freed and allocated each
 // time cost the runtime far more than the work at times: freeing the 9.5 GB of
 // 1024 waveforms of 500,000 spins took 1.5 ms or, once a run had allocated
@@ -60,8 +61,8 @@ void *dev_alloc(size_t bytes, hipError_t *e);
 // request of at least three quarters of its size.  The caller of pool_give
 // has waited for the device, as hipFree does.
 constexpr size_t kPoolShare = 16, kPoolBlocks = 256;
-void *pool_take(size_t bytes, size_t *got, hipError_t *e);
-void pool_give(void *p, size_t bytes);
+void *pool_take(size_t bytes, size_t *got, int *device, hipError_t *e);
+void pool_give(void *p, size_t bytes, int device);
 void pool_ref();
 void pool_unref();
 
@@ -70,11 +71,12 @@ struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
     size_t block = 0;  // bytes of the pool's block
+    int device = -1;   // that it lies on
     int alloc(size_t count) {
         n = count;
         if (count == 0) return DSIM_OK;
         hipError_t e = hipSuccess;
-        p = static_cast<T *>(POOL ? pool_take(count * sizeof(T), &block, &e)
+        p = static_cast<T *>(POOL ? pool_take(count * sizeof(T), &block, &device, &e)
                                   : dev_alloc(count * sizeof(T), &e));
         if (!p) {
             n = 0;
@@ -84,7 +86,7 @@ struct DevBuf {
         return DSIM_OK;
     }
     void release() {
-        if (p && POOL) pool_give(p, block);
+        if (p && POOL) pool_give(p, block, device);
         else if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;

@@ -1,0 +1,149 @@
+// Checks of the library's host code over the host-memory runtime: one case by
+// name, or all of them.
+#include "stub_hip.h"
+
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <string>
+#include <vector>
+
+#include <hip/hip_runtime_api.h>
+
+#include "../../dsim_amd/csrc/host_common.h"
+#include "../../dsim_amd/csrc/sim_internal.h"
+#include "../../include/dsim.h"
+#include "../../include/dsim_phase.h"
+#include "../../include/dsim_serve.h"
+
+static int fails = 0;
+#define EXPECT(c)                                                              \
+    do {                                                                       \
+        if (!(c)) {                                                            \
+            fprintf(stderr, "FAILED %s:%d: %s (%s)\n", __FILE__, __LINE__, #c, \
+                    dsim_last_error());                                        \
+            ++fails;                                                           \
+        }                                                                      \
+    } while (0)
+
+using dsim_host::PoolBuf;
+
+static int device_of(const void *p) { return stub::blocks.at(const_cast<void *>(p)).device; }
+
+static dsim_substrate *make_sub(uint32_t kind = DSIM_GRID_AABB, uint32_t n_tri = 0) {
+    std::vector<float> v(3 * 3 * (size_t)n_tri);
+    std::vector<uint32_t> t(3 * (size_t)n_tri), info(3 * (size_t)n_tri, 0);
+    for (uint32_t k = 0; k < 3 * n_tri; ++k) {
+        t[k] = k;
+        for (int a = 0; a < 3; ++a) v[3 * k + a] = 0.1f * (float)((k * 7 + a * 3) % 11) - 0.5f;
+    }
+    dsim_mesh m{3 * n_tri, v.data(), n_tri, t.data(), info.data()};
+    dsim_grid_params g{};
+    g.kind = kind;
+    for (int k = 0; k < 3; ++k) { g.dims[k] = 4; g.lo[k] = -1.0f; g.cell[k] = 0.5f; }
+    dsim_substrate *s = nullptr;
+    EXPECT(dsim_substrate_create(&m, &g, &s) == DSIM_OK);
+    return s;
+}
+
+static dsim_params params(uint32_t sort = 0) {
+    dsim_params p{};
+    p.dt = 0.005f;
+    for (int c = 0; c < 4; ++c) { p.std_dev[c] = 0.01f; p.t2[c] = INFINITY; }
+    p.reflection_type = 1;
+    p.mode = DSIM_MODE_PHYSICAL;
+    p.boundary = DSIM_BOUNDARY_PERIODIC;
+    p.rng = DSIM_RNG_PHILOX;
+    p.sort_interval = sort;
+    return p;
+}
+
+static dsim_sim *make_sim(dsim_substrate *s, uint32_t n, uint32_t sort = 0) {
+    const dsim_params p = params(sort);
+    dsim_sim *h = nullptr;
+    EXPECT(dsim_sim_create(s, &p, n, &h) == DSIM_OK);
+    return h;
+}
+
+// A block goes back under the device that it was allocated on, whatever device
+// is current then.
+static void pool_device() {
+    dsim_host::pool_ref();
+    PoolBuf<float> a, b, c;
+    hipSetDevice(1);
+    EXPECT(a.alloc(1000) == DSIM_OK);
+    const void *on1 = a.p;
+    hipSetDevice(0);
+    a.release();
+    EXPECT(b.alloc(1000) == DSIM_OK);
+    EXPECT(device_of(b.p) == 0);
+    hipSetDevice(1);
+    EXPECT(c.alloc(1000) == DSIM_OK);
+    EXPECT(c.p == on1 && device_of(c.p) == 1);
+    hipSetDevice(0);
+    b.release();
+    c.release();
+    dsim_host::pool_unref();
+    EXPECT(stub::blocks.empty());
+}
+
+// Each device's idle blocks are held to its own share.
+static void pool_bound() {
+    dsim_host::pool_ref();
+    const size_t lim[2] = {stub::total[0] / dsim_host::kPoolShare,
+                           stub::total[1] / dsim_host::kPoolShare};
+    std::vector<PoolBuf<uint8_t>> v[2];
+    for (int d : {0, 1}) {
+        hipSetDevice(d);
+        v[d].resize(4);
+        for (auto &b : v[d]) EXPECT(b.alloc(lim[d] / 3) == DSIM_OK);
+    }
+    for (int d : {0, 1}) {
+        hipSetDevice(1 - d);  // the other device is current when they are given back
+        for (auto &b : v[d]) b.release();
+    }
+    for (int d : {0, 1}) {
+        EXPECT(stub::used[d] <= lim[d]);
+        EXPECT(stub::used[d] >= lim[d] / 2);  // and one device does not push out the other's
+    }
+    hipSetDevice(0);
+    dsim_host::pool_unref();
+    EXPECT(stub::blocks.empty());
+}
+
+// Handles made and closed with different devices current.
+static void handle_device() {
+    hipSetDevice(0);
+    dsim_substrate *s0 = make_sub();
+    hipSetDevice(1);
+    dsim_substrate *s1 = make_sub();
+    dsim_sim *keep = make_sim(s1, 100), *h = make_sim(s1, 1000, 16);
+    hipSetDevice(0);
+    EXPECT(dsim_sim_destroy(h) == DSIM_OK);
+    const size_t before = stub::used[1];
+    dsim_sim *g = make_sim(s0, 1000, 16);
+    EXPECT(stub::used[1] == before);
+    size_t on0 = 0;
+    for (auto &kv : stub::blocks) on0 += kv.second.device == 0 ? kv.second.bytes : 0;
+    EXPECT(on0 >= 2 * 21 * 4 * 1000);  // both state blocks
+    EXPECT(dsim_sim_destroy(g) == DSIM_OK);
+    EXPECT(dsim_sim_destroy(keep) == DSIM_OK);
+    EXPECT(dsim_substrate_destroy(s0) == DSIM_OK && dsim_substrate_destroy(s1) == DSIM_OK);
+    EXPECT(stub::blocks.empty());
+}
+
+int main(int argc, char **argv) {
+    const std::pair<const char *, void (*)()> cases[] = {
+        {"pool_device", pool_device},
+        {"pool_bound", pool_bound},
+        {"handle_device", handle_device},
+    };
+    for (auto &c : cases) {
+        if (argc > 1 && strcmp(argv[1], c.first)) continue;
+        const int was = fails;
+        c.second();
+        printf("%s: %s\n", c.first, fails == was ? "ok" : "FAILED");
+    }
+    return fails != 0;
+}

@@ -127,6 +127,7 @@ struct LabelParams {
     // *n_retry.
     const uint32_t *row_start, *row_tri;
     const float4 *row_box;
+    uint32_t shared, shared_end;  // places of the entries that belong to every row
     uint32_t dims[3];
     float lo[3], hi[3], cell[3], inv_cell[3];
     uint2 *retry;

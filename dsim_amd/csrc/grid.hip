@@ -719,11 +719,45 @@ __device__ __forceinline__ float4 row_extent(const RowGeom &g, const float4 *box
                        g.C == 1 ? hi.y : hi.z);
 }
 
-// The triangles past the grid, after their count.
+// Ranges of the rows that a box of extents e may meet, from one cell to either
+// side.
+struct RowRange {
+    uint32_t b, c, wide, high;
+};
+__device__ __forceinline__ RowRange row_range(const RowGeom &g, const float4 e) {
+    const uint32_t nb = g.dims[g.B], nc = g.dims[g.C];
+    const float b0 = (e.x - g.lo[g.B]) / g.cell[g.B], b1 = (e.y - g.lo[g.B]) / g.cell[g.B];
+    const float c0 = (e.z - g.lo[g.C]) / g.cell[g.C], c1 = (e.w - g.lo[g.C]) / g.cell[g.C];
+    auto slack = [](float v) { return 1.0f + 1e-6f * fabsf(v); };
+    const int bl = (int)fminf(fmaxf(b0 - slack(b0), 0.0f), (float)(nb - 1));
+    const int bh = (int)fminf(fmaxf(b1 + slack(b1), 0.0f), (float)(nb - 1));
+    const int cl = (int)fminf(fmaxf(c0 - slack(c0), 0.0f), (float)(nc - 1));
+    const int ch = (int)fminf(fmaxf(c1 + slack(c1), 0.0f), (float)(nc - 1));
+    return RowRange{(uint32_t)bl, (uint32_t)cl, (uint32_t)max(bh - bl + 1, 0),
+                    (uint32_t)max(ch - cl + 1, 0)};
+}
+
+// The triangles past the grid, after their count; *ends (of all zero before):
+// the sum of their rows, in 64 bits.
 __global__ __launch_bounds__(kBlock) void k_row_outside(RowGeom g, uint32_t n_tri,
-                                                        const float4 *box, uint32_t *outside) {
+                                                        const float4 *box, uint32_t *outside,
+                                                        unsigned long long *ends) {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t < n_tri && past_grid(g, box, t)) outside[1 + atomicAdd(&outside[0], 1u)] = t;
+    if (t >= n_tri || !past_grid(g, box, t)) return;
+    outside[1 + atomicAdd(&outside[0], 1u)] = t;
+    const RowRange r = row_range(g, row_extent(g, box, t));
+    atomicAdd(ends, (unsigned long long)r.wide * r.high);
+}
+
+// The list that every row shares, at its place.
+__global__ __launch_bounds__(kBlock) void k_row_shared(RowGeom g, const uint32_t *outside,
+                                                       const float4 *box, uint32_t *tri,
+                                                       float4 *rec) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    if (j >= outside[0]) return;
+    const uint32_t t = outside[1 + j];
+    tri[j] = t;
+    rec[j] = row_extent(g, box, t);
 }
 
 // Their entries: in every row whose cells' boxes, computed as label_cell does,
@@ -735,22 +769,14 @@ __global__ __launch_bounds__(kBlock) void k_row_ends(RowGeom g, const uint32_t *
                                                      const float4 *box, uint32_t *count,
                                                      const uint32_t *start, uint32_t *tri,
                                                      float4 *rec) {
-    const uint32_t n = outside[0], nb = g.dims[g.B], nc = g.dims[g.C];
+    const uint32_t n = outside[0], nb = g.dims[g.B];
     for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
         const uint32_t t = outside[1 + j];
         const float4 e = row_extent(g, box, t);
-        // cell ranges to either side, then the boxes themselves
-        const float b0 = (e.x - g.lo[g.B]) / g.cell[g.B], b1 = (e.y - g.lo[g.B]) / g.cell[g.B];
-        const float c0 = (e.z - g.lo[g.C]) / g.cell[g.C], c1 = (e.w - g.lo[g.C]) / g.cell[g.C];
-        auto slack = [](float v) { return 1.0f + 1e-6f * fabsf(v); };
-        const int bl = (int)fminf(fmaxf(b0 - slack(b0), 0.0f), (float)(nb - 1));
-        const int bh = (int)fminf(fmaxf(b1 + slack(b1), 0.0f), (float)(nb - 1));
-        const int cl = (int)fminf(fmaxf(c0 - slack(c0), 0.0f), (float)(nc - 1));
-        const int ch = (int)fminf(fmaxf(c1 + slack(c1), 0.0f), (float)(nc - 1));
-        const uint32_t wide = (uint32_t)max(bh - bl + 1, 0);
-        const uint64_t all = (uint64_t)wide * (uint32_t)max(ch - cl + 1, 0);
+        const RowRange w = row_range(g, e);
+        const uint64_t all = (uint64_t)w.wide * w.high;
         for (uint64_t k = threadIdx.x; k < all; k += kBlock) {
-            const uint32_t b = bl + (uint32_t)(k % wide), c = cl + (uint32_t)(k / wide);
+            const uint32_t b = w.b + (uint32_t)(k % w.wide), c = w.c + (uint32_t)(k / w.wide);
             if (e.y < g.lo[g.B] + (float)b * g.cell[g.B] ||
                 e.x > g.lo[g.B] + (float)(b + 1) * g.cell[g.B] ||
                 e.w < g.lo[g.C] + (float)c * g.cell[g.C] ||
@@ -951,22 +977,35 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     const uint32_t n_rows = g.dims[g.B] * g.dims[g.C], n_blocks = std::min(nT, 1024u);
     TempBuf<uint8_t> temp;
     TempBuf<uint32_t> outside;  // and after it the rows' counts of their entries
+    TempBuf<unsigned long long> sum;
     int rc;
     size_t tb = 0;
     HIP_TRY(rocprim::exclusive_scan(nullptr, tb, R.start.p, R.start.p, 0u,
                                     (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
     if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = R.start.alloc((size_t)nC + 1)) ||
-        (rc = outside.alloc((size_t)nT + 1 + n_rows)))
+        (rc = outside.alloc((size_t)nT + 1 + n_rows)) || (rc = sum.alloc(1)))
         return rc;
     uint32_t *ends = outside.p + nT + 1;
     HIP_TRY(hipMemsetAsync(outside.p, 0, outside.n * 4, st));
-    if (nT) {
+    HIP_TRY(hipMemsetAsync(sum.p, 0, 8, st));
+    if (nT)
         hipLaunchKernelGGL(k_row_outside, dim3(blocks_for(nT)), dim3(kBlock), 0, st, g, nT,
-                           S->tri_aabb.p, outside.p);
+                           S->tri_aabb.p, outside.p, sum.p);
+    HIP_TRY(hipGetLastError());
+    uint32_t n_out = 0;
+    unsigned long long n_ends = 0;
+    HIP_TRY(hipMemcpyAsync(&n_out, outside.p, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&n_ends, sum.p, 8, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    const RowPlan plan = row_plan(nC, S->d_cell_tri.n, n_out, n_ends);
+    if (plan == kRowsNone) {
+        R.start.release();
+        return DSIM_OK;
+    }
+    if (plan == kRowsEnds && n_out)
         hipLaunchKernelGGL(k_row_ends<false>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
                            S->tri_aabb.p, ends, (const uint32_t *)nullptr, (uint32_t *)nullptr,
                            (float4 *)nullptr);
-    }
     hipLaunchKernelGGL(k_row_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
                        S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, R.start.p,
                        (uint32_t *)nullptr, (float4 *)nullptr);
@@ -977,7 +1016,10 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     uint32_t n = 0;
     HIP_TRY(hipMemcpyAsync(&n, R.start.p + nC, 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    const size_t n1 = std::max<uint32_t>(n, 1);  // a lane past its row's end reads entry 0
+    R.shared = n;
+    R.n_shared = plan == kRowsShared ? n_out : 0u;
+    // a lane past its row's end reads entry 0
+    const size_t n1 = std::max<size_t>((size_t)n + R.n_shared, 1);
     if (((uint64_t)nC + 1) * 4 + (uint64_t)n1 * 20 > most) {
         R.start.release();
         return DSIM_OK;
@@ -986,9 +1028,12 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     hipLaunchKernelGGL(k_row_lists<true>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
                        S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, R.start.p,
                        R.tri.p, R.box.p);
-    if (nT)
+    if (plan == kRowsEnds && n_out)
         hipLaunchKernelGGL(k_row_ends<true>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
                            S->tri_aabb.p, ends, R.start.p, R.tri.p, R.box.p);
+    if (R.n_shared)
+        hipLaunchKernelGGL(k_row_shared, dim3(blocks_for(R.n_shared)), dim3(kBlock), 0, st, g,
+                           outside.p, S->tri_aabb.p, R.tri.p + n, R.box.p + n);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     return DSIM_OK;

@@ -122,10 +122,26 @@ constexpr uint64_t kRowKeepBytes = 128ull << 20;
 struct RowLists {
     PoolBuf<uint32_t> start, tri;
     PoolBuf<float4> box;
+    uint32_t shared = 0, n_shared = 0;  // entries of every row (kRowsShared)
     void release() { start.release(); tri.release(); box.release(); }
     uint64_t bytes() const { return (start.n + tri.n) * 4 + box.n * 16; }
 };
-// Lists of more than `most` bytes are left empty.  Waits for st.
+// Where the triangles past the grid's face stand: an entry in every row that
+// their boxes meet (`ends` at most), or, where those would be more than the
+// grid's own cells and entries or than kRowEndsMax (320 MB; their counting, an
+// atomic addition each, would take tens of ms and more), once in a list that
+// every row shares.  Places are 32-bit: a grid whose entries alone pass that
+// gets no row lists, and its spins go through the pass over all triangles.
+enum RowPlan { kRowsNone, kRowsShared, kRowsEnds };
+constexpr uint64_t kRowEndsMax = 1ull << 24;
+inline RowPlan row_plan(uint64_t n_cells, uint64_t n_entries, uint64_t n_outside, uint64_t ends) {
+    constexpr uint64_t most = 0xFFFFFF00ull;
+    if (n_entries + n_outside > most) return kRowsNone;
+    if (ends > n_cells + n_entries || ends > kRowEndsMax || n_entries + ends > most)
+        return kRowsShared;
+    return kRowsEnds;
+}
+// Lists of more than `most` bytes, or none by row_plan, are left empty.  Waits for st.
 int build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t most, hipStream_t st);
 }  // namespace dsim_host
 

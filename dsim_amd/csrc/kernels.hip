@@ -2565,7 +2565,8 @@ __device__ __forceinline__ uint32_t label_cell(const LabelParams &P, float v, in
 // a crossing, and in a contiguous run of the row's cells (a convex triangle
 // meets a convex row of boxes in an interval), so every crossing is counted
 // once.  The others stand at the end of every row whose cells' boxes meet
-// theirs across the ray.
+// theirs across the ray, or, where that would be too many entries, in a list
+// that every spin walks after its row.
 //
 // What bounds it: the lines its gathers touch in the vector cache, and their
 // latency.
@@ -2675,21 +2676,26 @@ __global__ __launch_bounds__(256) void k_label_row(LabelParams P) {
         }
         wave_lds_sync();
     };
-    // two entries a lane and round: both loads are in flight together
-    while (__ballot(k < end)) {
-        const bool in0 = k < end, in1 = k + kRowLanes < end;
-        const uint32_t k0 = in0 ? k : 0u, k1 = in1 ? k + kRowLanes : k0;
-        const float4 b0 = P.row_box[k0], b1 = P.row_box[k1];
-        const float vb = s3[B], vc = s3[C];
-        const bool on0 = in0 && !(vb > b0.y || b0.x > vb || vc > b0.w || b0.z > vc);
-        const bool on1 = in1 && !(vb > b1.y || b1.x > vb || vc > b1.w || b1.z > vc);
-        push(on0, on0 ? P.row_tri[k0] : 0u);
-        push(on1, on1 ? P.row_tri[k1] : 0u);
-        while (queued >= 64u) {
-            queued -= 64u;
-            test(queued, 64u);
+    // the spin's row, then what every row shares
+    for (uint32_t part = 0; part < 2; ++part) {
+        // two entries a lane and round: both loads are in flight together
+        while (__ballot(k < end)) {
+            const bool in0 = k < end, in1 = k + kRowLanes < end;
+            const uint32_t k0 = in0 ? k : 0u, k1 = in1 ? k + kRowLanes : k0;
+            const float4 b0 = P.row_box[k0], b1 = P.row_box[k1];
+            const float vb = s3[B], vc = s3[C];
+            const bool on0 = in0 && !(vb > b0.y || b0.x > vb || vc > b0.w || b0.z > vc);
+            const bool on1 = in1 && !(vb > b1.y || b1.x > vb || vc > b1.w || b1.z > vc);
+            push(on0, on0 ? P.row_tri[k0] : 0u);
+            push(on1, on1 ? P.row_tri[k1] : 0u);
+            while (queued >= 64u) {
+                queued -= 64u;
+                test(queued, 64u);
+            }
+            k += 2 * kRowLanes;
         }
-        k += 2 * kRowLanes;
+        k = P.shared + g;
+        end = row ? P.shared_end : 0u;
     }
     test(0u, queued);
     if (!live || g != 0) return;

@@ -683,12 +683,7 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     // labeller first; the rest, and every re-cast, go through the tiled pass
     // over all triangles
     const dsim_substrate *sub = s->sub;
-    const bool rows = L.ray_axis && sub->kind != DSIM_GRID_REFERENCE && sub->n_cells > 0 &&
-                      s->n > 0;
-    constexpr size_t counters = dsim::kLabelGroups + 2;  // even: the uint2 queue follows
-    const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
-    // counters (groups, ambiguous, queued), then per spin the retry queue's
-    // entry and the place in the row order
+    bool rows = L.ray_axis && sub->kind != DSIM_GRID_REFERENCE && sub->n_cells > 0 && s->n > 0;
     dsim_host::RowLists own;  // of this call, where the substrate keeps none
     if (rows && !sub->rows.start.p)
         if (int rc = dsim_host::build_row_lists(sub, own, ~0ull, s->stream)) {
@@ -697,6 +692,11 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
             return rc;
         }
     const dsim_host::RowLists &lists = own.start.p ? own : sub->rows;
+    rows = rows && lists.start.p;  // no lists: more entries than places
+    constexpr size_t counters = dsim::kLabelGroups + 2;  // even: the uint2 queue follows
+    const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
+    // counters (groups, ambiguous, queued), then per spin the retry queue's
+    // entry and the place in the row order
     PoolBuf<uint32_t> work;
     if (int rc = work.alloc(words)) {
         own.release();
@@ -715,6 +715,8 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
         L.row_start = lists.start.p;
         L.row_tri = lists.tri.p;
         L.row_box = lists.box.p;
+        L.shared = lists.shared;
+        L.shared_end = lists.shared + lists.n_shared;
         for (int k = 0; k < 3; ++k) {
             L.dims[k] = sub->dims[k];
             L.lo[k] = sub->lo[k];

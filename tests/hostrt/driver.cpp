@@ -133,11 +133,33 @@ static void handle_device() {
     EXPECT(stub::blocks.empty());
 }
 
+// Where the labeller's row lists put the triangles past the grid: never more
+// than their 32-bit places hold, nor more than the grid's own size.
+static void row_plan() {
+    using namespace dsim_host;
+    // a grid of the crossing bundles: 1600 axons
+    EXPECT(row_plan(14'503'175, 16'000'000, 9'000, 60'000) == kRowsEnds);
+    EXPECT(row_plan(1'000'000, 3'000'000, 0, 0) == kRowsEnds);
+    // 1e5 walls across the far face of a grid of 4e4 rows: 4e9 entries
+    EXPECT(row_plan(4'000'000, 3'000'000, 100'000, 4'000'000'000ull) == kRowsShared);
+    // whose sum wraps to few in 32 bits
+    EXPECT(row_plan(1ull << 28, 100'000'000, 1 << 20, (1ull << 32) + 5) == kRowsShared);
+    EXPECT(row_plan(1ull << 28, 0xFFFFFF00ull - 10, 5, 11) == kRowsShared);
+    EXPECT(row_plan(1ull << 28, 0xFFFFFF00ull - 10, 10, 10) == kRowsEnds);
+    EXPECT(row_plan(1ull << 28, 0xFFFFFF00ull - 10, 11, 11) == kRowsNone);
+    EXPECT(row_plan(1ull << 28, 0xFFFFFFFFull, 2, 2) == kRowsNone);
+    EXPECT(row_plan(100, 50, 10, 150) == kRowsEnds);
+    EXPECT(row_plan(100, 50, 10, 151) == kRowsShared);
+    EXPECT(row_plan(1ull << 28, 1ull << 28, 10, kRowEndsMax) == kRowsEnds);
+    EXPECT(row_plan(1ull << 28, 1ull << 28, 10, kRowEndsMax + 1) == kRowsShared);
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
         {"pool_bound", pool_bound},
         {"handle_device", handle_device},
+        {"row_plan", row_plan},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

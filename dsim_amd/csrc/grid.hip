@@ -21,6 +21,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_reduce.hpp>
 #include <rocprim/device/device_scan.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
 #include <cmath>
@@ -1106,12 +1107,13 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
     const hipStream_t st = nullptr;
     DevBuf<float> dV;
     DevBuf<uint32_t> dT, dI, cnt, offs, keys, vals, keys2, vals2, ccount, ring, flag, maxc;
+    DevBuf<unsigned long long> total;
     DevBuf<uint8_t> temp;
     auto cleanup = [&] {
         dV.release(); dT.release(); dI.release(); cnt.release(); offs.release(); keys.release();
         vals.release();
         keys2.release(); vals2.release(); ccount.release(); ring.release(); flag.release();
-        maxc.release(); temp.release();
+        maxc.release(); total.release(); temp.release();
     };
     auto bail = [&](int code) {
         cleanup();
@@ -1134,7 +1136,7 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
         (rc = S->tri_aabb.alloc(nt1 * 2)) || (rc = cnt.alloc(nt1 + 1)) || (rc = offs.alloc(nt1 + 1)) ||
         (rc = S->d_cell_start.alloc((size_t)S->n_cells + 1)) ||
         (rc = ccount.alloc((size_t)S->n_cells + 1)) || (rc = maxc.alloc(1)) ||
-        (rc = flag.alloc(1)))
+        (rc = flag.alloc(1)) || (rc = total.alloc(1)))
         return bail(rc);
     if (nV) GRID_TRY(hipMemcpy(dV.p, mesh->vertices, (size_t)nV * 12, hipMemcpyHostToDevice));
     if (nT) {
@@ -1163,8 +1165,24 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
                                      (size_t)S->n_cells + 1, rocprim::plus<uint32_t>(), st));
     GRID_TRY(rocprim::reduce(nullptr, tb_red, ccount.p, maxc.p, 0u, (size_t)S->n_cells,
                              rocprim::maximum<uint32_t>(), st));
-    const size_t tb0 = std::max({tb_scan1, tb_scan2, tb_red, (size_t)1});
+    // the pairs in 64 bits: their places and numbers are 32-bit
+    const auto wide = rocprim::make_transform_iterator(
+        cnt.p, [] __device__(uint32_t v) { return (unsigned long long)v; });
+    size_t tb_sum = 0;
+    GRID_TRY(rocprim::reduce(nullptr, tb_sum, wide, total.p, 0ull, (size_t)nT,
+                             rocprim::plus<unsigned long long>(), st));
+    const size_t tb0 = std::max({tb_scan1, tb_scan2, tb_red, tb_sum, (size_t)1});
     if ((rc = temp.alloc(tb0))) return bail(rc);
+    unsigned long long n_listed = 0;
+    if (nT) {
+        GRID_TRY(rocprim::reduce(temp.p, tb_sum, wide, total.p, 0ull, (size_t)nT,
+                                 rocprim::plus<unsigned long long>(), st));
+        GRID_TRY(hipMemcpyAsync(&n_listed, total.p, 8, hipMemcpyDeviceToHost, st));
+        GRID_TRY(hipStreamSynchronize(st));
+    }
+    if (n_listed > 0xFFFFFFFFull)
+        return bail(fail(DSIM_ERR_ARG, "grid too fine: %llu entries in its cells, more than 2^32 - 1",
+                         n_listed));
     {
         size_t b = tb_scan1;
         GRID_TRY(rocprim::exclusive_scan(temp.p, b, cnt.p, offs.p, 0u, nT + 1,

@@ -42,6 +42,7 @@ struct StepParams {
     const uint32_t *walk_start;
     const uint2 *walk_ent;
     const float4 *walk_rec;
+    uint32_t n_entries;  // of the lists that the mode searches
     uint32_t walk_cell_major;
     float walk_eps;
     // per fine cell, a lower bound of the distance to any triangle in units of
@@ -90,7 +91,7 @@ struct StepParams {
     uint64_t step0;
     const float4 *inject;  // [iters][n]
     uint32_t *trace;       // [iters][n][5]
-    uint32_t *flags;       // status word: bit 0 collision loop guard hit
+    uint32_t *flags;       // status word: bit 0 collision loop guard hit, bit 2 entry out of range
     unsigned long long *stats;  // [kWalkStats] work counters (counting build of the walk)
     uint32_t *queue;       // [8] slot counters of the persistent walk, or null (fixed blocks)
     uint32_t queue_run;    // slots per queue run (persistent walk; set at launch)

@@ -613,6 +613,21 @@ __device__ __forceinline__ void queue_push(WaveScratch &L, bool c, uint2 tri, ui
     qlen += popc(b2);
 }
 
+// Entry k of the lists; one past their end, which a right numbering never
+// gives, is flagged and read as the first.  Takes 0.1 to 1.0 % of the walks'
+// time (acquisition of 1e4 spins 43.0 and 43.5 ms, of 1e6 379 and 381 ms); a
+// lane mask for the atomic, or the largest k kept to the round's end, 1.6 and
+// 1.3 % of the former.
+__device__ __forceinline__ uint32_t entry_checked(const StepParams &P, uint32_t k) {
+    if (__builtin_expect(__ballot(k >= P.n_entries) != 0ull, 0)) {  // one branch, no lane mask
+        if (k >= P.n_entries) {
+            atomicOr(P.flags, 4u);
+            k = 0;
+        }
+    }
+    return k;
+}
+
 // Test of pair j for its owner lane: whether the owner's segment may cross the
 // entry's facet, and the entry's triangles.
 template <int RECS>
@@ -625,7 +640,7 @@ __device__ __forceinline__ bool pair_crosses(const StepParams &P, const WaveScra
     uint32_t s = m.y;
     uint2 e = L.row[s];
     while (r >= e.y && s + 1 < kWaveRows) e = L.row[++s];
-    const uint32_t k = e.x + r;
+    const uint32_t k = entry_checked(P, e.x + r);
     tri = P.walk_ent[k];
     return walk_test<RECS>(P, k, tri.x, L.o[owner], L.p[owner]);
 }
@@ -1245,7 +1260,7 @@ __device__ __forceinline__ bool ref_pair(const StepParams &P, const RefScratch &
     uint32_t s = m.y;
     uint2 e = L.cell[s];
     while (r >= e.y && s + 1 < kRefCells) e = L.cell[++s];
-    const uint32_t k = e.x + r;
+    const uint32_t k = entry_checked(P, e.x + r);
     float4 a, d;
     uint32_t t;
     if (MAJOR) {

@@ -191,6 +191,10 @@ static int check_flags(dsim_sim *s, const uint32_t fl[4]) {
         HIP_TRY(hipMemsetAsync(s->flags(), 0, 16, s->stream));
         return fail(DSIM_ERR_OVERFLOW, "a spin exceeded 4096 collisions in one step");
     }
+    if (fl[0] & 4u) {
+        HIP_TRY(hipMemsetAsync(s->flags(), 0, 16, s->stream));
+        return fail(DSIM_ERR_STATE, "collision search numbered a grid entry out of range");
+    }
     return DSIM_OK;
 }
 
@@ -348,6 +352,7 @@ static dsim::StepParams step_params(dsim_sim *s) {
     P.walk_start = b->walk_start.p;
     P.walk_ent = b->walk_ent.p;
     P.walk_rec = b->walk_rec.p;
+    P.n_entries = (uint32_t)(s->prm.mode == DSIM_MODE_PHYSICAL ? b->walk_ent.n : b->d_cell_tri.n);
     P.walk_cell_major = b->kind != DSIM_GRID_TRIBOX;
     P.walk_eps = b->walk_eps;
     P.fine = s->prm.mode == DSIM_MODE_PHYSICAL ? b->d_fine.p : nullptr;

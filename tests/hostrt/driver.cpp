@@ -154,12 +154,53 @@ static void row_plan() {
     EXPECT(row_plan(1ull << 28, 1ull << 28, 10, kRowEndsMax + 1) == kRowsShared);
 }
 
+// An error flag of a step comes out of the next call that waits, once: on its
+// own, beside a signal's sums, in front of a state read in one copy (256 spins)
+// or in several (100,000), and before the caller's arrays are written.
+static void error_flags() {
+    dsim_substrate *s = make_sub();
+    for (uint32_t n : {256u, 100000u}) {
+        std::vector<float> pos(3 * n);
+        std::vector<dsim_spin_data> spins(n);
+        for (uint32_t bits : {1u, 4u}) {
+            const int code = bits == 1 ? DSIM_ERR_OVERFLOW : DSIM_ERR_STATE;
+            const char *word = bits == 1 ? "4096 collisions" : "out of range";
+            dsim_sim *h = make_sim(s, n);
+            EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK);
+            const float g[3] = {0, 0, 0};
+            for (int how = 0; how < 6; ++how) {
+                stub::flag_bits = bits;
+                EXPECT(dsim_integrate(h, g, 0.0f, 1) == DSIM_OK);
+                stub::flag_bits = 0;
+                double sig[5] = {-1, -1, -1, -1, -1};
+                pos.assign(3 * n, -7.0f);
+                memset(spins.data(), 0x5A, n * sizeof spins[0]);
+                const int rc = how == 0   ? dsim_sync(h)
+                               : how == 1 ? dsim_signal(h, sig)
+                               : how == 2 ? dsim_get_state_aos(h, pos.data(), spins.data(), nullptr)
+                               : how == 3 ? dsim_get_state_aos(h, nullptr, spins.data(), nullptr)
+                               : how == 4 ? dsim_get_state_aos(h, pos.data(), nullptr, nullptr)
+                                          : dsim_get_state_aos(h, nullptr, nullptr, nullptr);
+                EXPECT(rc == code && strstr(dsim_last_error(), word));
+                EXPECT(sig[0] == -1 && pos[0] == -7.0f && pos[3 * n - 1] == -7.0f);
+                EXPECT(spins[n - 1].insideFiber == 0x5A5A);
+                EXPECT(dsim_sync(h) == DSIM_OK && dsim_signal(h, sig) == DSIM_OK);
+                EXPECT(dsim_get_state_aos(h, pos.data(), spins.data(), nullptr) == DSIM_OK);
+                EXPECT(pos[3 * n - 1] == (float)(n - 1) + 2.0f);
+            }
+            EXPECT(dsim_sim_destroy(h) == DSIM_OK);
+        }
+    }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
         {"pool_bound", pool_bound},
         {"handle_device", handle_device},
         {"row_plan", row_plan},
+        {"error_flags", error_flags},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -14,7 +14,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 
-CASES = ["pool_device", "pool_bound", "handle_device", "row_plan"]
+CASES = ["pool_device", "pool_bound", "handle_device", "row_plan", "error_flags"]
 
 
 @pytest.fixture(scope="module")

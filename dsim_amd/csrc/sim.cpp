@@ -698,25 +698,24 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
         }
     const dsim_host::RowLists &lists = own.start.p ? own : sub->rows;
     rows = rows && lists.start.p;  // no lists: more entries than places
-    constexpr size_t counters = dsim::kLabelGroups + 2;  // even: the uint2 queue follows
-    const size_t words = counters + (rows ? 3 * (size_t)s->n : 0);
-    // counters (groups, ambiguous, queued), then per spin the retry queue's
-    // entry and the place in the row order
-    PoolBuf<uint32_t> work;
-    if (int rc = work.alloc(words)) {
-        own.release();
-        return rc;
-    }
-    uint32_t *w = work.p;
+    // The counters (groups, ambiguous, queued) stand in the readout's partial
+    // sums, and per spin the retry queue's entry and the place in the row order
+    // in the moments, which labelling ends: no memory is taken for them.
+    constexpr size_t counters = dsim::kLabelGroups + 2;
+    static_assert(counters * 4 <= (size_t)dsim::kSignalBlocks * 15 * 8, "room for the counters");
+    static_assert(F_MOMC + 3 - F_DISP >= 4, "three words a spin and one to align them");
+    uint32_t *w = reinterpret_cast<uint32_t *>(s->partial.p);
     L.group = w;
     L.n_ambiguous = w + counters - 2;
     L.n_retry = w + counters - 1;
     hipError_t e = hipMemsetAsync(w, 0, counters * 4, s->stream);
     if (rows) {
-        L.retry = reinterpret_cast<uint2 *>(w + counters);
+        s->moment_ready = false;
+        uint32_t *per_spin = s->state.p + (((size_t)F_DISP * s->n + 1) & ~(size_t)1);
+        L.retry = reinterpret_cast<uint2 *>(per_spin);
         const uint64_t row_bytes = (uint64_t)lists.tri.n * 20 + (uint64_t)sub->n_tri * 96;
         L.order = s->n >= dsim::kLabelOrderMin && row_bytes > dsim::kXcdL2Bytes
-                      ? w + counters + 2 * (size_t)s->n : nullptr;
+                      ? per_spin + 2 * (size_t)s->n : nullptr;
         L.row_start = lists.start.p;
         L.row_tri = lists.tri.p;
         L.row_box = lists.box.p;
@@ -737,7 +736,6 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     if (e == hipSuccess && n_ambiguous)
         e = hipMemcpyAsync(&ambiguous, L.n_ambiguous, 4, hipMemcpyDeviceToHost, s->stream);
     const hipError_t es = hipStreamSynchronize(s->stream);
-    work.release();
     own.release();
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "label: %s", hipGetErrorString(e));
@@ -822,7 +820,7 @@ hipStream_t dsim_host::sim_stream(const dsim_sim *s) { return s->stream; }
 
 uint64_t dsim_host::sim_footprint(uint32_t n, const dsim_params *p, uint32_t n_lines) {
     const uint64_t m = std::max<uint32_t>(n, 1);
-    uint64_t b = m * F_COUNT * 4 + m * 4 + 16 + (uint64_t)dsim::kSignalBlocks * 15 * 8 + 15 * 8;
+    uint64_t b = m * F_COUNT * 4 + 8 * 4 + (uint64_t)dsim::kSignalBlocks * 15 * 8 + 17 * 8;
     if (p->rng == DSIM_RNG_MWC) b += m * 8;
     if (p->sort_interval > 0 && p->mode == DSIM_MODE_PHYSICAL && p->rng == DSIM_RNG_PHILOX)
         b += m * F_COUNT * 4 + m * 16 + m * 8;  // second block, keys, values, sort scratch (about)

@@ -194,6 +194,40 @@ static void error_flags() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// Labelling takes no device memory of its own: it works on a full device, with
+// spin counts that leave its per-spin words unaligned, and leaves the fields it
+// does not end as they were.
+static void label_on_a_full_device() {
+    stub::keep_rows = true;
+    dsim_substrate *s = make_sub();
+    stub::keep_rows = false;
+    for (uint32_t n : {1u, 2u, 7u, 1000u, 40001u}) {
+        dsim_sim *h = make_sim(s, n);
+        EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK && dsim_moment_reset(h) == DSIM_OK);
+        const float *mag, *x0;
+        const uint32_t *label, *id;
+        dsim_host::sim_readout_fields(h, &mag, &label, &x0, &id);
+        const size_t was = stub::capacity[0];
+        const uint32_t rows = stub::n_label_rows;
+        stub::capacity[0] = stub::used[0];
+        uint32_t amb = 77;
+        EXPECT(dsim_label_spins(h, 1, 1, 1, 3, &amb) == DSIM_OK && amb == 0);
+        stub::capacity[0] = was;
+        EXPECT(stub::n_label_rows == rows + 1);
+        bool same = true;
+        for (uint32_t i = 0; i < n; ++i)
+            same &= mag[i] == 1.0f && label[i] == 7u << 8 && id[i] == i && x0[2 * n + i] == 0.25f;
+        EXPECT(same);
+        double sig[5];
+        EXPECT(dsim_integrate_moment(h, 1.0f, 1) == DSIM_ERR_STATE);  // the moments have ended
+        const float g[3] = {1, 0, 0};
+        EXPECT(dsim_signal_moment(h, 1, g, 1.0f, sig) == DSIM_ERR_STATE);
+        EXPECT(dsim_moment_reset(h) == DSIM_OK && dsim_integrate_moment(h, 1.0f, 1) == DSIM_OK);
+        EXPECT(dsim_sim_destroy(h) == DSIM_OK);
+    }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -201,6 +235,7 @@ int main(int argc, char **argv) {
         {"handle_device", handle_device},
         {"row_plan", row_plan},
         {"error_flags", error_flags},
+        {"label_on_a_full_device", label_on_a_full_device},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -21,6 +21,7 @@ size_t total[kDevices] = {1ull << 30, 1ull << 28}, capacity[kDevices] = {1ull <<
 uint64_t n_malloc, n_free;
 uint32_t flag_bits, n_label_rows, n_label_all, n_row_builds;
 uint64_t row_bytes;
+bool keep_rows;
 thread_local int device;
 thread_local hipError_t last = hipSuccess;
 hipError_t err(hipError_t e) {
@@ -227,7 +228,12 @@ hipError_t launch_walk_batch(const WalkTable *, uint32_t, bool, int, hipStream_t
 }  // namespace dsim
 
 namespace dsim_host {
-int build_walk_tables(dsim_substrate *, hipStream_t) { return DSIM_OK; }
+int build_walk_tables(dsim_substrate *S, hipStream_t) {
+    if (!stub::keep_rows) return DSIM_OK;
+    if (int rc = S->rows.start.alloc(16)) return rc;
+    if (int rc = S->rows.tri.alloc(4)) return rc;
+    return S->rows.box.alloc(4);
+}
 int build_row_lists(const dsim_substrate *, RowLists &R, uint64_t, hipStream_t) {
     ++stub::n_row_builds;
     if (int rc = R.start.alloc(16)) return rc;

@@ -21,4 +21,5 @@ extern uint64_t n_malloc, n_free;
 extern uint32_t flag_bits;         // error flags the next step launches raise
 extern uint32_t n_label_rows, n_label_all, n_row_builds;
 extern uint64_t row_bytes;         // of the row lists a call builds
+extern bool keep_rows;             // new substrates hold row lists
 }  // namespace stub

@@ -14,7 +14,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 
-CASES = ["pool_device", "pool_bound", "handle_device", "row_plan", "error_flags"]
+CASES = ["pool_device", "pool_bound", "handle_device", "row_plan", "error_flags",
+         "label_on_a_full_device"]
 
 
 @pytest.fixture(scope="module")

@@ -874,7 +874,8 @@ static int build_fine_clearance(dsim_substrate *S, hipStream_t st) {
     }
     f.half_diag = std::sqrt(h2) * 1.00001f;
     f.q = S->fine_q = smallest / kFineRange;
-    if (int rc = S->d_fine.alloc(n)) return rc;
+    if (int rc = S->d_fine.alloc(n))  // no table: every step searches
+        return rc == DSIM_ERR_NOMEM ? DSIM_OK : rc;
     hipLaunchKernelGGL(k_fine_clearance, dim3(blocks_for(n)), dim3(kBlock), 0, st, g, f,
                        S->d_cell_start.p, S->d_cell_tri.p, S->tri_mt.p, S->d_clearance.p,
                        S->d_fine.p);
@@ -976,9 +977,23 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     g.face = S->lo[g.A] + (float)S->dims[g.A] * S->cell[g.A];
     for (int k = 0; k < 3; ++k) { g.dims[k] = S->dims[k]; g.lo[k] = S->lo[k]; g.cell[k] = S->cell[k]; }
     const uint32_t n_rows = g.dims[g.B] * g.dims[g.C], n_blocks = std::min(nT, 1024u);
-    TempBuf<uint8_t> temp;
-    TempBuf<uint32_t> outside;  // and after it the rows' counts of their entries
-    TempBuf<unsigned long long> sum;
+    // Scratch of the pool, not of the runtime, whose hipFree waits for the whole
+    // device: a server makes lists while its requests step.  The pool does not
+    // wait, so an early return waits for the stream here.
+    struct Scratch {
+        hipStream_t st;
+        dsim_host::PoolBuf<uint8_t> temp;
+        dsim_host::PoolBuf<uint32_t> outside;  // and after it the rows' counts of their entries
+        dsim_host::PoolBuf<unsigned long long> sum;
+        bool waited = false;
+        ~Scratch() {
+            if (!waited) (void)hipStreamSynchronize(st);
+            temp.release(); outside.release(); sum.release();
+        }
+    } scratch{st, {}, {}, {}};
+    auto &temp = scratch.temp;
+    auto &outside = scratch.outside;
+    auto &sum = scratch.sum;
     int rc;
     size_t tb = 0;
     HIP_TRY(rocprim::exclusive_scan(nullptr, tb, R.start.p, R.start.p, 0u,
@@ -1037,12 +1052,16 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
                            outside.p, S->tri_aabb.p, R.tri.p + n, R.box.p + n);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
+    scratch.waited = true;
     return DSIM_OK;
 }
 
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
     if (S->kind != DSIM_GRID_REFERENCE)
-        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, st)) return rc;
+        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, st)) {
+            if (rc != DSIM_ERR_NOMEM) return rc;
+            S->rows.release();  // labelled without, or with those that a call can make
+        }
     if (S->kind == DSIM_GRID_REFERENCE)
         if (int rc = build_ref_tables(S, st)) return rc;
     if (int rc = build_search_lists(S, st)) return rc;

@@ -388,9 +388,10 @@ bool pool_trim() {
 void *dsim_host::dev_alloc(size_t bytes, hipError_t *e) {
     void *p = nullptr;
     *e = hipMalloc(&p, bytes);
+    if (*e != hipSuccess) (void)hipGetLastError();  // not the next launch's error
     if (*e != hipSuccess && pool_trim()) {
-        (void)hipGetLastError();
         *e = hipMalloc(&p, bytes);
+        if (*e != hipSuccess) (void)hipGetLastError();
     }
     return *e == hipSuccess ? p : nullptr;
 }

@@ -117,7 +117,8 @@ int build_walk_tables(dsim_substrate *S, hipStream_t st);
 // Row lists of the labeller (LabelParams::row_start).  A substrate keeps its own
 // up to kRowKeepBytes; of a larger grid they would be a third of its memory for
 // a call made once a spin set, so every labelling makes them and gives them
-// back (build_row_lists: 0.25 ms for 2.4e6 cells).
+// back (build_row_lists: 0.25 ms for 2.4e6 cells), or goes without where there
+// is no memory for them.
 constexpr uint64_t kRowKeepBytes = 128ull << 20;
 struct RowLists {
     PoolBuf<uint32_t> start, tri;

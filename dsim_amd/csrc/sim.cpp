@@ -694,10 +694,10 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
         if (int rc = dsim_host::build_row_lists(sub, own, ~0ull, s->stream)) {
             (void)hipStreamSynchronize(s->stream);
             own.release();
-            return rc;
+            if (rc != DSIM_ERR_NOMEM) return rc;
         }
     const dsim_host::RowLists &lists = own.start.p ? own : sub->rows;
-    rows = rows && lists.start.p;  // no lists: more entries than places
+    rows = rows && lists.start.p;  // no lists: no memory, or more entries than places
     // The counters (groups, ambiguous, queued) stand in the readout's partial
     // sums, and per spin the retry queue's entry and the place in the row order
     // in the moments, which labelling ends: no memory is taken for them.

@@ -228,6 +228,27 @@ static void label_on_a_full_device() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// A labelling that finds no memory for the row lists of a large grid goes
+// through the pass over all triangles, which needs none; no error stays behind.
+static void label_without_lists() {
+    dsim_substrate *s = make_sub();
+    dsim_sim *h = make_sim(s, 1000);
+    EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK);
+    stub::row_bytes = 1 << 20;
+    const size_t was = stub::capacity[0];
+    const uint32_t rows = stub::n_label_rows, all = stub::n_label_all;
+    for (size_t room : {(size_t)0, (size_t)100, (size_t)1 << 19}) {  // none, and for a part of them
+        stub::capacity[0] = stub::used[0] + room;
+        EXPECT(dsim_label_spins(h, 1, 1, 1, 3, nullptr) == DSIM_OK);
+    }
+    stub::capacity[0] = was;
+    EXPECT(stub::n_label_rows == rows && stub::n_label_all == all + 3);
+    EXPECT(dsim_label_spins(h, 1, 1, 1, 3, nullptr) == DSIM_OK);
+    EXPECT(stub::n_label_rows == rows + 1 && stub::n_label_all == all + 3);
+    EXPECT(dsim_sim_destroy(h) == DSIM_OK);
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -236,6 +257,7 @@ int main(int argc, char **argv) {
         {"row_plan", row_plan},
         {"error_flags", error_flags},
         {"label_on_a_full_device", label_on_a_full_device},
+        {"label_without_lists", label_without_lists},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -967,7 +967,7 @@ static int build_ref_tables(dsim_substrate *S, hipStream_t st) {
 }
 
 int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t most,
-                               hipStream_t st) {
+                               uint64_t room, hipStream_t st) {
     const uint32_t nT = S->n_tri, nC = S->n_cells;
     RowGeom g{};
     g.A = (int)S->label_axis;
@@ -998,6 +998,8 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     size_t tb = 0;
     HIP_TRY(rocprim::exclusive_scan(nullptr, tb, R.start.p, R.start.p, 0u,
                                     (size_t)nC + 1, rocprim::plus<uint32_t>(), st));
+    const uint64_t making = tb + ((uint64_t)nT + 1 + n_rows) * 4 + 64 + ((uint64_t)nC + 1) * 4;
+    if (!pool_room(making, room)) return DSIM_OK;
     if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = R.start.alloc((size_t)nC + 1)) ||
         (rc = outside.alloc((size_t)nT + 1 + n_rows)) || (rc = sum.alloc(1)))
         return rc;
@@ -1036,7 +1038,8 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     R.n_shared = plan == kRowsShared ? n_out : 0u;
     // a lane past its row's end reads entry 0
     const size_t n1 = std::max<size_t>((size_t)n + R.n_shared, 1);
-    if (((uint64_t)nC + 1) * 4 + (uint64_t)n1 * 20 > most) {
+    if (((uint64_t)nC + 1) * 4 + (uint64_t)n1 * 20 > most ||
+        !pool_room(making + (uint64_t)n1 * 20, room)) {
         R.start.release();
         return DSIM_OK;
     }
@@ -1058,7 +1061,7 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
 
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
     if (S->kind != DSIM_GRID_REFERENCE)
-        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, st)) {
+        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, ~0ull, st)) {
             if (rc != DSIM_ERR_NOMEM) return rc;
             S->rows.release();  // labelled without, or with those that a call can make
         }

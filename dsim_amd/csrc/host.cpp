@@ -442,6 +442,28 @@ void dsim_host::pool_give(void *p, size_t bytes, int device) {
     for (const PoolBlock &b : out) (void)hipFree(b.p);
 }
 
+void dsim_host::pool_trim_to(int device, uint64_t most) {
+    std::vector<PoolBlock> out;
+    {
+        std::lock_guard<std::mutex> l(pool_mu);
+        uint64_t held = 0;
+        for (const PoolBlock &b : pool) held += b.device == device ? b.bytes : 0;
+        while (held > most) {
+            out.push_back(pool_oldest(device));
+            held -= out.back().bytes;
+        }
+    }
+    for (const PoolBlock &b : out) (void)hipFree(b.p);
+}
+
+bool dsim_host::pool_room(uint64_t need, uint64_t room) {
+    if (room == ~0ull) return true;
+    int device = 0;
+    if (need > room || hipGetDevice(&device) != hipSuccess) return false;
+    pool_trim_to(device, room - need);
+    return true;
+}
+
 void dsim_host::pool_ref() {
     std::lock_guard<std::mutex> l(pool_mu);
     ++pool_users;

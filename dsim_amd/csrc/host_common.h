@@ -63,6 +63,12 @@ void *dev_alloc(size_t bytes, hipError_t *e);
 constexpr size_t kPoolShare = 16, kPoolBlocks = 256;
 void *pool_take(size_t bytes, size_t *got, int *device, hipError_t *e);
 void pool_give(void *p, size_t bytes, int device);
+// Idle blocks of the device given back, oldest first, until `most` bytes of them
+// are left.
+void pool_trim_to(int device, uint64_t most);
+// May `need` more bytes be taken out of `room` (~0 no limit), which idle blocks
+// of the current device share?  Gives back those that do not fit beside them.
+bool pool_room(uint64_t need, uint64_t room);
 void pool_ref();
 void pool_unref();
 
@@ -85,6 +91,8 @@ struct DevBuf {
         }
         return DSIM_OK;
     }
+    // Bytes of the block past the buffer's own.
+    uint64_t slack() const { return p && POOL ? block - n * sizeof(T) : 0; }
     void release() {
         if (p && POOL) pool_give(p, block, device);
         else if (p) (void)hipFree(p);
@@ -142,8 +150,11 @@ inline RowPlan row_plan(uint64_t n_cells, uint64_t n_entries, uint64_t n_outside
         return kRowsShared;
     return kRowsEnds;
 }
-// Lists of more than `most` bytes, or none by row_plan, are left empty.  Waits for st.
-int build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t most, hipStream_t st);
+// Lists of more than `most` bytes, or for which `room` is too small with the
+// scratch of their making (pool_room), or none by row_plan, are left empty.
+// Waits for st.
+int build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t most, uint64_t room,
+                    hipStream_t st);
 }  // namespace dsim_host
 
 #define HIP_TRY(expr)                                                                        \

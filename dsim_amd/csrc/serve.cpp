@@ -44,7 +44,8 @@ struct Req {
     dsim_substrate *sub = nullptr;
     std::vector<float> lobe_w, grads;
     std::vector<uint32_t> lobe_n;
-    uint64_t bytes = 0;
+    uint64_t bytes = 0;  // charged: the footprint, and what its blocks have above it
+    uint64_t slack = 0;
     dsim_sim *sim = nullptr;
     uint32_t lobe = 0, lobe_left = 0;
     uint32_t chunk = 0;  // steps of the current round
@@ -87,6 +88,7 @@ struct dsim_server {
     bool running = false, stopping = false;
     int loop_err = DSIM_OK;
     hipStream_t stream = nullptr;
+    int device = 0;
     Batch batch[4];  // [boundary * 2 + (grid entries read through cell_tri)]
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
@@ -112,8 +114,28 @@ void finish(dsim_server *S, Req *r, int status, int err, const std::string &msg)
     S->cv_done.notify_all();
 }
 
+// What is left of the budget beside the admitted requests.
+uint64_t budget_rest(dsim_server *S) {
+    std::lock_guard<std::mutex> l(S->mu);
+    return S->budget > S->used ? S->budget - S->used : 0;
+}
+
+// Charges what the pool gave the request's handle above its footprint.
+void charge_slack(dsim_server *S, Req *r) {
+    if (!r->sim) return;
+    const uint64_t b = dsim_host::sim_slack(r->sim);
+    std::lock_guard<std::mutex> l(S->mu);
+    S->used += b - r->slack;
+    r->bytes += b - r->slack;
+    r->slack = b;
+}
+
 // Creates the request's handle and prepares its spins (on its own stream).
+// The budget holds for all device memory of the library's handles: blocks that
+// wait in the pool for the next one count against what the admitted requests
+// leave, and so do row lists that the labelling makes for itself.
 int start_request(dsim_server *S, Req *r) {
+    dsim_host::pool_trim_to(S->device, budget_rest(S));
     dsim_params p{};
     p.dt = r->r.dt;
     for (int c = 0; c < 4; ++c) { p.std_dev[c] = r->r.std_dev[c]; p.t2[c] = r->r.t2[c]; }
@@ -134,6 +156,8 @@ int start_request(dsim_server *S, Req *r) {
     }
     int rc;
     if ((rc = dsim_sim_create(r->sub, &p, r->r.n_spins, &r->sim))) return rc;
+    charge_slack(S, r);
+    dsim_host::sim_list_room(r->sim, budget_rest(S));
     uint32_t amb = 0;
     if ((rc = voxel ? dsim_init_spins_box(r->sim, p.voxel_lo, p.voxel_hi)
                     : dsim_init_spins_uniform(r->sim, r->r.start_box)) ||
@@ -261,6 +285,7 @@ int run_round(dsim_server *S, uint32_t *n_active, uint32_t *n_queued) {
         int rc = r->r.n_lines ? dsim_signal_moment(r->sim, r->r.n_lines, r->grads.data(),
                                                    r->r.phase_constant, r->signals.data())
                               : dsim_sync(r->sim);
+        charge_slack(S, r);
         if (rc) finish(S, r, kFailed, rc, dsim_last_error());
         else finish(S, r, kDone, DSIM_OK, "");
     }
@@ -356,6 +381,7 @@ extern "C" int dsim_server_create(uint64_t hbm_budget, uint32_t round_steps,
     S->round_steps = round_steps ? round_steps : 256;
     S->max_spins = max_active_spins ? max_active_spins : (64u << 20);
     S->grid_blocks = walk_blocks(S->max_spins) + dsim::kMaxJobs;
+    (void)hipGetDevice(&S->device);
     hipError_t e = hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         delete S;

@@ -64,6 +64,7 @@ struct dsim_sim {
     uint64_t steps_since_sort = ~0ull;
     bool permuted = false;
     bool moment_ready = false;
+    uint64_t list_room = ~0ull;  // for the row lists that a labelling makes
     float wsum = 0.0f;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     double ms_done = 0.0;
@@ -691,7 +692,7 @@ extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
     bool rows = L.ray_axis && sub->kind != DSIM_GRID_REFERENCE && sub->n_cells > 0 && s->n > 0;
     dsim_host::RowLists own;  // of this call, where the substrate keeps none
     if (rows && !sub->rows.start.p)
-        if (int rc = dsim_host::build_row_lists(sub, own, ~0ull, s->stream)) {
+        if (int rc = dsim_host::build_row_lists(sub, own, ~0ull, s->list_room, s->stream)) {
             (void)hipStreamSynchronize(s->stream);
             own.release();
             if (rc != DSIM_ERR_NOMEM) return rc;
@@ -827,6 +828,17 @@ uint64_t dsim_host::sim_footprint(uint32_t n, const dsim_params *p, uint32_t n_l
     b += (uint64_t)n_lines * (12 + 256 * 15 * 8 + 15 * 8);  // readout
     return b;
 }
+
+uint64_t dsim_host::sim_slack(const dsim_sim *s) {
+    uint64_t b = s->partial.slack() + s->out.slack() + s->grads.slack() + s->inject.slack() +
+                 s->sort_tmp.slack() + s->stats.slack();
+    for (auto *u : {&s->state, &s->alt, &s->seed, &s->trace, &s->queue, &s->keys_a, &s->keys_b,
+                    &s->vals_a, &s->vals_b})
+        b += u->slack();
+    return b;
+}
+
+void dsim_host::sim_list_room(dsim_sim *s, uint64_t bytes) { s->list_room = bytes; }
 
 int dsim_host::sim_walk_traj(dsim_sim *s, uint32_t iters, float *traj) {
     if (int rc = check_sim(s)) return rc;

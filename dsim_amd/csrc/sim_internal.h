@@ -32,5 +32,10 @@ void sim_readout_fields(dsim_sim *s, const float **mag, const uint32_t **label, 
 uint32_t sim_spins(const dsim_sim *s);
 // Device bytes a handle of n spins holds, readout of n_lines lines included.
 uint64_t sim_footprint(uint32_t n, const dsim_params *p, uint32_t n_lines);
+// Bytes of the handle's blocks past what it asked for.
+uint64_t sim_slack(const dsim_sim *s);
+// Bytes that the handle's labelling may take for row lists of its own (without
+// them it goes through the pass over all triangles); no limit at creation.
+void sim_list_room(dsim_sim *s, uint64_t bytes);
 
 }  // namespace dsim_host

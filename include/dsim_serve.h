@@ -58,8 +58,11 @@ typedef struct {
     uint32_t ambiguous;               /* spins whose label stayed ambiguous */
 } dsim_request_stats;
 
-/* hbm_budget: device bytes the admitted requests may hold (the substrates are
- * not counted); round_steps: steps per request per round (0 = 256);
+/* hbm_budget: device bytes the admitted requests may hold, with the blocks that
+ * finished handles left for the next ones and the row lists that labelling on a
+ * large substrate makes for itself (where the budget has no room for those, the
+ * request is labelled without, slower); the substrates are not counted;
+ * round_steps: steps per request per round (0 = 256);
  * max_active_spins: spins in flight at most (0 = 64M). */
 int dsim_server_create(uint64_t hbm_budget, uint32_t round_steps, uint32_t max_active_spins,
                        dsim_server **out);

@@ -249,6 +249,78 @@ static void label_without_lists() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// A server's budget holds for all that its requests' handles take: their own
+// blocks, those that wait for the next handle, and row lists that a labelling
+// makes; lists that the budget has no room for are gone without.
+static void server_budget() {
+    dsim_substrate *s = make_sub();
+    const float lobe[1] = {1.0f}, g[60] = {1};
+    const uint32_t steps[1] = {300};
+    // the last: handles of 6100 spins in blocks that were of 8000, beside one of 8000
+    for (uint64_t rows : {0ull, 200'000ull, 5'000'000ull, 1ull}) {
+        stub::row_bytes = rows;
+        const bool tight = rows == 1;
+        dsim_params p = params();
+        const uint64_t one = dsim_host::sim_footprint(8000, &p, 20);
+        const uint64_t budget = tight ? one + dsim_host::sim_footprint(6100, &p, 20) + 1000
+                                      : 2 * one + one / 2;
+        dsim_server *S = nullptr;
+        EXPECT(dsim_server_create(budget, 0, 0, &S) == DSIM_OK);
+        uint32_t id = 0;
+        EXPECT(dsim_server_add_substrate(S, s, &id) == DSIM_OK);
+        std::vector<uint64_t> tickets;
+        auto submit = [&](uint32_t n) {
+            dsim_request q{};
+            q.substrate = id;
+            q.n_spins = n;
+            q.dt = 0.005f;
+            for (int c = 0; c < 4; ++c) { q.std_dev[c] = 0.01f; q.t2[c] = INFINITY; }
+            q.boundary = DSIM_BOUNDARY_PERIODIC;
+            q.start_box = 1.0f;
+            for (int k = 0; k < 3; ++k) q.label_extent[k] = 1.0f;
+            q.n_lobes = 1;
+            q.lobe_weight = lobe;
+            q.lobe_steps = steps;
+            q.n_lines = 20;
+            q.grads = g;
+            tickets.emplace_back();
+            EXPECT(dsim_server_submit(S, &q, &tickets.back()) == DSIM_OK);
+        };
+        submit(100);  // brings the job table, which is not a request's
+        uint32_t active = 1, queued = 1;
+        while (active || queued) EXPECT(dsim_server_round(S, &active, &queued) == DSIM_OK);
+        dsim_host::pool_trim_to(0, 0);
+        const size_t base = stub::used[0];
+        stub::peak[0] = base;
+        // falling and rising sizes: handles in blocks that were larger ones'
+        const uint32_t builds = stub::n_row_builds, all = stub::n_label_all;
+        for (uint32_t k = 0, u = 1; k < 200; ++k) {
+            u = u * 1664525u + 1013904223u;
+            submit(tight ? (k % 3 == 1 ? 6100 : 8000) : 1000 + (u >> 8) % 7001);
+            if (tight && k % 3 == 0)
+                for (active = 1; active;) EXPECT(dsim_server_round(S, &active, &queued) == DSIM_OK);
+            if (tight && k % 3 == 1) EXPECT(dsim_server_round(S, &active, &queued) == DSIM_OK);
+        }
+        active = queued = 1;
+        size_t rounds = 0;
+        while (active || queued) {
+            EXPECT(dsim_server_round(S, &active, &queued) == DSIM_OK);
+            if (++rounds > 1000) break;
+        }
+        EXPECT(rounds <= 1000);
+        EXPECT(stub::peak[0] - base <= budget);
+        if (stub::peak[0] - base > budget)
+            fprintf(stderr, "lists %llu: %zu of %llu\n", (unsigned long long)rows,
+                    stub::peak[0] - base, (unsigned long long)budget);
+        for (uint64_t t : tickets) EXPECT(dsim_server_wait(S, t, 0) == DSIM_OK);
+        if (rows > budget) EXPECT(stub::n_row_builds == builds && stub::n_label_all == all + 200);
+        else if (!tight) EXPECT(stub::n_row_builds > builds);
+        EXPECT(dsim_server_destroy(S) == DSIM_OK);
+    }
+    stub::row_bytes = 0;
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -258,6 +330,7 @@ int main(int argc, char **argv) {
         {"error_flags", error_flags},
         {"label_on_a_full_device", label_on_a_full_device},
         {"label_without_lists", label_without_lists},
+        {"server_budget", server_budget},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

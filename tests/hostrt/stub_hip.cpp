@@ -234,7 +234,8 @@ int build_walk_tables(dsim_substrate *S, hipStream_t) {
     if (int rc = S->rows.tri.alloc(4)) return rc;
     return S->rows.box.alloc(4);
 }
-int build_row_lists(const dsim_substrate *, RowLists &R, uint64_t, hipStream_t) {
+int build_row_lists(const dsim_substrate *, RowLists &R, uint64_t, uint64_t room, hipStream_t) {
+    if (!pool_room(stub::row_bytes + 96, room)) return DSIM_OK;
     ++stub::n_row_builds;
     if (int rc = R.start.alloc(16)) return rc;
     if (int rc = R.tri.alloc(4)) return rc;

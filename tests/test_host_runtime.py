@@ -15,7 +15,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 
 CASES = ["pool_device", "pool_bound", "handle_device", "row_plan", "error_flags",
-         "label_on_a_full_device", "label_without_lists"]
+         "label_on_a_full_device", "label_without_lists",
+         "server_budget"]
 
 
 @pytest.fixture(scope="module")

@@ -278,19 +278,45 @@ extern "C" int dsim_set_state_aos(dsim_sim *s, const float *pos, const dsim_spin
     return DSIM_OK;
 }
 
+// Positions and spin data field by field, which takes no device memory.
+static int get_state_fields(dsim_sim *s, float *pos, dsim_spin_data *spins) {
+    if (int rc = sync_and_check(s)) return rc;
+    const uint32_t n = s->n;
+    std::vector<uint32_t> id, v(n);
+    if (int rc = spin_ids(s, id)) return rc;
+    for (int k = 0; pos && k < 3; ++k) {
+        if (int rc = download_field(s, F_X + k, id, v.data())) return rc;
+        for (uint32_t i = 0; i < n; ++i) memcpy(&pos[3 * (size_t)i + k], &v[i], 4);
+    }
+    if (!spins) return DSIM_OK;
+    memset(spins, 0, n * sizeof(dsim_spin_data));
+    if (int rc = download_field(s, F_MAG, id, v.data())) return rc;
+    for (uint32_t i = 0; i < n; ++i) memcpy(&spins[i].signalMagnitude, &v[i], 4);
+    if (int rc = download_field(s, F_PHASE, id, v.data())) return rc;
+    for (uint32_t i = 0; i < n; ++i) memcpy(&spins[i].signalPhase, &v[i], 4);
+    if (int rc = download_field(s, F_LABEL, id, v.data())) return rc;
+    for (uint32_t i = 0; i < n; ++i) {
+        spins[i].compartmentType = (uint8_t)(v[i] & 0xFFu);
+        spins[i].insideFiber = (uint16_t)(v[i] >> 8);
+    }
+    return DSIM_OK;
+}
+
 extern "C" int dsim_get_state_aos(dsim_sim *s, float *pos, dsim_spin_data *spins,
                                   uint32_t *seeds) {
     if (int rc = check_sim(s)) return rc;
     const uint32_t n = s->n;
+    PoolBuf<uint32_t> pack;
     if (n == 0 || (!pos && !spins)) {
         if (int rc = sync_and_check(s)) return rc;
+    } else if (int nomem = pack.alloc(4 + (size_t)n * ((pos ? 3 : 0) + (spins ? 3 : 0)))) {
+        if (nomem != DSIM_ERR_NOMEM) return nomem;
+        if (int rc = get_state_fields(s, pos, spins)) return rc;
     } else {
         // error flags, positions and spin data in spin order, made on the device
         static_assert(sizeof(dsim_spin_data) == 12, "three words a spin");
         const size_t part = (size_t)n * 3;  // words
-        const size_t words = 4 + (pos ? part : 0) + (spins ? part : 0);
-        PoolBuf<uint32_t> pack;
-        if (int rc = pack.alloc(words)) return rc;
+        const size_t words = pack.n;
         uint32_t *d_pos = pos ? pack.p + 4 : nullptr;
         uint32_t *d_spins = spins ? pack.p + 4 + (pos ? part : 0) : nullptr;
         hipError_t e = dsim::launch_pack_state(n, s->f(F_X), s->f(F_Y), s->f(F_Z), s->f(F_MAG),

@@ -321,6 +321,42 @@ static void server_budget() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// State read-back on a full device: the same words, in spin order too.
+static void state_on_a_full_device() {
+    dsim_substrate *s = make_sub();
+    for (uint32_t n : {1u, 1000u, 100001u})
+        for (uint32_t sort : {0u, 1u}) {
+            dsim_sim *h = make_sim(s, n, sort);
+            std::vector<float> pos(3 * n), p2(3 * n, -1.0f);
+            std::vector<dsim_spin_data> spins(n), s2(n);
+            for (uint32_t i = 0; i < n; ++i) {
+                memset(&spins[i], 0, sizeof spins[i]);
+                memset(&s2[i], 0x5A, sizeof s2[i]);
+                for (int k = 0; k < 3; ++k) pos[3 * i + k] = (float)(i + k);
+                spins[i].signalMagnitude = (float)i + 0.5f;
+                spins[i].signalPhase = -(float)i;
+                spins[i].compartmentType = i % 4;
+                spins[i].insideFiber = (uint16_t)(i * 7);
+            }
+            EXPECT(dsim_set_state_aos(h, pos.data(), spins.data(), nullptr) == DSIM_OK);
+            const float g[3] = {0, 0, 0};
+            EXPECT(dsim_integrate(h, g, 0.0f, 3) == DSIM_OK);  // sorted: three reorders
+            const size_t was = stub::capacity[0];
+            stub::capacity[0] = stub::used[0];
+            EXPECT(dsim_get_state_aos(h, p2.data(), s2.data(), nullptr) == DSIM_OK);
+            EXPECT(pos == p2 && !memcmp(spins.data(), s2.data(), n * sizeof spins[0]));
+            p2.assign(3 * n, -1.0f);
+            EXPECT(dsim_get_state_aos(h, p2.data(), nullptr, nullptr) == DSIM_OK && pos == p2);
+            EXPECT(dsim_sync(h) == DSIM_OK);
+            stub::capacity[0] = was;
+            memset(s2.data(), 0x5A, n * sizeof s2[0]);
+            EXPECT(dsim_get_state_aos(h, nullptr, s2.data(), nullptr) == DSIM_OK);
+            EXPECT(!memcmp(spins.data(), s2.data(), n * sizeof spins[0]));
+            EXPECT(dsim_sim_destroy(h) == DSIM_OK);
+        }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -331,6 +367,7 @@ int main(int argc, char **argv) {
         {"label_on_a_full_device", label_on_a_full_device},
         {"label_without_lists", label_without_lists},
         {"server_budget", server_budget},
+        {"state_on_a_full_device", state_on_a_full_device},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

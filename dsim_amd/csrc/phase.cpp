@@ -4,6 +4,7 @@
 // readout (k_phase_partial).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include <hip/hip_runtime_api.h>
@@ -45,13 +46,38 @@ namespace {
 
 constexpr uint32_t kPhaseBlocks = 512;  // spin blocks of the readout
 
-constexpr uint64_t kStagingBytes = 64ull << 20;  // of get_phase's row blocks, at most
+// Of get_phase's row blocks, at most (two rows, if those are more).
+constexpr uint64_t kStagingBytes = 64ull << 20;
 
 // The pairs before any product, for a readout: zero.
 int clear_pairs(dsim_waveforms *W, hipStream_t st) {
     if (!W->empty) return DSIM_OK;
     HIP_TRY(hipMemsetAsync(W->phase.p, 0, W->phase.n * 4, st));
     W->empty = false;
+    return DSIM_OK;
+}
+
+// The pairs copied at their stride, without device memory.  The stream is idle.
+int get_phase_strided(dsim_waveforms *W, float *phase, float *comp) {
+    HIP_TRY(hipStreamSynchronize(dsim_host::sim_stream(W->sim)));
+    const size_t row = (size_t)W->n_wave * 4, pad = (size_t)W->n_wpad * 4;
+    if (phase)
+        HIP_TRY(hipMemcpy2D(phase, row, W->phase.p, pad, row, W->n, hipMemcpyDeviceToHost));
+    // a row holds two spins, in its halves
+    const uint32_t pairs = (W->n + 1) / 2;
+    std::vector<uint32_t> v;
+    for (uint32_t p0 = 0, m; comp && p0 < pairs; p0 += m) {
+        m = std::min<uint32_t>(pairs - p0, (uint32_t)std::max<uint64_t>(kStagingBytes / pad, 1));
+        v.resize((size_t)m * W->n_wpad);
+        HIP_TRY(hipMemcpy(v.data(), W->comp + (size_t)p0 * W->n_wpad, v.size() * 4,
+                          hipMemcpyDeviceToHost));
+        for (uint32_t s = 2 * p0; s < std::min(W->n, 2 * (p0 + m)); ++s)
+            for (uint32_t w = 0; w < W->n_wave; ++w) {
+                const uint32_t word = v[(size_t)(s / 2 - p0) * W->n_wpad + w];
+                const uint32_t bits = (s & 1u) ? word & 0xffff0000u : word << 16;
+                memcpy(&comp[(size_t)s * W->n_wave + w], &bits, 4);
+            }
+    }
     return DSIM_OK;
 }
 
@@ -219,12 +245,13 @@ extern "C" int dsim_waveforms_get_phase(dsim_waveforms *W, float *phase, float *
     // blocks of whole spin pairs, without the padded waveforms, through a
     // staging buffer: a copy of rows at a stride takes the runtime about 5 us
     // a row
-    const uint64_t row = (uint64_t)W->n_wave * 4;
+    const uint64_t row = (uint64_t)W->n_wave * 4, both = row * ((phase ? 1 : 0) + (comp ? 1 : 0));
     const uint32_t rows = (uint32_t)std::min<uint64_t>((W->n + 1u) & ~1u,
-                                                       std::max<uint64_t>(kStagingBytes / row & ~1ull, 2));
+                                                       std::max<uint64_t>(kStagingBytes / both & ~1ull, 2));
     PoolBuf<float> stage;
-    if (int rc = stage.alloc((size_t)rows * W->n_wave * 2)) return rc;
-    float *c_stage = stage.p + (size_t)rows * W->n_wave;
+    if (int rc = stage.alloc(rows * both / 4))
+        return rc == DSIM_ERR_NOMEM ? get_phase_strided(W, phase, comp) : rc;
+    float *c_stage = stage.p + (phase ? (size_t)rows * W->n_wave : 0);
     hipError_t e = hipSuccess;
     for (uint32_t s0 = 0; s0 < W->n && e == hipSuccess; s0 += rows) {
         const uint32_t m = std::min(rows, W->n - s0);

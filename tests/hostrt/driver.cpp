@@ -357,6 +357,44 @@ static void state_on_a_full_device() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// Phases read back through staging of at most 64 MB, whichever of the two
+// arrays is asked for, and on a full device.
+static void phases_read_back() {
+    dsim_substrate *s = make_sub();
+    for (uint32_t n : {1u, 8191u, 20001u}) {
+        dsim_sim *h = make_sim(s, n);
+        EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK && dsim_moment_reset(h) == DSIM_OK);
+        const uint32_t nw = 1003;
+        std::vector<float> g((size_t)32 * nw * 3, 1.0f);
+        dsim_waveforms *W = nullptr;
+        EXPECT(dsim_waveforms_create(h, nw, 32, g.data(), 1.0f, 32, &W) == DSIM_OK);
+        EXPECT(dsim_waveforms_run(W, 32, nullptr) == DSIM_OK);
+        dsim_host::pool_trim_to(0, 0);
+        const size_t m = (size_t)n * nw, was = stub::capacity[0], used = stub::used[0];
+        std::vector<float> p0(m), c0(m), p(m), c(m);
+        stub::peak[0] = used;
+        EXPECT(dsim_waveforms_get_phase(W, p0.data(), c0.data()) == DSIM_OK);
+        EXPECT(stub::peak[0] - used <= 64 << 20);
+        EXPECT(n < 8000 || stub::peak[0] - used > 60 << 20);
+        for (bool full : {false, true})
+            for (int which : {1, 2, 3}) {
+                dsim_host::pool_trim_to(0, 0);
+                stub::capacity[0] = full ? stub::used[0] : was;
+                stub::peak[0] = stub::used[0];
+                memset(p.data(), 0xA5, 4 * m);
+                memset(c.data(), 0xA5, 4 * m);
+                EXPECT(dsim_waveforms_get_phase(W, which & 1 ? p.data() : nullptr,
+                                                which & 2 ? c.data() : nullptr) == DSIM_OK);
+                EXPECT(stub::peak[0] - used <= (which == 3 || m > 16 << 20 ? 64u << 20 : 4 * (m + nw)));
+                EXPECT(!(which & 1) || !memcmp(p.data(), p0.data(), 4 * m));
+                EXPECT(!(which & 2) || !memcmp(c.data(), c0.data(), 4 * m));
+                stub::capacity[0] = was;
+            }
+        EXPECT(dsim_waveforms_destroy(W) == DSIM_OK && dsim_sim_destroy(h) == DSIM_OK);
+    }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -368,6 +406,7 @@ int main(int argc, char **argv) {
         {"label_without_lists", label_without_lists},
         {"server_budget", server_budget},
         {"state_on_a_full_device", state_on_a_full_device},
+        {"phases_read_back", phases_read_back},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

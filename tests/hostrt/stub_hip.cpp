@@ -72,6 +72,11 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) {
     return hipMemcpy(d, s, n, k);
 }
+hipError_t hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h,
+                       hipMemcpyKind) {
+    for (size_t r = 0; r < h; ++r) memcpy((char *)d + r * dp, (const char *)s + r * sp, w);
+    return hipSuccess;
+}
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) {
     if (!d) return err(hipErrorInvalidValue);
     memset(d, v, n);
@@ -174,7 +179,7 @@ hipError_t launch_phase_gemm(const float *, uint32_t, uint32_t n_pad, uint32_t, 
                              const uint16_t *, const uint16_t *, uint32_t, uint32_t, uint32_t n_wave,
                              float *phase, uint32_t *comp, bool, hipStream_t) {
     for (size_t k = 0; k < (size_t)n_pad * n_wave; ++k) phase[k] = (float)k;
-    for (size_t k = 0; k < (size_t)n_pad / 2 * n_wave; ++k) comp[k] = (uint32_t)k;
+    for (size_t k = 0; k < (size_t)n_pad / 2 * n_wave; ++k) comp[k] = (uint32_t)k * 2654435761u;
     return hipGetLastError();
 }
 hipError_t launch_phase_operands(const float *, uint32_t, uint32_t, uint32_t, float, uint16_t *,
@@ -187,7 +192,9 @@ hipError_t launch_phase_rows(uint32_t s0, uint32_t m, const float *phase, const 
     for (uint32_t r = 0; r < m; ++r)
         for (uint32_t w = 0; w < n_wave; ++w) {
             if (p_out) p_out[(size_t)r * n_wave + w] = phase[(size_t)(s0 + r) * n_wpad + w];
-            if (c_out) c_out[(size_t)r * n_wave + w] = (float)comp[(size_t)((s0 + r) / 2) * n_wpad + w];
+            const uint32_t word = comp[(size_t)((s0 + r) / 2) * n_wpad + w];
+            const uint32_t bits = ((s0 + r) & 1u) ? word & 0xffff0000u : word << 16;
+            if (c_out) memcpy(&c_out[(size_t)r * n_wave + w], &bits, 4);
         }
     return hipGetLastError();
 }

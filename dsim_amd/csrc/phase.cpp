@@ -108,16 +108,17 @@ extern "C" int dsim_waveforms_create(dsim_sim *sim, uint32_t n_wave, uint32_t n_
     const size_t nw = (size_t)std::max<uint32_t>(W->n_pad, 1) * nwp;
     const size_t n_sum = (size_t)nwp * 3, n_part = (size_t)kPhaseBlocks * nwp * 15;
     const size_t n_out = (size_t)nwp * 15;
-    PoolBuf<float> g;  // the gradients as given
+    const size_t n_given = (size_t)n_steps * n_wave * 3;
+    PoolBuf<float> g;  // the gradients as given, where the pairs have no room for them
     int rc;
-    if ((rc = g.alloc((size_t)n_steps * n_wave * 3)) ||
-        (rc = W->work.alloc(n_sum + n_part + n_out + (2 * ng * 2 + 7) / 8)) ||
+    if ((rc = W->work.alloc(n_sum + n_part + n_out + (2 * ng * 2 + 7) / 8)) ||
         (rc = W->traj.alloc((size_t)3 * chunk * W->n_pad)) ||
-        (rc = W->phase.alloc(nw + (size_t)std::max<uint32_t>(W->n_pad / 2, 1) * nwp))) {
-        g.release();
+        (rc = W->phase.alloc(nw + (size_t)std::max<uint32_t>(W->n_pad / 2, 1) * nwp)) ||
+        (W->phase.n < n_given && (rc = g.alloc(n_given)))) {
         delete W;
         return rc;
     }
+    float *given = g.p ? g.p : W->phase.p;  // nothing is in the pairs yet
     W->gsum = W->work.p;
     W->partial = W->gsum + n_sum;
     W->out = W->partial + n_part;
@@ -127,9 +128,9 @@ extern "C" int dsim_waveforms_create(dsim_sim *sim, uint32_t n_wave, uint32_t n_
     // The trajectory needs no clearing: padded spins reach only padded rows of
     // the pairs, which nothing reads.
     hipStream_t st = dsim_host::sim_stream(sim);
-    hipError_t e = hipMemcpyAsync(g.p, grads, g.n * 4, hipMemcpyHostToDevice, st);
+    hipError_t e = hipMemcpyAsync(given, grads, n_given * 4, hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
-        e = dsim::launch_phase_operands(g.p, n_steps, n_wave, nwp, pc, W->g_hi, W->g_lo, W->gsum, st);
+        e = dsim::launch_phase_operands(given, n_steps, n_wave, nwp, pc, W->g_hi, W->g_lo, W->gsum, st);
     const hipError_t es = hipStreamSynchronize(st);
     if (e == hipSuccess) e = es;
     g.release();

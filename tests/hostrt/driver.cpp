@@ -395,6 +395,30 @@ static void phases_read_back() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// A waveform handle's device memory is what its header says; preparing its
+// operands takes no more beside phases that are larger than the gradients.
+static void waveforms_memory() {
+    dsim_substrate *s = make_sub();
+    for (uint32_t n : {20001u, 127u}) {
+        dsim_sim *h = make_sim(s, n);
+        EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK && dsim_moment_reset(h) == DSIM_OK);
+        const uint32_t nw = 128, steps = 32;
+        std::vector<float> g((size_t)steps * nw * 3, 1.0f);
+        dsim_waveforms *W = nullptr;
+        const size_t pad = (n + 127) / 128 * 128, used = stub::used[0];
+        stub::peak[0] = used;
+        EXPECT(dsim_waveforms_create(h, nw, steps, g.data(), 1.0f, 32, &W) == DSIM_OK);
+        const size_t held = 6 * pad * nw + 4 * (size_t)nw * 3 * steps + 12 * pad * 32 +
+                            8 * ((size_t)nw * 18 + 512 * (size_t)nw * 15);  // sums of the readout
+        EXPECT(stub::used[0] - used == held);
+        EXPECT(stub::peak[0] - used == held);
+        std::vector<double> sig(5 * nw);
+        EXPECT(dsim_waveforms_signal(W, sig.data()) == DSIM_OK);
+        EXPECT(dsim_waveforms_destroy(W) == DSIM_OK && dsim_sim_destroy(h) == DSIM_OK);
+    }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -407,6 +431,7 @@ int main(int argc, char **argv) {
         {"server_budget", server_budget},
         {"state_on_a_full_device", state_on_a_full_device},
         {"phases_read_back", phases_read_back},
+        {"waveforms_memory", waveforms_memory},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -147,10 +147,17 @@ extern "C" int dsim_waveforms_set_buffer(dsim_waveforms *W, uint32_t buffer_step
     if (buffer_steps == 0 || buffer_steps % W->chunk)
         return fail(DSIM_ERR_ARG, "buffer_steps must be a positive multiple of chunk_steps (%u)",
                     W->chunk);
-    if (buffer_steps == W->buffer) return DSIM_OK;
+    if (buffer_steps == W->buffer && (W->traj.p || !W->n_pad)) return DSIM_OK;
     HIP_TRY(hipStreamSynchronize(dsim_host::sim_stream(W->sim)));
     W->traj.release();
-    if (int rc = W->traj.alloc((size_t)3 * buffer_steps * W->n_pad)) return rc;
+    if (int rc = W->traj.alloc((size_t)3 * buffer_steps * W->n_pad)) {
+        // the buffer as it was, or the smallest; a run without any is refused
+        if (W->traj.alloc((size_t)3 * W->buffer * W->n_pad)) {
+            W->buffer = W->chunk;
+            (void)W->traj.alloc((size_t)3 * W->buffer * W->n_pad);
+        }
+        return rc;
+    }
     W->buffer = buffer_steps;
     return DSIM_OK;
 }
@@ -167,6 +174,7 @@ extern "C" int dsim_waveforms_run(dsim_waveforms *W, uint32_t steps, float *traj
     if (steps % dsim::kPhaseSliceK || W->done + steps > W->n_steps)
         return fail(DSIM_ERR_ARG, "steps must be a multiple of %u within the waveforms' %u",
                     dsim::kPhaseSliceK, W->n_steps);
+    if (W->n_pad && !W->traj.p) return fail(DSIM_ERR_NOMEM, "no trajectory buffer");
     hipStream_t st = dsim_host::sim_stream(W->sim);
     hipEvent_t ev[3];
     for (auto &e : ev) HIP_TRY(hipEventCreate(&e));

@@ -367,6 +367,26 @@ extern "C" int dsim_get_step(dsim_sim *s, uint64_t *step) {
     return DSIM_OK;
 }
 
+// Room for m partial sums.  Without memory for them the handle keeps, or gets
+// back, those of a signal, which other calls rely on.
+static int need_partial(dsim_sim *s, size_t m) {
+    constexpr size_t base = (size_t)dsim::kSignalBlocks * 15;
+    m = std::max(m, base);
+    if (s->partial.n >= m) return DSIM_OK;
+    HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
+    PoolBuf<double> b;
+    if (b.alloc(m)) {
+        s->partial.release();
+        if (int rc = b.alloc(m)) {
+            (void)s->partial.alloc(base);
+            return rc;
+        }
+    }
+    s->partial.release();
+    s->partial = b;
+    return DSIM_OK;
+}
+
 static dsim::StepParams step_params(dsim_sim *s) {
     dsim::StepParams P{};
     dsim_substrate *b = s->sub;
@@ -566,6 +586,7 @@ extern "C" int dsim_integrate_injected(dsim_sim *s, const float g[3], float pc, 
 extern "C" int dsim_signal(dsim_sim *s, double out[5]) {
     if (int rc = check_sim(s)) return rc;
     if (!out) return fail(DSIM_ERR_ARG, "NULL out");
+    if (int rc = need_partial(s, 0)) return rc;
     hipError_t e = dsim::launch_signal(s->n, s->ff(F_MAG), s->ff(F_PHASE), s->f(F_LABEL),
                                        s->partial.p, dsim::kSignalBlocks, s->out.p, s->stream);
     if (e != hipSuccess) return fail(DSIM_ERR_HIP, "signal launch: %s", hipGetErrorString(e));
@@ -618,13 +639,7 @@ extern "C" int dsim_signal_moment(dsim_sim *s, uint32_t ndir, const float *g, fl
         s->grads.release();
         if (int rc = s->grads.alloc((size_t)ndir * 3)) return rc;
     }
-    if (s->partial.n < (size_t)ndir * nb * 15) {
-        HIP_TRY(hipStreamSynchronize(s->stream));  // the pool does not wait
-        s->partial.release();
-        if (int rc = s->partial.alloc(
-                (size_t)std::max<size_t>(ndir * (size_t)nb, dsim::kSignalBlocks) * 15))
-            return rc;
-    }
+    if (int rc = need_partial(s, (size_t)ndir * nb * 15)) return rc;
     PoolBuf<double> o;
     if (int rc = o.alloc((size_t)ndir * 15)) return rc;
     hipError_t e = hipMemcpyAsync(s->grads.p, g, (size_t)ndir * 12, hipMemcpyHostToDevice, s->stream);
@@ -696,6 +711,7 @@ extern "C" int dsim_init_spins_box(dsim_sim *s, const float lo[3], const float h
 extern "C" int dsim_label_spins(dsim_sim *s, float xmax, float ymax, float zmax,
                                 uint32_t max_tries, uint32_t *n_ambiguous) {
     if (int rc = check_sim(s)) return rc;
+    if (int rc = need_partial(s, 0)) return rc;
     dsim::LabelParams L{};
     L.tri_ref = s->sub->tri_ref.p;
     L.tri_mt = s->sub->tri_mt.p;

@@ -419,6 +419,44 @@ static void waveforms_memory() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// A buffer that cannot grow leaves the handle with one that works.
+static void failed_growth() {
+    dsim_substrate *s = make_sub();
+    dsim_sim *h = make_sim(s, 1000);
+    EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK && dsim_moment_reset(h) == DSIM_OK);
+    const size_t was = stub::capacity[0];
+    std::vector<float> g(3 * 4000, 1.0f);
+    std::vector<double> sig(5 * 4000);
+    double one[5] = {0};
+    for (uint32_t lines : {4000u, 100u, 4000u}) {
+        stub::capacity[0] = stub::used[0] + 100'000;  // room for the lines, not for their sums
+        EXPECT(dsim_signal_moment(h, lines, g.data(), 1.0f, sig.data()) == DSIM_ERR_NOMEM);
+        EXPECT(dsim_signal(h, one) == DSIM_OK && one[0] > 0);
+        stub::capacity[0] = was;
+        EXPECT(dsim_signal_moment(h, 90, g.data(), 1.0f, sig.data()) == DSIM_OK);
+    }
+    stub::capacity[0] = stub::used[0];
+    EXPECT(dsim_label_spins(h, 1, 1, 1, 3, nullptr) == DSIM_OK);
+    stub::capacity[0] = was;
+    EXPECT(dsim_moment_reset(h) == DSIM_OK);
+    std::vector<float> w((size_t)320 * 128 * 3, 1.0f);
+    dsim_waveforms *W = nullptr;
+    EXPECT(dsim_waveforms_create(h, 128, 320, w.data(), 1.0f, 32, &W) == DSIM_OK);
+    EXPECT(dsim_waveforms_set_buffer(W, 64) == DSIM_OK);
+    dsim_host::pool_trim_to(0, 0);
+    stub::capacity[0] = stub::used[0];
+    EXPECT(dsim_waveforms_set_buffer(W, 256) == DSIM_ERR_NOMEM);
+    EXPECT(dsim_waveforms_run(W, 160, nullptr) == DSIM_OK);
+    stub::capacity[0] = 0;  // not even the buffer that it had
+    EXPECT(dsim_waveforms_set_buffer(W, 256) == DSIM_ERR_NOMEM);
+    EXPECT(dsim_waveforms_run(W, 32, nullptr) == DSIM_ERR_NOMEM);
+    stub::capacity[0] = was;
+    EXPECT(dsim_waveforms_set_buffer(W, 32) == DSIM_OK);
+    EXPECT(dsim_waveforms_run(W, 160, nullptr) == DSIM_OK);
+    EXPECT(dsim_waveforms_destroy(W) == DSIM_OK && dsim_sim_destroy(h) == DSIM_OK);
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -432,6 +470,7 @@ int main(int argc, char **argv) {
         {"state_on_a_full_device", state_on_a_full_device},
         {"phases_read_back", phases_read_back},
         {"waveforms_memory", waveforms_memory},
+        {"failed_growth", failed_growth},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -764,6 +764,11 @@ extern "C" int dsim_thread_sync(void) {
     return DSIM_OK;
 }
 
+extern "C" int dsim_trim_memory(void) {
+    (void)pool_trim();
+    return DSIM_OK;
+}
+
 extern "C" int dsim_copy_from_device(void *host, const void *device, size_t bytes) {
     if (bytes == 0) return DSIM_OK;
     if (!host || !device) return fail(DSIM_ERR_ARG, "NULL pointer");

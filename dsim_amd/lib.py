@@ -98,6 +98,7 @@ def lib():
             "dsim_alloc_array": [C.POINTER(_vp), C.c_size_t],
             "dsim_free_array": [_vp],
             "dsim_thread_sync": [],
+            "dsim_trim_memory": [],
             "dsim_copy_from_device": [_vp, _vp, C.c_size_t],
             "dsim_copy_to_device": [_vp, _vp, C.c_size_t, C.c_size_t],
             "dsim_substrate_create": [C.POINTER(Mesh), C.POINTER(GridParams), C.POINTER(_vp)],
@@ -150,6 +151,12 @@ def device_count():
     n = C.c_int(0)
     check(lib().dsim_device_count(C.byref(n)))
     return n.value
+
+
+def trim_memory():
+    """Gives back the device memory of closed handles that waits for the next
+    ones (dsim_trim_memory), for other allocators of the process."""
+    check(lib().dsim_trim_memory())
 
 
 def _p(a, t):

@@ -136,6 +136,13 @@ int dsim_alloc_array(void **dev_ptr, size_t bytes);
 int dsim_free_array(void *dev_ptr);
 /* threadSync (spinSystem.cu:57-60): waits for all work on the device. */
 int dsim_thread_sync(void);
+/* No reference counterpart: gives back the device memory that no handle uses.
+ * While any simulation or server is alive, blocks of closed simulation and
+ * waveform handles (at most 1/16 of each device's memory) wait for the next
+ * handle; they go by themselves with the last one, and when an allocation of
+ * this library would fail, but another allocator of the process cannot ask for
+ * them.  May be called at any time, from any thread. */
+int dsim_trim_memory(void);
 /* copyArrayFromDevice (spinSystem.cu:68-75) without the GL buffer mapping. */
 int dsim_copy_from_device(void *host, const void *device, size_t bytes);
 /* copyArrayToDevice (spinSystem.cu:83-86): device + offset <- host. */

@@ -457,6 +457,29 @@ static void failed_growth() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// The caller can have the waiting blocks given back, on every device, while
+// handles are alive.
+static void trim() {
+    dsim_substrate *s = make_sub();
+    dsim_sim *keep = make_sim(s, 10);
+    size_t base[2];
+    for (int d : {0, 1}) {
+        hipSetDevice(d);
+        base[d] = stub::used[d];
+        PoolBuf<float> a, b;
+        EXPECT(a.alloc(100'000) == DSIM_OK && b.alloc(1000) == DSIM_OK);
+        a.release();
+        b.release();
+        EXPECT(stub::used[d] >= base[d] + 404'000);
+    }
+    hipSetDevice(0);
+    EXPECT(dsim_trim_memory() == DSIM_OK);
+    EXPECT(stub::used[0] == base[0] && stub::used[1] == base[1]);
+    EXPECT(dsim_trim_memory() == DSIM_OK);
+    EXPECT(dsim_sync(keep) == DSIM_OK && dsim_sim_destroy(keep) == DSIM_OK);
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -471,6 +494,7 @@ int main(int argc, char **argv) {
         {"phases_read_back", phases_read_back},
         {"waveforms_memory", waveforms_memory},
         {"failed_growth", failed_growth},
+        {"trim", trim},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

@@ -114,6 +114,18 @@ void finish(dsim_server *S, Req *r, int status, int err, const std::string &msg)
     S->cv_done.notify_all();
 }
 
+// Makes a device current for a scope.
+struct OnDevice {
+    int was = 0;
+    bool moved = false;
+    explicit OnDevice(int device) {
+        if (hipGetDevice(&was) == hipSuccess && was != device) moved = hipSetDevice(device) == hipSuccess;
+    }
+    ~OnDevice() {
+        if (moved) (void)hipSetDevice(was);
+    }
+};
+
 // What is left of the budget beside the admitted requests.
 uint64_t budget_rest(dsim_server *S) {
     std::lock_guard<std::mutex> l(S->mu);
@@ -223,6 +235,7 @@ int ensure_batch(dsim_server *S, int kind) {
 // for the step; (4) advance the bookkeeping; (5) release finished requests.
 int run_round(dsim_server *S, uint32_t *n_active, uint32_t *n_queued) {
     std::lock_guard<std::mutex> rl(S->round_mu);
+    const OnDevice on(S->device);  // the background loop's thread starts on device 0
     // (1) one batched launch per kind (boundary, record layout of the grid)
     // carries every prepared request of that kind.
     // A round lasts about total_blocks / kResidentBlocks times as long as one

@@ -480,6 +480,53 @@ static void trim() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// A server's handles lie on the device that was current at its creation, also
+// when another thread runs its rounds.
+static void server_device() {
+    hipSetDevice(1);
+    dsim_substrate *s = make_sub();
+    dsim_server *S = nullptr;
+    EXPECT(dsim_server_create(100 << 20, 0, 0, &S) == DSIM_OK);
+    uint32_t id = 0;
+    EXPECT(dsim_server_add_substrate(S, s, &id) == DSIM_OK);
+    const float lobe[1] = {1.0f}, g[3] = {1, 0, 0};
+    const uint32_t steps[1] = {300};
+    for (bool background : {true, false}) {
+        hipSetDevice(background ? 1 : 0);
+        dsim_trim_memory();
+        stub::peak[0] = stub::used[0];
+        stub::peak[1] = stub::used[1];
+        const size_t base = stub::used[1];
+        dsim_request q{};
+        q.substrate = id;
+        q.n_spins = 5000;
+        q.dt = 0.005f;
+        for (int c = 0; c < 4; ++c) { q.std_dev[c] = 0.01f; q.t2[c] = INFINITY; }
+        q.start_box = 1.0f;
+        q.n_lobes = 1;
+        q.lobe_weight = lobe;
+        q.lobe_steps = steps;
+        q.n_lines = 1;
+        q.grads = g;
+        uint64_t t = 0;
+        EXPECT(dsim_server_submit(S, &q, &t) == DSIM_OK);
+        if (background) {
+            EXPECT(dsim_server_start(S) == DSIM_OK);
+            EXPECT(dsim_server_wait(S, t, 30) == DSIM_OK);
+            EXPECT(dsim_server_stop(S) == DSIM_OK);
+        } else {
+            uint32_t a = 1, n = 1;
+            while (a || n) EXPECT(dsim_server_round(S, &a, &n) == DSIM_OK);
+            int d = -1;
+            EXPECT(hipGetDevice(&d) == hipSuccess && d == 0);
+        }
+        EXPECT(stub::peak[0] == 0 && stub::peak[1] >= base + 5000 * 21 * 4);
+    }
+    EXPECT(dsim_server_destroy(S) == DSIM_OK && dsim_substrate_destroy(s) == DSIM_OK);
+    hipSetDevice(0);
+    EXPECT(stub::blocks.empty());
+}
+
 int main(int argc, char **argv) {
     const std::pair<const char *, void (*)()> cases[] = {
         {"pool_device", pool_device},
@@ -495,6 +542,7 @@ int main(int argc, char **argv) {
         {"waveforms_memory", waveforms_memory},
         {"failed_growth", failed_growth},
         {"trim", trim},
+        {"server_device", server_device},
     };
     for (auto &c : cases) {
         if (argc > 1 && strcmp(argv[1], c.first)) continue;

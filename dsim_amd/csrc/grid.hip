@@ -429,8 +429,11 @@ struct FineGeom {
     float cell[3];      // fine cell edge
     float w[3];         // 0 on collapsed axes
     float half_diag, q;
+    float margin;       // kFineMargin for the substrate's coordinates
 };
-constexpr float kFineMargin = 1e-5f;  // covers FP32 rounding of positions, distances and lookups
+// Covers FP32 rounding of positions, distances and lookups at coordinates up to
+// 2 (times the substrate's margin_scale beyond).
+constexpr float kFineMargin = 1e-5f;
 constexpr float kFineRange = 32.0f;   // q = grid cell / kFineRange: bytes reach 8 grid cells
 
 struct D3 {
@@ -455,7 +458,7 @@ __device__ __forceinline__ double seg_dist2(D3 r, D3 e) {
 // from the edges the walk tests (the normal of a long thin triangle is off by
 // more than the margin in FP32); a degenerate triangle is its edges.
 // A triangle whose plane is farther than sqrt(enough) gives `enough`.
-__device__ double tri_dist2(const float4 *__restrict__ m, D3 c, D3 w, double enough) {
+__device__ double tri_dist2(const float4 *__restrict__ m, D3 c, D3 w, double enough, float margin) {
     const float4 v4 = m[1], a4 = m[2], b4 = m[3];
     const D3 e1 = D3{a4.x * w.x, a4.y * w.y, a4.z * w.z};
     const D3 e2 = D3{b4.x * w.x, b4.y * w.y, b4.z * w.z};
@@ -467,7 +470,7 @@ __device__ double tri_dist2(const float4 *__restrict__ m, D3 c, D3 w, double eno
     const D3 e3 = e2 - e1, r1 = r - e1;
     double d2 = fmin(fmin(seg_dist2(r, e1), seg_dist2(r, e2)), seg_dist2(r1, e3));
     if (nn > 0.0) {
-        const double k = -(double)kFineMargin * sqrt(nn);
+        const double k = -(double)margin * sqrt(nn);
         if (dotv(n, cross3(e1, r)) >= k * sqrt(dotv(e1, e1)) &&
             dotv(n, cross3(r, e2)) >= k * sqrt(dotv(e2, e2)) &&
             dotv(n, cross3(e3, r1)) >= k * sqrt(dotv(e3, e3))) {
@@ -514,11 +517,11 @@ __global__ __launch_bounds__(kBlock) void k_fine_clearance(Geom g, FineGeom f,
                 const uint64_t row = ((uint64_t)z * g.dims[1] + y) * g.dims[0];
                 const uint32_t k1 = start[row + a1[0] + 1];
                 for (uint32_t k = start[row + a0[0]]; k < k1; ++k)
-                    d2 = fmin(d2, tri_dist2(mt + (size_t)tri[k] * 4, p, w, d2));
+                    d2 = fmin(d2, tri_dist2(mt + (size_t)tri[k] * 4, p, w, d2, f.margin));
             }
         d = fmax(d, sqrt(d2) - f.half_diag);
     }
-    out[i] = (uint8_t)fmin(fmax(floor((d - kFineMargin) / f.q), 0.0), 255.0);
+    out[i] = (uint8_t)fmin(fmax(floor((d - f.margin) / f.q), 0.0), 255.0);
 }
 
 // ---- search lists of the walk ---------------------------------------------- //
@@ -577,11 +580,12 @@ __global__ __launch_bounds__(kBlock) void k_pair_triangles(uint32_t n_tri, const
 // Records of triangle t and its partner: the plane, and the lateral record
 // (d / W, m / W) with d the unit vector in the plane across the triangle's
 // longest edge and [m - W, m + W] the extent of both along d, widened by
-// kFineMargin; (0, 0, 0, 0), which bounds nothing, for a degenerate triangle.
+// kFineMargin (margins times); (0, 0, 0, 0), which bounds nothing, for a
+// degenerate triangle.
 // eps: the largest distance of a vertex from its own record's plane.
 __global__ __launch_bounds__(kBlock) void k_walk_records(uint32_t n_tri, const float4 *mt,
-                                                         const uint32_t *partner, float4 *rec,
-                                                         uint32_t *eps) {
+                                                         const uint32_t *partner, float margins,
+                                                         float4 *rec, uint32_t *eps) {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= n_tri) return;
     const float4 pl = mt[(size_t)t * 4];
@@ -610,13 +614,14 @@ __global__ __launch_bounds__(kBlock) void k_walk_records(uint32_t n_tri, const f
         u = partner[t];
         if (u == kNoTri) break;
     }
-    const double W = 0.5 * (hi - lo) + kFineMargin, m = 0.5 * (hi + lo);
-    const bool ok = dotv(d, d) > 0.5 && W < 1e30;  // false for a degenerate or NaN triangle
+    const double W = 0.5 * (hi - lo) + (double)kFineMargin * margins, m = 0.5 * (hi + lo);
+    // false for a degenerate or NaN triangle, or one off its own plane
+    const bool ok = dotv(d, d) > 0.5 && W < 1e30 && dev < margins;
     rec[(size_t)t * 2] = pl;
     rec[(size_t)t * 2 + 1] = ok ? make_float4((float)(d.x / W), (float)(d.y / W), (float)(d.z / W),
                                               (float)(m / W))
                                 : make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ok && dev < 1.0) atomicMax(eps, __float_as_uint((float)dev));
+    if (ok) atomicMax(eps, __float_as_uint((float)dev));
 }
 
 // Reference mode: per list entry the triangle's normal and its first vertex
@@ -873,6 +878,7 @@ static int build_fine_clearance(dsim_substrate *S, hipStream_t st) {
         S->fine_w[k] = f.w[k];
     }
     f.half_diag = std::sqrt(h2) * 1.00001f;
+    f.margin = kFineMargin * S->margins;
     f.q = S->fine_q = smallest / kFineRange;
     if (int rc = S->d_fine.alloc(n))  // no table: every step searches
         return rc == DSIM_ERR_NOMEM ? DSIM_OK : rc;
@@ -919,7 +925,7 @@ static int build_search_lists(dsim_substrate *S, hipStream_t st) {
         hipLaunchKernelGGL(k_pair_triangles, dim3(blocks_for(nT)), dim3(kBlock), 0, st, nT, keys2.p,
                            vals2.p, S->tri_mt.p, partner.p);
         hipLaunchKernelGGL(k_walk_records, dim3(blocks_for(nT)), dim3(kBlock), 0, st, nT, S->tri_mt.p,
-                           partner.p, rec.p, eps.p);
+                           partner.p, S->margins, rec.p, eps.p);
     }
     hipLaunchKernelGGL(k_walk_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, nC,
                        S->d_cell_start.p, S->d_cell_tri.p, partner.p, S->walk_start.p,
@@ -941,7 +947,7 @@ static int build_search_lists(dsim_substrate *S, hipStream_t st) {
     HIP_TRY(hipGetLastError());
     // side distances are off by the record's own error and by FP32 rounding at
     // coordinates up to 2 (three fused operations of half an ulp, 4e-7)
-    S->walk_eps = 2.0f * dev + 1e-6f;
+    S->walk_eps = 2.0f * dev + 1e-6f * S->margins;
     if (!cell_major) std::swap(S->walk_rec, static_cast<DevBuf<float4> &>(rec));
     HIP_TRY(hipStreamSynchronize(st));  // the temporary arrays are freed on return
     return DSIM_OK;
@@ -1124,6 +1130,7 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
     S->on_device = true;
     S->device_built = true;
     S->label_axis = dsim_host::label_axis_of(mesh);
+    S->margins = dsim_host::margin_scale(mesh, S);
 
     int rc = DSIM_OK;
     const hipStream_t st = nullptr;

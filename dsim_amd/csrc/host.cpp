@@ -324,6 +324,21 @@ int dsim_host::check_mesh(const dsim_mesh *mesh) {
     return DSIM_OK;
 }
 
+float dsim_host::margin_scale(const dsim_mesh *mesh, const dsim_substrate *S) {
+    float c = 2.0f;
+    auto see = [&c](float v) {
+        v = std::fabs(v);
+        if (std::isfinite(v) && v > c) c = v;
+    };
+    for (int k = 0; k < 3; ++k) {
+        see(S->lo[k]);
+        see(S->lo[k] + (float)S->dims[k] * S->cell[k]);
+    }
+    for (uint64_t k = 0; k < (uint64_t)mesh->n_vertices * 3 && mesh->n_triangles; ++k)
+        see(mesh->vertices[k]);
+    return 0.5f * c;
+}
+
 // Rings of exact clearance refinement (cells at ring distance <= this):
 // dsim_grid_params.clearance_rings - 2, or the grid kind's default.
 int64_t dsim_host::clearance_rings(const dsim_grid_params *g) {
@@ -663,6 +678,7 @@ extern "C" int dsim_substrate_create(const dsim_mesh *mesh, const dsim_grid_para
                           dsim_host::clearance_rings(grid), S->clearance);
     }
     S->label_axis = dsim_host::label_axis_of(mesh);
+    S->margins = dsim_host::margin_scale(mesh, S);
 
     if (!have_device) {  // host-only substrate: grid and helpers are inspectable, no sims
         *out = S;

@@ -11,6 +11,7 @@
 
 #include "../../include/dsim.h"
 
+struct dsim_substrate;
 namespace dsim_host {
 
 // Records a message for dsim_last_error() and returns code.
@@ -20,6 +21,11 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 int check_mesh(const dsim_mesh *mesh);
 // Axis (0 x, 1 y, 2 z) of the physical mode's labelling rays for a mesh.
 uint32_t label_axis_of(const dsim_mesh *mesh);
+// The margins of the walk's tables are set for coordinates up to 2,
+// the normalised ones; this is the factor for a mesh and grid beyond those, half
+// their largest finite coordinate (1 at least): the rounding that the margins
+// cover grows with it.
+float margin_scale(const dsim_mesh *mesh, const dsim_substrate *S);
 // Exact clearance refinement of exact-membership grids by default: rings 0-1.
 // Their exact distances cost a separating-axis gap per listed triangle of the
 // surrounding cells; measured on crossing substrates, refining rings 0-1 keeps
@@ -192,6 +198,7 @@ struct dsim_substrate {
     dsim_host::DevBuf<uint2> walk_ent;
     dsim_host::DevBuf<float4> walk_rec;
     float walk_eps = 0;  // bound of the error of a side distance (see walk_test, kernels.hip)
+    float margins = 1.0f;  // margin_scale of the mesh and grid
     // Fine clearance of the walk: one byte per fine cell, a lower bound of the distance to any registered triangle
     // in units of fine_q; axes with one grid cell are collapsed (fine_w 0).
     dsim_host::DevBuf<uint8_t> d_fine;

@@ -185,9 +185,9 @@ hipError_t launch_pack_state(uint32_t n, const uint32_t *x, const uint32_t *y, c
                              const uint32_t *id, const uint32_t *flags, uint32_t *out_flags,
                              uint32_t *pos, uint32_t *spins, hipStream_t s);
 hipError_t launch_label(const LabelParams &p, hipStream_t s);
-// Grid-row labelling of the first +x ray, then the tiled pass over the spins
-// it leaves (ambiguous rays, spins outside the grid).  The buffers of the
-// grid fields of p must be set; *n_outside and *n_retry must be zero.
+// Grid-row labelling of the first ray along the labelling axis, then the re-casts
+// of the spins it leaves (ambiguous rays, spins outside the grid).  The row lists
+// and the buffers of p must be set; the groups, *n_ambiguous and *n_retry zero.
 hipError_t launch_label_row(const LabelParams &p, hipStream_t s);
 // Batched physical-mode walk over a device-resident job table (periodic or
 // clamped boundary for every job of the launch).  recs: where the jobs' grid

@@ -180,7 +180,6 @@ __device__ __forceinline__ uint32_t ref_cell(float p, float lo, float cell, uint
     return (uint32_t)mx;
 }
 
-// The cells triangle t is listed in, in any order: fn(cell) for each.
 // Lanes that take a triangle's cells together.
 constexpr uint32_t kPairLanes = 16;
 

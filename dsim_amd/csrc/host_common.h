@@ -129,10 +129,15 @@ namespace dsim_host {
 int build_walk_tables(dsim_substrate *S, hipStream_t st);
 
 // Row lists of the labeller (LabelParams::row_start).  A substrate keeps its own
-// up to kRowKeepBytes; of a larger grid they would be a third of its memory for
-// a call made once a spin set, so every labelling makes them and gives them
-// back (build_row_lists: 0.25 ms for 2.4e6 cells), or goes without where there
-// is no memory for them.
+// up to kRowKeepBytes; above that every labelling makes them and gives them back,
+// or goes without where there is no memory for them.  On crossing bundles the
+// lists are about half of a substrate, for a call made once a spin set, and
+// making them adds about 0.3 ms to it for every 50 MiB of them.  Labelling 1e5
+// spins with lists kept / made by the call: 200 axons (61 MiB of lists) 0.22 /
+// 0.56 ms, 400 (108) 0.41 / 0.93, 800 (210) 0.80 / 1.72, 1600 (417) 2.07 / 4.02.
+// So the line trades memory for a factor of two in a call that walks of 20 ms and
+// more follow; it lies where the lists pass 100 MiB, below which a device full of
+// such substrates holds a thousand of them.
 constexpr uint64_t kRowKeepBytes = 128ull << 20;
 struct RowLists {
     PoolBuf<uint32_t> start, tri;

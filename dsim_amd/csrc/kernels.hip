@@ -431,9 +431,11 @@ __device__ __forceinline__ float clearance_at(const StepParams &P, float x, floa
 // (t, then index) order as a scan of the lane's cells in any order; the pair
 // holding the minimum then writes the hit for the lane.
 //
-// Bound: VALU issue (about 73 % of the slots at four waves a SIMD; the inner
-// turn takes some 230 instructions, a search round 350 and more).  1e6 spins,
-// 2000 axons, 12,000 steps: 380 ms, against 544 ms with a per-cell clearance
+// Bound: the instruction stream and the waits of four waves a SIMD.  1e6 spins,
+// 2000 axons: 878 VALU instructions a step of 64 spins (a turn takes some 230, a
+// search round 350 and more), 0.69 a CU and cycle, where the reference-mode
+// kernel reaches 1.03; and 151 bytes a spin-step from beyond L2 (65 % hits), 4.7
+// TB/s.  12,000 steps: 381 ms, against 544 ms with a per-cell clearance
 // budget (67 % of the steps searched, here 24 %, and 12 % again after a hit)
 // and one list entry a triangle (5.0 plane and 1.9 triangle tests a step, here
 // 1.8 and 0.9).
@@ -1633,7 +1635,14 @@ static void launch_one(const StepParams &p, uint32_t iters, hipStream_t s) {
     // same whatever its spins, and it ends with its slowest one.  Physical mode,
     // 1e4 spins: 55.8 ms at 64 spins a wave, 48.4 at 16, 45.6 at 8, 43.8 at 4; 1e5
     // spins: 29.9 ms at 64, 21.9 at 32 (3126 waves), 24.8 at 16 (6251, more than
-    // reside).  (The counting build keeps 64: its waves are counted.)
+    // reside).  The other modes, ms by this rule / at 64 a wave, for 5000, 32,000
+    // and 130,000 spins among 2000 axons: reference 7.4/16.0, 15.2/24.4,
+    // 28.1/33.4; injected 0.20/0.27, 0.27/0.31, 0.38/0.38; MWC draws 1.11/1.55,
+    // 1.57/1.80, 1.94/2.09; recording 3.1/4.3, 4.1/4.8, 5.5/5.8; crossing bundles
+    // alike.  Where nearly every step searches (16 axons, capped) the full waves'
+    // compaction pays from 65,000 spins on: reference 1.12/1.04, Philox 2.71/2.50,
+    // at 5000 0.71/0.90 and 1.79/2.25.  (The counting build keeps 64: its waves
+    // are counted.)
     uint32_t pw = 64;
     if constexpr (INSTR == kInstrNone)
         while (pw > 4 && (p.n + pw / 2 - 1) / (pw / 2) <= waves) pw /= 2;
@@ -2340,11 +2349,13 @@ hipError_t launch_signal(uint32_t n, const float *mag, const float *phase, const
 // Per-direction readout from gradient moments: phase_j = pc * g_j.(M + W x0).
 // Bound by the FP64 sine and cosine of every (spin, line) pair, and with few
 // pairs by the latency of the block sums; a block takes L lines of its spins,
-// which share the loads, the moment's x0 term and the counts.  10^6 spins, 65
-// lines: 205 us (250 with one line a block; 355 with sine and cosine apart, all
-// of a block's sums halved through LDS and zeros selected for the other
-// compartments); 60,000 spins, 13 lines: 14.6 us with one line, 19.2 with two
-// (26.1); 300,001 spins, 30 lines: 46.7 and 41.7 (65.5).
+// which share the loads, the moment's x0 term and the counts.  A readout of 10^6
+// spins, 65 lines: 181 to 197 us, 234 with one line a block (313 with sine and
+// cosine apart, all of a block's sums halved through LDS and zeros selected for
+// the other compartments).  The line of kReadoutPairs, one / two lines a block:
+// 60,000 spins, 13 lines 15.4 / 21.0 us, 100,000 and 65 42.8 / 47.7, 80,000 and
+// 52 (4.2M pairs) 32.8 / 35.9, 200,000 and 20 26.2 / 25.5, 300,001 and 30 42.8 /
+// 38.3.
 constexpr uint32_t kReadoutLines = 2;
 constexpr uint64_t kReadoutPairs = 4u << 20;
 template <uint32_t L>
@@ -2598,6 +2609,7 @@ __device__ __forceinline__ uint32_t label_cell(const LabelParams &P, float v, in
 // overlapping boxes a spin): 1.09 ms; walking the cells' lists with a search
 // for each triangle in the cell before, and a list of all triangles past the
 // grid's face for every spin, 42.7 ms.
+
 // Spins by row group for k_label_row (76 us for the ranks of 10^6 spins, bound
 // by the counts' atomics; 10 us for the rest): the group of each spin's row and its
 // rank there (the spins of a group in any order; labels do not depend on it),
@@ -3015,7 +3027,6 @@ hipError_t launch_moment_reset(uint32_t n, const float *x, const float *y, const
     return hipGetLastError();
 }
 
-// ------------------------------------------------------------------------ //
 // ------------------------------------------------------------------------ //
 // Spatial reordering of spins (Morton order of their grid cells), so that the
 // lanes of a wavefront walk the same cells and triangle records.

@@ -114,8 +114,9 @@ typedef struct {
     float voxel_hi[3];        /* all six zero means [-1, 1) on every axis (the cubic voxel)    */
     uint32_t fixed_blocks;    /* physical mode with Philox: 0 lets a persistent walk take over
                                * once every resident workgroup has two or more spins (each lane
-                               * takes its next spin as soon as one is done); 1 keeps one
-                               * 64-spin workgroup per block.  Results do not depend on it. */
+                               * takes its next spin as soon as one is done); 1 keeps fixed
+                               * blocks of spins, 64 each or, where they are few, 4 to 32.
+                               * Results do not depend on it. */
 } dsim_params;
 
 typedef struct dsim_substrate dsim_substrate;
@@ -176,9 +177,9 @@ int dsim_substrate_get_grid(const dsim_substrate *s, uint32_t *cell_start, uint3
 int dsim_substrate_get_helpers(const dsim_substrate *s, float *helpers);
 /* AABB grids only (no reference counterpart): per-cell lower bound of the
  * distance from any point of the cell to any triangle registered in the grid
- * [n_cells] (1e30 when there is none).  The physical step skips collision
- * detection while a spin that was inside the grid at its last check has
- * walked a path shorter than this clearance. */
+ * [n_cells] (1e30 when there is none).  The physical walk skips the collision
+ * search of a step shorter than the clearances of its two end points together,
+ * as a finer table made from this one bounds them. */
 int dsim_substrate_get_clearance(const dsim_substrate *s, float *clearance);
 /* No reference counterpart: the axis of the physical mode's labelling rays
  * (0 +x, 1 +y, 2 +z), chosen from the mesh so that the rays run across its

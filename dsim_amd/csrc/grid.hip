@@ -1065,8 +1065,9 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
 }
 
 int dsim_host::build_walk_tables(dsim_substrate *S, hipStream_t st) {
+    const uint64_t most = S->kind == DSIM_GRID_AABB ? ~0ull : kRowKeepBytes;
     if (S->kind != DSIM_GRID_REFERENCE)
-        if (int rc = build_row_lists(S, S->rows, kRowKeepBytes, ~0ull, st)) {
+        if (int rc = build_row_lists(S, S->rows, most, ~0ull, st)) {
             if (rc != DSIM_ERR_NOMEM) return rc;
             S->rows.release();  // labelled without, or with those that a call can make
         }

@@ -988,17 +988,16 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     struct Scratch {
         hipStream_t st;
         dsim_host::PoolBuf<uint8_t> temp;
-        dsim_host::PoolBuf<uint32_t> outside;  // and after it the rows' counts of their entries
-        dsim_host::PoolBuf<unsigned long long> sum;
+        // the sum of the rows to fill (two words), the triangles past the grid after
+        // their count, and the rows' counts of their entries
+        dsim_host::PoolBuf<uint32_t> outside;
         bool waited = false;
         ~Scratch() {
             if (!waited) (void)hipStreamSynchronize(st);
-            temp.release(); outside.release(); sum.release();
+            temp.release(); outside.release();
         }
-    } scratch{st, {}, {}, {}};
+    } scratch{st, {}, {}};
     auto &temp = scratch.temp;
-    auto &outside = scratch.outside;
-    auto &sum = scratch.sum;
     int rc;
     size_t tb = 0;
     HIP_TRY(rocprim::exclusive_scan(nullptr, tb, R.start.p, R.start.p, 0u,
@@ -1006,27 +1005,27 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
     const uint64_t making = tb + ((uint64_t)nT + 1 + n_rows) * 4 + 64 + ((uint64_t)nC + 1) * 4;
     if (!pool_room(making, room)) return DSIM_OK;
     if ((rc = temp.alloc(std::max(tb, (size_t)1))) || (rc = R.start.alloc((size_t)nC + 1)) ||
-        (rc = outside.alloc((size_t)nT + 1 + n_rows)) || (rc = sum.alloc(1)))
+        (rc = scratch.outside.alloc((size_t)nT + 3 + n_rows)))
         return rc;
-    uint32_t *ends = outside.p + nT + 1;
-    HIP_TRY(hipMemsetAsync(outside.p, 0, outside.n * 4, st));
-    HIP_TRY(hipMemsetAsync(sum.p, 0, 8, st));
+    unsigned long long *sum = reinterpret_cast<unsigned long long *>(scratch.outside.p);
+    uint32_t *outside = scratch.outside.p + 2, *ends = outside + nT + 1;
+    HIP_TRY(hipMemsetAsync(scratch.outside.p, 0, scratch.outside.n * 4, st));
     if (nT)
         hipLaunchKernelGGL(k_row_outside, dim3(blocks_for(nT)), dim3(kBlock), 0, st, g, nT,
-                           S->tri_aabb.p, outside.p, sum.p);
+                           S->tri_aabb.p, outside, sum);
     HIP_TRY(hipGetLastError());
-    uint32_t n_out = 0;
-    unsigned long long n_ends = 0;
-    HIP_TRY(hipMemcpyAsync(&n_out, outside.p, 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(&n_ends, sum.p, 8, hipMemcpyDeviceToHost, st));
+    uint32_t seen[3] = {0, 0, 0};
+    HIP_TRY(hipMemcpyAsync(seen, scratch.outside.p, 12, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    const uint32_t n_out = seen[2];
+    const uint64_t n_ends = seen[0] | (uint64_t)seen[1] << 32;
     const RowPlan plan = row_plan(nC, S->d_cell_tri.n, n_out, n_ends);
     if (plan == kRowsNone) {
         R.start.release();
         return DSIM_OK;
     }
     if (plan == kRowsEnds && n_out)
-        hipLaunchKernelGGL(k_row_ends<false>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
+        hipLaunchKernelGGL(k_row_ends<false>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside,
                            S->tri_aabb.p, ends, (const uint32_t *)nullptr, (uint32_t *)nullptr,
                            (float4 *)nullptr);
     hipLaunchKernelGGL(k_row_lists<false>, dim3(blocks_for(nC)), dim3(kBlock), 0, st, g, nC,
@@ -1053,11 +1052,11 @@ int dsim_host::build_row_lists(const dsim_substrate *S, RowLists &R, uint64_t mo
                        S->d_cell_start.p, S->d_cell_tri.p, S->tri_aabb.p, ends, R.start.p,
                        R.tri.p, R.box.p);
     if (plan == kRowsEnds && n_out)
-        hipLaunchKernelGGL(k_row_ends<true>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside.p,
+        hipLaunchKernelGGL(k_row_ends<true>, dim3(n_blocks), dim3(kBlock), 0, st, g, outside,
                            S->tri_aabb.p, ends, R.start.p, R.tri.p, R.box.p);
     if (R.n_shared)
         hipLaunchKernelGGL(k_row_shared, dim3(blocks_for(R.n_shared)), dim3(kBlock), 0, st, g,
-                           outside.p, S->tri_aabb.p, R.tri.p + n, R.box.p + n);
+                           outside, S->tri_aabb.p, R.tri.p + n, R.box.p + n);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     scratch.waited = true;
@@ -1136,13 +1135,12 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
     const hipStream_t st = nullptr;
     DevBuf<float> dV;
     DevBuf<uint32_t> dT, dI, cnt, offs, keys, vals, keys2, vals2, ccount, ring, flag, maxc;
-    DevBuf<unsigned long long> total;
     DevBuf<uint8_t> temp;
     auto cleanup = [&] {
         dV.release(); dT.release(); dI.release(); cnt.release(); offs.release(); keys.release();
         vals.release();
         keys2.release(); vals2.release(); ccount.release(); ring.release(); flag.release();
-        maxc.release(); total.release(); temp.release();
+        maxc.release(); temp.release();
     };
     auto bail = [&](int code) {
         cleanup();
@@ -1164,8 +1162,8 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
         (rc = S->tri_ref.alloc(nt1 * 4)) || (rc = S->tri_mt.alloc(nt1 * 4)) ||
         (rc = S->tri_aabb.alloc(nt1 * 2)) || (rc = cnt.alloc(nt1 + 1)) || (rc = offs.alloc(nt1 + 1)) ||
         (rc = S->d_cell_start.alloc((size_t)S->n_cells + 1)) ||
-        (rc = ccount.alloc((size_t)S->n_cells + 1)) || (rc = maxc.alloc(1)) ||
-        (rc = flag.alloc(1)) || (rc = total.alloc(1)))
+        (rc = ccount.alloc((size_t)S->n_cells + 1)) || (rc = maxc.alloc(4)) ||
+        (rc = flag.alloc(1)))
         return bail(rc);
     if (nV) GRID_TRY(hipMemcpy(dV.p, mesh->vertices, (size_t)nV * 12, hipMemcpyHostToDevice));
     if (nT) {
@@ -1197,29 +1195,27 @@ extern "C" int dsim_substrate_create_device(const dsim_mesh *mesh, const dsim_gr
     // the pairs in 64 bits: their places and numbers are 32-bit
     const auto wide = rocprim::make_transform_iterator(
         cnt.p, [] __device__(uint32_t v) { return (unsigned long long)v; });
+    unsigned long long *total = reinterpret_cast<unsigned long long *>(maxc.p + 2);
     size_t tb_sum = 0;
-    GRID_TRY(rocprim::reduce(nullptr, tb_sum, wide, total.p, 0ull, (size_t)nT,
+    GRID_TRY(rocprim::reduce(nullptr, tb_sum, wide, total, 0ull, (size_t)nT,
                              rocprim::plus<unsigned long long>(), st));
     const size_t tb0 = std::max({tb_scan1, tb_scan2, tb_red, tb_sum, (size_t)1});
     if ((rc = temp.alloc(tb0))) return bail(rc);
-    unsigned long long n_listed = 0;
-    if (nT) {
-        GRID_TRY(rocprim::reduce(temp.p, tb_sum, wide, total.p, 0ull, (size_t)nT,
+    if (nT)
+        GRID_TRY(rocprim::reduce(temp.p, tb_sum, wide, total, 0ull, (size_t)nT,
                                  rocprim::plus<unsigned long long>(), st));
-        GRID_TRY(hipMemcpyAsync(&n_listed, total.p, 8, hipMemcpyDeviceToHost, st));
-        GRID_TRY(hipStreamSynchronize(st));
-    }
-    if (n_listed > 0xFFFFFFFFull)
-        return bail(fail(DSIM_ERR_ARG, "grid too fine: %llu entries in its cells, more than 2^32 - 1",
-                         n_listed));
     {
         size_t b = tb_scan1;
         GRID_TRY(rocprim::exclusive_scan(temp.p, b, cnt.p, offs.p, 0u, nT + 1,
                                          rocprim::plus<uint32_t>(), st));
     }
-    uint32_t n_pairs = 0;
-    GRID_TRY(hipMemcpyAsync(&n_pairs, offs.p + nT, 4, hipMemcpyDeviceToHost, st));
+    unsigned long long n_listed = 0;
+    if (nT) GRID_TRY(hipMemcpyAsync(&n_listed, total, 8, hipMemcpyDeviceToHost, st));
     GRID_TRY(hipStreamSynchronize(st));
+    if (n_listed > 0xFFFFFFFFull)
+        return bail(fail(DSIM_ERR_ARG, "grid too fine: %llu entries in its cells, more than 2^32 - 1",
+                         n_listed));
+    const uint32_t n_pairs = (uint32_t)n_listed;
     const size_t np1 = std::max<uint32_t>(n_pairs, 1);
     if ((rc = keys.alloc(np1)) || (rc = vals.alloc(np1)) || (rc = keys2.alloc(np1)) ||
         (rc = S->d_cell_tri.alloc(np1)))

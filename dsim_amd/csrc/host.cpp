@@ -12,6 +12,7 @@
 #include <string>
 #include <thread>
 #include <mutex>
+#include <unordered_map>
 #include <vector>
 
 #include <hip/hip_runtime_api.h>
@@ -377,6 +378,17 @@ struct PoolBlock {
 std::mutex pool_mu;
 std::vector<PoolBlock> pool;  // oldest first
 uint64_t pool_users = 0;
+std::unordered_map<int, size_t> pool_limits;  // of the devices seen (asking took 2 us a block)
+
+// Bytes of idle blocks that the device may hold (under pool_mu).
+size_t pool_limit(int device) {
+    if (device < 0) return 0;
+    const auto it = pool_limits.find(device);
+    if (it != pool_limits.end()) return it->second;
+    size_t total = 0;
+    if (hipDeviceTotalMem(&total, device) != hipSuccess) return 0;
+    return pool_limits[device] = total / dsim_host::kPoolShare;
+}
 
 // The oldest block of the device (any for -1) out of the pool (under pool_mu).
 PoolBlock pool_oldest(int device) {
@@ -436,15 +448,12 @@ void *dsim_host::pool_take(size_t bytes, size_t *got, int *device, hipError_t *e
 }
 
 void dsim_host::pool_give(void *p, size_t bytes, int device) {
-    size_t total = 0;
-    if (device < 0 || hipDeviceTotalMem(&total, device) != hipSuccess) total = 0;
-    const size_t limit = total / kPoolShare;
     std::vector<PoolBlock> out;
-    if (bytes > limit) {
-        out.push_back({p, bytes, device});
-    } else {
+    {
         std::lock_guard<std::mutex> l(pool_mu);
-        pool.push_back({p, bytes, device});
+        const size_t limit = pool_limit(device);
+        if (bytes > limit) out.push_back({p, bytes, device});
+        else pool.push_back({p, bytes, device});
         size_t held = 0;  // idle on this device
         for (const PoolBlock &b : pool) held += b.device == device ? b.bytes : 0;
         while (held > limit) {

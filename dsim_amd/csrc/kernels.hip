@@ -1066,10 +1066,11 @@ __device__ __forceinline__ void walk_body(const StepParams &P, uint32_t block, u
                         if (STATS) ++shortcuts;
                     } else {
                         // the balls around the ends hold no triangle: search what
-                        // lies between
-                        const float r = __builtin_amdgcn_rcpf(len);
-                        t0 = fmaxf(clear * r, 0.0f);
-                        t1 = 1.0f - fmaxf(clear_p * r, 0.0f);
+                        // lies between; all of it where an end lies outside the
+                        // grid, whose cells need not list a triangle at a hit there
+                        const float r = clear + clear_p < 0.0f ? 0.0f : __builtin_amdgcn_rcpf(len);
+                        t0 = clear * r;
+                        t1 = 1.0f - clear_p * r;
                     }
                     clear = clear_p;  // unless the step ends elsewhere
                 }

@@ -514,9 +514,12 @@ static int run_steps(dsim_sim *s, dsim::StepParams P, uint32_t iters, int rng, b
         instr = dsim::kInstrStats;
     }
     uint32_t done = 0;
-    const uint32_t chunk = s->sorting() ? std::min(s->prm.steps_per_launch, s->prm.sort_interval)
-                                        : s->prm.steps_per_launch;
+    uint32_t chunk = s->sorting() ? std::min(s->prm.steps_per_launch, s->prm.sort_interval)
+                                  : s->prm.steps_per_launch;
     float *const traj0 = P.traj;  // row 0 of the trajectory buffer's tiles
+    // the tiles interleave their rows in chunks of four, so a launch may begin
+    // only where its first row (three a step) begins a chunk
+    if (traj0) chunk = std::max(chunk / dsim::kTrajChunk, 1u) * dsim::kTrajChunk;
     while (done < iters) {
         if (s->sorting() && s->steps_since_sort >= s->prm.sort_interval) {
             if (int rc = spatial_sort(s)) return rc;

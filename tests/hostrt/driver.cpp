@@ -395,6 +395,33 @@ static void phases_read_back() {
     EXPECT(dsim_substrate_destroy(s) == DSIM_OK && stub::blocks.empty());
 }
 
+// Trajectory rows stand in their place however the steps are split into launches.
+static void trajectory_launches() {
+    dsim_substrate *s = make_sub();
+    const uint32_t n = 200, steps = 96;
+    for (uint32_t sort : {0u, 1u, 5u, 10u, 64u})
+        for (uint32_t spl : {0u, 1u, 2u, 3u, 7u, 30u, 1000u}) {
+            dsim_params p = params(sort);
+            p.steps_per_launch = spl;
+            dsim_sim *h = nullptr;
+            dsim_waveforms *W = nullptr;
+            EXPECT(dsim_sim_create(s, &p, n, &h) == DSIM_OK);
+            EXPECT(dsim_init_spins_uniform(h, 1.0f) == DSIM_OK && dsim_moment_reset(h) == DSIM_OK);
+            std::vector<float> g((size_t)2 * steps * 3, 1.0f), tr((size_t)steps * 3 * n, -1.0f);
+            EXPECT(dsim_waveforms_create(h, 1, 2 * steps, g.data(), 1.0f, steps, &W) == DSIM_OK);
+            for (uint32_t first : {0u, steps}) {
+                EXPECT(dsim_waveforms_run(W, steps, tr.data()) == DSIM_OK);
+                size_t bad = 0;
+                for (size_t k = 0; k < tr.size(); ++k) bad += tr[k] != (float)(3 * first + k / n);
+                EXPECT(bad == 0);
+            }
+            EXPECT(dsim_waveforms_destroy(W) == DSIM_OK && dsim_sim_destroy(h) == DSIM_OK);
+        }
+    EXPECT(dsim_substrate_destroy(s) == DSIM_OK);
+    dsim_host::pool_trim_to(0, 0);
+    EXPECT(stub::blocks.empty());
+}
+
 // A waveform handle's device memory is what its header says; preparing its
 // operands takes no more beside phases that are larger than the gradients.
 static void waveforms_memory() {
@@ -539,6 +566,7 @@ int main(int argc, char **argv) {
         {"server_budget", server_budget},
         {"state_on_a_full_device", state_on_a_full_device},
         {"phases_read_back", phases_read_back},
+        {"trajectory_launches", trajectory_launches},
         {"waveforms_memory", waveforms_memory},
         {"failed_growth", failed_growth},
         {"trim", trim},

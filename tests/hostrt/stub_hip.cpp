@@ -219,14 +219,21 @@ hipError_t launch_sort_perm(const StepParams &p, uint32_t *, uint32_t *, uint32_
     return hipGetLastError();
 }
 // A step moves spin s to (s, s + 1, s + 2) and raises stub::flag_bits.
-hipError_t launch_step(const StepParams &p, uint32_t, int, int, int, int, bool, hipStream_t) {
+hipError_t launch_step(const StepParams &p, uint32_t iters, int, int, int, int, bool, hipStream_t) {
     *p.flags |= stub::flag_bits;
     for (uint32_t i = 0; i < p.n; ++i) {
         p.x[i] = (float)p.spin_id[i];
         p.y[i] = p.x[i] + 1.0f;
         p.z[i] = p.x[i] + 2.0f;
     }
-    if (p.traj) p.traj[0] = 0.0f;
+    // rows 3 * step + axis of the launch, in the tiles' chunks; each holds its number
+    for (uint32_t k = 0; p.traj && k < 3 * iters; ++k)
+        for (uint32_t i = 0; i < p.n; ++i) {
+            const uint32_t id = p.spin_id[i];
+            p.traj[(size_t)(id / kTrajTile) * p.traj_stride +
+                   (size_t)(k / kTrajChunk) * (kTrajTile * kTrajChunk) +
+                   (id % kTrajTile) * kTrajChunk + k % kTrajChunk] = (float)(3 * p.step0 + k);
+        }
     return hipGetLastError();
 }
 hipError_t launch_walk_batch(const WalkTable *, uint32_t, bool, int, hipStream_t) {

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
 CASES = ["pool_device", "pool_bound", "handle_device", "row_plan", "error_flags",
          "label_on_a_full_device", "label_without_lists",
          "server_budget", "state_on_a_full_device", "phases_read_back",
-         "waveforms_memory", "failed_growth", "trim", "server_device"]
+         "trajectory_launches", "waveforms_memory", "failed_growth", "trim", "server_device"]
 
 
 @pytest.fixture(scope="module")

@@ -109,7 +109,7 @@ typedef struct {
                                * every this many steps (0 = never), by recent rate of collision
                                * searches, then cell.  Results do not depend on it. */
     uint32_t steps_per_launch; /* steps fused per kernel launch (0 = 1024; with reordering at
-                                  most sort_interval) */
+                                  most sort_interval; waveform runs: a multiple of 4) */
     float voxel_lo[3];        /* periodic voxel [voxel_lo, voxel_hi) per axis, normalised;     */
     float voxel_hi[3];        /* all six zero means [-1, 1) on every axis (the cubic voxel)    */
     uint32_t fixed_blocks;    /* physical mode with Philox: 0 lets a persistent walk take over
